@@ -103,9 +103,11 @@ def draw(rng):
             layers = 2
         if dtype == "f32" or store != "plain":
             layers = 1
+            longest = math.isqrt((1 << 25) // heads)
+            if chunk > longest:
+                chunk = rng.randint(longest // 2, longest)
             batch = max(1, min(batch, (1 << 25) // (heads * chunk * (past + chunk))))
             past = min(past, max(0, (1 << 25) // (heads * chunk * batch) - chunk))
-            chunk = min(chunk, 1000)
         return _unnamed(_chunk("", dtype, store, batch, heads, kv_heads, dim, past, chunk, layers))
     if kind == "project":
         n, k = rng.choice([(4096, 4096), (1024, 4096), (14336, 4096), (4096, 14336), (2816, 1024), (1000, 2080)])
@@ -158,16 +160,28 @@ class _Inputs:
         return t.to(_TORCH[dtype])
 
 
-def _caches(case, x, store, batch, past, extra, layers):
-    """`layers` states whose caches hold `past` tokens and have room for `extra` more."""
-    dt, hkv, d = case["dtype"], case["kv_heads"], case["dim"]
+def _past_rows(case, x):
+    """The rows that a layer's key or value cache holds before the pass (None for none)."""
+    if case["past"]:
+        return x.normal((case["batch"], case["kv_heads"], case["past"], case["dim"]), case["dtype"], outliers=case["store"] != "plain")
+
+
+def _new_rows(case, x, batch, n, outliers=False):
+    """q, k and v of n tokens of each of `batch` sequences."""
+    hq, hkv, d, dt = case["heads"], case["kv_heads"], case["dim"], case["dtype"]
+    return x.normal((batch, hq, n, d), dt), x.normal((batch, hkv, n, d), dt, outliers=outliers), x.normal((batch, hkv, n, d), dt)
+
+
+def _caches(case, x, extra):
+    """A state per layer whose caches hold `past` tokens and have room for `extra` more."""
+    dt, hkv, d, past, batch = case["dtype"], case["kv_heads"], case["dim"], case["past"], case["batch"]
     states = []
-    for _ in range(layers):
-        st = ta.InPlaceKvSdpa(axis=2, causal=True, storage_format=store).state()
+    for _ in range(case["layers"]):
+        st = ta.InPlaceKvSdpa(axis=2, causal=True, storage_format=_STORE[case["store"]]).state()
         for c in (st.k, st.v):
             c.reserve(past + extra, like=((batch, hkv, 1, d), _NP[dt]))
-            if past:
-                rows = x.normal((batch, hkv, past, d), dt, outliers=store is not None)
+            rows = _past_rows(case, x)
+            if rows is not None:
                 torch.cuda.synchronize()
                 c.push(_wrap(rows))
                 ta.synchronize()
@@ -191,15 +205,15 @@ def _rotary(x, positions, dim, dtype):
 
 
 def _prepare_step(case, x):
-    b, hq, hkv, d, dt = case["batch"], case["heads"], case["kv_heads"], case["dim"], case["dtype"]
+    b, hkv, d, dt = case["batch"], case["kv_heads"], case["dim"], case["dtype"]
     past, n = case["past"], case["tokens"]
-    states = _caches(case, x, _STORE[case["store"]], b, past, n, case["layers"])
+    states = _caches(case, x, n)
     calls, outs, keep = [], [], []
     for t in range(n):
         cos, sin = _rotary(x, [past + t], d, dt)
         cs = [_wrap(r.reshape(1, 1, 1, d)) for r in (cos, sin)] if case["rope"] else []
         for st in states:
-            q, k, v = x.normal((b, hq, 1, d), dt), x.normal((b, hkv, 1, d), dt), x.normal((b, hkv, 1, d), dt)
+            q, k, v = _new_rows(case, x, b, 1)
             out = torch.empty_like(q)
             outs.append(out)
             keep += [q, k, v]
@@ -225,22 +239,30 @@ def _lengths(case, rng):
     return [int(n) for n in rng.integers(case["shortest"], case["longest"], size=case["seqs"], endpoint=True)]
 
 
+def _ragged_rows(case, x, lens):
+    """Keys, then values, of each sequence in turn."""
+    for length in lens:
+        for _ in range(2):
+            yield x.normal((1, case["kv_heads"], length, case["dim"]), case["dtype"], outliers=case["store"] != "plain")
+
+
 def _prepare_ragged(case, x):
     n, hq, hkv, d, dt = case["seqs"], case["heads"], case["kv_heads"], case["dim"], case["dtype"]
     lens = _lengths(case, np.random.default_rng(7))   # the lengths are the case's, not the seed's
+    rows_of = _ragged_rows(case, x, lens)
     ks, vs = [], []
     for length in lens:
         for many in (ks, vs):
             c = ta.InPlaceKvCache(2, _STORE[case["store"]])
             c.reserve(length + case["tokens"], like=((1, hkv, 1, d), _NP[dt]))
-            rows = x.normal((1, hkv, length, d), dt, outliers=case["store"] != "plain")
+            rows = next(rows_of)
             torch.cuda.synchronize()
             c.push(_wrap(rows))
             ta.synchronize()
             many.append(c)
     calls, outs = [], []
     for _ in range(case["tokens"]):
-        q, k, v = x.normal((n, hq, 1, d), dt), x.normal((n, hkv, 1, d), dt), x.normal((n, hkv, 1, d), dt)
+        q, k, v = _new_rows(case, x, n, 1)
         out = torch.empty_like(q)
         outs.append(out)
         calls.append((_wrap(q), _wrap(k), _wrap(v), _wrap(out)))
@@ -257,11 +279,11 @@ def _run_ragged(s):
 
 
 def _prepare_chunk(case, x):
-    b, hq, hkv, d, dt, n = case["batch"], case["heads"], case["kv_heads"], case["dim"], case["dtype"], case["chunk"]
-    states = _caches(case, x, _STORE[case["store"]], b, case["past"], n, case["layers"])
+    b, hkv, d, dt, n = case["batch"], case["kv_heads"], case["dim"], case["dtype"], case["chunk"]
+    states = _caches(case, x, n)
     calls, outs = [], []
     for st in states:
-        q, k, v = x.normal((b, hq, n, d), dt), x.normal((b, hkv, n, d), dt), x.normal((b, hkv, n, d), dt)
+        q, k, v = _new_rows(case, x, b, n)
         out = torch.empty_like(q)
         outs.append(out)
         calls.append((st, [_wrap(q), _wrap(k), _wrap(v)], _wrap(out)))
@@ -270,25 +292,35 @@ def _prepare_chunk(case, x):
     return {"past": case["past"], "caches": [c for st in states for c in (st.k, st.v)], "calls": calls, "outs": outs, "rope": False}
 
 
-def _q4_0_blocks(w):
-    """Canonical Q4_0 blocks of a [n, k] f32 tensor (18 bytes per 32 features: f16 scale, 16 bytes of code pairs)."""
+def _q4_0_codes(w):
+    """Scales (f32, one per 32 elements) and codes of a tensor's Q4_0 blocks."""
     g = w.reshape(-1, 32)
     at = g.abs().argmax(dim=1, keepdim=True)
     scale = g.gather(1, at) / -8.0
     inv = torch.where(scale == 0, torch.zeros_like(scale), 1.0 / scale)
-    codes = (g * inv + 8.5).clamp(0, 15).to(torch.uint8)
+    return scale, (g * inv + 8.5).clamp(0, 15).to(torch.uint8)
+
+
+def _q4_0_blocks(w):
+    """Canonical Q4_0 blocks of a [n, k] f32 tensor (18 bytes per 32 features: f16 scale, 16 bytes of code pairs)."""
+    scale, codes = _q4_0_codes(w)
     packed = codes[:, :16] | (codes[:, 16:] << 4)
     return torch.cat([scale.to(torch.float16).view(torch.uint8), packed], dim=1).reshape(-1)
+
+
+def _project_inputs(case, x):
+    """Each layer's weights [n, k] and activation rows."""
+    for _ in range(case["layers"]):
+        yield x.normal((case["n"], case["k"]), "f32", scale=0.03), x.normal((1, case["rows"], case["k"]), case["dtype"])
 
 
 def _prepare_project(case, x):
     m, n, k, dt = case["rows"], case["n"], case["k"], case["dtype"]
     calls, outs = [], []
-    for _ in range(case["layers"]):
-        blocks = _q4_0_blocks(x.normal((n, k), "f32", scale=0.03))
+    for weights, act in _project_inputs(case, x):
+        blocks = _q4_0_blocks(weights)
         torch.cuda.synchronize()
         w = ta.Q40Weights(_wrap(blocks), 1, n, k)
-        act = x.normal((1, m, k), dt)
         out = torch.empty((1, m, n), device="cuda", dtype=_TORCH[dt])
         outs.append(out)
         calls.append((w, _wrap(act), _wrap(out)))
@@ -302,12 +334,15 @@ def _run_project(s):
     return s["outs"]
 
 
+def _kivi_inputs(case, x):
+    """q, k and v of the prompt, then of each single token."""
+    return [_new_rows(case, x, case["batch"], n, outliers=True) for n in [case["prompt"]] + [1] * case["tokens"]]
+
+
 def _prepare_kivi(case, x):
-    b, hq, hkv, d, dt = case["batch"], case["heads"], case["kv_heads"], case["dim"], case["dtype"]
     st = ta.QuantizedKvSdpa(axis=2).state()
     calls, outs = [], []
-    for n in [case["prompt"]] + [1] * case["tokens"]:
-        q, k, v = x.normal((b, hq, n, d), dt), x.normal((b, hkv, n, d), dt, outliers=True), x.normal((b, hkv, n, d), dt)
+    for q, k, v in _kivi_inputs(case, x):
         out = torch.empty_like(q)
         outs.append(out)
         calls.append(([_wrap(q), _wrap(k), _wrap(v)], _wrap(out)))
@@ -337,6 +372,124 @@ def prepare(case, seed):
 
 def run(state):
     return state["run"](state["state"])
+
+
+# ---- the same in 64 bits -----------------------------------------------------------------------------------
+
+
+def _round_half_away(t):
+    return torch.trunc(t.double() + torch.copysign(torch.full_like(t.double(), 0.5), t.double()))
+
+
+def _stored(rows, store):
+    """What a cache of this format holds for these rows, in f64."""
+    if store == "plain":
+        return rows.double()
+    w = rows.float()
+    if store == "q4_0":
+        scale, codes = _q4_0_codes(w)
+        codes = codes.double() - 8.0
+    else:
+        g = w.reshape(-1, 32)
+        scale = g.gather(1, g.abs().argmax(dim=1, keepdim=True)) / 127.0
+        inv = torch.where(scale == 0, torch.zeros_like(scale), 1.0 / scale)
+        codes = _round_half_away(g * inv).clamp(-128, 127)
+    return (codes * scale.to(torch.float16).double()).reshape(rows.shape)
+
+
+def _attend(q, k, v, causal):
+    """Attention of q [hq, n, d] over k and v [hkv, t, d], all f64; causal: the last row of q is the last token."""
+    hq, n, d = q.shape
+    hkv, t, _ = k.shape
+    kt, out = k.transpose(1, 2).contiguous(), torch.empty_like(q)
+    step = max(1, (1 << 27) // (hq * t))
+    for i in range(0, n, step):
+        rows = q[:, i : i + step]
+        m = rows.shape[1]
+        s = torch.matmul(rows.reshape(hkv, -1, d), kt) / math.sqrt(d)
+        if causal:
+            sees = torch.arange(t, device="cuda")[None, :] <= (t - n) + torch.arange(i, i + m, device="cuda")[:, None]
+            s.view(hkv, -1, m, t).masked_fill_(~sees, -math.inf)
+        out[:, i : i + step] = torch.matmul(torch.softmax(s, dim=-1), v).reshape(hq, m, d)
+    return out
+
+
+def _rotate(t, cos, sin):
+    half = t.shape[-1] // 2
+    return t * cos.double() + torch.cat([-t[..., half:], t[..., :half]], dim=-1) * sin.double()
+
+
+def _exact_cached(case, x):
+    """Steps and chunks: a pass of single tokens over a layer is one causal pass of all of them."""
+    b, store, n = case["batch"], case["store"], case["layers"]
+    past = [[_past_rows(case, x) for _ in range(2)] for _ in range(n)]
+    single = case["kind"] == "step"
+    tokens = case["tokens"] if single else 1
+    new = [[_new_rows(case, x, b, 1 if single else case["chunk"]) for _ in range(n)] for _ in range(tokens)]   # [token][layer]
+    outs, kept = [[None] * n for _ in range(tokens)], []
+    for layer in range(n):
+        q, k, v = (torch.cat([new[t][layer][i] for t in range(tokens)], dim=2).double() for i in range(3))
+        if case.get("rope"):
+            cos, sin = _rotary(x, [case["past"] + t for t in range(tokens)], case["dim"], case["dtype"])
+            q, k = _rotate(q, cos, sin), _rotate(k, cos, sin)
+            if store != "plain":
+                k = k.to(_TORCH[case["dtype"]])   # the type that is quantised
+        out = torch.empty_like(q)
+        for i in range(b):
+            ki, vi = (_stored(new_rows[i], store) if rows is None else torch.cat([_stored(rows[i], store), _stored(new_rows[i], store)], dim=1)
+                      for rows, new_rows in zip(past[layer], (k, v)))
+            out[i] = _attend(q[i], ki, vi, True)
+        for t in range(tokens):
+            outs[t][layer] = out[:, :, t : t + 1] if single else out
+        kept += [k, v]
+    return [o for per in outs for o in per] + (kept if store == "plain" else [])
+
+
+def _exact_ragged(case, x):
+    lens = _lengths(case, np.random.default_rng(7))
+    past = list(_ragged_rows(case, x, lens))
+    new = [_new_rows(case, x, case["seqs"], 1) for _ in range(case["tokens"])]
+    q, k, v = (torch.cat([t[i] for t in new], dim=2) for i in range(3))
+    out = torch.empty(q.shape, device="cuda", dtype=torch.float64)
+    for i in range(case["seqs"]):
+        ki, vi = (torch.cat([_stored(past[2 * i + j][0], case["store"]), _stored(r[i], case["store"])], dim=1) for j, r in enumerate((k, v)))
+        out[i] = _attend(q[i].double(), ki, vi, True)
+    return [out[:, :, t : t + 1] for t in range(case["tokens"])]
+
+
+def _exact_project(case, x):
+    outs = []
+    for weights, act in _project_inputs(case, x):
+        scale, codes = _q4_0_codes(weights)
+        w = ((codes.double() - 8.0) * scale.to(torch.float16).double()).reshape(weights.shape)
+        outs.append(torch.matmul(act.double(), w.t().contiguous()))
+    return outs
+
+
+def _exact_kivi(case, x):
+    """Keys: 8-bit codes of a channel, written with the smallest value and the widest range up to their token and read with
+    the newest ones; values: 8-bit codes per token.  Every token of a call sees all of the cache."""
+    new = _kivi_inputs(case, x)
+    k, v = (torch.cat([t[i] for t in new], dim=2).float() for i in (1, 2))
+    lo = torch.cummin(k, dim=2).values
+    scale = torch.cummax((k - lo) / 255.0, dim=2).values.clamp(min=1.0)
+    codes = _round_half_away((k - lo) / scale).clamp(0, 255)
+    vlo, vhi = v.amin(dim=3, keepdim=True), v.amax(dim=3, keepdim=True)
+    vscale = torch.where(vhi > vlo, (vhi - vlo) / 255.0, torch.ones_like(vlo))
+    values = vlo.double() + _round_half_away((v - vlo) / vscale).clamp(0, 255) * vscale.double()
+    outs, t = [], 0
+    for q, _, _ in new:
+        t += q.shape[2]
+        keys = lo[:, :, t - 1 : t].double() + codes[:, :, :t] * scale[:, :, t - 1 : t].double()
+        outs.append(torch.stack([_attend(q[i].double(), keys[i], values[i, :, :t].contiguous(), False) for i in range(case["batch"])]))
+    return outs
+
+
+_EXACT = {"step": _exact_cached, "ragged": _exact_ragged, "chunk": _exact_cached, "project": _exact_project, "kivi": _exact_kivi}
+
+
+def exact(case, seed):
+    return _EXACT[case["kind"]](case, _Inputs(seed))
 
 
 # ---- what a pass cannot do without ---------------------------------------------------------------------------
