@@ -1143,6 +1143,7 @@ static int dispatch_sdpa(const SdpaArgs &a, hipStream_t s) {
     if (a.Sq == 1) rc = is_quant(a.kv_fmt) ? launch_sdpa_decode_quant(a, s) : launch_sdpa_decode(a, s);
     if (rc == 2 && a.Sq > 1) rc = launch_sdpa_prefill_pp(a, s);
     if (rc == 2) rc = launch_sdpa_prefill(a, s);
+    if (rc == 2 && a.Sq > 1) rc = launch_sdpa_prefill_f32(a, s);
     if (rc == 2) rc = launch_sdpa_generic(a, s);
     return rc;
 }
