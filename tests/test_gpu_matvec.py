@@ -58,7 +58,7 @@ def test_matvec_matches_the_oracle(rt, dt, wb, ab, m, n, k):
 # features: one wave per row group and k share (1, 2, 4 or 8 shares by the matrix's size), activations whole in LDS or
 # in chunks (8 rows of 14336 features, 16 of 8192), row groups that do not fill a workgroup's set, several rounds per
 # workgroup (20000 rows x 128 features), batches that share weights, and more than 16 rows (the matrix-matrix kernel
-# reading tiles; 17 rows of f32 in groups of 8).
+# reading tiles; 7 f32 rows and more: q4_matmul_f32.hip).
 TILED_SHAPES = [
     (1, 1, 1, 16, 128), (1, 1, 1, 48, 256), (2, 2, 1, 80, 384), (1, 2, 2, 1024, 4096), (1, 1, 3, 1024, 4096), (1, 3, 2, 4096, 1024), (1, 1, 1, 14336, 4096), (1, 1, 3, 4096, 14336),
     (1, 1, 8, 14336, 4096), (1, 1, 8, 4096, 14336), (1, 1, 16, 1040, 8192), (2, 4, 5, 272, 2176), (1, 1, 7, 20000, 128),
@@ -98,6 +98,46 @@ def test_tiled_weights_match_the_f64_product(rt, monkeypatch, dt, wb, ab, m, n, 
         monkeypatch.delenv("TROCM_Q4_ROWS_TOO")
         assert np.array_equal(only_tiles.blocks(), blocks)
         assert rel_err(tract_amd.GgmlGemm().eval(act, only_tiles).to_numpy(), want) <= tol
+
+
+# 7 f32 rows and more: tiles of 16 x 16, 16 x 32, 32 x 32, 32 x 64 and 64 x 64 (activation rows x weight rows) chosen by the
+# shape, ragged edges of each, k of one block, of one block past a unit of four, of fewer units than waves and of several
+# units per wave; as planes and as tiles (n a multiple of 16 and k of 128)
+@pytest.mark.parametrize("wb,ab,m,n,k", [
+    (1, 1, 7, 1, 32), (1, 1, 17, 33, 160), (2, 4, 15, 47, 1056), (1, 1, 33, 8200, 288), (1, 1, 130, 4100, 96), (1, 1, 600, 2060, 2080),
+    (1, 1, 7, 16, 128), (2, 4, 16, 1040, 1152), (1, 1, 24, 4112, 1152), (1, 1, 40, 8208, 256), (1, 1, 100, 4112, 1024), (1, 1, 600, 2064, 2176)])
+def test_f32_rows_are_summed_as_f32(rt, wb, ab, m, n, k):
+    rng = np.random.default_rng(n + k + m)
+    blocks = orc.quant(Q4, (rng.standard_normal((wb, n, k)) * 0.05).astype(np.float32))
+    act = rng.standard_normal((ab, m, k)).astype(np.float32) * (10.0 ** rng.uniform(-6, 6, (ab, m, 1))).astype(np.float32)
+    got = tract_amd.GgmlGemm().eval(act, tract_amd.Q40Weights(blocks, wb, n, k)).to_numpy().astype(np.float64)
+    want = f64_product(blocks, act, np.float32)
+    # products are exact; at most k / 32 / 8 + 8 + 6 additions stand one after the other, each rounding by 2^-24 of a partial
+    # sum that is no larger than the sum of the magnitudes
+    wd = np.repeat(np.abs(orc.dequant(Q4, blocks, np.float32).astype(np.float64)), ab // wb, axis=0)
+    bound = np.einsum("bmk,bnk->bmn", np.abs(act.astype(np.float64)), wd) * (k / 256 + 15) * 2.0 ** -24
+    assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.parametrize("m,n,k", [(9, 40, 96), (40, 4112, 256)])
+def test_f32_rows_with_infinities_and_huge_values(rt, m, n, k):
+    """An infinity, a NaN or values whose unscaled sum would overflow: the products with the dequantised weights, in that row
+    only."""
+    rng = np.random.default_rng(k)
+    blocks = orc.quant(Q4, (rng.standard_normal((1, n, k)) * 0.05).astype(np.float32))
+    act = rng.standard_normal((1, m, k)).astype(np.float32)
+    act[0, 1, 3], act[0, 2, 40], act[0, 4, :] = np.inf, np.nan, 1e38
+    act[0, 5, 64:] *= np.float32(1e-30)
+    got = tract_amd.GgmlGemm().eval(act, tract_amd.Q40Weights(blocks, 1, n, k)).to_numpy()
+    with np.errstate(all="ignore"):
+        want = f64_product(blocks, act, np.float32).astype(np.float32)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    big = np.isinf(want)
+    np.testing.assert_array_equal(got[big], want[big])
+    fine = np.isfinite(want)
+    fine[0, 4] = False   # cancelling terms of 1e36: against their magnitude
+    assert np.all(np.abs(got[0, 4] - want[0, 4]) <= 1e38 * 0.5 * k * 2.0 ** -20)
+    assert rel_err(got[fine], want[fine].astype(np.float64)) <= 1e-5
 
 
 def test_tiles_and_planes_hold_the_same_weights(rt, monkeypatch):

@@ -135,6 +135,9 @@ int launch_q4_0_matvec_mfma(const void *codes, const void *scales, int64_t w_bat
 // tiled: `codes` are tiles of 16 rows x 128 features (q4_tiled.hip), `scales` is unused.
 int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, int64_t n, int64_t k, const void *act,
                        int act_dtype, int64_t act_batch, int64_t m, void *out, hipStream_t s, int tiled = 0);
+// The same for f32 activations (q4_matmul_f32.hip; faster than the kernels above from 7 rows on).  Returns 2 when not covered.
+int launch_q4_0_matmul_f32(const void *codes, const void *scales, int64_t w_batch, int64_t n, int64_t k, const void *act,
+                           int64_t act_batch, int64_t m, void *out, hipStream_t s, int tiled);
 // Q4_0 weights tiled by 16 rows x 128 features (n a multiple of 16, k of 128): the layout, its inverse, and the product
 // with m rows of f16 or f32 activations (q4_tiled.hip).
 bool q4_0_tiled_layout_fits(int64_t n, int64_t k);

@@ -278,6 +278,12 @@ int launch_q4_0_matvec(const void *codes, const void *scales, int64_t w_batch, i
         const int rc = launch_q4_0_matmul(codes, scales, w_batch, n, k, act, act_dtype, act_batch, m, out, s);
         if (rc != 2) return rc;
     }
+    // f32 rows from 7 on: one pass over the weights for all of them (us for 1000 x 2080, here | there: 5 rows 7.2 | 7.3, 6 rows
+    // 8.0 | 7.3, 8 rows 11.6 | 7.4)
+    if (act_dtype == TROCM_F32 && m >= 7) {
+        const int rc = launch_q4_0_matmul_f32(codes, scales, w_batch, n, k, act, act_batch, m, out, s, 0);
+        if (rc != 2) return rc;
+    }
     // What it does not take runs as groups of 8 rows (each group streams the weights once): correct
     // for any m, efficient only for the few rows of a decode step.
     for (int64_t i0 = 0; i0 < m; i0 += 8) {

@@ -530,7 +530,8 @@ int launch_q4_0_tiled_export(const void *tiles, void *blocks, int64_t rows, int6
 }
 
 // Tiled weights x activations for any m: f16 rows in groups of up to 16 (more than 16 rows go to the matrix-matrix
-// kernel first, which reads the same tiles, when it takes the call), f32 rows in groups of up to 8.
+// kernel first, which reads the same tiles, when it takes the call), up to 6 f32 rows (more go to q4_matmul_f32.hip; in
+// groups of 8 what that refuses).
 int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int64_t k, const void *act, int act_dtype,
                              int64_t act_batch, int64_t m, void *out, hipStream_t s) {
     if (n >= (1ll << 30) || k >= (1ll << 30) || act_batch > 65535) return fail("q4_0_matvec: shape too large");
@@ -542,6 +543,12 @@ int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int6
     static const int matmul_from = env_int("TROCM_Q4_MATMUL_FROM", 17);
     if (act_dtype == TROCM_F16 && m >= matmul_from && m > 16) {
         const int rc = launch_q4_0_matmul(tiles, nullptr, w_batch, n, k, act, act_dtype, act_batch, m, out, s, 1);
+        if (rc != 2) return rc;
+    }
+    // f32 rows from 7 on: one pass over the weights for all of them (us, here | there, 6 rows and 7: 14336 x 4096 16.4 | 17.5
+    // and 18.2 | 17.6, 4096 x 4096 9.5 | 8.7 and 13.0 | 8.8, 4096 x 14336 31.2 | 24.8 and 34.4 | 25.1)
+    if (act_dtype == TROCM_F32 && m >= 7) {
+        const int rc = launch_q4_0_matmul_f32(tiles, nullptr, w_batch, n, k, act, act_batch, m, out, s, 1);
         if (rc != 2) return rc;
     }
     const int64_t es = act_dtype == TROCM_F16 ? 2 : 4, step = act_dtype == TROCM_F16 ? 16 : 8;
