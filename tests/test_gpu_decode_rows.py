@@ -1,0 +1,77 @@
+"""A few queries per sequence as columns of the decode tiles, new tokens read from the call's input and stored by the attention
+launch, against a float64 restatement and the bytes that were appended."""
+import numpy as np
+import pytest
+
+import tract_amd as ta
+from oracle import oracle as orc
+from tests.cases import textbook_sdpa
+from tests.gpu_util import rt  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def _f16(rng, *shape):
+    return rng.standard_normal(shape, dtype=np.float32).astype(np.float16)
+
+
+# Rows of a kv head (group size * q_len) at 8, 16 and 32, one more than each, two and more groups of which the last overlaps
+# its neighbour; lengths at and around a tile of 32 keys and four of them (one tile per wave), all new tokens, new tokens in
+# two tiles; one split, splits merged in the kernel (8 rows) and by the second launch
+@pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [
+    (1, 2, 1, 128, 0, 4), (1, 4, 4, 64, 27, 8), (2, 3, 1, 128, 31, 3), (1, 16, 2, 64, 29, 2), (2, 17, 1, 128, 300, 2),
+    (1, 8, 2, 128, 1021, 8), (1, 11, 1, 128, 127, 3), (2, 14, 2, 64, 700, 5), (1, 7, 1, 128, 2000, 17), (1, 6, 2, 128, 255, 16),
+    (3, 4, 4, 128, 64, 33), (1, 5, 1, 64, 0, 64), (4, 32, 8, 128, 500, 8), (1, 32, 8, 128, 6000, 2)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_rows_of_several_queries(rt, B, Hq, Hkv, D, past, n, causal):
+    rng = np.random.default_rng(B + 10 * Hq + past + n)
+    q = (_f16(rng, B, Hq, n, D) / np.float16(np.sqrt(D))).astype(np.float16) * np.float16(4)
+    k, v = _f16(rng, B, Hkv, past + n, D), _f16(rng, B, Hkv, past + n, D)
+    st = ta.InPlaceKvSdpa(axis=2, causal=causal).state()
+    if past:
+        st.k.push(k[:, :, :past]), st.v.push(v[:, :, :past])
+    got = st.eval([q, np.ascontiguousarray(k[:, :, past:]), np.ascontiguousarray(v[:, :, past:])]).to_numpy().astype(np.float64)
+    want = textbook_sdpa(q, k, v, causal=causal)
+    # probabilities and results are rounded to f16 (2^-11): twice 2^-11 of a row's largest |v|, which its result cannot exceed
+    assert np.abs(got - want).max() <= 2 * 2.0 ** -11 * np.abs(v.astype(np.float64)).max()
+    assert np.linalg.norm(got - want) <= 2.0 ** -10 * np.linalg.norm(want)
+    assert st.k.len() == st.v.len() == past + n
+    assert st.k.valid_contiguous().tobytes() == k.tobytes()
+    assert st.v.valid_contiguous().tobytes() == v.tobytes()
+    # without the append, over the same cache
+    again = ta.Sdpa(datum_type=np.float16, is_causal=causal).eval(q, k, v).to_numpy().astype(np.float64)
+    assert np.abs(again - want).max() <= 2 * 2.0 ** -11 * np.abs(v.astype(np.float64)).max()
+
+
+@pytest.mark.parametrize("fmt_name", ["Q8_0", "Q4_0"])
+@pytest.mark.parametrize("B,Hq,Hkv,past,n", [(1, 4, 4, 30, 2), (2, 8, 2, 600, 4), (1, 8, 2, 1021, 8), (1, 14, 2, 700, 5), (2, 3, 1, 31, 5)])
+def test_rows_over_a_quantised_cache(rt, fmt_name, B, Hq, Hkv, past, n):
+    fmt = {"Q8_0": ta.Q8_0, "Q4_0": ta.Q4_0}[fmt_name]
+    rng = np.random.default_rng(Hq + past + n)
+    D = 128
+    q = (_f16(rng, B, Hq, n, D) / np.float16(np.sqrt(D))).astype(np.float16)
+    k, v = _f16(rng, B, Hkv, past + n, D), _f16(rng, B, Hkv, past + n, D)
+    k[:, :, :, 5] *= np.float16(12)
+    st = ta.InPlaceKvSdpa(axis=2, causal=True, storage_format=fmt).state()
+    st.k.push(k[:, :, :past]), st.v.push(v[:, :, :past])
+    got = st.eval([q, np.ascontiguousarray(k[:, :, past:]), np.ascontiguousarray(v[:, :, past:])]).to_numpy().astype(np.float64)
+    kd, vd = (orc.dequant(fmt, orc.quant(fmt, t), np.float16) for t in (k, v))
+    # as above, over the dequantised blocks
+    assert np.abs(got - textbook_sdpa(q, kd, vd, causal=True)).max() <= 2 * 2.0 ** -11 * np.abs(vd.astype(np.float64)).max()
+    assert st.k.valid_contiguous().tobytes() == orc.quant(fmt, k).tobytes()
+
+
+def test_rows_growing_a_cache_in_steps(rt):
+    """Chunks of changing length, some routed here and some to the prefill kernel, across capacity doublings."""
+    rng = np.random.default_rng(11)
+    B, Hq, Hkv, D = 2, 8, 2, 128
+    st = ta.InPlaceKvSdpa(axis=2, causal=True).state()
+    ks, vs = [], []
+    for n in (3, 5, 1, 8, 40, 2, 70, 4, 1, 6):
+        q = (_f16(rng, B, Hq, n, D) / np.float16(np.sqrt(D))).astype(np.float16)
+        ks.append(_f16(rng, B, Hkv, n, D)), vs.append(_f16(rng, B, Hkv, n, D))
+        got = st.eval([q, ks[-1], vs[-1]]).to_numpy().astype(np.float64)
+        k, v = np.concatenate(ks, axis=2), np.concatenate(vs, axis=2)
+        assert np.abs(got - textbook_sdpa(q, k, v, causal=True)).max() <= 2 * 2.0 ** -11 * np.abs(v.astype(np.float64)).max()
+        assert st.k.valid_contiguous().tobytes() == k.tobytes()
+        assert st.v.valid_contiguous().tobytes() == v.tobytes()

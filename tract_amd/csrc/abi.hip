@@ -1141,6 +1141,7 @@ static int dispatch_sdpa(const SdpaArgs &a, hipStream_t s) {
     if (a.B == 0 || a.Hq == 0 || a.Sq == 0 || a.D == 0) return 0;
     int rc = 2;
     if (a.Sq == 1) rc = is_quant(a.kv_fmt) ? launch_sdpa_decode_quant(a, s) : launch_sdpa_decode(a, s);
+    if (rc == 2 && a.Sq > 1) rc = launch_sdpa_decode_rows(a, s);
     if (rc == 2 && a.Sq > 1) rc = launch_sdpa_prefill_pp(a, s);
     if (rc == 2) rc = launch_sdpa_prefill(a, s);
     if (rc == 2 && a.Sq > 1) rc = launch_sdpa_prefill_f32(a, s);
@@ -1330,6 +1331,27 @@ int trocm_inplace_kv_sdpa_eval(const void *q, const void *k_new, const void *v_n
             if (rc == 0) {
                 kc->len += 1;
                 vc->len += 1;
+                return 0;
+            }
+            if (rc != 2) return rc;
+        }
+    }
+    // A few tokens at once on an f16 cache: likewise (4 x 5000 tokens, 8 new ones, 32 heads over 8: 26.4 us with an append
+    // launch, 24.8 without; 1 x 229: 14.9, 12.6).
+    if (n_new > 1 && is_dense && dtype == TROCM_F16 && kc->fmt == TROCM_F16 && vc->fmt == TROCM_F16 && q && k_new && v_new && out &&
+        kc->window == 0 && vc->window == 0 && kc->B == vc->B && kc->H == vc->H && kc->D == vc->D && kc->len == vc->len && q_heads % kc->H == 0) {
+        hipStream_t s;
+        if (resolve_stream(stream, &s)) return 1;
+        if (append_prepare(kc, k_new, dtype, kv_new_strides, n_new, s)) return 1;
+        if (append_prepare(vc, v_new, dtype, kv_new_strides, n_new, s)) return 1;
+        if (kc->cap == vc->cap) {
+            SdpaArgs a;
+            cached_args(a, q, dtype, q_heads, n_new, kc, vc, kc->len + n_new, out, scale, causal, workspace, workspace_bytes);
+            a.k_new = k_new, a.v_new = v_new;
+            const int rc = launch_sdpa_decode_rows(a, s);
+            if (rc == 0) {
+                kc->len += n_new;
+                vc->len += n_new;
                 return 0;
             }
             if (rc != 2) return rc;

@@ -204,6 +204,7 @@ int launch_sdpa_decode_kivi(const KiviSdpaArgs &a, hipStream_t s);
 int launch_sdpa_prefill(const SdpaArgs &a, hipStream_t s);
 // MFMA prefill for q_len >= 32: staggered waves, GQA heads sharing K/V tiles, key splits across
 // workgroups (partials in the workspace after the counter area).  Returns 2 when not covered.
+int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s);   // a few queries per sequence (sdpa_decode_mfma.hip)
 int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s);
 // The same for f32 q, K and V (2..: any number of queries), on the f32 matrix instruction.  Returns 2 when not covered.
 int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s);

@@ -47,6 +47,9 @@ struct DecodeDev {
     // matrix-core kernels, 8-row records with at most 4 real heads, in-kernel merge of up to 8 splits: rows 4..7 are neither
     // combined, stored nor merged (TROCM_DECODE_LIVE_TRIM=0 keeps them)
     int live_trim;
+    // several queries per sequence (sdpa_decode_rows_kernel): q_len, whether row r stops at its query's token, the rows of a
+    // kv head (group size * q_len) and the groups of g_real of them
+    int q_len, causal, n_rows, n_groups;
 };
 inline int decode_live_trim() {
     static const int on = getenv("TROCM_DECODE_LIVE_TRIM") ? atoi(getenv("TROCM_DECODE_LIVE_TRIM")) : 1;

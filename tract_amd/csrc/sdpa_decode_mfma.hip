@@ -85,6 +85,8 @@ struct MfmaWork {
     int *counter;                 // in-kernel merge by the last workgroup to arrive (dense batches, GP <= 8)
     int64_t part_first, part_stride;   // partial records of this sequence-head: first, first + stride, ...
     const char *mask;             // additive mask row of this kv head's first query head, token 0 (MASK instantiations)
+    int64_t row0;                 // ROWS instantiations: the first q / output row, and its place among its kv head's rows
+    int row_in_head0;
 };
 
 // The tail every formulation shares: the four waves' records (O[GP][D], m[GP], l[GP], in `lds_raw`, kCombStride floats
@@ -205,7 +207,8 @@ __device__ __forceinline__ auto rope_piece128(const _Float16 *row, const char *c
     return rope_finish<N>(rope_load128<N>(row, cosr, sinr, f0));
 }
 
-template <int D, int GP, int FMT, bool MASK = false, bool W16 = false, bool ROPE = false>
+// ROWS: the columns are rows of several queries (launch_sdpa_decode_rows), each of which sees its own number of tokens.
+template <int D, int GP, int FMT, bool MASK = false, bool W16 = false, bool ROPE = false, bool ROWS = false>
 __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaWork &wk) {
     static_assert(!W16 || GP <= 16, "the 16-wide layout: at most 16 heads");
     static_assert(!ROPE || (W16 && FMT == TROCM_F16 && !MASK), "the rotation is built for f16 rows on the 16-wide tiles");
@@ -233,10 +236,14 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
     const int g = p.g_real;
     _Float16 *tile = reinterpret_cast<_Float16 *>(lds_raw + w * kTileBytes);
 
-    const int64_t head0 = (int64_t)b * p.Hq + (int64_t)kvh * g;
+    static_assert(!ROWS || (!MASK && !ROPE), "several queries: no mask input, rotated before");
+    const int64_t head0 = ROWS ? wk.row0 : (int64_t)b * p.Hq + (int64_t)kvh * g;
     const _Float16 *qrow = reinterpret_cast<const _Float16 *>(p.q) + (head0 + min(hcol, g - 1)) * D;
     const char *kbase = wk.kbase, *vbase = wk.vbase;
     const int T = wk.T;
+    // Tokens that this lane's row sees, and the tokens that every row sees: tiles up to there need no comparison
+    const int t_row = ROWS && p.causal ? T - (p.q_len - 1) + (wk.row_in_head0 + min(hcol, g - 1)) % p.q_len : T;
+    const int t_all = ROWS && p.causal ? T - (p.q_len - 1) : T;
     const int tile_begin = wk.tile_begin, tile_end = wk.tile_end;
 
     // this lane's chunks of a tile: chunk j*64 + lane = (row, 16-byte chunk of the row)
@@ -261,11 +268,18 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
     // compiler sizes a wait for the path with the fewest operations in flight, so every tile of every wave waited for
     // its newest loads as well -- 1.6 us of a 47.6 us launch, with or without a new token.)
     const int new_pos = wk.new_pos;
-    const int64_t new_row = ((int64_t)b * p.Hkv + kvh) * D * 2;
+    const int64_t new_row = ((int64_t)b * p.Hkv + kvh) * (ROWS ? p.q_len : 1) * D * 2;   // (ROWS: q_len new tokens, from new_pos on)
     // (ROPE: the step's q and k_new rows are rotated on the way in, with the sequence's cos / sin rows)
     const char *cos_row = ROPE ? p.rope_cos + (int64_t)b * p.rope_stride_b : nullptr;
     const char *sin_row = ROPE ? p.rope_sin + (int64_t)b * p.rope_stride_b : nullptr;
-    if constexpr (!QUANT) {
+    if constexpr (!QUANT && ROWS) {
+        if (new_pos >= 0 && wk.tile_begin == 0 && wk.row_in_head0 == 0)
+            for (int c = tid; c < 2 * CPR * p.q_len; c += kThreads) {
+                const int tensor = c >= CPR * p.q_len, rc = c - tensor * CPR * p.q_len;   // row * CPR + chunk
+                char *dst = const_cast<char *>(tensor ? vbase : kbase) + (int64_t)(new_pos + rc / CPR) * p.kv_stride_t + rc % CPR * 16;
+                *reinterpret_cast<u32x4 *>(dst) = *reinterpret_cast<const u32x4 *>((tensor ? p.v_new : p.k_new) + new_row + (int64_t)rc * 16);
+            }
+    } else if constexpr (!QUANT) {
         if (new_pos >= 0 && w == 0 && wk.tile_begin == 0 && lane < 2 * CPR) {
             const int dc = lane % CPR;
             const char *src = (lane < CPR ? p.k_new : p.v_new) + new_row + dc * 16;
@@ -326,7 +340,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
     auto fetch = [&](const char *base0, const char *fresh, int t, u32x4 (&dst)[NLD], bool rotate = false) {
         const int t0 = t * kTile;
         const char *base = base0 + (int64_t)t0 * p.kv_stride_t;
-        if (t0 + kTile <= T && !(new_pos >= t0 && new_pos < t0 + kTile)) {
+        if (t0 + kTile <= T && !(new_pos >= (ROWS ? 0 : t0) && new_pos < t0 + kTile)) {
 #pragma unroll
             for (int j = 0; j < NLD; j++) dst[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(base + g_off[j]));
         } else {   // the sequence's last tile (rows past the end repeat the last token, masked below) or the new token's
@@ -334,8 +348,8 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
             for (int j = 0; j < NLD; j++) {
                 const int c = j * 64 + lane, row = min(c / CPR, T - 1 - t0), dc = c % CPR;
                 const char *cache_ptr = base + (uint32_t)row * (uint32_t)p.kv_stride_t + (uint32_t)dc * 16u;
-                const bool is_new = t0 + row == new_pos;
-                const u32x4 ld = *reinterpret_cast<const u32x4 *>(is_new ? fresh + new_row + dc * 16 : cache_ptr);
+                const bool is_new = ROWS ? new_pos >= 0 && t0 + row >= new_pos : t0 + row == new_pos;
+                const u32x4 ld = *reinterpret_cast<const u32x4 *>(is_new ? fresh + new_row + (ROWS ? (t0 + row - new_pos) * D * 2 : 0) + dc * 16 : cache_ptr);
                 // (ROPE: the lane's chunk of the rotated new key, made once ahead of the loop; dc = lane % CPR for every j.
                 // A select after the load, not a branch around it: with a load that some lanes skip the compiler can no
                 // longer count what is in flight and every wait of the loop becomes a wait for everything.)
@@ -479,14 +493,14 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const int tok = t0 + 16 * mb + 4 * q4 + r;
-                    s16[mb][r] = (t0 + kTile <= T || tok < T) ? s16[mb][r] * p.scale_log2 : -INFINITY;
+                    s16[mb][r] = (t0 + kTile <= t_all || tok < t_row) ? s16[mb][r] * p.scale_log2 : -INFINITY;
                     if constexpr (MASK) s16[mb][r] = __builtin_fmaf((float)mk[mb][r], 1.4426950408889634f, s16[mb][r]);
                     tmax = fmaxf(tmax, s16[mb][r]);
                 }
             tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
             tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
             const float m_new = fmaxf(m_run, tmax);   // finite without a mask: every tile holds at least one valid token
-            const float m_ref16 = (MASK && m_new == -INFINITY) ? 0.0f : m_new;   // masked out entirely with -inf: no NaN
+            const float m_ref16 = ((MASK || ROWS) && m_new == -INFINITY) ? 0.0f : m_new;   // masked out entirely with -inf: no NaN
             float psum = 0.0f;
 #pragma unroll
             for (int i = 0; i < 8; i++) {
@@ -517,7 +531,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
         }
         // ---- online softmax of this lane's head over its 16 tokens: token = t0 + 8*(r/4) + 4*hb + r%4 ----
         float tmax = -INFINITY;
-        if (QUANT && t0 + kTile <= T) {   // (the f16 instantiation has no register to spare for a second copy of this)
+        if (QUANT && t0 + kTile <= t_all) {   // (the f16 instantiation has no register to spare for a second copy of this)
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 s[r] *= p.scale_log2;
@@ -527,7 +541,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int tok = t0 + 8 * (r >> 2) + 4 * hb + (r & 3);
-                s[r] = (t0 + kTile <= T || tok < T) ? s[r] * p.scale_log2 : -INFINITY;
+                s[r] = (t0 + kTile <= t_all || tok < t_row) ? s[r] * p.scale_log2 : -INFINITY;
                 if constexpr (MASK) s[r] = __builtin_fmaf((float)mk[r >> 2][r & 3], 1.4426950408889634f, s[r]);
                 tmax = fmaxf(tmax, s[r]);
             }
@@ -535,7 +549,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
         const float m_new = fmaxf(m_run, tmax);   // finite without a mask: every tile holds at least one valid token
         // a tile (so far: a row) masked out entirely with -inf must leave the state untouched, not NaN
-        const float m_ref = (MASK && m_new == -INFINITY) ? 0.0f : m_new;
+        const float m_ref = ((MASK || ROWS) && m_new == -INFINITY) ? 0.0f : m_new;
         float psum = 0.0f;
 #pragma unroll
         for (int st = 0; st < 2; st++)
@@ -1948,6 +1962,44 @@ __global__ __launch_bounds__(kThreads, (QB ? QB % 10 : 2)) void sdpa_decode_mfma
         decode_mfma_body<D, GP, FMT, MASK, W16>(p, wk);
 }
 
+// Several queries per sequence: grid (splits, kv_heads * row groups, batch).  Row r = head r / q_len, query r % q_len of a
+// kv head's G q_len rows (consecutive in q and in the output); group i takes g_real of them from i g_real on, the last
+// group the last g_real (rows of two groups are written twice, with the same bits).
+template <int D, int GP, int FMT, bool W16>
+__global__ __launch_bounds__(kThreads, 2) void sdpa_decode_rows_kernel(DecodeDev p) {
+    const int split = blockIdx.x, kvh = blockIdx.y / p.n_groups, group = blockIdx.y % p.n_groups, b = blockIdx.z;
+    MfmaWork wk;
+    wk.seq = b, wk.kvh = kvh;
+    wk.kbase = p.k + (int64_t)b * p.kv_stride_b + (int64_t)kvh * p.kv_stride_h;
+    wk.vbase = p.v + (int64_t)b * p.kv_stride_b + (int64_t)kvh * p.kv_stride_h;
+    wk.ksbase = wk.vsbase = nullptr;
+    if constexpr (FMT != TROCM_F16) {
+        wk.ksbase = p.k_scales + (int64_t)b * p.sc_stride_b + (int64_t)kvh * p.sc_stride_h;
+        wk.vsbase = p.v_scales + (int64_t)b * p.sc_stride_b + (int64_t)kvh * p.sc_stride_h;
+    }
+    wk.T = p.T;
+    wk.tile_begin = split * kWaves, wk.tile_end = (p.T + kTile - 1) / kTile, wk.tile_step = kWaves * p.nsplit;
+    wk.skew_period = 0, wk.skew_split = split, wk.nsplit = p.nsplit;
+    const int64_t bh = (int64_t)b * gridDim.y + blockIdx.y;
+    wk.slot = bh * p.nsplit + split;
+    wk.new_pos = p.k_new ? p.new_pos : -1;
+    wk.counter = p.counters ? p.counters + bh : nullptr;
+    wk.part_first = bh * p.nsplit, wk.part_stride = 1;
+    wk.mask = nullptr;
+    wk.row_in_head0 = min(group * p.g_real, p.n_rows - p.g_real);
+    wk.row0 = ((int64_t)b * p.Hkv + kvh) * p.n_rows + wk.row_in_head0;
+    decode_mfma_body<D, GP, FMT, false, W16, false, true>(p, wk);
+}
+
+// Merge launch of the above: grid (kv_heads * row groups, batch, rows of a group), D threads.
+template <int D, int GP>
+__global__ __launch_bounds__(D) void sdpa_decode_rows_merge_kernel(DecodeDev p) {
+    const int kvh = blockIdx.x / p.n_groups, group = blockIdx.x % p.n_groups, b = blockIdx.y, r = blockIdx.z;
+    const int64_t bh = (int64_t)b * gridDim.x + blockIdx.x;
+    const int64_t row = ((int64_t)b * p.Hkv + kvh) * p.n_rows + min(group * p.g_real, p.n_rows - p.g_real) + r;
+    merge_head<__half, D, GP>(p, bh * p.nsplit, 1, p.nsplit, r, reinterpret_cast<__half *>(p.out) + row * D, threadIdx.x);
+}
+
 // Ragged batch: grid (work items, kv_heads); an item is a tile range of one sequence (the host's plan).
 template <int D, int GP, int FMT, bool W16 = false, int QB = 0>
 __global__ __launch_bounds__(kThreads, (QB ? QB % 10 : 2)) void sdpa_decode_mfma_ragged_kernel(DecodeDev p, const RaggedItem *__restrict__ items) {
@@ -2084,6 +2136,24 @@ int launch_quant(const DecodeDev &p, int gp, dim3 grid, hipStream_t s) {
         case 8: return launch_gp<128, 8, FMT>(p, grid, s);
         case 16: return launch_gp<128, 16, FMT>(p, grid, s);
         default: return launch_gp<128, 32, FMT>(p, grid, s);
+    }
+}
+
+template <int D, int GP, int FMT>
+int launch_rows(const DecodeDev &p, dim3 grid, hipStream_t s) {
+    hipLaunchKernelGGL((sdpa_decode_rows_kernel<D, GP, FMT, (GP <= 16)>), grid, dim3(kThreads), 0, s, p);
+    if (p.nsplit > 1 && p.counters == nullptr)
+        hipLaunchKernelGGL((sdpa_decode_rows_merge_kernel<D, GP>), dim3(grid.y, grid.z, p.g_real), dim3(D), 0, s, p);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail("sdpa_decode (rows) launch failed: %s", hipGetErrorString(e));
+    return 0;
+}
+template <int D, int FMT>
+int launch_rows_gp(const DecodeDev &p, int gp, dim3 grid, hipStream_t s) {
+    switch (gp) {
+        case 8: return launch_rows<D, 8, FMT>(p, grid, s);
+        case 16: return launch_rows<D, 16, FMT>(p, grid, s);
+        default: return launch_rows<D, 32, FMT>(p, grid, s);
     }
 }
 
@@ -2308,6 +2378,80 @@ int launch_sdpa_decode_mfma(const SdpaArgs &a, hipStream_t s) {
         p.counters = (int *)a.workspace;
     dim3 grid(nsplit, (unsigned)a.Hkv, (unsigned)a.B);
     return a.D == 128 ? launch_d<128>(p, gp, grid, s) : launch_d<64>(p, gp, grid, s);
+}
+
+// A few queries per sequence (proposed tokens to verify, short chunks) over a cache: the rows of a kv head, its G heads
+// times q_len queries, are the columns of the decode tiles, in groups of up to 32.  Like a decode step it is bound by the
+// stream of K and V (one group) and the chain of a short launch; the prefill kernels stage whole tiles for 32 queries per
+// head whatever q_len is, or read K and V once per query head.  Partial results stay f32 (the prefill kernels': f16).
+// a.k_new: the last q_len tokens are read from the call's input and stored to the cache by this launch, no append launch.
+// Measured, a call with its append, before | now: 4 x 5000 tokens, 6 queries, 32 heads over 8 31.1 | 24.6 us; 1 x 8000
+// 29.3 | 18.4; 1 x 229 13.6 | 10.9; 32 heads over 32, 1 x 8000 185.9 | 26.7; 14 over 2, 4 x 5000 108.8 | 20.5.
+// 2 = not taken.
+int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s) {
+    if (a.Sq < 2 || a.Sk < 1 || a.mask || a.q_dtype != TROCM_F16 || a.Hq % a.Hkv) return 2;
+    const bool quant = is_quant(a.kv_fmt);
+    if (!quant && a.kv_fmt != TROCM_F16) return 2;
+    if (a.D != 128 && (a.D != 64 || quant)) return 2;
+    if (a.causal && a.Sk < a.Sq) return 2;   // some queries would see nothing
+    if (a.Sk > (1ll << 30) || a.B > 65535 || a.kv_stride_t >= (1ll << 24)) return 2;
+    if ((uintptr_t)a.k % 16 || (uintptr_t)a.v % 16 || (uintptr_t)a.q % 16 || (uintptr_t)a.out % 8) return 2;
+    const int64_t G = a.Hq / a.Hkv;
+    if (a.Sq > 64 || G > 1024) return 2;
+    const int64_t rows = G * a.Sq, n_groups = (rows + 31) / 32, per = (rows + n_groups - 1) / n_groups;
+    const int gp = per <= 8 ? 8 : per <= 16 ? 16 : 32;
+    if (a.Hkv * n_groups > 65535) return 2;
+    const int64_t BH = a.B * a.Hkv * n_groups;
+    // One group reads K and V once: always (us with the append, prefill kernel | here: 32 heads over 8, 4 x 5000 tokens, 4
+    // queries 30.7 | 20.3, 8 queries 30.9 | 24.8; 1 x 229, 8 queries 13.1 | 12.6; Q4_0, 1 x 2000, 4 queries 24.1 | 15.1).  More
+    // groups read them again: against the prefill kernel that shares a tile among the heads of a group (an even G, and every
+    // quantised cache) while the launch is small (BH counts workgroups per split: 2 x 2000 tokens, 12 queries, BH 32 25.0 | 16.1;
+    // 4 x 5000, 64 31.2 | 30.5; 8 x 1000, 128 18.7 | 23.2); against the one that reads them per head up to 64 queries
+    // (14 heads over 2, 3 x 4000 tokens, 16 queries 88.8 | 25.0, 64 queries 90.0 | 34.4; 32 over 32, 48 queries 101.3 | 84.6,
+    // 100 queries 105.5 | 130.7).
+    if (n_groups > 1 && (quant || G % 2 == 0) && (n_groups > 4 || BH > 64)) return 2;
+    // (a short quantised cache and more than 16 rows: one staged tile of the prefill kernel, 14 heads over 2, 229 tokens, 6
+    // queries, Q4_0 13.6 | 14.1)
+    if (quant && gp == 32 && a.Sk < 512) return 2;
+    DecodeDev p;
+    memset(&p, 0, sizeof(p));
+    p.q = (const char *)a.q, p.out = (char *)a.out, p.k = (const char *)a.k, p.v = (const char *)a.v;
+    if (quant) {   // cache planes: dense token rows (strides arrive in elements of the logical rows)
+        if (a.kv_stride_t != a.D || !a.k_scales || !a.v_scales || a.kv_stride_h % a.D || a.kv_stride_b % a.D) return 2;
+        if ((uintptr_t)a.k_scales % 8 || (uintptr_t)a.v_scales % 8) return 2;
+        const int64_t rb = a.kv_fmt == TROCM_Q8_0 ? a.D : a.D / 2, rh = a.kv_stride_h / a.D, rbatch = a.kv_stride_b / a.D;
+        p.kv_stride_t = rb, p.kv_stride_h = rh * rb, p.kv_stride_b = rbatch * rb;
+        p.k_scales = (const char *)a.k_scales, p.v_scales = (const char *)a.v_scales;
+        p.sc_stride_h = rh * (a.D / 32) * 2, p.sc_stride_b = rbatch * (a.D / 32) * 2;
+    } else {
+        if ((a.kv_stride_b * 2) % 16 || (a.kv_stride_h * 2) % 16 || (a.kv_stride_t * 2) % 16) return 2;
+        p.kv_stride_b = a.kv_stride_b * 2, p.kv_stride_h = a.kv_stride_h * 2, p.kv_stride_t = a.kv_stride_t * 2;
+    }
+    p.T = (int)a.Sk, p.Hq = (int)a.Hq, p.Hkv = (int)a.Hkv, p.g_real = (int)per;
+    if (a.k_new) {   // the last q_len tokens come from the call's input and are stored by the launch
+        if (quant || !a.v_new || (uintptr_t)a.k_new % 16 || (uintptr_t)a.v_new % 16 || a.Sk < a.Sq) return 2;
+        p.k_new = (const char *)a.k_new, p.v_new = (const char *)a.v_new, p.new_pos = (int)(a.Sk - a.Sq);
+    }
+    p.q_len = (int)a.Sq, p.causal = a.causal, p.n_rows = (int)rows, p.n_groups = (int)n_groups;
+    p.scale_log2 = a.scale * 1.4426950408889634f;
+    const int n_tiles = (int)((a.Sk + kTile - 1) / kTile);
+    // A workgroup per compute unit, never a few more; two with several groups and more than 8 tiles per wave (40 heads over 8,
+    // 4 x 5000 tokens, 8 queries 38.7 -> 33.4 us).  Records of more than 8 rows are merged by a second launch, which up to
+    // two tiles per wave costs more than the split gives.
+    int64_t resident = num_compute_units();
+    int nsplit = choose_decode_splits(BH, gp, n_tiles, 1);
+    if (n_groups > 1 && n_tiles >= 32 * nsplit) nsplit = choose_decode_splits(BH, gp, n_tiles, 2), resident *= 2;
+    if (nsplit > 1 && BH * nsplit > resident && resident >= BH) nsplit = (int)(resident / BH);
+    if (gp > 8 && n_tiles <= 2 * kWaves) nsplit = 1;
+    p.nsplit = fit_decode_splits(nsplit, BH, gp, a.D, a.workspace, a.workspace_bytes);
+    p.live_trim = decode_live_trim();
+    p.part_ml = (float *)((char *)a.workspace + kWsCounterBytes);
+    p.part_o = p.part_ml + (size_t)BH * p.nsplit * 2 * gp;
+    if (gp <= 8 && p.nsplit > 1 && p.nsplit <= kWideMergeMax && BH <= (int64_t)(kWsCounterBytes / sizeof(int))) p.counters = (int *)a.workspace;
+    const dim3 grid((unsigned)p.nsplit, (unsigned)(a.Hkv * n_groups), (unsigned)a.B);
+    if (a.kv_fmt == TROCM_Q8_0) return launch_rows_gp<128, TROCM_Q8_0>(p, gp, grid, s);
+    if (a.kv_fmt == TROCM_Q4_0) return launch_rows_gp<128, TROCM_Q4_0>(p, gp, grid, s);
+    return a.D == 128 ? launch_rows_gp<128, TROCM_F16>(p, gp, grid, s) : launch_rows_gp<64, TROCM_F16>(p, gp, grid, s);
 }
 
 }  // namespace trocm
