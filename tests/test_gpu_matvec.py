@@ -119,6 +119,23 @@ def test_f32_rows_are_summed_as_f32(rt, wb, ab, m, n, k):
     assert np.all(np.abs(got - want) <= bound)
 
 
+# 9 f16 rows and more with few tiles, or planes whose k is no multiple of 64: tiles of 16 x 16, 16 x 32, 32 x 32, 32 x 64 and
+# 64 x 64 chosen by the shape, ragged edges, k of one block, one past a unit, fewer units than waves, several per wave
+@pytest.mark.parametrize("wb,ab,m,n,k", [
+    (1, 1, 9, 1, 32), (2, 4, 17, 33, 160), (1, 1, 33, 1001, 1056), (1, 1, 257, 1000, 288), (1, 1, 600, 2060, 2080), (1, 1, 900, 2050, 96),
+    (1, 1, 9, 16, 128), (2, 4, 16, 272, 1152), (1, 1, 64, 1024, 4096), (1, 1, 31, 4096, 2176), (1, 1, 70, 528, 128)])
+def test_f16_rows_times_exact_codes(rt, wb, ab, m, n, k):
+    rng = np.random.default_rng(n + k + m)
+    blocks = orc.quant(Q4, (rng.standard_normal((wb, n, k)) * 0.05).astype(np.float32))
+    act = rng.standard_normal((ab, m, k)).astype(np.float16)
+    got = tract_amd.GgmlGemm().eval(act, tract_amd.Q40Weights(blocks, wb, n, k)).to_numpy().astype(np.float64)
+    want = f64_product(blocks, act, np.float32)   # (the weights are not rounded to f16)
+    # products are exact; at most k / 32 / 8 + 10 f32 additions stand one after the other, and the result is rounded to f16
+    wd = np.repeat(np.abs(orc.dequant(Q4, blocks, np.float32).astype(np.float64)), ab // wb, axis=0)
+    bound = np.einsum("bmk,bnk->bmn", np.abs(act.astype(np.float64)), wd) * (k / 256 + 11) * 2.0 ** -24 + np.abs(want) * 2.0 ** -11 + 2.0 ** -25
+    assert np.all(np.abs(got - want) <= bound)
+
+
 @pytest.mark.parametrize("m,n,k", [(9, 40, 96), (40, 4112, 256)])
 def test_f32_rows_with_infinities_and_huge_values(rt, m, n, k):
     """An infinity, a NaN or values whose unscaled sum would overflow: the products with the dequantised weights, in that row

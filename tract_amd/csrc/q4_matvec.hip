@@ -274,7 +274,12 @@ int launch_q4_0_matvec(const void *codes, const void *scales, int64_t w_batch, i
         const int rc = launch_q4_0_matvec_mfma(codes, scales, w_batch, n, k, act, act_dtype, act_batch, m, out, s);
         if (rc != 2) return rc;
     }
-    if (m > 8) {   // the matrix-matrix arm (q4_matmul.hip) for f16 activations
+    // the matrix-matrix arms for f16 activations: k shared among waves for few tiles and for a k that q4_matmul.hip does not take
+    if (m > 8 && act_dtype == TROCM_F16 && (k % 64 || q4_0_matmul_waves_fits(n, m, act_batch))) {
+        const int rc = launch_q4_0_matmul_waves(codes, scales, w_batch, n, k, act, act_batch, m, out, s, 0);
+        if (rc != 2) return rc;
+    }
+    if (m > 8) {   // ... and q4_matmul.hip
         const int rc = launch_q4_0_matmul(codes, scales, w_batch, n, k, act, act_dtype, act_batch, m, out, s);
         if (rc != 2) return rc;
     }

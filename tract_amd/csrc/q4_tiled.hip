@@ -537,6 +537,12 @@ int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int6
     if (n >= (1ll << 30) || k >= (1ll << 30) || act_batch > 65535) return fail("q4_0_matvec: shape too large");
     // (a row group's records are addressed through one buffer descriptor: 32-bit offsets)
     if ((k / 128) * kTile >= (1ll << 31)) return fail("q4_0_matvec: rows of %lld features are too long for the tiled layout", (long long)k);
+    // 9 f16 rows and more with few tiles (us, the kernel above | there: 5 rows of 4096 x 14336 12.2 | 12.5; 9 rows 18.4 | 13.6,
+    // 16 rows 23.1 | 18.3, of 4096 x 4096 8.3 | 8.0)
+    if (act_dtype == TROCM_F16 && m >= 9 && q4_0_matmul_waves_fits(n, m, act_batch)) {
+        const int rc = launch_q4_0_matmul_waves(tiles, nullptr, w_batch, n, k, act, act_batch, m, out, s, 1);
+        if (rc != 2) return rc;
+    }
     // Up to 16 f16 rows take one pass through the kernel above, more go to the matrix-matrix kernel (us, two passes here |
     // one launch there with 32 activation rows per workgroup: 24 rows of 14336 x 4096 21.3 | 13.5, of 4096 x 4096
     // 12.9 | 10.0, of 1024 x 4096 12.4 | 8.9, of 4096 x 14336 35.5 | 32.3; 17 rows of the last 29.0 | 32.3).
