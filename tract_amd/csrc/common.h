@@ -197,8 +197,10 @@ struct KiviSdpaArgs {
     void *out;
     const uint8_t *k_codes, *v_codes;    // [B * Hkv, cap_rows, 128]
     int64_t k_cap_rows, v_cap_rows;
-    const float *k_chan_scale;           // [B * Hkv, 128]
-    const float *v_tok_scale, *v_tok_lo; // [B * Hkv, v_cap_rows]
+    const float *k_chan_lo, *k_chan_scale;         // [B * Hkv, 128]; the launch writes what the new token makes of them
+    float *k_chan_lo_next, *k_chan_scale_next;     // to these
+    const float *v_tok_scale, *v_tok_lo;           // [B * Hkv, v_cap_rows]
+    const void *k_new, *v_new;                     // the last of the T tokens, f16 [B * Hkv, 128]: coded and stored by the launch
     int64_t B, Hq, Hkv, T;
     float scale;
     void *workspace;

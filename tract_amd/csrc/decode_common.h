@@ -40,7 +40,9 @@ struct DecodeDev {
     int64_t mask_stride_b, mask_stride_h;
     // affine u8 caches (decode_mfma_kivi_body): the Keys' per-channel scales, f32 [B * Hkv, D]; k_scales / v_scales then
     // point at the Values' per-token scale and lo planes, f32 [B, Hkv, cap_rows], sc_stride_* their byte strides
-    const float *chan_scale;
+    // ... and their los; what the new token makes of both is written to the _next planes
+    const float *chan_scale, *chan_lo;
+    float *chan_scale_next, *chan_lo_next;
     // fused append with RoPE (f16, 16-wide tiles): cos / sin rows of D halves, one per sequence rope_stride_b bytes apart
     const char *rope_cos, *rope_sin;
     int64_t rope_stride_b;

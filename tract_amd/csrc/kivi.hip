@@ -24,7 +24,9 @@
 #include <hip/hip_fp16.h>
 #include <new>
 #include <type_traits>
+#include <utility>
 #include "common.h"
+#include "affine.h"
 
 namespace trocm {
 namespace {
@@ -32,47 +34,6 @@ namespace {
 constexpr int kKeyBlock = 32;   // quant_dyn_kv_cache.rs:153
 
 __device__ __forceinline__ float ld(const float *p) { return *p; }
-// A value on its way into fminf / fmaxf: a signalling NaN is quieted first.  v_min_f32 / v_max_f32 answer NaN for a
-// signalling one, and the next operation of the chain, which ignores that NaN, has then lost what came before it;
-// f32::min / f32::max skip every NaN alike.
-__device__ __forceinline__ float quiet(float x) { return __builtin_canonicalizef(x); }
-
-// Exchanges between lanes on the vector ALU (DPP modifiers and the lane-swap instructions) instead of through the LDS
-// crossbar (`__shfl_xor` = ds_bpermute_b32: the per-token ingest spent 14 of its 101 us on eight of those per lane).
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, false));
-}
-// x of lane (l ^ M) for M = 8, 16, 32 combined with this lane's by OP (min or max): exact partners.
-template <int M, typename Op>
-__device__ __forceinline__ float xor_combine(float x, Op op) {
-    static_assert(M == 8 || M == 16 || M == 32, "lane distances 8, 16, 32");
-    if constexpr (M == 8) {
-        return op(x, dpp_move<0x128>(x));                       // row_ror:8 within a row of 16 lanes
-    } else {   // rows 2k and 2k + 1 (halves of the wave) trade places between the two results: one of them is this lane's own
-        unsigned a = __builtin_bit_cast(unsigned, x), b = a;
-        asm("" : "+v"(b));   // two registers: the instruction swaps in place, and both results are read
-        const auto sw = M == 16 ? __builtin_amdgcn_permlane16_swap(a, b, false, false) : __builtin_amdgcn_permlane32_swap(a, b, false, false);
-        unsigned s0 = sw[0], s1 = sw[1];
-        asm("" : "+v"(s0), "+v"(s1));   // (this compiler folds op(sw[0], sw[1]) to sw[0] when both operands were one value: the minimum was lost)
-        return op(__builtin_bit_cast(float, s0), __builtin_bit_cast(float, s1));
-    }
-}
-// Minimum and maximum over aligned groups of N lanes (8, 16, 32, 64), left in every lane of the group.  (Any order of
-// exchanges gives the same bits: both are exact.)  Quads, halves of a row and rows by DPP, then pairs of rows, then the
-// two halves of the wave.
-template <int N>
-__device__ __forceinline__ void group_min_max(float &lo, float &hi) {
-    static_assert(N == 8 || N == 16 || N == 32 || N == 64, "groups of 8, 16, 32 or 64 lanes");
-    auto mn = [](float a, float b) { return fminf(a, b); };
-    auto mx = [](float a, float b) { return fmaxf(a, b); };
-    lo = fminf(lo, dpp_move<0xB1>(lo)), hi = fmaxf(hi, dpp_move<0xB1>(hi));       // quad_perm [1,0,3,2]
-    lo = fminf(lo, dpp_move<0x4E>(lo)), hi = fmaxf(hi, dpp_move<0x4E>(hi));       // quad_perm [2,3,0,1]
-    lo = fminf(lo, dpp_move<0x141>(lo)), hi = fmaxf(hi, dpp_move<0x141>(hi));     // row_half_mirror: the other quad of 8 lanes
-    if constexpr (N >= 16) lo = fminf(lo, dpp_move<0x140>(lo)), hi = fmaxf(hi, dpp_move<0x140>(hi));   // row_mirror: the other half of the row
-    if constexpr (N >= 32) lo = xor_combine<16>(lo, mn), hi = xor_combine<16>(hi, mx);
-    if constexpr (N >= 64) lo = xor_combine<32>(lo, mn), hi = xor_combine<32>(hi, mx);
-}
 __device__ __forceinline__ float ld(const __half *p) { return __half2float(*p); }
 
 // f32 -> f16 as its own instruction: without the barrier the compiler may fold the preceding multiply and add
@@ -81,24 +42,6 @@ __device__ __forceinline__ void st(float *p, float x) { *p = x; }
 __device__ __forceinline__ void st(__half *p, float x) {
     asm volatile("" : "+v"(x));
     *p = __float2half_rn(x);
-}
-
-// f32::round(): half away from zero, as trunc(x + copysign(0.49999997, x)) (the float below 0.5; the sum rounds to
-// nearest even, so an exact half ties up to the integer and anything less stays below it; exact for every float,
-// checked exhaustively on the host for the exponents where it matters; inf and NaN pass through).
-__device__ __forceinline__ float round_half_away(float x) {
-    return truncf(__fadd_rn(x, __builtin_copysignf(0.49999997f, x)));
-}
-
-// ((x - lo) / scale).round().clamp(0.0, lv) as u8   (quant_dyn_kv_cache.rs:128, :190; kv_quant.rs:110, :219)
-__device__ __forceinline__ uint32_t affine_code(float x, float lo, float scale, float lv) {
-    float q = round_half_away(__fdiv_rn(__fsub_rn(x, lo), scale));
-    if (!(q == q)) return 0;            // clamp keeps NaN, the cast turns it into 0
-    q = q < 0.0f ? 0.0f : (q > lv ? lv : q);
-    return (uint32_t)q;
-}
-__device__ __forceinline__ float affine_scale(float lo, float hi, float lv) {   // :127, :186
-    return hi > lo ? __fdiv_rn(__fsub_rn(hi, lo), lv) : 1.0f;
 }
 
 // The same codes without a division per element.  With inv = RN(1 / scale) the product q0 = RN((x - lo) * inv) lies
@@ -946,6 +889,7 @@ struct trocm_kivi_cache {
     int64_t len = 0, n_sink = 0, n_rows = 0, n_res = 0, cap_rows = 0;
     float *sink = nullptr, *residual = nullptr, *lo = nullptr, *scale = nullptr;
     uint8_t *codes = nullptr;
+    float *running = nullptr, *lo_next = nullptr, *scale_next = nullptr;   // per-channel layout: the allocation behind lo and scale; the other set
     void *deq = nullptr;      // dequantised copy handed to attention by trocm_quantized_kv_sdpa_eval
     size_t deq_bytes = 0;
     float *scan = nullptr;    // chunk results of a prompt pushed into the running Key store (kept for the next prompt)
@@ -1005,14 +949,9 @@ static int kivi_alloc_fixed(trocm_kivi_cache *c, hipStream_t s) {
         kivi_malloc((void **)&c->residual, (size_t)c->BH * kKeyBlock * c->D * 4, "the partial key block"))
         return 1;
     if (c->layout == TROCM_KIVI_RUNNING_CHANNEL && !c->lo) {
-        const int64_t n = c->BH * c->D;
-        float *lo = nullptr, *scale = nullptr;
-        if (kivi_malloc((void **)&lo, (size_t)n * 4, "running key parameters")) return 1;
-        if (kivi_malloc((void **)&scale, (size_t)n * 4, "running key parameters")) {
-            (void)hipFree(lo);
-            return 1;
-        }
-        c->lo = lo, c->scale = scale;
+        const int64_t n = c->BH * c->D;   // two sets, and a decode step reads one and writes the other
+        if (kivi_malloc((void **)&c->running, (size_t)n * 4 * 4, "running key parameters")) return 1;
+        c->lo = c->running, c->scale = c->running + n, c->lo_next = c->running + 2 * n, c->scale_next = c->running + 3 * n;
         kivi_fill_running_kernel<<<dim3((unsigned)((n + 255) / 256)), 256, 0, s>>>(c->lo, c->scale, n);
         TROCM_HIP(hipGetLastError());
     }
@@ -1281,8 +1220,11 @@ int trocm_kivi_cache_destroy(trocm_kivi_cache *c) {
     if (!c) return 0;
     (void)hipFree(c->sink);
     (void)hipFree(c->residual);
-    (void)hipFree(c->lo);
-    (void)hipFree(c->scale);
+    if (!c->running) {
+        (void)hipFree(c->lo);
+        (void)hipFree(c->scale);
+    }
+    (void)hipFree(c->running);
     (void)hipFree(c->codes);
     (void)hipFree(c->deq);
     (void)hipFree(c->scan);
@@ -1441,6 +1383,41 @@ int trocm_quantized_kv_sdpa_eval(const void *q, const void *k_new, const void *v
         for (trocm_kivi_cache *c : {k_cache, v_cache})
             if (kivi_grow_buffer(&c->deq, &c->deq_bytes, need, s, "the dequantised copy of a quantised store")) return 1;
     }
+    // A decode step of f16 queries: the attention launch codes the new token itself and writes its row and the Keys' new
+    // parameters, the latter into the set that it does not read (a prompt of 2 x 1500 tokens and 16 steps, 32 heads over 8: 390.0 us with a
+    // launch for each push, 368.5 without).  The dequantised copies a prompt left behind are not needed again: released
+    // behind an event.
+    if (fused_attention && workspace) {
+        KiviSdpaArgs a;
+        a.q = q, a.out = out;
+        a.k_codes = k_cache->codes, a.v_codes = v_cache->codes;
+        a.k_cap_rows = k_cache->cap_rows, a.v_cap_rows = v_cache->cap_rows;
+        a.k_chan_lo = k_cache->lo, a.k_chan_scale = k_cache->scale;
+        a.k_chan_lo_next = k_cache->lo_next, a.k_chan_scale_next = k_cache->scale_next;
+        a.v_tok_scale = v_cache->scale, a.v_tok_lo = v_cache->lo;
+        a.k_new = k_new, a.v_new = v_new;
+        a.B = k_cache->B, a.Hq = q_heads, a.Hkv = k_cache->H, a.T = k_cache->len + 1;
+        a.scale = scale == scale ? scale : 1.0f / sqrtf((float)k_cache->D);   // NaN asks for the default (sdpa.rs:93-95)
+        a.workspace = workspace, a.workspace_bytes = workspace_bytes;
+        const int rc = launch_sdpa_decode_kivi(a, s);
+        if (rc == 0) {
+            std::swap(k_cache->lo, k_cache->lo_next), std::swap(k_cache->scale, k_cache->scale_next);
+            for (trocm_kivi_cache *c : {k_cache, v_cache}) {
+                c->n_rows += 1, c->len += 1;
+                if (c->deq) {
+                    if (defer_device_free(c->deq, nullptr, s)) return 1;
+                    c->deq = nullptr;
+                    c->deq_bytes = 0;
+                }
+            }
+            return 0;
+        }
+        if (rc != 2) return rc;
+        // (the launch declined: the dequantising path needs its buffers after all)
+        const size_t need = (size_t)k_cache->BH * (k_cache->len + 1) * k_cache->D * elem_bytes(dtype);
+        for (trocm_kivi_cache *c : {k_cache, v_cache})
+            if (kivi_grow_buffer(&c->deq, &c->deq_bytes, need, s, "the dequantised copy of a quantised store")) return 1;
+    }
     // a decode step on the op's own stores: both rows pushed by one launch
     if (n_new == 1 && k_cache->D == 128 && k_cache->layout == TROCM_KIVI_RUNNING_CHANNEL && v_cache->layout == TROCM_KIVI_PER_TOKEN &&
         k_cache->bits == 8 && v_cache->bits == 8 && k_cache->sink_tokens == 0 && v_cache->sink_tokens == 0 &&
@@ -1459,34 +1436,6 @@ int trocm_quantized_kv_sdpa_eval(const void *q, const void *k_new, const void *v
         if (trocm_kivi_cache_append(v_cache, v_new, dtype, n_new, s)) return 1;
     }
     const int64_t T = k_cache->len, D = k_cache->D;
-    // One token of f16 queries over the op's own stores (Keys under running per-channel parameters, Values per token, u8
-    // codes, nothing kept in f32): attention straight over the codes, no dequantised copy.  TROCM_KIVI_FUSED=0 keeps
-    // the dequantising path below, which serves every other case.
-    if (fused_attention) {
-        KiviSdpaArgs a;
-        a.q = q, a.out = out;
-        a.k_codes = k_cache->codes, a.v_codes = v_cache->codes;
-        a.k_cap_rows = k_cache->cap_rows, a.v_cap_rows = v_cache->cap_rows;
-        a.k_chan_scale = k_cache->scale;
-        a.v_tok_scale = v_cache->scale, a.v_tok_lo = v_cache->lo;
-        a.B = k_cache->B, a.Hq = q_heads, a.Hkv = k_cache->H, a.T = T;
-        a.scale = scale == scale ? scale : 1.0f / sqrtf((float)D);   // NaN asks for the default (sdpa.rs:93-95)
-        a.workspace = workspace, a.workspace_bytes = workspace_bytes;
-        const int rc = workspace ? launch_sdpa_decode_kivi(a, s) : 2;
-        if (rc == 0) {   // the dequantised copies a prompt left behind are not needed again: released behind an event
-            for (trocm_kivi_cache *c : {k_cache, v_cache})
-                if (c->deq) {
-                    if (defer_device_free(c->deq, nullptr, s)) return 1;
-                    c->deq = nullptr;
-                    c->deq_bytes = 0;
-                }
-        }
-        if (rc != 2) return rc;
-        // (the launch declined: the dequantising path needs its buffers after all)
-        const size_t need = (size_t)k_cache->BH * T * D * elem_bytes(dtype);
-        for (trocm_kivi_cache *c : {k_cache, v_cache})
-            if (kivi_grow_buffer(&c->deq, &c->deq_bytes, need, s, "the dequantised copy of a quantised store")) return 1;
-    }
     for (trocm_kivi_cache *c : {k_cache, v_cache})
         if (kivi_dequantize(c, c->deq, dtype, s, false)) return 1;
     const int64_t strides[3] = {k_cache->H * T * D, T * D, D};

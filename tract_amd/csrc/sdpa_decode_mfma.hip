@@ -28,6 +28,7 @@
 #include <type_traits>
 #include "decode_common.h"
 #include "quant_block.h"
+#include "affine.h"
 
 namespace trocm {
 namespace {
@@ -1646,6 +1647,7 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
     constexpr int kCombStride = GP * D + 2 * GP;
     constexpr int kLdsBytes = kWaves * (kWaveBytes > kCombStride * 4 ? kWaveBytes : kCombStride * 4);
     __shared__ __attribute__((aligned(16))) unsigned char lds_raw[kLdsBytes];
+    __shared__ __attribute__((aligned(16))) unsigned char lds_new[2 * RB];   // the new token's Key codes, its Value codes
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1662,21 +1664,59 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
     const int tile_begin = wk.tile_begin, tile_end = wk.tile_end;
     // lanes 0..31 carry the scale of token `lane` of a tile, lanes 32..63 the lo of token `lane - 32`
     const float *par_row = reinterpret_cast<const float *>(lane < kTile ? wk.ksbase : wk.vsbase);
+    const int64_t chan0 = ((int64_t)b * p.Hkv + kvh) * D;
+    // The step's new token, the last of the sequence: coded by the wave whose tiles include it, as kivi_step_push_kernel
+    // would, into `lds_new` (no other wave reads it), its row in the planes and the Keys' next parameters.
+    const int new_pos = wk.new_pos;
+    const bool owner = tile_begin + w <= new_pos / kTile && new_pos / kTile < tile_end && (new_pos / kTile - tile_begin - w) % wk.tile_step == 0;
+    float new_scale = 0.0f, new_lo = 0.0f;   // of the new Value row
+    if (owner) {
+        const float2 lo2 = *reinterpret_cast<const float2 *>(p.chan_lo + chan0 + 2 * lane), sc2 = *reinterpret_cast<const float2 *>(p.chan_scale + chan0 + 2 * lane);
+        const half2_t k2 = *reinterpret_cast<const half2_t *>(p.k_new + (chan0 + 2 * lane) * 2), v2 = *reinterpret_cast<const half2_t *>(p.v_new + (chan0 + 2 * lane) * 2);
+        float klo[2] = {lo2.x, lo2.y}, ks[2] = {sc2.x, sc2.y};
+        uint32_t kc = 0, vc = 0;
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const float val = (float)k2[e];
+            if (val < klo[e]) klo[e] = val;
+            const float range = __fsub_rn(val, klo[e]);
+            if (range > 0.0f) {
+                const float ns = __fdiv_rn(range, 255.0f);
+                if (ns > ks[e]) ks[e] = ns;
+            }
+            kc |= affine_code(val, klo[e], ks[e], 255.0f) << (8 * e);
+        }
+        const float v0 = (float)v2[0], v1 = (float)v2[1];
+        float vlo = fminf(fminf(INFINITY, quiet(v0)), quiet(v1)), vhi = fmaxf(fmaxf(-INFINITY, quiet(v0)), quiet(v1));
+        group_min_max<64>(vlo, vhi);
+        new_lo = vlo, new_scale = affine_scale(vlo, vhi, 255.0f);
+        vc = affine_code(v0, new_lo, new_scale, 255.0f) | (affine_code(v1, new_lo, new_scale, 255.0f) << 8);
+        reinterpret_cast<uint16_t *>(lds_new)[lane] = (uint16_t)kc, reinterpret_cast<uint16_t *>(lds_new + RB)[lane] = (uint16_t)vc;
+        reinterpret_cast<uint16_t *>(const_cast<char *>(wk.kbase) + (int64_t)new_pos * RB)[lane] = (uint16_t)kc;
+        reinterpret_cast<uint16_t *>(const_cast<char *>(wk.vbase) + (int64_t)new_pos * RB)[lane] = (uint16_t)vc;
+        *reinterpret_cast<float2 *>(p.chan_lo_next + chan0 + 2 * lane) = float2{klo[0], klo[1]};
+        *reinterpret_cast<float2 *>(p.chan_scale_next + chan0 + 2 * lane) = float2{ks[0], ks[1]};
+        if (lane == 0) {
+            reinterpret_cast<float *>(const_cast<char *>(wk.ksbase))[new_pos] = new_scale;
+            reinterpret_cast<float *>(const_cast<char *>(wk.vsbase))[new_pos] = new_lo;
+        }
+    }
 
     u32x4 kpre[PF][NLD], vpre[PF][NLD];
     float ppre[PF];
     auto fetch = [&](int t, u32x4 (&kd)[NLD], u32x4 (&vd)[NLD], float &par) {
         const int t0 = t * kTile;
         const char *kb = wk.kbase + (int64_t)t0 * RB, *vb = wk.vbase + (int64_t)t0 * RB;
-        if (t0 + kTile <= T) {
+        if (t0 + kTile < T) {
 #pragma unroll
             for (int j = 0; j < NLD; j++) {
                 kd[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(kb + (j * 64 + lane) * 16));
                 vd[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(vb + (j * 64 + lane) * 16));
             }
             par = par_row[t0 + (lane & (kTile - 1))];
-        } else {   // rows past the end of the sequence repeat its last token (their scores are masked below)
-            const int last = T - 1 - t0;
+        } else {   // the tile of the new token: rows from it on repeat the one before (row 0 of the tile if there is none) and
+                   // are replaced, or masked, below
+            const int last = max(T - 2 - t0, 0);
 #pragma unroll
             for (int j = 0; j < NLD; j++) {
                 const int c = j * 64 + lane, row = min(c / CPR, last), dc = c % CPR;
@@ -1710,10 +1750,40 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
     half8_t qf[NB];
     float ks_max = 0.0f;
     float4_t ksv[NB][2];
+    // (what the new token makes of the scales: a division only where its range can move one, as in kivi_run_chunk_vec_kernel)
+    float4_t lov[NB][2];
+    half8_t kn[NB];
 #pragma unroll
     for (int blk = 0; blk < NB; blk++) {
-        ksv[blk][0] = *reinterpret_cast<const float4_t *>(ksc + 32 * blk + 8 * q4);
-        ksv[blk][1] = *reinterpret_cast<const float4_t *>(ksc + 32 * blk + 8 * q4 + 4);
+        kn[blk] = *reinterpret_cast<const half8_t *>(p.k_new + (chan0 + 32 * blk + 8 * q4) * 2);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            ksv[blk][h] = *reinterpret_cast<const float4_t *>(ksc + 32 * blk + 8 * q4 + 4 * h);
+            lov[blk][h] = *reinterpret_cast<const float4_t *>(p.chan_lo + chan0 + 32 * blk + 8 * q4 + 4 * h);
+        }
+    }
+    bool wider = false;
+#pragma unroll
+    for (int blk = 0; blk < NB; blk++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) {   // lov becomes the range
+            const float val = (float)kn[blk][i], lo = lov[blk][i >> 2][i & 3];
+            const float range = __fsub_rn(val, val < lo ? val : lo);
+            lov[blk][i >> 2][i & 3] = range;
+            wider = wider || range > ksv[blk][i >> 2][i & 3] * 254.9f;
+        }
+    if (__builtin_amdgcn_ballot_w64(wider) != 0) {
+#pragma unroll
+        for (int blk = 0; blk < NB; blk++)
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                if (lov[blk][i >> 2][i & 3] > 0.0f) {
+                    const float ns = __fdiv_rn(lov[blk][i >> 2][i & 3], 255.0f);
+                    if (ns > ksv[blk][i >> 2][i & 3]) ksv[blk][i >> 2][i & 3] = ns;
+                }
+    }
+#pragma unroll
+    for (int blk = 0; blk < NB; blk++) {
 #pragma unroll
         for (int i = 0; i < 8; i++) ks_max = fmaxf(ks_max, fabsf(ksv[blk][i >> 2][i & 3]));
     }
@@ -1764,6 +1834,13 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
             *reinterpret_cast<u32x4 *>(lds_v + v_slot[j]) = vpre[ST][j];
         }
         lds_vp[lane] = ppre[ST];
+        if (owner && new_pos < t0 + kTile) {   // (new_pos is in the wave's last tile)
+            const int r = new_pos - t0, dc = lane & (CPR - 1);
+            if (lane < 2 * CPR)
+                *reinterpret_cast<u32x4 *>(lane < CPR ? lds_k + r * RB + 16 * (dc ^ key_k(r)) : lds_v + r * RB + 16 * (dc ^ key_v(r))) =
+                    *reinterpret_cast<const u32x4 *>(lds_new + 16 * lane);
+            if ((lane & (kTile - 1)) >= r) lds_vp[lane] = lane < kTile ? new_scale : new_lo;
+        }
         if (more) fetch(t + PF * tstep, kpre[ST], vpre[ST], ppre[ST]);
         // ---- codes x scaled query features, all 128 channels into one accumulator ------------------------------------
         float sc8[8];
@@ -2272,7 +2349,8 @@ int launch_sdpa_decode_kivi(const KiviSdpaArgs &a, hipStream_t s) {
     const int gp = decode_mfma_group(g_real);
     if (gp == 0 || gp > 16) return 2;
     if (a.T <= 0 || a.T > (1ll << 30) || a.B > 65535 || a.Hkv > 65535 || !(a.scale > 0.0f)) return 2;
-    if ((uintptr_t)a.q % 16 || (uintptr_t)a.k_codes % 16 || (uintptr_t)a.v_codes % 16 || (uintptr_t)a.k_chan_scale % 16) return 2;
+    if ((uintptr_t)a.q % 16 || (uintptr_t)a.k_codes % 16 || (uintptr_t)a.v_codes % 16 || (uintptr_t)a.k_chan_scale % 16 || (uintptr_t)a.k_chan_lo % 16) return 2;
+    if ((uintptr_t)a.k_new % 16 || (uintptr_t)a.v_new % 16 || (uintptr_t)a.k_chan_scale_next % 16 || (uintptr_t)a.k_chan_lo_next % 16) return 2;
     const int64_t BH = a.B * a.Hkv;
     const int n_tiles = (int)((a.T + kTile - 1) / kTile);
     int nsplit = fit_decode_splits(choose_decode_splits(BH, gp, n_tiles, 2), BH, gp, 128, a.workspace, a.workspace_bytes);
@@ -2286,7 +2364,8 @@ int launch_sdpa_decode_kivi(const KiviSdpaArgs &a, hipStream_t s) {
     p.kv_stride_h = a.k_cap_rows * 128, p.kv_stride_b = a.Hkv * p.kv_stride_h, p.kv_stride_t = 128;
     p.k_scales = (const char *)a.v_tok_scale, p.v_scales = (const char *)a.v_tok_lo;
     p.sc_stride_h = a.v_cap_rows * 4, p.sc_stride_b = a.Hkv * p.sc_stride_h;
-    p.chan_scale = a.k_chan_scale;
+    p.chan_scale = a.k_chan_scale, p.chan_lo = a.k_chan_lo, p.chan_scale_next = a.k_chan_scale_next, p.chan_lo_next = a.k_chan_lo_next;
+    p.k_new = (const char *)a.k_new, p.v_new = (const char *)a.v_new;
     p.T = (int)a.T;
     p.tiles_per_split = tps, p.nsplit = nsplit;
     p.Hq = (int)a.Hq, p.Hkv = (int)a.Hkv, p.g_real = (int)g_real;
