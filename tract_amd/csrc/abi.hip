@@ -149,6 +149,8 @@ struct DeferredFree {
     void *data, *scales;
     trocm_kv_pool *pool;   // NULL: planes of their own (hipFree)
     hipEvent_t done;
+    size_t bytes;          // of `data`, 0: not to be handed out again
+    hipStream_t stream;    // that `done` was recorded on
 };
 static std::mutex g_deferred_mu;
 static std::vector<DeferredFree> g_deferred;
@@ -199,10 +201,20 @@ static void reap_deferred(bool wait, trocm_kv_pool *only_pool = nullptr, bool un
     }
 }
 
+static bool stream_is_capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 // Hand the planes over to the deferred list, guarded by an event recorded on `s` now.
-static int defer_free(trocm_kv_pool *pool, void *data, void *scales, hipStream_t s) {
+static int defer_free(trocm_kv_pool *pool, void *data, void *scales, hipStream_t s, size_t bytes = 0) {
     if (!data && !scales) return 0;
-    DeferredFree d{data, scales, pool, nullptr};
+    if (bytes && stream_is_capturing(s)) bytes = 0;   // (a graph may read it again whenever it is replayed)
+    DeferredFree d{data, scales, pool, nullptr, bytes, s};
     hipError_t e = hipEventCreateWithFlags(&d.done, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventRecord(d.done, s);
     if (e != hipSuccess) {   // no event: fall back to waiting for the stream
@@ -219,7 +231,26 @@ static int defer_free(trocm_kv_pool *pool, void *data, void *scales, hipStream_t
 // The same service for the other stateful objects of the library (the affine-quantised stores): device memory that
 // work queued on `s` may still read is released by a later call, not by waiting for the stream here.
 namespace trocm {
-int defer_device_free(void *a, void *b, hipStream_t s) { return defer_free(nullptr, a, b, s); }
+int defer_device_free(void *a, void *b, hipStream_t s, size_t bytes) { return defer_free(nullptr, a, b, s, bytes); }
+// Memory on the list that was handed over with its size and serves `need` bytes without wasting more than it holds, for work on
+// `s`: what the same stream left behind (its work comes first in any case), or what nothing reads any more.  NULL: none.
+void *reuse_device_free(size_t need, hipStream_t s, size_t *bytes) {
+    if (need == 0 || stream_is_capturing(s)) return nullptr;
+    std::lock_guard<std::mutex> lock(g_deferred_mu);
+    for (size_t i = 0; i < g_deferred.size(); i++) {
+        const DeferredFree d = g_deferred[i];
+        if (d.pool || d.scales || d.bytes < need || d.bytes / 2 > need) continue;
+        const bool usable = hipEventQuery(d.done) == hipSuccess || (d.stream == s && hipStreamWaitEvent(s, d.done, 0) == hipSuccess);
+        (void)hipGetLastError();   // "not ready" is an answer, not a failure
+        if (!usable) continue;
+        g_deferred[i] = g_deferred.back();
+        g_deferred.pop_back();
+        (void)hipEventDestroy(d.done);
+        *bytes = d.bytes;
+        return d.data;
+    }
+    return nullptr;
+}
 void reap_device_frees(bool wait) { reap_deferred(wait); }
 }  // namespace trocm
 

@@ -76,7 +76,9 @@ struct AppendPair {
 int launch_append_pair(const AppendPair &a, hipStream_t s);
 // Device memory that work queued on `s` may still read: released by a later call, once an event recorded on `s` now has
 // completed (abi.hip).  reap_device_frees(wait) releases what has completed (wait: everything).
-int defer_device_free(void *a, void *b, hipStream_t s);
+// With its size, `a` may be handed out again before that (reuse_device_free).
+int defer_device_free(void *a, void *b, hipStream_t s, size_t bytes = 0);
+void *reuse_device_free(size_t need, hipStream_t s, size_t *bytes);
 void reap_device_frees(bool wait);
 // empty kernel (kind 0) or read-only streaming kernel (kind 1) on a given launch shape
 int launch_floor(int kind, const void *src, size_t bytes, int workgroups, int threads, void *sink, hipStream_t s);

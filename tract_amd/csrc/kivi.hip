@@ -1006,10 +1006,11 @@ static int kivi_ensure_rows(trocm_kivi_cache *c, int64_t need, hipStream_t s) {
 // A scratch buffer that only grows (by doubling); the one it replaces is released behind an event.
 static int kivi_grow_buffer(void **buf, size_t *have, size_t need, hipStream_t s, const char *what) {
     if (*have >= need) return 0;
-    const size_t cap = *have * 2 > need ? *have * 2 : need;
-    void *fresh = nullptr;
-    if (kivi_malloc(&fresh, cap, what)) return 1;
-    if (*buf && defer_device_free(*buf, nullptr, s)) return 1;
+    size_t cap = *have * 2 > need ? *have * 2 : need;
+    // what an earlier prompt left behind, else new memory
+    void *fresh = reuse_device_free(cap, s, &cap);
+    if (!fresh && kivi_malloc(&fresh, cap, what)) return 1;
+    if (*buf && defer_device_free(*buf, nullptr, s, *have)) return 1;
     *buf = fresh;
     *have = cap;
     return 0;
@@ -1405,7 +1406,7 @@ int trocm_quantized_kv_sdpa_eval(const void *q, const void *k_new, const void *v
             for (trocm_kivi_cache *c : {k_cache, v_cache}) {
                 c->n_rows += 1, c->len += 1;
                 if (c->deq) {
-                    if (defer_device_free(c->deq, nullptr, s)) return 1;
+                    if (defer_device_free(c->deq, nullptr, s, c->deq_bytes)) return 1;
                     c->deq = nullptr;
                     c->deq_bytes = 0;
                 }
