@@ -1,0 +1,82 @@
+"""The affine u8 stores: single tokens coded by the attention launch, prompts in chunks of every length, prompt buffers that are
+handed out again.  Stored bytes and parameters against the oracle, bit for bit."""
+import numpy as np
+import pytest
+
+import tract_amd
+from oracle import oracle as orc
+from tests.gpu_util import rt  # noqa: F401
+from tract_amd import kivi
+from tract_amd.runtime import Stream
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+def _same(got, want):
+    assert got["packed"].tobytes() == want["packed"].tobytes()
+    assert got["lo"].tobytes() == want["lo"].tobytes() and got["scale"].tobytes() == want["scale"].tobytes()
+
+
+# from the first token on, across tiles of 32 and the four waves of a workgroup; 4, 8 and 16 heads per kv head (records of 8 and
+# of 16 rows); minima and ranges that move late, constant rows, a range of exactly zero
+@pytest.mark.parametrize("B,Hq,Hkv,steps", [(1, 8, 2, 140), (2, 16, 2, 70), (1, 16, 1, 40)])
+def test_single_tokens_from_an_empty_store(rt, B, Hq, Hkv, steps):
+    rng = np.random.default_rng(steps)
+    st = tract_amd.QuantizedKvSdpa(axis=2).state()
+    kc, vc = orc.KiviCache(True, running=True), orc.KiviCache(False, running=True)
+    for t in range(steps):
+        q = (rng.standard_normal((B, Hq, 1, D)) / np.sqrt(D)).astype(np.float16)
+        k, v = rng.standard_normal((B, Hkv, 1, D)).astype(np.float16), rng.standard_normal((B, Hkv, 1, D)).astype(np.float16)
+        k[:, :, :, 3] *= np.float16(1 + 8 * t)      # ranges beyond 255: the scale moves with every token
+        k[:, :, :, 4] = np.float16(-t)
+        if t % 9 == 4:
+            v[:] = np.float16(-3.25)
+        got = st.eval([q, k, v]).to_numpy().astype(np.float64)
+        kc.ingest(k.astype(np.float32)), vc.ingest(v.astype(np.float32))
+        if t < 3 or t % 31 == 0 or t == steps - 1:
+            want = orc.flash_sdpa(q.astype(np.float32), kc.dequantized(), vc.dequantized(), causal=False)
+            assert np.abs(got - want).max() <= 2e-2, t   # (the tolerance of the existing step tests: f16 products over a sharp softmax)
+            _same(st.k.state(), kc.state()), _same(st.v.state(), vc.state())
+
+
+# chunks of 8, 16, 32 and 64 tokens, one token more and less than each change, on top of earlier state
+@pytest.mark.parametrize("lengths", [(63, 64, 65), (512, 5, 513), (4096, 1), (4097, 70), (8193,)])
+def test_prompts_in_chunks_of_every_length(rt, lengths):
+    rng = np.random.default_rng(lengths[0])
+    cache = kivi.KiviCache(kivi.KIVI_RUNNING_CHANNEL, 8, 0, 1, 2, D)
+    ref = orc.KiviCache(True, running=True)
+    for n in lengths:
+        x = (rng.standard_normal((1, 2, n, D)) * 100).astype(np.float16)
+        x[0, 1, :, 9] = np.linspace(5, -600, n).astype(np.float16)
+        x[0, 0, n // 2, 3] = np.nan
+        cache.append(x)
+        ref.ingest(x.astype(np.float32))
+        _same(cache.state(), ref.state())
+
+
+def test_sessions_that_reuse_their_prompt_buffers(rt):
+    """Prompt, steps, reset, again, on two streams in turn without a wait in between: the buffers a prompt left behind serve a
+    later one, and every session gives what it gave alone."""
+    rng = np.random.default_rng(3)
+    data = []
+    for n in (300, 200, 260):
+        data.append([((rng.standard_normal((1, 8, m, D)) / np.sqrt(D)).astype(np.float16), rng.standard_normal((1, 2, m, D)).astype(np.float16),
+                      rng.standard_normal((1, 2, m, D)).astype(np.float16)) for m in (n, 1, 1)])
+    alone = []
+    for calls in data:
+        st = tract_amd.QuantizedKvSdpa(axis=2).state()
+        alone.append([st.eval(list(c)).to_numpy() for c in calls])
+    streams = [Stream(), Stream()]
+    states = [tract_amd.QuantizedKvSdpa(axis=2).state() for _ in streams]
+    device = [[[tract_amd.DeviceTensor.from_numpy(t) for t in c] for c in calls] for calls in data]
+    outs = []
+    for turn in range(6):
+        i, calls = turn % 3, device[turn % 3]
+        st, s = states[turn % 2], streams[turn % 2]
+        if st.k is not None:
+            st.k.reset(stream=s), st.v.reset(stream=s)
+        outs.append((i, s, [st.eval(c, stream=s) for c in calls]))
+    for i, s, got in outs:
+        for g, w in zip(got, alone[i]):
+            assert np.array_equal(g.to_numpy(s), w)

@@ -246,6 +246,10 @@ __global__ void kivi_running_push_kernel(const SrcT *__restrict__ src, int64_t S
 // chunks with two short scans over the chunk results between them give every token the parameters the token-by-token
 // loop would have had at its push.
 constexpr int kRunChunk = 64;
+// From this many tokens on a prompt is cut into chunks by the 128-bit passes (a call with its attention, us, walked by a thread
+// per channel | in chunks: 40 tokens 47.3 | 47.1, 64 52.9 | 50.7, 250 108.4 | 62.5); the passes below, one channel per
+// thread, from four chunks on.
+constexpr int64_t kScanFrom = 64;
 
 // pass 1: first minimal value of each chunk and channel (+inf for a chunk of NaNs)
 template <typename SrcT>
@@ -501,13 +505,13 @@ __device__ __forceinline__ void settle(uint4 &w) { asm volatile("" : "+v"(w.x), 
 template <typename SrcT, int LPR, int PASS>
 __global__ void __launch_bounds__(256) kivi_run_chunk_vec_kernel(const SrcT *__restrict__ src, int64_t S, int n, int n_chunks,
                                                                  float *__restrict__ a, float *__restrict__ b,
-                                                                 uint8_t *__restrict__ codes, int64_t cap_rows, int64_t row0,
+                                                                 uint8_t *__restrict__ codes, int64_t cap_rows, int64_t row0, int chunk,
                                                                  float *__restrict__ c3 = nullptr) {
     constexpr int D = LPR * 8, CPW = 256 / LPR;
     const int bh = blockIdx.y, k = blockIdx.x * CPW + (int)threadIdx.x / LPR, sub = (int)threadIdx.x % LPR;
     if (k >= n_chunks) return;
     const int64_t at = ((int64_t)bh * n_chunks + k) * D + sub * 8;
-    const int t0 = k * kRunChunk, t1 = min(n, t0 + kRunChunk);
+    const int t0 = k * chunk, t1 = min(n, t0 + chunk);
     const SrcT *row = src + ((int64_t)bh * S + t0) * D + sub * 8;
     // PASS 3 takes the chunk's rows in groups of 8.  Loads and stores share a counter and are not ordered against each
     // other, so a wait for a row with a store outstanding is a wait for all memory traffic: with the loads of just the
@@ -1017,7 +1021,14 @@ static int kivi_grow_buffer(void **buf, size_t *have, size_t need, hipStream_t s
 }
 
 static bool kivi_prompt_scan(const trocm_kivi_cache *c, int64_t rem) {
-    return c->layout == TROCM_KIVI_RUNNING_CHANNEL && rem >= 4 * kRunChunk && (rem + kRunChunk - 1) / kRunChunk <= 65535;
+    return c->layout == TROCM_KIVI_RUNNING_CHANNEL && rem >= kScanFrom && (rem + kRunChunk - 1) / kRunChunk <= 65535;
+}
+// Tokens per chunk of the 128-bit passes.  A lane walks its chunk, a trip to memory per group of 8 tokens, and the scan walks the
+// chunks, 16 per trip: short prompts are cut finer, which also spreads them over more compute units (us with the attention, in
+// chunks of 64 | 32 | 16 | 8: 300 tokens 99.4 | 79.1 | 68.6 | 64.1, 2 x 1500 198.8 | 181.5 | 176.5 | 179.9, 3000 283.9 | 273.2 |
+// 268.4 | 277.8, 6000 707.1 | 694.1 | 701.2 | 730.1).
+static int kivi_vec_chunk(int64_t rem) {
+    return rem <= 512 ? 8 : rem <= 4096 ? 16 : rem <= 8192 ? 32 : kRunChunk;
 }
 
 // Everything an append of S tokens may have to allocate, before anything is launched or counted: a call that fails here
@@ -1031,7 +1042,7 @@ static int kivi_prepare(trocm_kivi_cache *c, int64_t S, hipStream_t s) {
     if (c->layout == TROCM_KIVI_BLOCK_CHANNEL) rows = c->n_rows + (c->n_res + rem) / kKeyBlock * kKeyBlock;
     if (rows > c->n_rows && kivi_ensure_rows(c, rows, s)) return 1;
     if (kivi_prompt_scan(c, rem)) {
-        const size_t need = (size_t)c->BH * ((rem + kRunChunk - 1) / kRunChunk) * c->D * 3 * sizeof(float);   // (three results per chunk and channel on the 128-bit path)
+        const size_t need = (size_t)c->BH * ((rem + kivi_vec_chunk(rem) - 1) / kivi_vec_chunk(rem)) * c->D * 3 * sizeof(float);   // (three results per chunk and channel on the 128-bit path)
         if (kivi_grow_buffer((void **)&c->scan, &c->scan_bytes, need, s, "the chunk results of a prompt")) return 1;
     }
     return 0;
@@ -1104,19 +1115,20 @@ static int kivi_append_t(trocm_kivi_cache *c, const SrcT *src, int64_t S, hipStr
             c->n_res += rem;
         }
     } else if (rem > 0) {
-        const int64_t n_chunks = (rem + kRunChunk - 1) / kRunChunk;
-        if (kivi_prompt_scan(c, rem)) {   // a prompt: chunks side by side (scratch: two floats per chunk and channel)
+        const bool vec = ((uintptr_t)(src + t0 * D) & 15) == 0 && (D == 64 || D == 128 || D == 256 || D == 512);
+        const int chunk = vec ? kivi_vec_chunk(rem) : kRunChunk;
+        const int64_t n_chunks = (rem + chunk - 1) / chunk;
+        if (kivi_prompt_scan(c, rem) && (vec || rem >= 4 * kRunChunk)) {   // a prompt: chunks side by side (scratch: two floats per chunk and channel)
             float *tmp = c->scan;
             const size_t plane = (size_t)c->BH * n_chunks * D;
             const SrcT *from = src + t0 * D;
             const dim3 scan((unsigned)((D + 63) / 64), BH);
-            const bool vec = ((uintptr_t)from & 15) == 0 && (D == 64 || D == 128 || D == 256 || D == 512);
 #define KIVI_RUN_VEC(LPR)                                                                                                              \
     do {                                                                                                                               \
         const dim3 vgrid((unsigned)((n_chunks + 256 / LPR - 1) / (256 / LPR)), BH);                                                    \
-        kivi_run_chunk_vec_kernel<SrcT, LPR, 12><<<vgrid, 256, 0, s>>>(from, S, (int)rem, (int)n_chunks, tmp, tmp + plane, c->codes, c->cap_rows, c->n_rows, tmp + 2 * plane); \
+        kivi_run_chunk_vec_kernel<SrcT, LPR, 12><<<vgrid, 256, 0, s>>>(from, S, (int)rem, (int)n_chunks, tmp, tmp + plane, c->codes, c->cap_rows, c->n_rows, chunk, tmp + 2 * plane); \
         kivi_run_scan_both_kernel<<<scan, 64, 0, s>>>(tmp, tmp + plane, tmp + 2 * plane, D, (int)n_chunks, c->lo, c->scale);         \
-        kivi_run_chunk_vec_kernel<SrcT, LPR, 3><<<vgrid, 256, 0, s>>>(from, S, (int)rem, (int)n_chunks, tmp, tmp + plane, c->codes, c->cap_rows, c->n_rows); \
+        kivi_run_chunk_vec_kernel<SrcT, LPR, 3><<<vgrid, 256, 0, s>>>(from, S, (int)rem, (int)n_chunks, tmp, tmp + plane, c->codes, c->cap_rows, c->n_rows, chunk); \
     } while (0)
             if (vec) {
                 if (D == 64) KIVI_RUN_VEC(8); else if (D == 128) KIVI_RUN_VEC(16); else if (D == 256) KIVI_RUN_VEC(32); else KIVI_RUN_VEC(64);
