@@ -177,12 +177,12 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32_kernel(PrefillF3
         // A key that a row does not see must not reach its sum, and 0 times an infinity or a NaN of V would: in a tile
         // with such keys the products take V's finite values only, and the others are added to the rows that do see them.
         if (edge) {
-            bool all_finite = true;
+            float probe = 0.0f;   // NaN once one is not finite (one register; a condition per element takes 86 scalar ones too many)
 #pragma unroll
             for (int i = 0; i < 16; i++)
 #pragma unroll
-                for (int t = 0; t < T; t++) all_finite = all_finite && finite(vreg[i][t]);
-            if (__any(!all_finite)) {
+                for (int t = 0; t < T; t++) probe = fmaf(vreg[i][t], 0.0f, probe);
+            if (__any(probe != 0.0f)) {
 #pragma unroll 1
                 for (int kk = 0; kk < 32; kk++) {
                     // p of (row = lane % 32, key kk): register 4 (kk / 8) + kk % 4 of the half (kk / 4) % 2
@@ -214,26 +214,30 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32_kernel(PrefillF3
     }
 
     // ---- the waves' results: out = sum_w e^(m_w - M) O_w / sum_w e^(m_w - M) l_w -------------------------------
-    l_run += __shfl_xor(l_run, 32, 64);
-    if (hb == 0) lds_m[w][l32] = m_run, lds_l[w][l32] = l_run;
+    // (the thread's number taken anew: what the tail makes of it would otherwise be kept through the loop, in scratch memory)
+    int tid_end = tid;
+    asm("" : "+v"(tid_end));
+    const int l_end = tid_end & 31, h_end = (tid_end >> 5) & 1;
+    l_run += __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(((tid_end & 63) ^ 32) * 4, __builtin_bit_cast(int, l_run)));
+    if (h_end == 0) lds_m[w][l_end] = m_run, lds_l[w][l_end] = l_run;
     __syncthreads();   // (and every wave is done with q)
-    float m_all = lds_m[0][l32];
+    float m_all = lds_m[0][l_end];
 #pragma unroll
-    for (int i = 1; i < kWaves; i++) m_all = fmaxf(m_all, lds_m[i][l32]);
+    for (int i = 1; i < kWaves; i++) m_all = fmaxf(m_all, lds_m[i][l_end]);
     const float wgt = expf(m_run - ref_of(m_all));
-    float *mine = &lds[w * kRows * ROW + l32 * ROW];
+    float *mine = &lds[w * kRows * ROW + l_end * ROW];
 #pragma unroll
     for (int r = 0; r < 16; r++) {
         vec x;
 #pragma unroll
         for (int t = 0; t < T; t++) x[t] = o[t][r] * wgt;
-        *reinterpret_cast<vec *>(mine + T * (8 * (r / 4) + 4 * hb + r % 4)) = x;
+        *reinterpret_cast<vec *>(mine + T * (8 * (r / 4) + 4 * h_end + r % 4)) = x;
     }
     __syncthreads();
     const int64_t wb = (int64_t)bh * p.n_rt + rt, n_wb = (int64_t)p.n_bh * p.n_rt;
 #pragma unroll
     for (int j = 0; j < kRows * D / 4 / kThreads; j++) {
-        const int f = j * kThreads + tid, r = f / (D / 4), c = f % (D / 4);
+        const int f = j * kThreads + tid_end, r = f / (D / 4), c = f % (D / 4);
         f32x4 sum = *reinterpret_cast<const f32x4 *>(&lds[r * ROW + 4 * c]);
         float mm = lds_m[0][r];
 #pragma unroll
