@@ -343,7 +343,11 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
         const char *base = base0 + (int64_t)t0 * p.kv_stride_t;
         if (t0 + kTile <= T && !(new_pos >= (ROWS ? 0 : t0) && new_pos < t0 + kTile)) {
 #pragma unroll
-            for (int j = 0; j < NLD; j++) dst[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(base + g_off[j]));
+            for (int j = 0; j < NLD; j++) {
+                // (ROWS, 32 columns: the rows' distance in scalar registers, the lane's offsets have no vector registers left)
+                const char *at = ROWS && !W16 ? base + (uint64_t)((uint32_t)(j * (64 / CPR)) * (uint32_t)p.kv_stride_t) + g_off[0] : base + g_off[j];
+                dst[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(at));
+            }
         } else {   // the sequence's last tile (rows past the end repeat the last token, masked below) or the new token's
 #pragma unroll
             for (int j = 0; j < NLD; j++) {
@@ -603,7 +607,17 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
         }
     }
     if constexpr (W16) l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
+    // (ROWS, 32 columns: the lane's number taken anew, else what the tail makes of it is kept through the loop, in scratch memory)
+    int l32_end = l32, hb_end = hb;
+    if constexpr (ROWS && !W16) {
+        int lane_end = tid;
+        asm volatile("" : "+v"(lane_end));
+        lane_end &= 63;
+        l32_end = lane_end & 31, hb_end = lane_end >> 5;
+        l_run += __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane_end ^ 32) * 4, __builtin_bit_cast(int, l_run)));
+    } else {
+        l_run += __shfl_xor(l_run, 32, 64);
+    }
 
     // ---- merge the 4 waves through LDS (the K/V tiles are dead) --------------------------------------------
     __syncthreads();
@@ -618,18 +632,18 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
                 cw[GP * D + GP + l16] = l_run;
             }
         }
-    } else if (l32 < GP) {
+    } else if (l32_end < GP) {
         float *cw = comb + w * kCombStride;
 #pragma unroll
         for (int db = 0; db < DB; db++)
 #pragma unroll
             for (int rq = 0; rq < 4; rq++) {
                 float4_t f4 = {o[db][4 * rq], o[db][4 * rq + 1], o[db][4 * rq + 2], o[db][4 * rq + 3]};
-                *reinterpret_cast<float4_t *>(cw + l32 * D + 32 * db + 8 * rq + 4 * hb) = f4;
+                *reinterpret_cast<float4_t *>(cw + l32_end * D + 32 * db + 8 * rq + 4 * hb_end) = f4;
             }
-        if (hb == 0) {
-            cw[GP * D + l32] = m_run;
-            cw[GP * D + GP + l32] = l_run;
+        if (hb_end == 0) {
+            cw[GP * D + l32_end] = m_run;
+            cw[GP * D + GP + l32_end] = l_run;
         }
     }
     wave_records_to_output<D, GP>(p, wk, lds_raw, head0, g, tid);
@@ -1762,7 +1776,7 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
             lov[blk][h] = *reinterpret_cast<const float4_t *>(p.chan_lo + chan0 + 32 * blk + 8 * q4 + 4 * h);
         }
     }
-    bool wider = false;
+    float excess = 0.0f;
 #pragma unroll
     for (int blk = 0; blk < NB; blk++)
 #pragma unroll
@@ -1770,9 +1784,9 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
             const float val = (float)kn[blk][i], lo = lov[blk][i >> 2][i & 3];
             const float range = __fsub_rn(val, val < lo ? val : lo);
             lov[blk][i >> 2][i & 3] = range;
-            wider = wider || range > ksv[blk][i >> 2][i & 3] * 254.9f;
+            excess = fmaxf(excess, fmaf(ksv[blk][i >> 2][i & 3], -254.9f, range));   // (a NaN moves no scale and is skipped)
         }
-    if (__builtin_amdgcn_ballot_w64(wider) != 0) {
+    if (__builtin_amdgcn_ballot_w64(excess > 0.0f) != 0) {
 #pragma unroll
         for (int blk = 0; blk < NB; blk++)
 #pragma unroll
