@@ -1776,7 +1776,7 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
             lov[blk][h] = *reinterpret_cast<const float4_t *>(p.chan_lo + chan0 + 32 * blk + 8 * q4 + 4 * h);
         }
     }
-    float excess = 0.0f;
+    uint64_t wider = 0;   // (of the wave, joined as they come: a condition per channel and lane takes more scalar registers than there are)
 #pragma unroll
     for (int blk = 0; blk < NB; blk++)
 #pragma unroll
@@ -1784,9 +1784,9 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
             const float val = (float)kn[blk][i], lo = lov[blk][i >> 2][i & 3];
             const float range = __fsub_rn(val, val < lo ? val : lo);
             lov[blk][i >> 2][i & 3] = range;
-            excess = fmaxf(excess, fmaf(ksv[blk][i >> 2][i & 3], -254.9f, range));   // (a NaN moves no scale and is skipped)
+            wider |= __builtin_amdgcn_ballot_w64(range > ksv[blk][i >> 2][i & 3] * 254.9f);
         }
-    if (__builtin_amdgcn_ballot_w64(excess > 0.0f) != 0) {
+    if (wider != 0) {
 #pragma unroll
         for (int blk = 0; blk < NB; blk++)
 #pragma unroll
@@ -2478,8 +2478,9 @@ int launch_sdpa_decode_mfma(const SdpaArgs &a, hipStream_t s) {
 // stream of K and V (one group) and the chain of a short launch; the prefill kernels stage whole tiles for 32 queries per
 // head whatever q_len is, or read K and V once per query head.  Partial results stay f32 (the prefill kernels': f16).
 // a.k_new: the last q_len tokens are read from the call's input and stored to the cache by this launch, no append launch.
-// Measured, a call with its append, before | now: 4 x 5000 tokens, 6 queries, 32 heads over 8 31.1 | 24.6 us; 1 x 8000
-// 29.3 | 18.4; 1 x 229 13.6 | 10.9; 32 heads over 32, 1 x 8000 185.9 | 26.7; 14 over 2, 4 x 5000 108.8 | 20.5.
+// Measured, a call with its append, before | now: 4 x 5000 tokens, 6 queries, 32 heads over 8 31.1 | 24.6 us (four layers in
+// turn 113.2 | 106.1, 100.1 since nothing is kept in scratch memory); 1 x 8000 29.3 | 18.4; 1 x 229 13.6 | 10.9; 32 heads
+// over 32, 1 x 8000 185.9 | 26.7; 14 over 2, 4 x 5000 108.8 | 20.5.
 // 2 = not taken.
 int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s) {
     if (a.Sq < 2 || a.Sk < 1 || a.mask || a.q_dtype != TROCM_F16 || a.Hq % a.Hkv) return 2;
