@@ -75,3 +75,53 @@ def test_rows_growing_a_cache_in_steps(rt):
         assert np.abs(got - textbook_sdpa(q, k, v, causal=True)).max() <= 2 * 2.0 ** -11 * np.abs(v.astype(np.float64)).max()
         assert st.k.valid_contiguous().tobytes() == k.tobytes()
         assert st.v.valid_contiguous().tobytes() == v.tobytes()
+
+
+# 8, 16 and 32 rows per kv head and two groups; one tile, several per wave, splits; a token that only the last query sees, one in
+# the middle of the new ones, one in a tile that all see; Q8_0: a value that is no number takes its block with it
+@pytest.mark.parametrize("fmt,B,Hq,Hkv,D,past,n", [
+    (None, 1, 2, 2, 128, 0, 6), (None, 2, 4, 2, 128, 37, 8), (None, 1, 8, 2, 128, 0, 8), (None, 1, 3, 1, 128, 1500, 8), (None, 1, 1, 1, 64, 30, 40),
+    (None, 2, 4, 2, 64, 700, 6), (ta.Q8_0, 1, 2, 2, 128, 0, 6), (ta.Q8_0, 2, 4, 2, 128, 37, 8), (ta.Q8_0, 1, 3, 1, 128, 1500, 8)])
+def test_rows_do_not_see_what_later_tokens_hold(rt, fmt, B, Hq, Hkv, D, past, n):
+    rng = np.random.default_rng(past + n)
+    q = (_f16(rng, B, Hq, n, D) / np.float16(np.sqrt(D))).astype(np.float16)
+    k, v = _f16(rng, B, Hkv, past + n, D), _f16(rng, B, Hkv, past + n, D)
+    v[0, 0, past + n - 1, 5], v[B - 1, Hkv - 1, past + n // 2, D - 1] = np.inf, -np.inf
+    v[0, Hkv - 1, past + 1, 40] = np.nan
+    if past:
+        v[B - 1, 0, past // 2, 17] = np.inf
+    st = ta.InPlaceKvSdpa(axis=2, causal=True, storage_format=fmt).state()
+    if past:
+        st.k.push(k[:, :, :past]), st.v.push(v[:, :, :past])
+    else:   # the caches exist before the call: keys and values travel with it
+        st.k.reserve(n, like=((B, Hkv, 1, D), np.float16)), st.v.reserve(n, like=((B, Hkv, 1, D), np.float16))
+    got = st.eval([q, np.ascontiguousarray(k[:, :, past:]), np.ascontiguousarray(v[:, :, past:])]).to_numpy().astype(np.float64)
+    if fmt is not None:
+        with np.errstate(all="ignore"):
+            k, v = (orc.dequant(fmt, orc.quant(fmt, t), np.float16) for t in (k, v))
+    bad = np.repeat(~np.isfinite(v), Hq // Hkv, axis=1)
+    reached = np.logical_or.accumulate(bad, axis=2)[:, :, past:]   # [B, Hq, n, D]: query i sees tokens up to past + i
+    np.testing.assert_array_equal(~np.isfinite(got), reached)
+    want = textbook_sdpa(q, k, np.where(np.isfinite(v), v, np.float16(0)), causal=True)
+    assert np.abs(got - want)[~reached].max() <= 2 * 2.0 ** -11 * np.abs(v[np.isfinite(v)].astype(np.float64)).max()
+    if fmt is None:
+        assert got[0, 0, n - 1, 5] == np.inf   # (one infinity, no other term that is not finite)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [(1, 2, 2, 128, 0, 6), (1, 4, 2, 128, 900, 8), (2, 8, 2, 64, 40, 8), (1, 3, 1, 128, 33, 20)])
+def test_rows_with_scores_that_are_no_numbers(rt, B, Hq, Hkv, D, past, n):
+    rng = np.random.default_rng(past + n + 1)
+    q = (_f16(rng, B, Hq, n, D) / np.float16(np.sqrt(D))).astype(np.float16)
+    k, v = _f16(rng, B, Hkv, past + n, D), _f16(rng, B, Hkv, past + n, D)
+    q[0, 1, 2, 7] = np.nan
+    k[B - 1, 0, past + 4, 3] = np.nan
+    st = ta.InPlaceKvSdpa(axis=2, causal=True).state()
+    if past:
+        st.k.push(k[:, :, :past]), st.v.push(v[:, :, :past])
+    got = st.eval([q, np.ascontiguousarray(k[:, :, past:]), np.ascontiguousarray(v[:, :, past:])]).to_numpy().astype(np.float64)
+    nan = np.zeros(got.shape, bool)
+    nan[0, 1, 2] = True
+    nan[B - 1, : Hq // Hkv, 4:] = True
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    want = textbook_sdpa(np.nan_to_num(q), np.nan_to_num(k), v, causal=True)
+    assert np.abs(got - want)[~nan].max() <= 2 * 2.0 ** -11 * np.abs(v.astype(np.float64)).max()

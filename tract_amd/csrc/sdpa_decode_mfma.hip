@@ -584,6 +584,55 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
             for (int j = 0; j < NLD; j++) *reinterpret_cast<u32x4 *>(tile + v_slot[j]) = vpre[j];
             if (more) fetch(vbase, p.v_new, tn, vpre);
         }
+        // ROWS: a token that a row does not see must not reach its sum, and a weight of 0 times an infinity or a NaN would: in
+        // a tile with such tokens the product takes V's finite values only, and the others (any positive weight leaves them as
+        // they are) are added to the rows that see them.  (Ordinary values: 4 to 8 LDS reads and their test in the last tiles.)
+        if constexpr (ROWS) {
+            if (t0 + kTile > t_all) {
+                constexpr int CH = kTile * D / 8 / 64;   // 16-byte chunks of the tile per lane
+                auto odd_halves = [](uint32_t x) { return ((x & 0x7C007C00u) + 0x04000400u) & 0x80008000u; };
+                uint32_t odd = 0;
+#pragma unroll
+                for (int j = 0; j < CH; j++) {
+                    const int c = j * 64 + lane;
+                    const u32x4 x = *reinterpret_cast<const u32x4 *>(tile + c / (D / 8) * VROW + c % (D / 8) * 8);
+                    odd |= odd_halves(x.x) | odd_halves(x.y) | odd_halves(x.z) | odd_halves(x.w);
+                }
+                if (__builtin_amdgcn_ballot_w64(odd != 0) != 0) {
+                    auto unless_finite = [](_Float16 x) { return __builtin_isfinite((float)x) ? 0.0f : (float)x; };
+#pragma unroll 1
+                    for (int kk = 0; kk < kTile; kk++) {
+                        const bool seen = t0 + kk < t_row;
+                        if constexpr (W16) {
+#pragma unroll
+                            for (int fb = 0; fb < D / 16; fb++) {
+                                const half4_t x = *reinterpret_cast<const half4_t *>(tile + kk * VROW + 16 * fb + 4 * q4);
+#pragma unroll
+                                for (int i = 0; i < 4; i++) o16[fb][i] += seen ? unless_finite(x[i]) : 0.0f;
+                            }
+                        } else {
+#pragma unroll
+                            for (int db = 0; db < DB; db++)
+#pragma unroll
+                                for (int rq = 0; rq < 4; rq++) {
+                                    const half4_t x = *reinterpret_cast<const half4_t *>(tile + kk * VROW + 32 * db + 8 * rq + 4 * hb);
+#pragma unroll
+                                    for (int i = 0; i < 4; i++) o[db][4 * rq + i] += seen ? unless_finite(x[i]) : 0.0f;
+                                }
+                        }
+                    }
+#pragma unroll 1
+                    for (int j = 0; j < CH; j++) {
+                        const int c = j * 64 + lane;
+                        u32x4 *at = reinterpret_cast<u32x4 *>(tile + c / (D / 8) * VROW + c % (D / 8) * 8);
+                        u32x4 x = *at;
+#pragma unroll
+                        for (int i = 0; i < 4; i++) x[i] &= ~((odd_halves(x[i]) >> 15) * 0xFFFFu);
+                        *at = x;
+                    }
+                }
+            }
+        }
         // ---- O^T += V^T P^T ---------------------------------------------------------------------------------
         const _Float16 *vsrc = tile + vsrc_off;
         if constexpr (W16) {
@@ -617,6 +666,13 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
         l_run += __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane_end ^ 32) * 4, __builtin_bit_cast(int, l_run)));
     } else {
         l_run += __shfl_xor(l_run, 32, 64);
+    }
+
+    // ROWS: a row with a score that is no number has none in its result either, as in the prefill kernels (a sum of NaN would
+    // read as "no token seen" below; its outputs are NaN already)
+    if constexpr (ROWS) {
+        const bool nan = l_run != l_run;
+        m_run = nan ? 0.0f : m_run, l_run = nan ? 1.0f : l_run;
     }
 
     // ---- merge the 4 waves through LDS (the K/V tiles are dead) --------------------------------------------
