@@ -125,3 +125,29 @@ def test_rows_with_scores_that_are_no_numbers(rt, B, Hq, Hkv, D, past, n):
     np.testing.assert_array_equal(np.isnan(got), nan)
     want = textbook_sdpa(np.nan_to_num(q), np.nan_to_num(k), v, causal=True)
     assert np.abs(got - want)[~nan].max() <= 2 * 2.0 ** -11 * np.abs(v.astype(np.float64)).max()
+
+
+# the output over q, over the new keys and over the new values: 5 query heads per kv head in 6 groups of rows, more workgroups
+# than run at once; as many kv heads as query heads, two groups
+@pytest.mark.parametrize("B,Hq,Hkv,past,n", [(16, 40, 8, 300, 33), (4, 32, 32, 100, 33)])
+@pytest.mark.parametrize("over", ["q", "k", "v"])
+def test_rows_stored_over_the_calls_own_inputs(rt, over, B, Hq, Hkv, past, n):
+    rng = np.random.default_rng(n + Hq)
+    D = 128
+    q = (_f16(rng, B, Hq, n, D) / np.float16(np.sqrt(D))).astype(np.float16)
+    k, v = _f16(rng, B, Hkv, past + n, D), _f16(rng, B, Hkv, past + n, D)
+    results = []
+    for shared in (False, True):
+        st = ta.InPlaceKvSdpa(axis=2, causal=True).state()
+        st.k.push(k[:, :, :past]), st.v.push(v[:, :, :past])
+        tensors = {"q": q, "k": k[:, :, past:], "v": v[:, :, past:]}
+        args = {name: ta.DeviceTensor.from_numpy(t) for name, t in tensors.items()}
+        out = ta.DeviceTensor(q.shape, np.float16)
+        if shared:   # the input at the start of the output's memory
+            whole = np.zeros(q.size, np.float16)
+            whole[: tensors[over].size] = np.ascontiguousarray(tensors[over]).reshape(-1)
+            out = ta.DeviceTensor.from_numpy(whole.reshape(q.shape))
+            args[over] = ta.DeviceTensor(tensors[over].shape, np.float16, ptr=out.ptr, owner=out)
+        results.append(st.eval_into(args["q"], args["k"], args["v"], out).to_numpy())
+        assert st.k.valid_contiguous().tobytes() == k.tobytes() and st.v.valid_contiguous().tobytes() == v.tobytes()
+    np.testing.assert_array_equal(results[1], results[0])

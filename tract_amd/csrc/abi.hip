@@ -1324,6 +1324,11 @@ static int inplace_eval_check(const char *what, const void *q, const void *k_new
     return 0;
 }
 
+// Whether `n` bytes at a and `m` bytes at b have memory in common.
+static bool ranges_meet(const void *a, size_t n, const void *b, size_t m) {
+    return (uintptr_t)a < (uintptr_t)b + m && (uintptr_t)b < (uintptr_t)a + n;
+}
+
 int trocm_inplace_kv_sdpa_eval(const void *q, const void *k_new, const void *v_new, int dtype, int64_t q_heads,
                                int64_t n_new, const int64_t *kv_new_strides, trocm_kv_cache *kc, trocm_kv_cache *vc,
                                void *out, float scale, int causal, void *workspace, size_t workspace_bytes,
@@ -1368,8 +1373,10 @@ int trocm_inplace_kv_sdpa_eval(const void *q, const void *k_new, const void *v_n
         }
     }
     // A few tokens at once on an f16 cache: likewise (4 x 5000 tokens, 8 new ones, 32 heads over 8: 26.4 us with an append
-    // launch, 24.8 without; 1 x 229: 14.9, 12.6).
-    if (n_new > 1 && is_dense && dtype == TROCM_F16 && kc->fmt == TROCM_F16 && vc->fmt == TROCM_F16 && q && k_new && v_new && out &&
+    // launch, 24.8 without; 1 x 229: 14.9, 12.6).  Not where the output lies over the new rows: one workgroup stores results
+    // while another still reads them.
+    const size_t new_bytes = (size_t)kc->B * kc->H * n_new * kc->D * 2, out_bytes = (size_t)kc->B * q_heads * n_new * kc->D * 2;
+    if (n_new > 1 && is_dense && !ranges_meet(out, out_bytes, k_new, new_bytes) && !ranges_meet(out, out_bytes, v_new, new_bytes) && dtype == TROCM_F16 && kc->fmt == TROCM_F16 && vc->fmt == TROCM_F16 && q && k_new && v_new && out &&
         kc->window == 0 && vc->window == 0 && kc->B == vc->B && kc->H == vc->H && kc->D == vc->D && kc->len == vc->len && q_heads % kc->H == 0) {
         hipStream_t s;
         if (resolve_stream(stream, &s)) return 1;

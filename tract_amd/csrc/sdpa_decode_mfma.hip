@@ -86,8 +86,8 @@ struct MfmaWork {
     int *counter;                 // in-kernel merge by the last workgroup to arrive (dense batches, GP <= 8)
     int64_t part_first, part_stride;   // partial records of this sequence-head: first, first + stride, ...
     const char *mask;             // additive mask row of this kv head's first query head, token 0 (MASK instantiations)
-    int64_t row0;                 // ROWS instantiations: the first q / output row, and its place among its kv head's rows
-    int row_in_head0;
+    int64_t row0;                 // ROWS instantiations: the first q / output row, its place among its kv head's rows, how many
+    int row_in_head0, rows;
 };
 
 // The tail every formulation shares: the four waves' records (O[GP][D], m[GP], l[GP], in `lds_raw`, kCombStride floats
@@ -234,7 +234,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
     const int l16 = lane & 15, q4 = lane >> 4;
     const int hcol = W16 ? l16 : l32;   // the head (column of the score tile) of this lane
     const int kvh = wk.kvh, b = wk.seq;
-    const int g = p.g_real;
+    const int g = ROWS ? wk.rows : p.g_real;
     _Float16 *tile = reinterpret_cast<_Float16 *>(lds_raw + w * kTileBytes);
 
     static_assert(!ROWS || (!MASK && !ROPE), "several queries: no mask input, rotated before");
@@ -2110,8 +2110,8 @@ __global__ __launch_bounds__(kThreads, (QB ? QB % 10 : 2)) void sdpa_decode_mfma
 }
 
 // Several queries per sequence: grid (splits, kv_heads * row groups, batch).  Row r = head r / q_len, query r % q_len of a
-// kv head's G q_len rows (consecutive in q and in the output); group i takes g_real of them from i g_real on, the last
-// group the last g_real (rows of two groups are written twice, with the same bits).
+// kv head's G q_len rows (consecutive in q and in the output); group i takes up to g_real of them from i g_real on.  (Not one
+// of them twice: the output may lie over q, whose rows must not be read once another group has stored its results.)
 template <int D, int GP, int FMT, bool W16>
 __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_rows_kernel(DecodeDev p) {
     const int split = blockIdx.x, kvh = blockIdx.y / p.n_groups, group = blockIdx.y % p.n_groups, b = blockIdx.z;
@@ -2133,7 +2133,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_rows_kernel(DecodeDev
     wk.counter = p.counters ? p.counters + bh : nullptr;
     wk.part_first = bh * p.nsplit, wk.part_stride = 1;
     wk.mask = nullptr;
-    wk.row_in_head0 = min(group * p.g_real, p.n_rows - p.g_real);
+    wk.row_in_head0 = group * p.g_real, wk.rows = min(p.g_real, p.n_rows - wk.row_in_head0);
     wk.row0 = ((int64_t)b * p.Hkv + kvh) * p.n_rows + wk.row_in_head0;
     decode_mfma_body<D, GP, FMT, false, W16, false, true>(p, wk);
 }
@@ -2143,7 +2143,8 @@ template <int D, int GP>
 __global__ __launch_bounds__(D) void sdpa_decode_rows_merge_kernel(DecodeDev p) {
     const int kvh = blockIdx.x / p.n_groups, group = blockIdx.x % p.n_groups, b = blockIdx.y, r = blockIdx.z;
     const int64_t bh = (int64_t)b * gridDim.x + blockIdx.x;
-    const int64_t row = ((int64_t)b * p.Hkv + kvh) * p.n_rows + min(group * p.g_real, p.n_rows - p.g_real) + r;
+    if (group * p.g_real + r >= p.n_rows) return;
+    const int64_t row = ((int64_t)b * p.Hkv + kvh) * p.n_rows + group * p.g_real + r;
     merge_head<__half, D, GP>(p, bh * p.nsplit, 1, p.nsplit, r, reinterpret_cast<__half *>(p.out) + row * D, threadIdx.x);
 }
 
