@@ -208,6 +208,9 @@ __device__ __forceinline__ auto rope_piece128(const _Float16 *row, const char *c
     return rope_finish<N>(rope_load128<N>(row, cosr, sinr, f0));
 }
 
+// All bits of those halves of a pair that are infinite or NaN.
+__device__ __forceinline__ uint32_t not_finite(uint32_t pair) { return ((((pair & 0x7C007C00u) + 0x04000400u) & 0x80008000u) >> 15) * 0xFFFFu; }
+
 // ROWS: the columns are rows of several queries (launch_sdpa_decode_rows), each of which sees its own number of tokens.
 template <int D, int GP, int FMT, bool MASK = false, bool W16 = false, bool ROPE = false, bool ROWS = false>
 __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaWork &wk) {
@@ -448,6 +451,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
         }
         return (nsp * sr + sp + se) * kWaves + w;
     };
+    bool any_left_out = false;   // ROWS: a value of V was left out of a product
     int tn = advance(t);
     for (; t < tile_end; t = tn, tn = advance(tn)) {
         const int t0 = t * kTile;
@@ -576,61 +580,46 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
         }
         }
         // ---- V tile -> the same LDS tile (every K fragment has been consumed), next V into flight ------
+        // ROWS: a token that a row does not see must not reach its sum, and a weight of 0 times an infinity or a NaN would: in
+        // a tile with such tokens the product takes V's finite values only (one operation per two values finds out whether
+        // there are others), the others follow after the loop.
+        const bool edge = ROWS && t0 + kTile > t_all;
+        bool left_out = false;
+        half2_t probe = {(_Float16)0.0f, (_Float16)0.0f};   // NaN once one is not finite
+        const half2_t none = probe;
         if constexpr (QUANT) {
             stash_q(vpre, vsc, v_slot);
+            if (edge) {
+#pragma unroll
+                for (int j = 0; j < kTile * D / 8 / 64; j++) {
+                    const u32x4 x = *reinterpret_cast<const u32x4 *>(tile + (j * 64 + lane) / (D / 8) * VROW + (j * 64 + lane) % (D / 8) * 8);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) probe = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, (uint32_t)x[i]), none, probe);
+                }
+                left_out = __any(!(probe.x == none.x) || !(probe.y == none.y));
+            }
             if (more) fetch_q(vbase, wk.vsbase, tn, vpre, vsc);
         } else {
+            if (edge) {
+#pragma unroll
+                for (int j = 0; j < NLD; j++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) probe = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, (uint32_t)vpre[j][i]), none, probe);
+                left_out = __any(!(probe.x == none.x) || !(probe.y == none.y));
+            }
 #pragma unroll
             for (int j = 0; j < NLD; j++) *reinterpret_cast<u32x4 *>(tile + v_slot[j]) = vpre[j];
             if (more) fetch(vbase, p.v_new, tn, vpre);
         }
-        // ROWS: a token that a row does not see must not reach its sum, and a weight of 0 times an infinity or a NaN would: in
-        // a tile with such tokens the product takes V's finite values only, and the others (any positive weight leaves them as
-        // they are) are added to the rows that see them.  (Ordinary values: 4 to 8 LDS reads and their test in the last tiles.)
-        if constexpr (ROWS) {
-            if (t0 + kTile > t_all) {
-                constexpr int CH = kTile * D / 8 / 64;   // 16-byte chunks of the tile per lane
-                auto odd_halves = [](uint32_t x) { return ((x & 0x7C007C00u) + 0x04000400u) & 0x80008000u; };
-                uint32_t odd = 0;
-#pragma unroll
-                for (int j = 0; j < CH; j++) {
-                    const int c = j * 64 + lane;
-                    const u32x4 x = *reinterpret_cast<const u32x4 *>(tile + c / (D / 8) * VROW + c % (D / 8) * 8);
-                    odd |= odd_halves(x.x) | odd_halves(x.y) | odd_halves(x.z) | odd_halves(x.w);
-                }
-                if (__builtin_amdgcn_ballot_w64(odd != 0) != 0) {
-                    auto unless_finite = [](_Float16 x) { return __builtin_isfinite((float)x) ? 0.0f : (float)x; };
+        if (ROWS && __builtin_expect(left_out, 0)) {
+            any_left_out = true;
 #pragma unroll 1
-                    for (int kk = 0; kk < kTile; kk++) {
-                        const bool seen = t0 + kk < t_row;
-                        if constexpr (W16) {
+            for (int c = lane; c < kTile * D / 8; c += 64) {
+                u32x4 *at = reinterpret_cast<u32x4 *>(tile + c / (D / 8) * VROW + c % (D / 8) * 8);
+                u32x4 x = *at;
 #pragma unroll
-                            for (int fb = 0; fb < D / 16; fb++) {
-                                const half4_t x = *reinterpret_cast<const half4_t *>(tile + kk * VROW + 16 * fb + 4 * q4);
-#pragma unroll
-                                for (int i = 0; i < 4; i++) o16[fb][i] += seen ? unless_finite(x[i]) : 0.0f;
-                            }
-                        } else {
-#pragma unroll
-                            for (int db = 0; db < DB; db++)
-#pragma unroll
-                                for (int rq = 0; rq < 4; rq++) {
-                                    const half4_t x = *reinterpret_cast<const half4_t *>(tile + kk * VROW + 32 * db + 8 * rq + 4 * hb);
-#pragma unroll
-                                    for (int i = 0; i < 4; i++) o[db][4 * rq + i] += seen ? unless_finite(x[i]) : 0.0f;
-                                }
-                        }
-                    }
-#pragma unroll 1
-                    for (int j = 0; j < CH; j++) {
-                        const int c = j * 64 + lane;
-                        u32x4 *at = reinterpret_cast<u32x4 *>(tile + c / (D / 8) * VROW + c % (D / 8) * 8);
-                        u32x4 x = *at;
-#pragma unroll
-                        for (int i = 0; i < 4; i++) x[i] &= ~((odd_halves(x[i]) >> 15) * 0xFFFFu);
-                        *at = x;
-                    }
-                }
+                for (int i = 0; i < 4; i++) x[i] &= ~not_finite(x[i]);
+                *at = x;
             }
         }
         // ---- O^T += V^T P^T ---------------------------------------------------------------------------------
@@ -653,6 +642,45 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
                     const half8_t vf = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
                     o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[st], o[db], 0, 0, 0);
                 }
+        }
+    }
+    // ROWS: the values of V that were left out, whatever their weight, to the rows that see them
+    if constexpr (ROWS) {
+        if (__builtin_expect(any_left_out, 0)) {
+#pragma unroll 1
+            for (int te = tile_begin + w; te < tile_end; te += tstep) {
+                const int t0 = te * kTile;
+                if (t0 + kTile <= t_all) continue;
+                if constexpr (QUANT) {
+                    fetch_q(vbase, wk.vsbase, te, vpre, vsc);
+                    stash_q(vpre, vsc, v_slot);
+                } else {
+                    fetch(vbase, p.v_new, te, vpre);
+#pragma unroll
+                    for (int j = 0; j < NLD; j++) *reinterpret_cast<u32x4 *>(tile + v_slot[j]) = vpre[j];
+                }
+#pragma unroll 1
+                for (int kk = 0; kk < kTile; kk++) {
+                    const uint32_t seen = t0 + kk < t_row ? ~0u : 0u;
+                    if constexpr (W16) {
+#pragma unroll
+                        for (int fb = 0; fb < D / 16; fb++) {
+                            const uint2 x = *reinterpret_cast<const uint2 *>(tile + kk * VROW + 16 * fb + 4 * q4);
+                            const half2_t a = __builtin_bit_cast(half2_t, x.x & not_finite(x.x) & seen), b = __builtin_bit_cast(half2_t, x.y & not_finite(x.y) & seen);
+                            o16[fb] += float4_t{(float)a.x, (float)a.y, (float)b.x, (float)b.y};
+                        }
+                    } else {
+#pragma unroll
+                        for (int db = 0; db < DB; db++)
+#pragma unroll
+                            for (int rq = 0; rq < 4; rq++) {
+                                const uint2 x = *reinterpret_cast<const uint2 *>(tile + kk * VROW + 32 * db + 8 * rq + 4 * hb);
+                                const half2_t a = __builtin_bit_cast(half2_t, x.x & not_finite(x.x) & seen), b = __builtin_bit_cast(half2_t, x.y & not_finite(x.y) & seen);
+                                o[db][4 * rq] += (float)a.x, o[db][4 * rq + 1] += (float)a.y, o[db][4 * rq + 2] += (float)b.x, o[db][4 * rq + 3] += (float)b.y;
+                            }
+                    }
+                }
+            }
         }
     }
     if constexpr (W16) l_run += __shfl_xor(l_run, 16, 64);
