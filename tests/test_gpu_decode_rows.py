@@ -21,7 +21,7 @@ def _f16(rng, *shape):
 @pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [
     (1, 2, 1, 128, 0, 4), (1, 4, 4, 64, 27, 8), (2, 3, 1, 128, 31, 3), (1, 16, 2, 64, 29, 2), (2, 17, 1, 128, 300, 2),
     (1, 8, 2, 128, 1021, 8), (1, 11, 1, 128, 127, 3), (2, 14, 2, 64, 700, 5), (1, 7, 1, 128, 2000, 17), (1, 6, 2, 128, 255, 16),
-    (3, 4, 4, 128, 64, 33), (1, 5, 1, 64, 0, 64), (4, 32, 8, 128, 500, 8), (1, 32, 8, 128, 6000, 2)])
+    (3, 4, 4, 128, 64, 33), (16, 16, 8, 128, 600, 12), (1, 5, 1, 64, 0, 64), (4, 32, 8, 128, 500, 8), (1, 32, 8, 128, 6000, 2)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_rows_of_several_queries(rt, B, Hq, Hkv, D, past, n, causal):
     rng = np.random.default_rng(B + 10 * Hq + past + n)

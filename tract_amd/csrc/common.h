@@ -211,9 +211,12 @@ struct KiviSdpaArgs {
 int launch_sdpa_decode_kivi(const KiviSdpaArgs &a, hipStream_t s);
 // MFMA prefill.  Returns 2 when the shape is not covered.
 int launch_sdpa_prefill(const SdpaArgs &a, hipStream_t s);
+// A few f16 queries per sequence on the decode tiles (sdpa_decode_mfma.hip).  Returns 2 when not covered, or when
+// sdpa_decode_rows_fits says that the prefill kernels are faster.
+int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s);
+bool sdpa_decode_rows_fits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int kv_fmt);
 // MFMA prefill for q_len >= 32: staggered waves, GQA heads sharing K/V tiles, key splits across
 // workgroups (partials in the workspace after the counter area).  Returns 2 when not covered.
-int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s);   // a few queries per sequence (sdpa_decode_mfma.hip)
 int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s);
 // The same for f32 q, K and V (2..: any number of queries), on the f32 matrix instruction.  Returns 2 when not covered.
 int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s);

@@ -2558,6 +2558,44 @@ int launch_sdpa_decode_mfma(const SdpaArgs &a, hipStream_t s) {
     return a.D == 128 ? launch_d<128>(p, gp, grid, s) : launch_d<64>(p, gp, grid, s);
 }
 
+// Whether launch_sdpa_decode_rows is faster than the prefill kernels.  Figures: us for a call with its append, prefill kernel |
+// here, two layers in turn; BH counts workgroups per key range.
+//
+// Up to 16 rows per kv head: always.  One group of 17 to 32 rows reads K and V once, as the prefill kernel does that shares a
+// tile among `shared` heads of a group (sdpa_prefill_pp.hip: 4, 2 or 1); `reads` counts how often K and V are read here against
+// there.  What decides beyond that is whether workgroups of 32 rows fill the chip as well as its workgroups of 256.
+bool sdpa_decode_rows_fits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int kv_fmt) {
+    if (Sq < 2 || Sq > 64 || Hkv < 1 || Hq / Hkv > 1024) return false;
+    const int64_t G = Hq / Hkv, rows = G * Sq, n_groups = (rows + 31) / 32, BH = B * Hkv * n_groups, cus = num_compute_units();
+    if (rows <= 16) return true;
+    const int64_t shared = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
+    const bool fewer_reads = n_groups * shared < G, same_reads = n_groups * shared == G;
+    if (is_quant(kv_fmt)) {
+        if (n_groups > 4) return false;
+        // Odd groups are read per head there: 40 heads over 8, 1 x 850 tokens, 16 queries 29.4 | 34.2, 1 x 2000 46.7 | 33.7; 14 over 2,
+        // 8 x 500, 16 queries 43.9 | 36.9, 2 x 650 tokens 28.7 | 31.2, 4 x 850, 3 queries 40.1 | 32.2.
+        if (G % 2 && G > 1) return BH <= 64 && Sk >= (B * Hq >= 96 ? 512 : B * Hq >= 64 ? 600 : B * Hq >= 40 ? 800 : 1000);
+        // 64 heads over 8, 3 queries: 4 x 500 28.8 | 32.2, 4 x 650 32.1 | 31.3, 8 x 2000 66.2 | 45.0
+        if (fewer_reads) return Sk >= 512;
+        // 32 heads over 8, 8 queries: 1 x 500 tokens 28.1 | 31.9, 1 x 650 31.5 | 30.4; 8 x 650 33.2 | 38.7, 8 x 2000 46.6 | 47.1, 8 x 3000
+        // 56.5 | 54.8; 16 x 1200 48.7 | 47.9; 32 x 550 51.2 | 50.0.  32 over 32, 32 queries: 2 x 1300 34.0 | 39.0, 2 x 3000 58.8 | 58.7.
+        if (same_reads) return Sk >= (BH >= cus ? 550 : G % 4 ? 2048 : BH <= 32 ? 600 : BH >= 128 ? 1200 : 2048);
+        // 32 over 8, 16 queries: 2 x 2000 50.0 | 37.2; 4 x 2000 43.9 | 46.7, 8 x 2000 48.2 | 62.6
+        return BH <= 32 && Sk >= 1000;
+    }
+    // Odd groups (sdpa_prefill.hip, a workgroup per head and 64 queries): up to a workgroup per compute unit (24 heads over 8,
+    // 64 queries: 8 x 314 tokens 35.4 | 43.5 with 384, 4 x 1064 55.0 | 46.0 with 192; 32 over 32, 33 queries, 4 x 1033, 256: 65.0 |
+    // 54.5), as many as do not read more (40 over 8, 16 x 283, 33 queries 60.2 | 53.5), or two per compute unit where it
+    // needs a second round (24 over 8, 16 x 283, 33 queries 57.0 | 46.4).
+    if (G % 2) return n_groups == 1 || BH <= cus || 4 * n_groups <= 5 * G || (BH <= 2 * cus && B * Hq > cus);
+    // 16 heads over 8, 16 queries: 8 x 616 tokens 27.6 | 29.2, 8 x 400 26.4 | 25.9, 8 x 8000 114 | 98; 16 x 1516 48.7 | 52.1
+    if (n_groups == 1) return G != 2 || BH < 64 || Sk <= 512 || Sk >= 2560;
+    // 32 over 8: 22 queries 1 x 8000 tokens 52.2 | 42.2, 2 x 8000 62.4 | 81.0, 2 x 1500 41.7 | 33.4; 16 queries 4 x 3000 45.1 | 50.9.  16 over
+    // 8, 22 queries: 4 x 3000 40.1 | 50.4, 2 x 3000 38.0 | 31.3.  12 over 2, 10 queries, 10 x 8000: groups of 2 heads there.
+    if (n_groups > 4 || BH > 64) return false;
+    return fewer_reads || same_reads || BH <= 32 || Sk <= 512 || (G != 2 && (G % 4 || Sk <= 2560));
+}
+
 // A few queries per sequence (proposed tokens to verify, short chunks) over a cache: the rows of a kv head, its G heads
 // times q_len queries, are the columns of the decode tiles, in groups of up to 32.  Like a decode step it is bound by the
 // stream of K and V (one group) and the chain of a short launch; the prefill kernels stage whole tiles for 32 queries per
@@ -2581,17 +2619,7 @@ int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s) {
     const int gp = per <= 8 ? 8 : per <= 16 ? 16 : 32;
     if (a.Hkv * n_groups > 65535) return 2;
     const int64_t BH = a.B * a.Hkv * n_groups;
-    // One group reads K and V once: always (us with the append, prefill kernel | here: 32 heads over 8, 4 x 5000 tokens, 4
-    // queries 30.7 | 20.3, 8 queries 30.9 | 24.8; 1 x 229, 8 queries 13.1 | 12.6; Q4_0, 1 x 2000, 4 queries 24.1 | 15.1).  More
-    // groups read them again: against the prefill kernel that shares a tile among the heads of a group (an even G, and every
-    // quantised cache) while the launch is small (BH counts workgroups per split: 2 x 2000 tokens, 12 queries, BH 32 25.0 | 16.1;
-    // 4 x 5000, 64 31.2 | 30.5; 8 x 1000, 128 18.7 | 23.2); against the one that reads them per head up to 64 queries
-    // (14 heads over 2, 3 x 4000 tokens, 16 queries 88.8 | 25.0, 64 queries 90.0 | 34.4; 32 over 32, 48 queries 101.3 | 84.6,
-    // 100 queries 105.5 | 130.7).
-    if (n_groups > 1 && (quant || G % 2 == 0) && (n_groups > 4 || BH > 64)) return 2;
-    // (a short quantised cache and more than 16 rows: one staged tile of the prefill kernel, 14 heads over 2, 229 tokens, 6
-    // queries, Q4_0 13.6 | 14.1)
-    if (quant && gp == 32 && a.Sk < 512) return 2;
+    if (!sdpa_decode_rows_fits(a.B, a.Hq, a.Hkv, a.Sq, a.Sk, a.kv_fmt)) return 2;
     DecodeDev p;
     memset(&p, 0, sizeof(p));
     p.q = (const char *)a.q, p.out = (char *)a.out, p.k = (const char *)a.k, p.v = (const char *)a.v;
@@ -2615,13 +2643,16 @@ int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s) {
     p.scale_log2 = a.scale * 1.4426950408889634f;
     const int n_tiles = (int)((a.Sk + kTile - 1) / kTile);
     // A workgroup per compute unit, never a few more; two with several groups and more than 8 tiles per wave (40 heads over 8,
-    // 4 x 5000 tokens, 8 queries 38.7 -> 33.4 us).  Records of more than 8 rows are merged by a second launch, which up to
-    // two tiles per wave costs more than the split gives.
+    // 4 x 5000 tokens, 8 queries 38.7 -> 33.4 us), 32 where one range of keys fills the chip (32 over 32, 4 x 1064, 64 queries 83.0
+    // split, 58.5 not).  Records of more than 8 rows are merged by a second launch, the dearer the more of them there are:
+    // below these lengths it costs more than the split gives (us of two layers, split | not: BH 128, 10 tiles 38.5 | 27.3, 20 tiles
+    // 39.2 | 33.5, 33 tiles equal; BH 64, 9 tiles 26.9 | 23.2, 20 tiles equal; BH 32, 9 tiles 24.4 | 22.9, 16 tiles 26.5 | 29.5;
+    // quantised caches, whose waves take longer for a tile: BH 64, 16 tiles 27.1 | 28.9).
     int64_t resident = num_compute_units();
     int nsplit = choose_decode_splits(BH, gp, n_tiles, 1);
-    if (n_groups > 1 && n_tiles >= 32 * nsplit) nsplit = choose_decode_splits(BH, gp, n_tiles, 2), resident *= 2;
+    if (n_groups > 1 && n_tiles >= (nsplit == 1 ? 128 : 32 * nsplit)) nsplit = choose_decode_splits(BH, gp, n_tiles, 2), resident *= 2;
     if (nsplit > 1 && BH * nsplit > resident && resident >= BH) nsplit = (int)(resident / BH);
-    if (gp > 8 && n_tiles <= 2 * kWaves) nsplit = 1;
+    if (gp > 8 && nsplit > 1 && n_tiles <= 8 + (quant ? 16 : 48) / nsplit) nsplit = 1;
     p.nsplit = fit_decode_splits(nsplit, BH, gp, a.D, a.workspace, a.workspace_bytes);
     p.live_trim = decode_live_trim();
     p.part_ml = (float *)((char *)a.workspace + kWsCounterBytes);
