@@ -531,7 +531,7 @@ int launch_q4_0_tiled_export(const void *tiles, void *blocks, int64_t rows, int6
 
 // Tiled weights x activations for any m: f16 rows in groups of up to 16 (more than 16 rows go to the matrix-matrix
 // kernel first, which reads the same tiles, when it takes the call), up to 6 f32 rows (more go to q4_matmul_f32.hip; in
-// groups of 8 what that refuses).
+// groups of 8 what that refuses, and few rows of tall matrices).
 int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int64_t k, const void *act, int act_dtype,
                              int64_t act_batch, int64_t m, void *out, hipStream_t s) {
     if (n >= (1ll << 30) || k >= (1ll << 30) || act_batch > 65535) return fail("q4_0_matvec: shape too large");
@@ -551,9 +551,17 @@ int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int6
         const int rc = launch_q4_0_matmul(tiles, nullptr, w_batch, n, k, act, act_dtype, act_batch, m, out, s, 1);
         if (rc != 2) return rc;
     }
-    // f32 rows from 7 on: one pass over the weights for all of them (us, here | there, 6 rows and 7: 14336 x 4096 16.4 | 17.5
-    // and 18.2 | 17.6, 4096 x 4096 9.5 | 8.7 and 13.0 | 8.8, 4096 x 14336 31.2 | 24.8 and 34.4 | 25.1)
-    if (act_dtype == TROCM_F32 && m >= 7) {
+    // f32 rows from 7 on: one pass over the weights for all of them (us, here | there, 6 rows and 7: 4096 x 4096 9.5 | 8.7 and 13.0 |
+    // 8.8, 4096 x 14336 31.2 | 24.8 and 34.4 | 25.1).  Its workgroups of 16 activation rows take 16 or 32 weight rows each, one workgroup
+    // per compute unit: few rows of a tall matrix need several rounds of them, while a pass of 8 rows here streams the weights at
+    // the memory's rate.
+    // 7 and 8 rows: 32768 x 4096 27.6 | 40.3, 32768 x 128 4.8 | 7.2, 14336 x 4096 16.5 | 19.3, 14336 x 1024 7.0 | 6.4, 24576 x 4096 28.9 |
+    // 22.3; 12 rows, two passes: 128256 x 512 24.6 | 31.2, 128256 x 4096 165 | 153, 65536 x
+    // 2048 40.9 | 45.0, 65536 x 1024 23.6 | 24.1, 65536 x 128 12.9 | 13.7; 17 rows: 128256 x 128 26.0 | 28.1, 128256 x 512 48.0 | 32.2.
+    const bool stream = m <= 8 ? n > 24576 || (n > 12288 && n <= 16384 && k >= 2048)
+                      : m <= 16 ? n >= 57344 && k < 4096 && (n > 98304 || k < 256 || k >= 2048)
+                                : m <= 24 && n > 98304 && k < 256;
+    if (act_dtype == TROCM_F32 && m >= 7 && !stream) {
         const int rc = launch_q4_0_matmul_f32(tiles, nullptr, w_batch, n, k, act, act_batch, m, out, s, 1);
         if (rc != 2) return rc;
     }
