@@ -80,3 +80,24 @@ def test_sessions_that_reuse_their_prompt_buffers(rt):
     for i, s, got in outs:
         for g, w in zip(got, alone[i]):
             assert np.array_equal(g.to_numpy(s), w)
+
+
+# rows that start one and two elements past an aligned address: the same bits, and the step that needs no dequantised copy
+@pytest.mark.parametrize("off_k,off_v", [(1, 0), (0, 1), (2, 3), (1, 1)])
+def test_single_tokens_at_any_element(rt, off_k, off_v):
+    rng = np.random.default_rng(off_k + 10 * off_v)
+    B, Hq, Hkv = 2, 8, 2
+    data = [((rng.standard_normal((B, Hq, n, D)) / np.sqrt(D)).astype(np.float16), rng.standard_normal((B, Hkv, n, D)).astype(np.float16),
+             rng.standard_normal((B, Hkv, n, D)).astype(np.float16)) for n in (40, 1, 1, 1)]
+
+    def shifted(x, off):
+        t = tract_amd.DeviceTensor.from_numpy(np.concatenate([np.zeros(off, np.float16), x.reshape(-1)]))
+        return tract_amd.DeviceTensor(x.shape, np.float16, ptr=t.ptr.value + 2 * off, owner=t)
+
+    aligned, moved = tract_amd.QuantizedKvSdpa(axis=2).state(), tract_amd.QuantizedKvSdpa(axis=2).state()
+    for q, k, v in data:
+        step = k.shape[2] == 1
+        want = aligned.eval([q, k, v]).to_numpy()
+        got = moved.eval([tract_amd.DeviceTensor.from_numpy(q), shifted(k, off_k) if step else k, shifted(v, off_v) if step else v]).to_numpy()
+        np.testing.assert_array_equal(got, want)
+        _same(moved.k.state(), aligned.k.state()), _same(moved.v.state(), aligned.v.state())

@@ -1731,6 +1731,9 @@ __device__ __forceinline__ void decode_mfma_qdiag_body(const DecodeDev &p, const
 // with the token scales folded into the probabilities (one operand for the whole row) and the second term one scalar per
 // head, added to every feature after the loop.  Lane layout, LDS tiles and the combine are those of the block-scaling
 // body; wk.ksbase / wk.vsbase are the Values' per-token scale and lo rows (f32).
+// The new token's rows may start at any element (one load of the whole width all the same: unaligned access is on).
+typedef half2_t half2_any_t __attribute__((aligned(2)));
+typedef half8_t half8_any_t __attribute__((aligned(2)));
 template <int GP, int PF>
 __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const MfmaWork &wk) {
     static_assert(GP <= 16, "the 16-wide layout: at most 16 heads");
@@ -1770,7 +1773,7 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
     float new_scale = 0.0f, new_lo = 0.0f;   // of the new Value row
     if (owner) {
         const float2 lo2 = *reinterpret_cast<const float2 *>(p.chan_lo + chan0 + 2 * lane), sc2 = *reinterpret_cast<const float2 *>(p.chan_scale + chan0 + 2 * lane);
-        const half2_t k2 = *reinterpret_cast<const half2_t *>(p.k_new + (chan0 + 2 * lane) * 2), v2 = *reinterpret_cast<const half2_t *>(p.v_new + (chan0 + 2 * lane) * 2);
+        const half2_t k2 = *reinterpret_cast<const half2_any_t *>(p.k_new + (chan0 + 2 * lane) * 2), v2 = *reinterpret_cast<const half2_any_t *>(p.v_new + (chan0 + 2 * lane) * 2);
         float klo[2] = {lo2.x, lo2.y}, ks[2] = {sc2.x, sc2.y};
         uint32_t kc = 0, vc = 0;
 #pragma unroll
@@ -1853,7 +1856,7 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
     half8_t kn[NB];
 #pragma unroll
     for (int blk = 0; blk < NB; blk++) {
-        kn[blk] = *reinterpret_cast<const half8_t *>(p.k_new + (chan0 + 32 * blk + 8 * q4) * 2);
+        kn[blk] = *reinterpret_cast<const half8_any_t *>(p.k_new + (chan0 + 32 * blk + 8 * q4) * 2);
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             ksv[blk][h] = *reinterpret_cast<const float4_t *>(ksc + 32 * blk + 8 * q4 + 4 * h);
@@ -2449,7 +2452,7 @@ int launch_sdpa_decode_kivi(const KiviSdpaArgs &a, hipStream_t s) {
     if (gp == 0 || gp > 16) return 2;
     if (a.T <= 0 || a.T > (1ll << 30) || a.B > 65535 || a.Hkv > 65535 || !(a.scale > 0.0f)) return 2;
     if ((uintptr_t)a.q % 16 || (uintptr_t)a.k_codes % 16 || (uintptr_t)a.v_codes % 16 || (uintptr_t)a.k_chan_scale % 16 || (uintptr_t)a.k_chan_lo % 16) return 2;
-    if ((uintptr_t)a.k_new % 16 || (uintptr_t)a.v_new % 16 || (uintptr_t)a.k_chan_scale_next % 16 || (uintptr_t)a.k_chan_lo_next % 16) return 2;
+    if ((uintptr_t)a.k_new % 2 || (uintptr_t)a.v_new % 2 || (uintptr_t)a.k_chan_scale_next % 16 || (uintptr_t)a.k_chan_lo_next % 16) return 2;
     const int64_t BH = a.B * a.Hkv;
     const int n_tiles = (int)((a.T + kTile - 1) / kTile);
     int nsplit = fit_decode_splits(choose_decode_splits(BH, gp, n_tiles, 2), BH, gp, 128, a.workspace, a.workspace_bytes);
