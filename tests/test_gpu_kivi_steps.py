@@ -1,12 +1,15 @@
 """The affine u8 stores: single tokens coded by the attention launch, prompts in chunks of every length, prompt buffers that are
 handed out again.  Stored bytes and parameters against the oracle, bit for bit."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import tract_amd
 from oracle import oracle as orc
 from tests.gpu_util import rt  # noqa: F401
-from tract_amd import kivi
+from tract_amd import _lib, kivi
+from tract_amd._lib import call
 from tract_amd.runtime import Stream
 
 pytestmark = pytest.mark.gpu
@@ -101,3 +104,54 @@ def test_single_tokens_at_any_element(rt, off_k, off_v):
         got = moved.eval([tract_amd.DeviceTensor.from_numpy(q), shifted(k, off_k) if step else k, shifted(v, off_v) if step else v]).to_numpy()
         np.testing.assert_array_equal(got, want)
         _same(moved.k.state(), aligned.k.state()), _same(moved.v.state(), aligned.v.state())
+
+
+def test_a_recorded_step_replayed_in_later_sessions(rt):
+    """A step recorded into a graph, replayed after other prompts of the same length with numbers of single tokens in between
+    that are odd and even: every replay gives what the step gives in a new session."""
+    rng = np.random.default_rng(17)
+    B, Hq, Hkv, n = 2, 8, 2, 41
+
+    def tokens(m, scale=1.0):
+        return [(rng.standard_normal((B, h, m, D)) * s).astype(np.float16) for h, s in ((Hq, D ** -0.5), (Hkv, scale), (Hkv, scale))]
+
+    def eager(calls):
+        st = tract_amd.QuantizedKvSdpa(axis=2).state()
+        return [st.eval(c).to_numpy() for c in calls][-1]
+
+    hip, s, held = _lib.load(), Stream(), [tract_amd.DeviceTensor.from_numpy(t) for t in tokens(1)]
+    out = tract_amd.DeviceTensor((B, Hq, 1, D), np.float16)
+    st = tract_amd.QuantizedKvSdpa(axis=2).state()
+
+    def put(step):
+        for t, x in zip(held, step):
+            call("trocm_h2d", t.ptr, x.ctypes.data_as(C.c_void_p), t.nbytes, s.handle)
+            s.synchronize()
+
+    def check(rc):
+        assert rc == 0, rc
+
+    def on_device(step):
+        return [tract_amd.DeviceTensor.from_numpy(t, s) for t in step]
+
+    graph, runnable = C.c_void_p(), C.c_void_p()
+    for session, more in enumerate((0, 1, 2, 3)):
+        scale = 4.0 ** -session   # (ranges of an earlier session would give other codes)
+        prompt, first, step = tokens(n, scale), tokens(1, scale), tokens(1, scale)
+        if session:
+            for _ in range(more):
+                st.eval(on_device(tokens(1, 30.0)), stream=s)
+            st.k.reset(stream=s), st.v.reset(stream=s)
+        for c in (prompt, first):
+            st.eval(on_device(c), stream=s)
+        put(step)
+        if session == 0:
+            check(hip.hipStreamBeginCapture(s.handle, 2))
+            st.eval(held, stream=s, out=out)
+            check(hip.hipStreamEndCapture(s.handle, C.byref(graph)))
+            check(hip.hipGraphInstantiate(C.byref(runnable), graph, None, None, C.c_size_t(0)))
+        for _ in range(2):   # (the same token again: the same row and parameters)
+            check(hip.hipGraphLaunch(runnable, s.handle))
+            np.testing.assert_array_equal(out.to_numpy(s), eager([prompt, first, step]))
+    check(hip.hipGraphExecDestroy(runnable))
+    check(hip.hipGraphDestroy(graph))

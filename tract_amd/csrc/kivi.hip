@@ -24,7 +24,6 @@
 #include <hip/hip_fp16.h>
 #include <new>
 #include <type_traits>
-#include <utility>
 #include "common.h"
 #include "affine.h"
 
@@ -216,15 +215,21 @@ __global__ void __launch_bounds__(256) kivi_finalize_blocks_kernel(const SrcT *_
     }
 }
 
+// The running parameters [BH, D] that a push starts from and those it leaves (the same memory, or the other set).
+struct RunSets {
+    const float *lo, *scale;
+    float *lo_next, *scale_next;
+};
+
 // Keys with running parameters, a thread per (head row, channel), tokens in order (QuantKeyCache::push_token):
 // lo follows the minimum, scale only grows, each token is coded under the parameters current at its push.
 template <typename SrcT>
 __global__ void kivi_running_push_kernel(const SrcT *__restrict__ src, int64_t S, int n, int D, uint8_t *__restrict__ codes,
-                                         int64_t cap_rows, int64_t row0, float *__restrict__ lo_io, float *__restrict__ scale_io) {
+                                         int64_t cap_rows, int64_t row0, RunSets sets) {
     const int bh = blockIdx.y;
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= D) return;
-    float lo = lo_io[(int64_t)bh * D + c], scale = scale_io[(int64_t)bh * D + c];
+    float lo = sets.lo[(int64_t)bh * D + c], scale = sets.scale[(int64_t)bh * D + c];
     for (int t = 0; t < n; t++) {
         const float val = ld(src + ((int64_t)bh * S + t) * D + c);
         if (val < lo) lo = val;
@@ -235,8 +240,8 @@ __global__ void kivi_running_push_kernel(const SrcT *__restrict__ src, int64_t S
         }
         codes[((int64_t)bh * cap_rows + row0 + t) * D + c] = (uint8_t)affine_code(val, lo, scale, 255.0f);
     }
-    lo_io[(int64_t)bh * D + c] = lo;
-    scale_io[(int64_t)bh * D + c] = scale;
+    sets.lo_next[(int64_t)bh * D + c] = lo;
+    sets.scale_next[(int64_t)bh * D + c] = scale;
 }
 
 // The same push for a long run of tokens (a prompt), in chunks of kRunChunk tokens that are scanned side by side.
@@ -266,10 +271,10 @@ __global__ void kivi_run_chunk_min_kernel(const SrcT *__restrict__ src, int64_t 
 }
 // scan 1: lo at the start of every chunk (in place), and the final lo into the store.  Sixteen chunk results are
 // requested together: one dependent load per chunk made this a chain of memory latencies (32 us for 128 chunks).
-__global__ void kivi_run_scan_min_kernel(float *__restrict__ cmin, int D, int n_chunks, float *__restrict__ lo_io) {
+__global__ void kivi_run_scan_min_kernel(float *__restrict__ cmin, int D, int n_chunks, RunSets sets) {
     const int bh = blockIdx.y, c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= D) return;
-    float lo = lo_io[(int64_t)bh * D + c];
+    float lo = sets.lo[(int64_t)bh * D + c];
     float *col = cmin + (int64_t)bh * n_chunks * D + c;
     for (int k0 = 0; k0 < n_chunks; k0 += 16) {
         float m[16];
@@ -281,7 +286,7 @@ __global__ void kivi_run_scan_min_kernel(float *__restrict__ cmin, int D, int n_
             if (m[i] < lo) lo = m[i];
         }
     }
-    lo_io[(int64_t)bh * D + c] = lo;
+    sets.lo_next[(int64_t)bh * D + c] = lo;
 }
 // pass 2: the largest scale candidate of each chunk and channel (0 when no token of the chunk has a positive range)
 template <typename SrcT>
@@ -303,10 +308,10 @@ __global__ void kivi_run_chunk_scale_kernel(const SrcT *__restrict__ src, int64_
     cmax[((int64_t)bh * n_chunks + k) * D + c] = best;
 }
 // scan 2: scale at the start of every chunk (in place), and the final scale into the store
-__global__ void kivi_run_scan_scale_kernel(float *__restrict__ cmax, int D, int n_chunks, float *__restrict__ scale_io) {
+__global__ void kivi_run_scan_scale_kernel(float *__restrict__ cmax, int D, int n_chunks, RunSets sets) {
     const int bh = blockIdx.y, c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= D) return;
-    float scale = scale_io[(int64_t)bh * D + c];
+    float scale = sets.scale[(int64_t)bh * D + c];
     float *col = cmax + (int64_t)bh * n_chunks * D + c;
     for (int k0 = 0; k0 < n_chunks; k0 += 16) {
         float m[16];
@@ -318,7 +323,7 @@ __global__ void kivi_run_scan_scale_kernel(float *__restrict__ cmax, int D, int 
             if (m[i] > scale) scale = m[i];
         }
     }
-    scale_io[(int64_t)bh * D + c] = scale;
+    sets.scale_next[(int64_t)bh * D + c] = scale;
 }
 // The 128-bit path makes one pass for both scans.  Per chunk and channel it leaves the first minimal value (`cmin`), the
 // largest value (`cmax`) and the widest range against the chunk's own running minimum (`cown`).  A token's range is
@@ -328,11 +333,11 @@ __global__ void kivi_run_scan_scale_kernel(float *__restrict__ cmax, int D, int 
 // start come out of one walk over the chunks.  NaN values take part in nothing (every comparison with them is false),
 // exactly as in the token-by-token loop.  In place: cmin becomes the chunk's starting lo, cmax its starting scale.
 __global__ void kivi_run_scan_both_kernel(float *__restrict__ cmin, float *__restrict__ cmax, const float *__restrict__ cown, int D,
-                                          int n_chunks, float *__restrict__ lo_io, float *__restrict__ scale_io) {
+                                          int n_chunks, RunSets sets) {
     const int bh = blockIdx.y, c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= D) return;
-    float lo = lo_io[(int64_t)bh * D + c];
-    const float scale0 = scale_io[(int64_t)bh * D + c];
+    float lo = sets.lo[(int64_t)bh * D + c];
+    const float scale0 = sets.scale[(int64_t)bh * D + c];
     // The walk carries the widest RANGE so far, not the scale: the quotient by 255 grows with the range, so the largest
     // quotient is the quotient of the widest range, and the divisions (one per chunk, for the scale its tokens start
     // from) stay off the chain from chunk to chunk, which is a subtraction and two comparisons.  Sixteen chunks'
@@ -387,9 +392,9 @@ __global__ void kivi_run_scan_both_kernel(float *__restrict__ cmin, float *__res
         step(cmin[at], cmax[at], cown[at], lo_in, w_in);
         cmin[at] = lo_in, cmax[at] = start_scale(w_in);
     }
-    lo_io[(int64_t)bh * D + c] = lo;
+    sets.lo_next[(int64_t)bh * D + c] = lo;
     const float ns = widest > 0.0f ? __fdiv_rn(widest, 255.0f) : 0.0f;
-    scale_io[(int64_t)bh * D + c] = ns > scale0 ? ns : scale0;
+    sets.scale_next[(int64_t)bh * D + c] = ns > scale0 ? ns : scale0;
 }
 // pass 3: the codes, every chunk starting from its own parameters
 template <typename SrcT>
@@ -673,14 +678,14 @@ __global__ void __launch_bounds__(256) kivi_quant_tokens_vec_kernel(const SrcT *
 template <typename SrcT>
 __global__ void __launch_bounds__(128) kivi_step_push_kernel(const SrcT *__restrict__ k_src, const SrcT *__restrict__ v_src,
                                                              uint8_t *__restrict__ k_codes, int64_t k_cap_rows, int64_t k_row0,
-                                                             float *__restrict__ k_lo_io, float *__restrict__ k_scale_io,
+                                                             RunSets sets,
                                                              uint8_t *__restrict__ v_codes, int64_t v_cap_rows, int64_t v_row0,
                                                              float *__restrict__ v_lo_out, float *__restrict__ v_scale_out) {
     constexpr int D = 128;
     const int bh = blockIdx.x;
     if (blockIdx.y == 0) {
         const int c = threadIdx.x;
-        float lo = k_lo_io[(int64_t)bh * D + c], scale = k_scale_io[(int64_t)bh * D + c];
+        float lo = sets.lo[(int64_t)bh * D + c], scale = sets.scale[(int64_t)bh * D + c];
         const float val = ld(k_src + (int64_t)bh * D + c);
         if (val < lo) lo = val;
         const float range = __fsub_rn(val, lo);
@@ -689,8 +694,8 @@ __global__ void __launch_bounds__(128) kivi_step_push_kernel(const SrcT *__restr
             if (ns > scale) scale = ns;
         }
         k_codes[((int64_t)bh * k_cap_rows + k_row0) * D + c] = (uint8_t)affine_code(val, lo, scale, 255.0f);
-        k_lo_io[(int64_t)bh * D + c] = lo;
-        k_scale_io[(int64_t)bh * D + c] = scale;
+        sets.lo_next[(int64_t)bh * D + c] = lo;
+        sets.scale_next[(int64_t)bh * D + c] = scale;
     } else {
         const int sub = threadIdx.x;
         if (sub >= 16) return;   // (the exchanges below stay inside the first 16 lanes)
@@ -893,12 +898,28 @@ struct trocm_kivi_cache {
     int64_t len = 0, n_sink = 0, n_rows = 0, n_res = 0, cap_rows = 0;
     float *sink = nullptr, *residual = nullptr, *lo = nullptr, *scale = nullptr;
     uint8_t *codes = nullptr;
-    float *running = nullptr, *lo_next = nullptr, *scale_next = nullptr;   // per-channel layout: the allocation behind lo and scale; the other set
+    // Running layout: two sets of (lo, scale), so that a decode step need not write the one that it reads.  Which of them is the
+    // current one follows from the number of coded rows (kivi_run_sets): a launch recorded into a graph finds its parameters whenever
+    // the store holds as many as when it was recorded, whatever came in between.
+    float *running = nullptr;
     void *deq = nullptr;      // dequantised copy handed to attention by trocm_quantized_kv_sdpa_eval
     size_t deq_bytes = 0;
     float *scan = nullptr;    // chunk results of a prompt pushed into the running Key store (kept for the next prompt)
     size_t scan_bytes = 0;
 };
+
+// The set that a push of `rows` coded rows starts from, and the one that it leaves.
+static RunSets kivi_run_sets(const trocm_kivi_cache *c, int64_t rows) {
+    const int64_t n = c->BH * c->D;
+    float *from = c->running + (c->n_rows & 1) * 2 * n, *to = c->running + ((c->n_rows + rows) & 1) * 2 * n;
+    return RunSets{from, from + n, to, to + n};
+}
+// After every change of the number of coded rows: lo and scale are the current set.
+static void kivi_select_set(trocm_kivi_cache *c) {
+    if (!c->running) return;
+    const RunSets r = kivi_run_sets(c, 0);
+    c->lo = r.lo_next, c->scale = r.scale_next;
+}
 
 static int64_t param_pitch(const trocm_kivi_cache *c, int64_t cap_rows) {
     switch (c->layout) {
@@ -953,9 +974,9 @@ static int kivi_alloc_fixed(trocm_kivi_cache *c, hipStream_t s) {
         kivi_malloc((void **)&c->residual, (size_t)c->BH * kKeyBlock * c->D * 4, "the partial key block"))
         return 1;
     if (c->layout == TROCM_KIVI_RUNNING_CHANNEL && !c->lo) {
-        const int64_t n = c->BH * c->D;   // two sets, and a decode step reads one and writes the other
+        const int64_t n = c->BH * c->D;
         if (kivi_malloc((void **)&c->running, (size_t)n * 4 * 4, "running key parameters")) return 1;
-        c->lo = c->running, c->scale = c->running + n, c->lo_next = c->running + 2 * n, c->scale_next = c->running + 3 * n;
+        kivi_select_set(c);
         kivi_fill_running_kernel<<<dim3((unsigned)((n + 255) / 256)), 256, 0, s>>>(c->lo, c->scale, n);
         TROCM_HIP(hipGetLastError());
     }
@@ -1115,6 +1136,7 @@ static int kivi_append_t(trocm_kivi_cache *c, const SrcT *src, int64_t S, hipStr
             c->n_res += rem;
         }
     } else if (rem > 0) {
+        const RunSets sets = kivi_run_sets(c, rem);
         const bool vec = ((uintptr_t)(src + t0 * D) & 15) == 0 && (D == 64 || D == 128 || D == 256 || D == 512);
         const int chunk = vec ? kivi_vec_chunk(rem) : kRunChunk;
         const int64_t n_chunks = (rem + chunk - 1) / chunk;
@@ -1127,7 +1149,7 @@ static int kivi_append_t(trocm_kivi_cache *c, const SrcT *src, int64_t S, hipStr
     do {                                                                                                                               \
         const dim3 vgrid((unsigned)((n_chunks + 256 / LPR - 1) / (256 / LPR)), BH);                                                    \
         kivi_run_chunk_vec_kernel<SrcT, LPR, 12><<<vgrid, 256, 0, s>>>(from, S, (int)rem, (int)n_chunks, tmp, tmp + plane, c->codes, c->cap_rows, c->n_rows, chunk, tmp + 2 * plane); \
-        kivi_run_scan_both_kernel<<<scan, 64, 0, s>>>(tmp, tmp + plane, tmp + 2 * plane, D, (int)n_chunks, c->lo, c->scale);         \
+        kivi_run_scan_both_kernel<<<scan, 64, 0, s>>>(tmp, tmp + plane, tmp + 2 * plane, D, (int)n_chunks, sets);         \
         kivi_run_chunk_vec_kernel<SrcT, LPR, 3><<<vgrid, 256, 0, s>>>(from, S, (int)rem, (int)n_chunks, tmp, tmp + plane, c->codes, c->cap_rows, c->n_rows, chunk); \
     } while (0)
             if (vec) {
@@ -1135,18 +1157,19 @@ static int kivi_append_t(trocm_kivi_cache *c, const SrcT *src, int64_t S, hipStr
             } else {
                 const dim3 grid((unsigned)((D + 63) / 64), (unsigned)n_chunks, BH);
                 kivi_run_chunk_min_kernel<SrcT><<<grid, 64, 0, s>>>(from, S, (int)rem, D, (int)n_chunks, tmp);
-                kivi_run_scan_min_kernel<<<scan, 64, 0, s>>>(tmp, D, (int)n_chunks, c->lo);
+                kivi_run_scan_min_kernel<<<scan, 64, 0, s>>>(tmp, D, (int)n_chunks, sets);
                 kivi_run_chunk_scale_kernel<SrcT><<<grid, 64, 0, s>>>(from, S, (int)rem, D, (int)n_chunks, tmp, tmp + plane);
-                kivi_run_scan_scale_kernel<<<scan, 64, 0, s>>>(tmp + plane, D, (int)n_chunks, c->scale);
+                kivi_run_scan_scale_kernel<<<scan, 64, 0, s>>>(tmp + plane, D, (int)n_chunks, sets);
                 kivi_run_chunk_codes_kernel<SrcT><<<grid, 64, 0, s>>>(from, S, (int)rem, D, (int)n_chunks, tmp, tmp + plane, c->codes, c->cap_rows, c->n_rows);
             }
 #undef KIVI_RUN_VEC
             TROCM_HIP(hipGetLastError());
         } else {
-            kivi_running_push_kernel<SrcT><<<dim3((unsigned)((D + 127) / 128), BH), 128, 0, s>>>(src + t0 * D, S, (int)rem, D, c->codes, c->cap_rows, c->n_rows, c->lo, c->scale);
+            kivi_running_push_kernel<SrcT><<<dim3((unsigned)((D + 127) / 128), BH), 128, 0, s>>>(src + t0 * D, S, (int)rem, D, c->codes, c->cap_rows, c->n_rows, sets);
             TROCM_HIP(hipGetLastError());
         }
         c->n_rows += rem;
+        kivi_select_set(c);
     }
     c->len += S;
     return 0;
@@ -1250,6 +1273,7 @@ int trocm_kivi_cache_reset(trocm_kivi_cache *c, void *stream) {
     hipStream_t s;
     if (resolve_stream(stream, &s)) return 1;
     c->len = c->n_sink = c->n_rows = c->n_res = 0;
+    kivi_select_set(c);
     if (c->layout == TROCM_KIVI_RUNNING_CHANNEL && c->lo) {
         const int64_t n = c->BH * c->D;
         kivi_fill_running_kernel<<<dim3((unsigned)((n + 255) / 256)), 256, 0, s>>>(c->lo, c->scale, n);
@@ -1340,6 +1364,7 @@ int trocm_kivi_cache_clone(const trocm_kivi_cache *c, trocm_kivi_cache **out, vo
         n->n_sink = c->n_sink;
         n->n_rows = c->n_rows;
         n->n_res = c->n_res;
+        kivi_select_set(n);
         if (!rc && c->n_sink) rc = copy_rows(n->sink, c->sink_tokens * c->D * 4, c->sink, c->sink_tokens * c->D * 4, c->n_sink * c->D * 4, c->BH, s);
         if (!rc && c->n_res) rc = copy_rows(n->residual, (int64_t)kKeyBlock * c->D * 4, c->residual, (int64_t)kKeyBlock * c->D * 4, c->n_res * c->D * 4, c->BH, s);
         if (!rc && c->n_rows) rc = copy_rows(n->codes, n->cap_rows * c->row_bytes, c->codes, c->cap_rows * c->row_bytes, c->n_rows * c->row_bytes, c->BH, s);
@@ -1405,8 +1430,9 @@ int trocm_quantized_kv_sdpa_eval(const void *q, const void *k_new, const void *v
         a.q = q, a.out = out;
         a.k_codes = k_cache->codes, a.v_codes = v_cache->codes;
         a.k_cap_rows = k_cache->cap_rows, a.v_cap_rows = v_cache->cap_rows;
-        a.k_chan_lo = k_cache->lo, a.k_chan_scale = k_cache->scale;
-        a.k_chan_lo_next = k_cache->lo_next, a.k_chan_scale_next = k_cache->scale_next;
+        const RunSets sets = kivi_run_sets(k_cache, 1);
+        a.k_chan_lo = sets.lo, a.k_chan_scale = sets.scale;
+        a.k_chan_lo_next = sets.lo_next, a.k_chan_scale_next = sets.scale_next;
         a.v_tok_scale = v_cache->scale, a.v_tok_lo = v_cache->lo;
         a.k_new = k_new, a.v_new = v_new;
         a.B = k_cache->B, a.Hq = q_heads, a.Hkv = k_cache->H, a.T = k_cache->len + 1;
@@ -1414,9 +1440,9 @@ int trocm_quantized_kv_sdpa_eval(const void *q, const void *k_new, const void *v
         a.workspace = workspace, a.workspace_bytes = workspace_bytes;
         const int rc = launch_sdpa_decode_kivi(a, s);
         if (rc == 0) {
-            std::swap(k_cache->lo, k_cache->lo_next), std::swap(k_cache->scale, k_cache->scale_next);
             for (trocm_kivi_cache *c : {k_cache, v_cache}) {
                 c->n_rows += 1, c->len += 1;
+                kivi_select_set(c);
                 if (c->deq) {
                     if (defer_device_free(c->deq, nullptr, s, c->deq_bytes)) return 1;
                     c->deq = nullptr;
@@ -1436,14 +1462,15 @@ int trocm_quantized_kv_sdpa_eval(const void *q, const void *k_new, const void *v
         k_cache->bits == 8 && v_cache->bits == 8 && k_cache->sink_tokens == 0 && v_cache->sink_tokens == 0 &&
         ((uintptr_t)v_new & 15) == 0 && (k_cache->len + 1) * 128 < (1ll << 31)) {
         const dim3 grid((unsigned)k_cache->BH, 2);
+        const RunSets sets = kivi_run_sets(k_cache, 1);
         if (dtype == TROCM_F16)
             kivi_step_push_kernel<__half><<<grid, 128, 0, s>>>((const __half *)k_new, (const __half *)v_new, k_cache->codes, k_cache->cap_rows, k_cache->n_rows,
-                                                               k_cache->lo, k_cache->scale, v_cache->codes, v_cache->cap_rows, v_cache->n_rows, v_cache->lo, v_cache->scale);
+                                                               sets, v_cache->codes, v_cache->cap_rows, v_cache->n_rows, v_cache->lo, v_cache->scale);
         else
             kivi_step_push_kernel<float><<<grid, 128, 0, s>>>((const float *)k_new, (const float *)v_new, k_cache->codes, k_cache->cap_rows, k_cache->n_rows,
-                                                              k_cache->lo, k_cache->scale, v_cache->codes, v_cache->cap_rows, v_cache->n_rows, v_cache->lo, v_cache->scale);
+                                                              sets, v_cache->codes, v_cache->cap_rows, v_cache->n_rows, v_cache->lo, v_cache->scale);
         TROCM_HIP(hipGetLastError());
-        for (trocm_kivi_cache *c : {k_cache, v_cache}) c->n_rows += 1, c->len += 1;
+        for (trocm_kivi_cache *c : {k_cache, v_cache}) c->n_rows += 1, c->len += 1, kivi_select_set(c);
     } else {
         if (trocm_kivi_cache_append(k_cache, k_new, dtype, n_new, s)) return 1;
         if (trocm_kivi_cache_append(v_cache, v_new, dtype, n_new, s)) return 1;
