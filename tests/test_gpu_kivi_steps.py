@@ -155,3 +155,23 @@ def test_a_recorded_step_replayed_in_later_sessions(rt):
             np.testing.assert_array_equal(out.to_numpy(s), eager([prompt, first, step]))
     check(hip.hipGraphExecDestroy(runnable))
     check(hip.hipGraphDestroy(graph))
+
+
+@pytest.mark.parametrize("over", ["k", "v"])
+def test_a_step_stored_over_its_own_new_rows(rt, over):
+    """More workgroups than run at once, so that some read their rows after others have stored results."""
+    rng = np.random.default_rng(23)
+    B, Hq, Hkv = 192, 32, 8
+    data = [tuple((rng.standard_normal((B, h, n, D)) * c).astype(np.float16) for h, c in ((Hq, D ** -0.5), (Hkv, 1), (Hkv, 1))) for n in (33, 1, 1)]
+    apart, shared = tract_amd.QuantizedKvSdpa(axis=2).state(), tract_amd.QuantizedKvSdpa(axis=2).state()
+    for q, k, v in data:
+        want = apart.eval([q, k, v]).to_numpy()
+        args = {name: tract_amd.DeviceTensor.from_numpy(t) for name, t in (("q", q), ("k", k), ("v", v))}
+        out = tract_amd.DeviceTensor(q.shape, np.float16)
+        if k.shape[2] == 1:
+            whole = np.zeros(q.size, np.float16)
+            whole[: k.size] = (k if over == "k" else v).reshape(-1)
+            out = tract_amd.DeviceTensor.from_numpy(whole.reshape(q.shape))
+            args[over] = tract_amd.DeviceTensor(k.shape, np.float16, ptr=out.ptr, owner=out)
+        np.testing.assert_array_equal(shared.eval([args["q"], args["k"], args["v"]], out=out).to_numpy(), want)
+        _same(shared.k.state(), apart.k.state()), _same(shared.v.state(), apart.v.state())

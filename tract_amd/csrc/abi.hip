@@ -1324,11 +1324,6 @@ static int inplace_eval_check(const char *what, const void *q, const void *k_new
     return 0;
 }
 
-// Whether `n` bytes at a and `m` bytes at b have memory in common.
-static bool ranges_meet(const void *a, size_t n, const void *b, size_t m) {
-    return (uintptr_t)a < (uintptr_t)b + m && (uintptr_t)b < (uintptr_t)a + n;
-}
-
 int trocm_inplace_kv_sdpa_eval(const void *q, const void *k_new, const void *v_new, int dtype, int64_t q_heads,
                                int64_t n_new, const int64_t *kv_new_strides, trocm_kv_cache *kc, trocm_kv_cache *vc,
                                void *out, float scale, int causal, void *workspace, size_t workspace_bytes,

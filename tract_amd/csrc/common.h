@@ -74,6 +74,10 @@ struct AppendPair {
     int64_t dst_stride[3];
 };
 int launch_append_pair(const AppendPair &a, hipStream_t s);
+// Whether `n` bytes at a and `m` bytes at b have memory in common.
+inline bool ranges_meet(const void *a, size_t n, const void *b, size_t m) {
+    return (uintptr_t)a < (uintptr_t)b + m && (uintptr_t)b < (uintptr_t)a + n;
+}
 // Device memory that work queued on `s` may still read: released by a later call, once an event recorded on `s` now has
 // completed (abi.hip).  reap_device_frees(wait) releases what has completed (wait: everything).
 // With its size, `a` may be handed out again before that (reuse_device_free).
@@ -202,7 +206,7 @@ struct KiviSdpaArgs {
     const float *k_chan_lo, *k_chan_scale;         // [B * Hkv, 128]; the launch writes what the new token makes of them
     float *k_chan_lo_next, *k_chan_scale_next;     // to these
     const float *v_tok_scale, *v_tok_lo;           // [B * Hkv, v_cap_rows]
-    const void *k_new, *v_new;                     // the last of the T tokens, f16 [B * Hkv, 128]: coded and stored by the launch
+    const void *k_new, *v_new;                     // the last of the T tokens, f16 [B * Hkv, 128]: coded and stored by the launch (NULL: it is stored)
     int64_t B, Hq, Hkv, T;
     float scale;
     void *workspace;

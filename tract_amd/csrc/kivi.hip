@@ -1421,28 +1421,53 @@ int trocm_quantized_kv_sdpa_eval(const void *q, const void *k_new, const void *v
         for (trocm_kivi_cache *c : {k_cache, v_cache})
             if (kivi_grow_buffer(&c->deq, &c->deq_bytes, need, s, "the dequantised copy of a quantised store")) return 1;
     }
+    // Pushes the call's rows; a decode step on the op's own stores: both by one launch.
+    auto push = [&]() -> int {
+        if (n_new == 1 && k_cache->D == 128 && k_cache->layout == TROCM_KIVI_RUNNING_CHANNEL && v_cache->layout == TROCM_KIVI_PER_TOKEN &&
+            k_cache->bits == 8 && v_cache->bits == 8 && k_cache->sink_tokens == 0 && v_cache->sink_tokens == 0 &&
+            ((uintptr_t)v_new & 15) == 0 && (k_cache->len + 1) * 128 < (1ll << 31)) {
+            const dim3 grid((unsigned)k_cache->BH, 2);
+            const RunSets sets = kivi_run_sets(k_cache, 1);
+            if (dtype == TROCM_F16)
+                kivi_step_push_kernel<__half><<<grid, 128, 0, s>>>((const __half *)k_new, (const __half *)v_new, k_cache->codes, k_cache->cap_rows, k_cache->n_rows,
+                                                                   sets, v_cache->codes, v_cache->cap_rows, v_cache->n_rows, v_cache->lo, v_cache->scale);
+            else
+                kivi_step_push_kernel<float><<<grid, 128, 0, s>>>((const float *)k_new, (const float *)v_new, k_cache->codes, k_cache->cap_rows, k_cache->n_rows,
+                                                                  sets, v_cache->codes, v_cache->cap_rows, v_cache->n_rows, v_cache->lo, v_cache->scale);
+            TROCM_HIP(hipGetLastError());
+            for (trocm_kivi_cache *c : {k_cache, v_cache}) c->n_rows += 1, c->len += 1, kivi_select_set(c);
+            return 0;
+        }
+        return trocm_kivi_cache_append(k_cache, k_new, dtype, n_new, s) || trocm_kivi_cache_append(v_cache, v_new, dtype, n_new, s);
+    };
     // A decode step of f16 queries: the attention launch codes the new token itself and writes its row and the Keys' new
     // parameters, the latter into the set that it does not read (a prompt of 2 x 1500 tokens and 16 steps, 32 heads over 8: 390.0 us with a
-    // launch for each push, 368.5 without).  The dequantised copies a prompt left behind are not needed again: released
+    // launch for each push, 368.5 without).  Pushed ahead of it where the output lies over the new rows: one workgroup stores
+    // results while another still reads them.  The dequantised copies a prompt left behind are not needed again: released
     // behind an event.
+    bool pushed = false;
     if (fused_attention && workspace) {
+        const size_t new_bytes = (size_t)k_cache->BH * 128 * 2, out_bytes = (size_t)k_cache->B * q_heads * 128 * 2;
+        if (ranges_meet(out, out_bytes, k_new, new_bytes) || ranges_meet(out, out_bytes, v_new, new_bytes)) {
+            if (push()) return 1;
+            pushed = true;
+        }
         KiviSdpaArgs a;
         a.q = q, a.out = out;
         a.k_codes = k_cache->codes, a.v_codes = v_cache->codes;
         a.k_cap_rows = k_cache->cap_rows, a.v_cap_rows = v_cache->cap_rows;
-        const RunSets sets = kivi_run_sets(k_cache, 1);
+        const RunSets sets = kivi_run_sets(k_cache, pushed ? 0 : 1);
         a.k_chan_lo = sets.lo, a.k_chan_scale = sets.scale;
         a.k_chan_lo_next = sets.lo_next, a.k_chan_scale_next = sets.scale_next;
         a.v_tok_scale = v_cache->scale, a.v_tok_lo = v_cache->lo;
-        a.k_new = k_new, a.v_new = v_new;
-        a.B = k_cache->B, a.Hq = q_heads, a.Hkv = k_cache->H, a.T = k_cache->len + 1;
+        a.k_new = pushed ? nullptr : k_new, a.v_new = pushed ? nullptr : v_new;
+        a.B = k_cache->B, a.Hq = q_heads, a.Hkv = k_cache->H, a.T = k_cache->len + (pushed ? 0 : 1);
         a.scale = scale == scale ? scale : 1.0f / sqrtf((float)k_cache->D);   // NaN asks for the default (sdpa.rs:93-95)
         a.workspace = workspace, a.workspace_bytes = workspace_bytes;
         const int rc = launch_sdpa_decode_kivi(a, s);
         if (rc == 0) {
             for (trocm_kivi_cache *c : {k_cache, v_cache}) {
-                c->n_rows += 1, c->len += 1;
-                kivi_select_set(c);
+                if (!pushed) c->n_rows += 1, c->len += 1, kivi_select_set(c);
                 if (c->deq) {
                     if (defer_device_free(c->deq, nullptr, s, c->deq_bytes)) return 1;
                     c->deq = nullptr;
@@ -1453,28 +1478,11 @@ int trocm_quantized_kv_sdpa_eval(const void *q, const void *k_new, const void *v
         }
         if (rc != 2) return rc;
         // (the launch declined: the dequantising path needs its buffers after all)
-        const size_t need = (size_t)k_cache->BH * (k_cache->len + 1) * k_cache->D * elem_bytes(dtype);
+        const size_t need = (size_t)k_cache->BH * (k_cache->len + (pushed ? 0 : 1)) * k_cache->D * elem_bytes(dtype);
         for (trocm_kivi_cache *c : {k_cache, v_cache})
             if (kivi_grow_buffer(&c->deq, &c->deq_bytes, need, s, "the dequantised copy of a quantised store")) return 1;
     }
-    // a decode step on the op's own stores: both rows pushed by one launch
-    if (n_new == 1 && k_cache->D == 128 && k_cache->layout == TROCM_KIVI_RUNNING_CHANNEL && v_cache->layout == TROCM_KIVI_PER_TOKEN &&
-        k_cache->bits == 8 && v_cache->bits == 8 && k_cache->sink_tokens == 0 && v_cache->sink_tokens == 0 &&
-        ((uintptr_t)v_new & 15) == 0 && (k_cache->len + 1) * 128 < (1ll << 31)) {
-        const dim3 grid((unsigned)k_cache->BH, 2);
-        const RunSets sets = kivi_run_sets(k_cache, 1);
-        if (dtype == TROCM_F16)
-            kivi_step_push_kernel<__half><<<grid, 128, 0, s>>>((const __half *)k_new, (const __half *)v_new, k_cache->codes, k_cache->cap_rows, k_cache->n_rows,
-                                                               sets, v_cache->codes, v_cache->cap_rows, v_cache->n_rows, v_cache->lo, v_cache->scale);
-        else
-            kivi_step_push_kernel<float><<<grid, 128, 0, s>>>((const float *)k_new, (const float *)v_new, k_cache->codes, k_cache->cap_rows, k_cache->n_rows,
-                                                              sets, v_cache->codes, v_cache->cap_rows, v_cache->n_rows, v_cache->lo, v_cache->scale);
-        TROCM_HIP(hipGetLastError());
-        for (trocm_kivi_cache *c : {k_cache, v_cache}) c->n_rows += 1, c->len += 1, kivi_select_set(c);
-    } else {
-        if (trocm_kivi_cache_append(k_cache, k_new, dtype, n_new, s)) return 1;
-        if (trocm_kivi_cache_append(v_cache, v_new, dtype, n_new, s)) return 1;
-    }
+    if (!pushed && push()) return 1;
     const int64_t T = k_cache->len, D = k_cache->D;
     for (trocm_kivi_cache *c : {k_cache, v_cache})
         if (kivi_dequantize(c, c->deq, dtype, s, false)) return 1;

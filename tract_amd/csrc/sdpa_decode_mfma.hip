@@ -1766,10 +1766,10 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
     // lanes 0..31 carry the scale of token `lane` of a tile, lanes 32..63 the lo of token `lane - 32`
     const float *par_row = reinterpret_cast<const float *>(lane < kTile ? wk.ksbase : wk.vsbase);
     const int64_t chan0 = ((int64_t)b * p.Hkv + kvh) * D;
-    // The step's new token, the last of the sequence: coded by the wave whose tiles include it, as kivi_step_push_kernel
-    // would, into `lds_new` (no other wave reads it), its row in the planes and the Keys' next parameters.
-    const int new_pos = wk.new_pos;
-    const bool owner = tile_begin + w <= new_pos / kTile && new_pos / kTile < tile_end && (new_pos / kTile - tile_begin - w) % wk.tile_step == 0;
+    // The step's new token (if it is not stored yet), the last of the sequence: coded by the wave whose tiles include it, as
+    // kivi_step_push_kernel would, into `lds_new` (no other wave reads it), its row in the planes and the Keys' next parameters.
+    const int new_pos = wk.new_pos, stored = new_pos >= 0 ? T - 1 : T;
+    const bool owner = new_pos >= 0 && tile_begin + w <= new_pos / kTile && new_pos / kTile < tile_end && (new_pos / kTile - tile_begin - w) % wk.tile_step == 0;
     float new_scale = 0.0f, new_lo = 0.0f;   // of the new Value row
     if (owner) {
         const float2 lo2 = *reinterpret_cast<const float2 *>(p.chan_lo + chan0 + 2 * lane), sc2 = *reinterpret_cast<const float2 *>(p.chan_scale + chan0 + 2 * lane);
@@ -1808,16 +1808,16 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
     auto fetch = [&](int t, u32x4 (&kd)[NLD], u32x4 (&vd)[NLD], float &par) {
         const int t0 = t * kTile;
         const char *kb = wk.kbase + (int64_t)t0 * RB, *vb = wk.vbase + (int64_t)t0 * RB;
-        if (t0 + kTile < T) {
+        if (t0 + kTile <= stored) {
 #pragma unroll
             for (int j = 0; j < NLD; j++) {
                 kd[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(kb + (j * 64 + lane) * 16));
                 vd[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(vb + (j * 64 + lane) * 16));
             }
             par = par_row[t0 + (lane & (kTile - 1))];
-        } else {   // the tile of the new token: rows from it on repeat the one before (row 0 of the tile if there is none) and
-                   // are replaced, or masked, below
-            const int last = max(T - 2 - t0, 0);
+        } else {   // the last tile: rows from the end, or the new token, on repeat the one before (row 0 of the tile if there
+                   // is none) and are replaced, or masked, below
+            const int last = max(stored - 1 - t0, 0);
 #pragma unroll
             for (int j = 0; j < NLD; j++) {
                 const int c = j * 64 + lane, row = min(c / CPR, last), dc = c % CPR;
@@ -1856,32 +1856,34 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
     half8_t kn[NB];
 #pragma unroll
     for (int blk = 0; blk < NB; blk++) {
-        kn[blk] = *reinterpret_cast<const half8_any_t *>(p.k_new + (chan0 + 32 * blk + 8 * q4) * 2);
+        if (new_pos >= 0) kn[blk] = *reinterpret_cast<const half8_any_t *>(p.k_new + (chan0 + 32 * blk + 8 * q4) * 2);
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             ksv[blk][h] = *reinterpret_cast<const float4_t *>(ksc + 32 * blk + 8 * q4 + 4 * h);
             lov[blk][h] = *reinterpret_cast<const float4_t *>(p.chan_lo + chan0 + 32 * blk + 8 * q4 + 4 * h);
         }
     }
-    uint64_t wider = 0;   // (of the wave, joined as they come: a condition per channel and lane takes more scalar registers than there are)
-#pragma unroll
-    for (int blk = 0; blk < NB; blk++)
-#pragma unroll
-        for (int i = 0; i < 8; i++) {   // lov becomes the range
-            const float val = (float)kn[blk][i], lo = lov[blk][i >> 2][i & 3];
-            const float range = __fsub_rn(val, val < lo ? val : lo);
-            lov[blk][i >> 2][i & 3] = range;
-            wider |= __builtin_amdgcn_ballot_w64(range > ksv[blk][i >> 2][i & 3] * 254.9f);
-        }
-    if (wider != 0) {
+    if (new_pos >= 0) {
+        uint64_t wider = 0;   // (of the wave, joined as they come: a condition per channel and lane takes more scalar registers than there are)
 #pragma unroll
         for (int blk = 0; blk < NB; blk++)
 #pragma unroll
-            for (int i = 0; i < 8; i++)
-                if (lov[blk][i >> 2][i & 3] > 0.0f) {
-                    const float ns = __fdiv_rn(lov[blk][i >> 2][i & 3], 255.0f);
-                    if (ns > ksv[blk][i >> 2][i & 3]) ksv[blk][i >> 2][i & 3] = ns;
-                }
+            for (int i = 0; i < 8; i++) {   // lov becomes the range
+                const float val = (float)kn[blk][i], lo = lov[blk][i >> 2][i & 3];
+                const float range = __fsub_rn(val, val < lo ? val : lo);
+                lov[blk][i >> 2][i & 3] = range;
+                wider |= __builtin_amdgcn_ballot_w64(range > ksv[blk][i >> 2][i & 3] * 254.9f);
+            }
+        if (wider != 0) {
+#pragma unroll
+            for (int blk = 0; blk < NB; blk++)
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    if (lov[blk][i >> 2][i & 3] > 0.0f) {
+                        const float ns = __fdiv_rn(lov[blk][i >> 2][i & 3], 255.0f);
+                        if (ns > ksv[blk][i >> 2][i & 3]) ksv[blk][i >> 2][i & 3] = ns;
+                    }
+        }
     }
 #pragma unroll
     for (int blk = 0; blk < NB; blk++) {
