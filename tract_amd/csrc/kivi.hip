@@ -1466,14 +1466,14 @@ int trocm_quantized_kv_sdpa_eval(const void *q, const void *k_new, const void *v
         a.workspace = workspace, a.workspace_bytes = workspace_bytes;
         const int rc = launch_sdpa_decode_kivi(a, s);
         if (rc == 0) {
-            for (trocm_kivi_cache *c : {k_cache, v_cache}) {
-                if (!pushed) c->n_rows += 1, c->len += 1, kivi_select_set(c);
+            if (!pushed)   // (both counts before anything that can fail: the stores stay level)
+                for (trocm_kivi_cache *c : {k_cache, v_cache}) c->n_rows += 1, c->len += 1, kivi_select_set(c);
+            for (trocm_kivi_cache *c : {k_cache, v_cache})
                 if (c->deq) {
                     if (defer_device_free(c->deq, nullptr, s, c->deq_bytes)) return 1;
                     c->deq = nullptr;
                     c->deq_bytes = 0;
                 }
-            }
             return 0;
         }
         if (rc != 2) return rc;
