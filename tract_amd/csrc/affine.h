@@ -1,6 +1,7 @@
 // Affine codes as the quantised caches of the reference form them (quant_dyn_kv_cache.rs:118-192; kv_quant.rs:105-236): shared by
-// the stores' own kernels and the attention launch that takes a step's new token.  Every operation that rounds is an intrinsic:
-// nothing here depends on contraction.
+// the stores' own kernels and the attention launch that takes a step's new token.  The codes are the same in every file that
+// includes this, whether it is compiled with contraction or without: __fadd_rn and its like are plain operators here, so the
+// functions turn contraction off themselves.
 #pragma once
 #include <hip/hip_fp16.h>
 #include "common.h"
@@ -54,17 +55,20 @@ __device__ __forceinline__ void group_min_max(float &lo, float &hi) {
 // nearest even, so an exact half ties up to the integer and anything less stays below it; exact for every float,
 // checked exhaustively on the host for the exponents where it matters; inf and NaN pass through).
 __device__ __forceinline__ float round_half_away(float x) {
+#pragma clang fp contract(off)
     return truncf(__fadd_rn(x, __builtin_copysignf(0.49999997f, x)));
 }
 
 // ((x - lo) / scale).round().clamp(0.0, lv) as u8   (quant_dyn_kv_cache.rs:128, :190; kv_quant.rs:110, :219)
 __device__ __forceinline__ uint32_t affine_code(float x, float lo, float scale, float lv) {
+#pragma clang fp contract(off)
     float q = round_half_away(__fdiv_rn(__fsub_rn(x, lo), scale));
     if (!(q == q)) return 0;            // clamp keeps NaN, the cast turns it into 0
     q = q < 0.0f ? 0.0f : (q > lv ? lv : q);
     return (uint32_t)q;
 }
 __device__ __forceinline__ float affine_scale(float lo, float hi, float lv) {   // :127, :186
+#pragma clang fp contract(off)
     return hi > lo ? __fdiv_rn(__fsub_rn(hi, lo), lv) : 1.0f;
 }
 

@@ -1772,6 +1772,7 @@ __device__ __forceinline__ void decode_mfma_kivi_body(const DecodeDev &p, const 
     const bool owner = new_pos >= 0 && tile_begin + w <= new_pos / kTile && new_pos / kTile < tile_end && (new_pos / kTile - tile_begin - w) % wk.tile_step == 0;
     float new_scale = 0.0f, new_lo = 0.0f;   // of the new Value row
     if (owner) {
+#pragma clang fp contract(off)
         const float2 lo2 = *reinterpret_cast<const float2 *>(p.chan_lo + chan0 + 2 * lane), sc2 = *reinterpret_cast<const float2 *>(p.chan_scale + chan0 + 2 * lane);
         const half2_t k2 = *reinterpret_cast<const half2_any_t *>(p.k_new + (chan0 + 2 * lane) * 2), v2 = *reinterpret_cast<const half2_any_t *>(p.v_new + (chan0 + 2 * lane) * 2);
         float klo[2] = {lo2.x, lo2.y}, ks[2] = {sc2.x, sc2.y};
