@@ -158,6 +158,28 @@ def test_f32_rows_with_infinities_and_huge_values(rt, m, n, k):
     assert rel_err(got[fine], want[fine].astype(np.float64)) <= 1e-5
 
 
+# planes: rows of every magnitude down to subnormal numbers, next to ordinary ones, rows of zeros, values of both kinds in one row
+@pytest.mark.parametrize("m,n,k", [(9, 40, 96), (16, 273, 1152), (40, 4110, 256), (150, 2063, 1024)])
+def test_f32_rows_of_tiny_values_keep_their_bits(rt, m, n, k):
+    rng = np.random.default_rng(m)
+    blocks = orc.quant(Q4, (rng.standard_normal((1, n, k)) * 0.05).astype(np.float32))
+    act = rng.standard_normal((1, m, k)).astype(np.float32)
+    act[0, 1] *= np.float32(1e-33)
+    act[0, 2] *= np.float32(1e-36)
+    act[0, 3] = np.float32(3) * np.float32(1e-38) * act[0, 3]
+    act[0, 4] = 0.0
+    act[0, 5, : k // 2] *= np.float32(1e-36)
+    act[0, 6:, 64:] *= np.float32(1e-30)
+    got = tract_amd.GgmlGemm().eval(act, tract_amd.Q40Weights(blocks, 1, n, k)).to_numpy().astype(np.float64)
+    want = f64_product(blocks, act, np.float32)
+    # one after the other in f32: products and sums round by 2^-24 each, k / 8 of them per wave and 15 beyond; subnormal
+    # results by 2^-150 each
+    wd = np.abs(orc.dequant(Q4, blocks, np.float32).astype(np.float64))
+    bound = np.einsum("bmk,bnk->bmn", np.abs(act.astype(np.float64)), wd) * (k / 4 + 15) * 2.0 ** -24 + k * 2.0 ** -149
+    assert np.all(np.abs(got - want) <= bound)
+    assert np.linalg.norm((got - want)[0, 2]) <= 1e-6 * np.linalg.norm(want[0, 2])
+
+
 def test_tiles_and_planes_hold_the_same_weights(rt, monkeypatch):
     """The same matrix as tiles and (TROCM_Q4_TILED=0 at creation) as planes of codes and scales: equal exports, and
     products that agree to the tolerance of either."""

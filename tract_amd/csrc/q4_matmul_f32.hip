@@ -3,10 +3,12 @@
 //   out[b, i, j] = sum_k act[b, i, k] * dequant(W[b / ratio, j, k]),   f32 activations and results
 //
 // The f32 side of the matrix-matrix arm of GgmlGemm (cuda/src/kernels/matmul/mod.rs:605-610).  Arithmetic: an activation is
-// the exact sum of three bf16 numbers of 8 significant bits (x = b1 + b2 + b3 by truncation and exact remainders), a code
-// - 8 is one bf16 number, so every product of v_mfma_f32_*_bf16 is exact and its sums are f32.  A quantisation block
-// (32 features) is summed from zero, smallest part first, its f16 scale multiplies the block's sum, and the blocks are
-// added in f32.
+// the sum of three bf16 numbers of 8 significant bits (x = b1 + b2 + b3 by truncation and exact remainders; exact from 2^-110
+// on, below that within 2^-133), a code - 8 is one bf16 number, so every product of v_mfma_f32_*_bf16 is exact and its sums are
+// f32.  A quantisation block (32 features) is summed from zero, smallest part first, its f16 scale multiplies the block's sum,
+// and the blocks are added in f32.  Blocks with values that have no such three parts (`kBig` and more, infinities) are done in
+// f32; planes' blocks also where a lane's values are so small that 2^-133 counts among them (tiled weights are split the same way
+// by the kernel for few rows, q4_tiled.hip; the test costs 2 % of 150 rows of 4096 x 4096).
 //
 // A workgroup of 8 waves owns SUB MS (activation rows) x SUB NI (weight rows) of the result.  Its waves share k, not the
 // tile: wave w takes units (4 blocks, a record of tiled weights) w, w + 8, ..  Both operands then go from memory straight
@@ -37,7 +39,8 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kW = 8;          // waves per workgroup
 constexpr int kTile = 1152;    // bytes of a record of tiled weights (q4_tiled.hip)
-constexpr float kBig = 0x1p118f;   // from here on a block's unscaled sum could overflow: such blocks are done in f32
+constexpr float kBig = 0x1p118f;     // from here on a block's unscaled sum could overflow
+constexpr float kSmall = 0x1p-100f;  // from here on what the split loses, 2^-133, is less than 2^-32 of the largest value
 
 struct MatMulF32 {
     const uint8_t *codes;     // planes: [w_batch, n, k/2]; tiles: [w_batch, n / 16, k / 128] records
@@ -173,8 +176,14 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
     // result register r of a lane: activation row SUB i + out_row(r) of the workgroup's, weight row SUB j + lane % SUB
     auto out_row = [&](int r) { return SUB == 32 ? 8 * (r / 4) + 4 * grp + r % 4 : 4 * grp + r; };
 
-    // A block with values so large that its unscaled sum could overflow, or with infinities, whose remainders are no
-    // numbers: products with the dequantised weights, one after the other.
+    // Whether a block is one of those, by the largest magnitude among a lane's 8 values of each of its activation rows.
+    auto needs_f32 = [](const float (&big)[MS]) {
+        bool any = false;
+#pragma unroll
+        for (int i = 0; i < MS; i++) any = any || big[i] >= kBig || (!TILED && big[i] < kSmall && big[i] > 0.0f);
+        return __any(any);
+    };
+    // Products with the dequantised weights, one after the other.
     auto slow_block = [&](int blk) {
         const float *act = p.act + (int64_t)b * p.m * p.k + blk * 32;
 #pragma unroll 1
@@ -227,7 +236,9 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
             }
             __builtin_amdgcn_sched_barrier(0);   // (a block's fragments live only as long as the block)
             bf16x8_t part[3][MS][KST];   // the smallest first
-            float big = 0.0f;
+            float big[MS];
+#pragma unroll
+            for (int i = 0; i < MS; i++) big[i] = 0.0f;
 #pragma unroll
             for (int i = 0; i < MS; i++)
 #pragma unroll
@@ -236,7 +247,7 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
                         const float x0 = cur.x[i][st][e >> 1][2 * (e & 1)], x1 = cur.x[i][st][e >> 1][2 * (e & 1) + 1];
-                        big = fmaxf(fmaxf(fabsf(x0), fabsf(x1)), big);
+                        big[i] = fmaxf(fmaxf(fabsf(x0), fabsf(x1)), big[i]);
                         const float r0 = rest(x0), r1 = rest(x1);
                         b1[e] = upper2(x0, x1), b2[e] = upper2(r0, r1), b3[e] = upper2(rest(r0), rest(r1));
                     }
@@ -244,7 +255,7 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
                     part[1][i][st] = __builtin_bit_cast(bf16x8_t, b2);
                     part[2][i][st] = __builtin_bit_cast(bf16x8_t, b1);
                 }
-            if (__any(big >= kBig)) {   // after the loop
+            if (needs_f32(big)) {   // after the loop
                 skipped = true;
                 continue;
             }
@@ -276,15 +287,17 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
     if (skipped) {
         for (u = w; u < units; u += kW)
             for (int blk = 4 * u; blk < min(4 * u + 4, nb); blk++) {
-                float big = 0.0f;
+                float big[MS];
                 load_a(cur, blk);
+#pragma unroll
+                for (int i = 0; i < MS; i++) big[i] = 0.0f;
 #pragma unroll
                 for (int i = 0; i < MS; i++)
 #pragma unroll
                     for (int st = 0; st < KST; st++)
 #pragma unroll
-                        for (int e = 0; e < 8; e++) big = fmaxf(big, fabsf(cur.x[i][st][e >> 2][e & 3]));
-                if (__any(big >= kBig)) slow_block(blk);
+                        for (int e = 0; e < 8; e++) big[i] = fmaxf(big[i], fabsf(cur.x[i][st][e >> 2][e & 3]));
+                if (needs_f32(big)) slow_block(blk);
             }
     }
 
