@@ -175,3 +175,45 @@ def test_a_step_stored_over_its_own_new_rows(rt, over):
             args[over] = tract_amd.DeviceTensor(k.shape, np.float16, ptr=out.ptr, owner=out)
         np.testing.assert_array_equal(shared.eval([args["q"], args["k"], args["v"]], out=out).to_numpy(), want)
         _same(shared.k.state(), apart.k.state()), _same(shared.v.state(), apart.v.state())
+
+
+def test_a_recorded_prompt_keeps_its_copies(rt):
+    """A prompt and a step recorded together: the step hands the prompt's dequantised copies back, and they stay the graph's
+    whatever is released or allocated between its replays."""
+    rng = np.random.default_rng(29)
+    B, Hq, Hkv, n = 1, 8, 2, 70
+
+    def tokens(m):
+        return [(rng.standard_normal((B, h, m, D)) * c).astype(np.float16) for h, c in ((Hq, D ** -0.5), (Hkv, 1), (Hkv, 1))]
+
+    hip, s = _lib.load(), Stream()
+    calls = [tokens(n), tokens(1)]
+    alone = tract_amd.QuantizedKvSdpa(axis=2).state()
+    want = [alone.eval(c).to_numpy() for c in calls]
+    held = [[tract_amd.DeviceTensor.from_numpy(t) for t in c] for c in calls]
+    outs = [tract_amd.DeviceTensor(c[0].shape, np.float16) for c in calls]
+    st = tract_amd.QuantizedKvSdpa(axis=2).state()
+    for c in calls:   # (rows, workspace and scratch are there; the copies go to the list and are released)
+        st.eval([tract_amd.DeviceTensor.from_numpy(t) for t in c], stream=s)
+    s.synchronize()
+    call("trocm_release_unused", 1)
+    st.k.reset(stream=s), st.v.reset(stream=s)
+    s.synchronize()
+    graph, runnable = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(s.handle, 2) == 0
+    for c, out in zip(held, outs):
+        st.eval(c, stream=s, out=out)
+    assert hip.hipStreamEndCapture(s.handle, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(runnable), graph, None, None, C.c_size_t(0)) == 0
+    others = []
+    for _ in range(3):
+        others.append(tract_amd.QuantizedKvSdpa(axis=2).state())
+        for c, w in zip(calls, want):
+            np.testing.assert_array_equal(others[-1].eval([tract_amd.DeviceTensor.from_numpy(t) for t in c], stream=s).to_numpy(s), w)
+        call("trocm_release_unused", 1)
+        st.k.reset(stream=s), st.v.reset(stream=s)   # (a replay is a session from the start)
+        assert hip.hipGraphLaunch(runnable, s.handle) == 0
+        for out, w in zip(outs, want):
+            np.testing.assert_array_equal(out.to_numpy(s), w)
+    assert hip.hipGraphExecDestroy(runnable) == 0
+    assert hip.hipGraphDestroy(graph) == 0

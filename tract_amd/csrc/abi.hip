@@ -213,7 +213,9 @@ static bool stream_is_capturing(hipStream_t s) {
 // Hand the planes over to the deferred list, guarded by an event recorded on `s` now.
 static int defer_free(trocm_kv_pool *pool, void *data, void *scales, hipStream_t s, size_t bytes = 0) {
     if (!data && !scales) return 0;
-    if (bytes && stream_is_capturing(s)) bytes = 0;   // (a graph may read it again whenever it is replayed)
+    // What is handed over while `s` is being recorded, the graph uses again whenever it is replayed: it is never released.  (An
+    // event recorded there is part of the graph: asked once the recording has ended, it answers that all is done.)
+    if (stream_is_capturing(s)) return 0;
     DeferredFree d{data, scales, pool, nullptr, bytes, s};
     hipError_t e = hipEventCreateWithFlags(&d.done, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventRecord(d.done, s);
