@@ -1,5 +1,7 @@
 """A few queries per sequence as columns of the decode tiles, new tokens read from the call's input and stored by the attention
 launch, against a float64 restatement and the bytes that were appended."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -7,6 +9,7 @@ import tract_amd as ta
 from oracle import oracle as orc
 from tests.cases import textbook_sdpa
 from tests.gpu_util import rt  # noqa: F401
+from tract_amd._lib import call
 
 pytestmark = pytest.mark.gpu
 
@@ -151,3 +154,30 @@ def test_rows_stored_over_the_calls_own_inputs(rt, over, B, Hq, Hkv, past, n):
         results.append(st.eval_into(args["q"], args["k"], args["v"], out).to_numpy())
         assert st.k.valid_contiguous().tobytes() == k.tobytes() and st.v.valid_contiguous().tobytes() == v.tobytes()
     np.testing.assert_array_equal(results[1], results[0])
+
+
+# no scratch, counters only, room for two ranges of keys, what the library asks for; K and V as [batch, token, head, feature]
+# with 8 elements between rows; 8, 16 and 32 rows per kv head in f16, 20 f32 rows
+@pytest.mark.parametrize("dtype,Hq,n", [(np.float16, 4, 4), (np.float16, 8, 4), (np.float16, 8, 8), (np.float16, 6, 23), (np.float32, 8, 5)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_scratch_limits_and_strided_rows(rt, dtype, Hq, n, causal):
+    rng = np.random.default_rng(n)
+    B, Hkv, D, T, pad = 2, 2, 128, 2600, 8
+    q = (rng.standard_normal((B, Hq, n, D)) / np.sqrt(D)).astype(dtype)
+    kv = rng.standard_normal((2, B, T, Hkv * D + pad)).astype(dtype)
+    k, v = (x[:, :, : Hkv * D].reshape(B, T, Hkv, D).transpose(0, 2, 1, 3) for x in kv)
+    want = textbook_sdpa(q, k, v, causal=causal)
+    dq, dk, dv = (ta.DeviceTensor.from_numpy(t) for t in (q, kv[0], kv[1]))
+    row = Hkv * D + pad
+    strides = (C.c_int64 * 3)(T * row, D, row)
+    full = ta.Workspace(B, Hq, n, D)
+    counters = 64 * 1024
+    two = counters + 256 + 2 * B * Hkv * -(-Hq // Hkv * n // 32) * 32 * (D + 4) * 4
+    for size in (0, counters, min(two, full.nbytes), full.nbytes):
+        out = ta.DeviceTensor.from_numpy(np.full(q.shape, 7, dtype))
+        call("trocm_sdpa", dq.ptr, dk.ptr, dv.ptr, None, out.ptr, ta.F16 if dtype == np.float16 else ta.F32, B, Hq, Hkv, n, T, D, strides, 1, 1,
+             C.c_float(float("nan")), int(causal), full.ptr if size else None, size, None)
+        got = out.to_numpy().astype(np.float64)
+        # f16: as above; f32: sums of D products and 2600 weights, 2^-24 of the score in the exponent
+        tol = 2 * 2.0 ** -11 * np.abs(v.astype(np.float64)).max() if dtype == np.float16 else 2e-5 * np.abs(want).max()
+        assert np.abs(got - want).max() <= tol, size
