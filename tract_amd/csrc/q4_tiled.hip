@@ -555,10 +555,10 @@ int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int6
     // 8.8, 4096 x 14336 31.2 | 24.8 and 34.4 | 25.1).  Its workgroups of 16 activation rows take 16 or 32 weight rows each, one workgroup
     // per compute unit: few rows of a tall matrix need several rounds of them, while a pass of 8 rows here streams the weights at
     // the memory's rate.
-    // 7 and 8 rows: 32768 x 4096 27.6 | 40.3, 32768 x 128 4.8 | 7.2, 14336 x 4096 16.5 | 19.3, 14336 x 1024 7.0 | 6.4, 24576 x 4096 28.9 |
-    // 22.3; 12 rows, two passes: 128256 x 512 24.6 | 31.2, 128256 x 4096 165 | 153, 65536 x
+    // 7 and 8 rows: 32768 x 4096 27.6 | 40.3, 32768 x 128 4.8 | 7.2, 24576 x 4096 28.9 | 22.3, 14336 x 1024 7.0 | 6.4 (14336 x 4096
+    // 16.5 | 19.3 goes there for its smaller error against 64 bits, 1.5e-7 | 9.9e-8); 12 rows, two passes: 128256 x 512 24.6 | 31.2, 128256 x 4096 165 | 153, 65536 x
     // 2048 40.9 | 45.0, 65536 x 1024 23.6 | 24.1, 65536 x 128 12.9 | 13.7; 17 rows: 128256 x 128 26.0 | 28.1, 128256 x 512 48.0 | 32.2.
-    const bool stream = m <= 8 ? n > 24576 || (n > 12288 && n <= 16384 && k >= 2048)
+    const bool stream = m <= 8 ? n > 24576
                       : m <= 16 ? n >= 57344 && k < 4096 && (n > 98304 || k < 256 || k >= 2048)
                                 : m <= 24 && n > 98304 && k < 256;
     if (act_dtype == TROCM_F32 && m >= 7 && !stream) {
