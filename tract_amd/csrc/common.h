@@ -141,7 +141,8 @@ int launch_q4_0_matvec_mfma(const void *codes, const void *scales, int64_t w_bat
 // tiled: `codes` are tiles of 16 rows x 128 features (q4_tiled.hip), `scales` is unused.
 int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, int64_t n, int64_t k, const void *act,
                        int act_dtype, int64_t act_batch, int64_t m, void *out, hipStream_t s, int tiled = 0);
-// The same for f32 activations (q4_matmul_f32.hip; faster than the kernels above from 7 rows on).  Returns 2 when not covered.
+// The same for f32 activations (q4_matmul_f32.hip; faster than the kernels above from 7 rows on, but for few rows of tall tiled
+// matrices).  Returns 2 when not covered.
 int launch_q4_0_matmul_f32(const void *codes, const void *scales, int64_t w_batch, int64_t n, int64_t k, const void *act,
                            int64_t act_batch, int64_t m, void *out, hipStream_t s, int tiled);
 // The same for f16 activations with k shared among the waves of a workgroup (q4_matmul_waves.hip), any m and k of whole blocks;

@@ -369,7 +369,9 @@ int launch_q4_0_matmul_f32(const void *codes, const void *scales, int64_t w_batc
     typedef std::integral_constant<int, 32> I32;
     // The shape that takes the least time: rounds of workgroups, one per compute unit, times the time of a round measured at
     // 4096 features (us, more than one round).  (150 rows of 4096 x 4096: 64 x 64 37.6 us, 32 x 64 38.3, 32 x 32 46.3; 24 rows:
-    // 16 x 32 11.7, 16 x 16 16.1, 32 x 32 15.7; 512 rows of 2816 x 1024: 32 x 64 20.7, 64 x 64 25.8.)
+    // 16 x 32 11.7, 16 x 16 16.1, 32 x 32 15.7; 512 rows of 2816 x 1024: 32 x 64 20.7, 64 x 64 25.8.)  Below 1024 features, where
+    // some waves have no unit, a launch takes its 4 to 5 us and is still the faster side (groups of 8 rows | here: 7 rows of
+    // 4096 x 32 7.1 | 4.1, of 4096 x 512 5.4 | 4.2; 40 rows of 16384 x 128 23.7 | 7.7, of 1000 x 96 24.7 | 4.5).
     struct Shape { int sub, ms, ni, us; };
     const Shape shapes[] = {{16, 1, 1, 7}, {16, 1, 2, 11}, {32, 1, 1, 15}, {32, 1, 2, 18}, {32, 2, 2, 34}};
     int best = 0;

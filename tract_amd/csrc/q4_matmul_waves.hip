@@ -249,7 +249,8 @@ int launch_q4_0_matmul_waves(const void *codes, const void *scales, int64_t w_ba
     p.act = (const _Float16 *)act, p.out = (_Float16 *)out;
     p.n = (int)n, p.k = (int)k, p.m = (int)m, p.ratio = (int)(act_batch / w_batch);
     // The shape that takes the least time: rounds of workgroups times the time of a round (1000 x 2080: 64 rows 16 x 16 7.9 us,
-    // 16 x 32 11.2; 200 rows 32 x 32 13.1, 16 x 32 19.7; 476 rows 32 x 64 20.2, 32 x 32 23.7, 64 x 64 23.5).
+    // 16 x 32 11.2; 200 rows 32 x 32 13.1, 16 x 32 19.7; 476 rows 32 x 64 20.2, 32 x 32 23.7, 64 x 64 23.5).  Below 1024 features,
+    // where some waves have no unit (before | here: 9 rows of 4096 x 512 4.9 | 4.4, 128 rows 4.6 | 4.5, 16 rows of 320 x 992 8.3 | 5.0).
     int best = 0;
     int64_t best_cost = 0;
     for (int c = 0; c < 5; c++) {

@@ -968,11 +968,11 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
     if (forced_hg && G % forced_hg == 0 && (forced_hg == 1 || forced_hg == 2 || forced_hg == 4)) hg = forced_hg;
     const int block_m = 32 * kWavesPP / hg;
     const int64_t n_qtiles = (a.Sq + block_m - 1) / block_m;
-    // Waves whose 32-query block lies past q_len idle.  With several heads per workgroup that is still
-    // the better kernel for a few queries over a long cache (speculative decoding, tiny chunks): the
-    // K/V tiles are read once per kv head instead of once per query head (8 x 32 heads x 4 queries over
-    // 8192 tokens: 66 us against 183 us).  With one head per workgroup short prompts go to the smaller kernel.
-    // (Quantised caches have no smaller kernel: they stay here whatever the prompt length.)
+    // Waves whose 32-query block lies past q_len idle.  Few queries come here with a mask, from short quantised caches, or
+    // as more groups of 32 rows than pay on the decode tiles (sdpa_decode_rows_fits).  With several heads per workgroup this is
+    // still the better of the two prefill kernels for them: K and V are read once per kv head instead of once per query
+    // head (8 x 32 heads x 4 queries over 8192 tokens: 66 us against 183 us).  With one head per workgroup short prompts
+    // go to the smaller kernel.  (Quantised caches have no smaller kernel: they stay here whatever the prompt length.)
     if (hg == 1 && !quant && a.Sq * 2 < n_qtiles * block_m) return 2;
 
     PrefillPP p;
