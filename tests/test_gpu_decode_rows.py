@@ -47,7 +47,8 @@ def test_rows_of_several_queries(rt, B, Hq, Hkv, D, past, n, causal):
 
 
 @pytest.mark.parametrize("fmt_name", ["Q8_0", "Q4_0"])
-@pytest.mark.parametrize("B,Hq,Hkv,past,n", [(1, 4, 4, 30, 2), (2, 8, 2, 600, 4), (1, 8, 2, 1021, 8), (1, 14, 2, 700, 5), (2, 3, 1, 31, 5)])
+@pytest.mark.parametrize("B,Hq,Hkv,past,n", [(1, 4, 4, 30, 2), (2, 8, 2, 600, 4), (1, 8, 2, 1021, 8), (1, 14, 2, 700, 5), (2, 3, 1, 31, 5),
+                                              (32, 5, 1, 290, 9), (6, 40, 8, 600, 4)])   # odd groups of many heads, two row groups and one
 def test_rows_over_a_quantised_cache(rt, fmt_name, B, Hq, Hkv, past, n):
     fmt = {"Q8_0": ta.Q8_0, "Q4_0": ta.Q4_0}[fmt_name]
     rng = np.random.default_rng(Hq + past + n)

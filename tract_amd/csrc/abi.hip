@@ -1373,7 +1373,7 @@ int trocm_inplace_kv_sdpa_eval(const void *q, const void *k_new, const void *v_n
     // launch, 24.8 without; 1 x 229: 14.9, 12.6).  Not where the output lies over the new rows: one workgroup stores results
     // while another still reads them.
     const size_t new_bytes = (size_t)kc->B * kc->H * n_new * kc->D * 2, out_bytes = (size_t)kc->B * q_heads * n_new * kc->D * 2;
-    if (n_new > 1 && is_dense && sdpa_decode_rows_fits(kc->B, q_heads, kc->H, n_new, kc->len + n_new, TROCM_F16) &&
+    if (n_new > 1 && is_dense && sdpa_decode_rows_fits(kc->B, q_heads, kc->H, n_new, kc->len + n_new, kc->D, TROCM_F16) &&
         !ranges_meet(out, out_bytes, k_new, new_bytes) && !ranges_meet(out, out_bytes, v_new, new_bytes) && dtype == TROCM_F16 && kc->fmt == TROCM_F16 && vc->fmt == TROCM_F16 && q && k_new && v_new && out &&
         kc->window == 0 && vc->window == 0 && kc->B == vc->B && kc->H == vc->H && kc->D == vc->D && kc->len == vc->len && q_heads % kc->H == 0) {
         hipStream_t s;

@@ -219,7 +219,7 @@ int launch_sdpa_prefill(const SdpaArgs &a, hipStream_t s);
 // A few f16 queries per sequence on the decode tiles (sdpa_decode_mfma.hip).  Returns 2 when not covered, or when
 // sdpa_decode_rows_fits says that the prefill kernels are faster.
 int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s);
-bool sdpa_decode_rows_fits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int kv_fmt);
+bool sdpa_decode_rows_fits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D, int kv_fmt);
 // MFMA prefill for q_len >= 32: staggered waves, GQA heads sharing K/V tiles, key splits across
 // workgroups (partials in the workspace after the counter area).  Returns 2 when not covered.
 int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s);

@@ -2564,13 +2564,15 @@ int launch_sdpa_decode_mfma(const SdpaArgs &a, hipStream_t s) {
     return a.D == 128 ? launch_d<128>(p, gp, grid, s) : launch_d<64>(p, gp, grid, s);
 }
 
-// Whether launch_sdpa_decode_rows is faster than the prefill kernels.  Figures: us for a call with its append, prefill kernel |
-// here, two layers in turn; BH counts workgroups per key range.
+// Whether launch_sdpa_decode_rows is faster than the prefill kernels.  Figures: us of two layers' calls with their appends, prefill
+// kernel | here; BH counts workgroups per key range.
 //
 // Up to 16 rows per kv head: always.  One group of 17 to 32 rows reads K and V once, as the prefill kernel does that shares a
 // tile among `shared` heads of a group (sdpa_prefill_pp.hip: 4, 2 or 1); `reads` counts how often K and V are read here against
 // there.  What decides beyond that is whether workgroups of 32 rows fill the chip as well as its workgroups of 256.
-bool sdpa_decode_rows_fits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int kv_fmt) {
+// Over 3000 shapes of more than 16 rows (batch 1 to 16, 200 to 8192 tokens, 2 to 64 queries) the line costs 3 % against the faster
+// side of each call in the geometric mean, and 8 % at most against the prefill kernels.
+bool sdpa_decode_rows_fits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D, int kv_fmt) {
     if (Sq < 2 || Sq > 64 || Hkv < 1 || Hq / Hkv > 1024) return false;
     const int64_t G = Hq / Hkv, rows = G * Sq, n_groups = (rows + 31) / 32, BH = B * Hkv * n_groups, cus = num_compute_units();
     if (rows <= 16) return true;
@@ -2578,28 +2580,36 @@ bool sdpa_decode_rows_fits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64
     const bool fewer_reads = n_groups * shared < G, same_reads = n_groups * shared == G;
     if (is_quant(kv_fmt)) {
         if (n_groups > 4) return false;
-        // Odd groups are read per head there: 40 heads over 8, 1 x 850 tokens, 16 queries 29.4 | 34.2, 1 x 2000 46.7 | 33.7; 14 over 2,
-        // 8 x 500, 16 queries 43.9 | 36.9, 2 x 650 tokens 28.7 | 31.2, 4 x 850, 3 queries 40.1 | 32.2.
-        if (G % 2 && G > 1) return BH <= 64 && Sk >= (B * Hq >= 96 ? 512 : B * Hq >= 64 ? 600 : B * Hq >= 40 ? 800 : 1000);
-        // 64 heads over 8, 3 queries: 4 x 500 28.8 | 32.2, 4 x 650 32.1 | 31.3, 8 x 2000 66.2 | 45.0
-        if (fewer_reads) return Sk >= 512;
-        // 32 heads over 8, 8 queries: 1 x 500 tokens 28.1 | 31.9, 1 x 650 31.5 | 30.4; 8 x 650 33.2 | 38.7, 8 x 2000 46.6 | 47.1, 8 x 3000
-        // 56.5 | 54.8; 16 x 1200 48.7 | 47.9; 32 x 550 51.2 | 50.0.  32 over 32, 32 queries: 2 x 1300 34.0 | 39.0, 2 x 3000 58.8 | 58.7.
-        if (same_reads) return Sk >= (BH >= cus ? 550 : G % 4 ? 2048 : BH <= 32 ? 600 : BH >= 128 ? 1200 : 2048);
-        // 32 over 8, 16 queries: 2 x 2000 50.0 | 37.2; 4 x 2000 43.9 | 46.7, 8 x 2000 48.2 | 62.6
-        return BH <= 32 && Sk >= 1000;
+        // 32 heads over 32, 2 groups: 2 x 2600 tokens, BH 128 1.1 to 1.3 times the prefill kernel's time; one: 8 x 1400, BH 256 0.57,
+        // 4 x 1000, BH 128 0.70, 1 x 700, BH 32 1.09
+        if (G == 1) return n_groups == 1 && Sk >= (BH >= 96 ? 512 : 2048);
+        // Odd groups are read per head there, by a workgroup per head: what decides is how many of those there are.  40 heads over
+        // 8, 16 x 3781 tokens, 4 queries 473 | 83; 16 x 593, 4 queries 99 | 40; 24 over 8, 12 x 7471, 15 queries 604 | 169; 40 over 8, 1 x 936, 4
+        // queries 32.9 | 29.5, 1 x 824, 17 queries 31.3 | 36.5; 24 over 8, 2 x 730, 15 queries 40.1 | 36.0.
+        if (G % 2) return B * Hq >= 160 || Sk >= (B * Hq >= 80 ? 512 : B * Hq >= 64 ? 600 : B * Hq >= 48 ? 700 : 900);
+        // 64 heads over 8: 8 x 2000 tokens, 3 queries 66.2 | 45.0; 12 over 2, 6 queries: 6 x 619 31.0 | 33.0
+        if (fewer_reads) return Sk >= (G % 4 && BH < 16 ? 900 : 512);
+        // 32 heads over 8: 12 x 643 tokens, 7 queries 49.8 | 41.5; 8 x 650, 8 queries 33.2 | 38.7; 16 x 623, 5 queries 39.5 | 42.0; 16 over
+        // 8: 2 x 926, 14 queries 34.6 | 31.6, 8 x 1707 42.8 | 45.6; 64 over 8: 3 x 1087, 6 queries 25.1 | 19.0 (one layer), 4 x 882, 8
+        // queries 37.6 | 40.0.
+        if (same_reads) return Sk >= (BH >= 64 && BH < 80 && G < 8 ? 1200 : BH >= 80 ? 550 : G % 4 ? 900 : 700);
+        // 32 over 8: 2 x 962, 14 queries 37.1 | 33.6, 1 x 906, 16 queries 37.1 | 31.1; 16 over 8, 2 x 6759, 39 queries 65.8 | 70.4
+        return BH <= (n_groups < 4 ? 48 : 32) && Sk >= 900;
     }
     // Odd groups (sdpa_prefill.hip, a workgroup per head and 64 queries): up to a workgroup per compute unit (24 heads over 8,
     // 64 queries: 8 x 314 tokens 35.4 | 43.5 with 384, 4 x 1064 55.0 | 46.0 with 192; 32 over 32, 33 queries, 4 x 1033, 256: 65.0 |
-    // 54.5), as many as do not read more (40 over 8, 16 x 283, 33 queries 60.2 | 53.5), or two per compute unit where it
-    // needs a second round (24 over 8, 16 x 283, 33 queries 57.0 | 46.4).
-    if (G % 2) return n_groups == 1 || BH <= cus || 4 * n_groups <= 5 * G || (BH <= 2 * cus && B * Hq > cus);
-    // 16 heads over 8, 16 queries: 8 x 616 tokens 27.6 | 29.2, 8 x 400 26.4 | 25.9, 8 x 8000 114 | 98; 16 x 1516 48.7 | 52.1
-    if (n_groups == 1) return G != 2 || BH < 64 || Sk <= 512 || Sk >= 2560;
-    // 32 over 8: 22 queries 1 x 8000 tokens 52.2 | 42.2, 2 x 8000 62.4 | 81.0, 2 x 1500 41.7 | 33.4; 16 queries 4 x 3000 45.1 | 50.9.  16 over
-    // 8, 22 queries: 4 x 3000 40.1 | 50.4, 2 x 3000 38.0 | 31.3.  12 over 2, 10 queries, 10 x 8000: groups of 2 heads there.
+    // 54.5); where it needs a second round as many as do not read more (40 over 8, 33 queries: 16 x 283 60.2 | 53.5, 16 x 4445 561 |
+    // 487, but one round, 6 x 3389, 38 queries 154 | 194) or two per compute unit (24 over 8, 16 x 283, 33 queries 57.0 | 46.4); rows
+    // of 64 features up to 2048 tokens (40 over 8, 8 x 1550, 63 queries 108 | 81, 12 x 6860 380 | 425).
+    if (G % 2) return n_groups == 1 || BH <= cus || (B * Hq > cus && (4 * n_groups <= 5 * G || BH <= 2 * cus)) || (D == 64 && Sk <= 2048);
+    // 16 heads over 8: 16 queries, 8 x 616 tokens 27.6 | 29.2, 8 x 400 26.4 | 25.9, 8 x 8000 114 | 98, 16 x 1516 48.7 | 52.1; 12 x 2051,
+    // 15 queries 78.7 | 54.1
+    if (n_groups == 1) return D == 64 || G != 2 || BH < 64 || (BH >= 80 && BH < 128) || Sk <= 512 || Sk >= 2560;
+    // 32 over 8: 22 queries 1 x 8000 tokens 52.2 | 42.2, 2 x 8000 62.4 | 81.0, 2 x 1500 41.7 | 33.4; 16 queries 4 x 3000 45.1 | 50.9, 3 x 3235
+    // 113 | 101 (15 queries, four layers), 3 x 5719 61.9 | 65.3 (11).  16 over 8, 22 queries: 4 x 3000 40.1 | 50.4, 2 x 3000 38.0 | 31.3.  12 over
+    // 2, 10 queries, 10 x 8000: groups of 2 heads there.  64 features: 32 over 8, 4 x 8144, 13 queries 53.8 | 42.7.
     if (n_groups > 4 || BH > 64) return false;
-    return fewer_reads || same_reads || BH <= 32 || Sk <= 512 || (G != 2 && (G % 4 || Sk <= 2560));
+    return D == 64 || fewer_reads || same_reads || BH <= (G == 2 ? 32 : 48) || Sk <= 512 || (G != 2 && (G % 4 || Sk <= 2560));
 }
 
 // A few queries per sequence (proposed tokens to verify, short chunks) over a cache: the rows of a kv head, its G heads
@@ -2626,7 +2636,7 @@ int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s) {
     const int gp = per <= 8 ? 8 : per <= 16 ? 16 : 32;
     if (a.Hkv * n_groups > 65535) return 2;
     const int64_t BH = a.B * a.Hkv * n_groups;
-    if (!sdpa_decode_rows_fits(a.B, a.Hq, a.Hkv, a.Sq, a.Sk, a.kv_fmt)) return 2;
+    if (!sdpa_decode_rows_fits(a.B, a.Hq, a.Hkv, a.Sq, a.Sk, a.D, a.kv_fmt)) return 2;
     DecodeDev p;
     memset(&p, 0, sizeof(p));
     p.q = (const char *)a.q, p.out = (char *)a.out, p.k = (const char *)a.k, p.v = (const char *)a.v;
