@@ -24,7 +24,7 @@ def _f16(rng, *shape):
 @pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [
     (1, 2, 1, 128, 0, 4), (1, 4, 4, 64, 27, 8), (2, 3, 1, 128, 31, 3), (1, 16, 2, 64, 29, 2), (2, 17, 1, 128, 300, 2),
     (1, 8, 2, 128, 1021, 8), (1, 11, 1, 128, 127, 3), (2, 14, 2, 64, 700, 5), (1, 7, 1, 128, 2000, 17), (1, 6, 2, 128, 255, 16),
-    (3, 4, 4, 128, 64, 33), (16, 16, 8, 128, 600, 12), (1, 5, 1, 64, 0, 64), (4, 32, 8, 128, 500, 8), (1, 32, 8, 128, 6000, 2)])
+    (3, 4, 4, 128, 64, 33), (16, 16, 8, 128, 600, 12), (12, 8, 8, 64, 1300, 10), (1, 5, 1, 64, 0, 64), (4, 32, 8, 128, 500, 8), (1, 32, 8, 128, 6000, 2)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_rows_of_several_queries(rt, B, Hq, Hkv, D, past, n, causal):
     rng = np.random.default_rng(B + 10 * Hq + past + n)
@@ -48,7 +48,8 @@ def test_rows_of_several_queries(rt, B, Hq, Hkv, D, past, n, causal):
 
 @pytest.mark.parametrize("fmt_name", ["Q8_0", "Q4_0"])
 @pytest.mark.parametrize("B,Hq,Hkv,past,n", [(1, 4, 4, 30, 2), (2, 8, 2, 600, 4), (1, 8, 2, 1021, 8), (1, 14, 2, 700, 5), (2, 3, 1, 31, 5),
-                                              (32, 5, 1, 290, 9), (6, 40, 8, 600, 4)])   # odd groups of many heads, two row groups and one
+                                              (32, 5, 1, 290, 9), (6, 40, 8, 600, 4),   # odd groups of many heads, two row groups and one
+                                              (1, 8, 2, 60, 4), (1, 8, 2, 61, 4)])   # 64 tokens and 65
 def test_rows_over_a_quantised_cache(rt, fmt_name, B, Hq, Hkv, past, n):
     fmt = {"Q8_0": ta.Q8_0, "Q4_0": ta.Q4_0}[fmt_name]
     rng = np.random.default_rng(Hq + past + n)

@@ -2567,7 +2567,8 @@ int launch_sdpa_decode_mfma(const SdpaArgs &a, hipStream_t s) {
 // Whether launch_sdpa_decode_rows is faster than the prefill kernels.  Figures: us of two layers' calls with their appends, prefill
 // kernel | here; BH counts workgroups per key range.
 //
-// Up to 16 rows per kv head: always.  One group of 17 to 32 rows reads K and V once, as the prefill kernel does that shares a
+// Up to 16 rows per kv head: always (over up to 64 quantised tokens the prefill kernel's one staged tile is faster, 32 heads over 8,
+// 1 x 41 tokens, 4 queries 17.3 | 19.8, but lets an infinity of a later token into every row).  One group of 17 to 32 rows reads K and V once, as the prefill kernel does that shares a
 // tile among `shared` heads of a group (sdpa_prefill_pp.hip: 4, 2 or 1); `reads` counts how often K and V are read here against
 // there.  What decides beyond that is whether workgroups of 32 rows fill the chip as well as its workgroups of 256.
 // Over 3000 shapes of more than 16 rows (batch 1 to 16, 200 to 8192 tokens, 2 to 64 queries) the line costs 3 % against the faster
@@ -2659,7 +2660,9 @@ int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s) {
     p.q_len = (int)a.Sq, p.causal = a.causal, p.n_rows = (int)rows, p.n_groups = (int)n_groups;
     p.scale_log2 = a.scale * 1.4426950408889634f;
     const int n_tiles = (int)((a.Sk + kTile - 1) / kTile);
-    // A workgroup per compute unit, never a few more; two with several groups and more than 8 tiles per wave (40 heads over 8,
+    // A workgroup per compute unit, never a few more, but for up to 16 rows of 64 features, whose workgroups are light (8 heads over
+    // 8, 12 x 5549 tokens, 10 queries, two layers 63.4 us in 2 ranges, 56.9 in 3; 32 over 32, 6 x 2610 55.1 in 1, 48.9 in 2; no
+    // difference below 64 workgroups per range); two with several groups and more than 8 tiles per wave (40 heads over 8,
     // 4 x 5000 tokens, 8 queries 38.7 -> 33.4 us), 32 where one range of keys fills the chip (32 over 32, 4 x 1064, 64 queries 83.0
     // split, 58.5 not).  Records of more than 8 rows are merged by a second launch, the dearer the more of them there are:
     // below these lengths it costs more than the split gives (us of two layers, split | not: BH 128, 10 tiles 38.5 | 27.3, 20 tiles
@@ -2668,7 +2671,8 @@ int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s) {
     int64_t resident = num_compute_units();
     int nsplit = choose_decode_splits(BH, gp, n_tiles, 1);
     if (n_groups > 1 && n_tiles >= (nsplit == 1 ? 128 : 32 * nsplit)) nsplit = choose_decode_splits(BH, gp, n_tiles, 2), resident *= 2;
-    if (nsplit > 1 && BH * nsplit > resident && resident >= BH) nsplit = (int)(resident / BH);
+    const bool light = a.D == 64 && gp <= 16 && BH >= 64 && n_tiles >= 32;
+    if (nsplit > 1 && BH * nsplit > resident && resident >= BH && !light) nsplit = (int)(resident / BH);
     if (gp > 8 && nsplit > 1 && n_tiles <= 8 + (quant ? 16 : 48) / nsplit) nsplit = 1;
     p.nsplit = fit_decode_splits(nsplit, BH, gp, a.D, a.workspace, a.workspace_bytes);
     p.live_trim = decode_live_trim();
