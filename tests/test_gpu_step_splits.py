@@ -1,0 +1,31 @@
+"""Single tokens over numbers of sequence-heads that do not divide the compute units: one range, a few, more than the narrow
+and the wide merge take."""
+import numpy as np
+import pytest
+
+import tract_amd as ta
+from oracle import oracle as orc
+from tests.gpu_util import rt  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("store", ["plain", "Q8_0", "Q4_0"])
+@pytest.mark.parametrize("B,Hq,Hkv,D,T", [(1, 8, 1, 128, 5000), (3, 32, 8, 128, 1100), (12, 8, 8, 128, 390), (28, 32, 8, 128, 129), (1, 16, 2, 128, 127),
+                                           (13, 14, 2, 128, 260), (13, 8, 2, 64, 515)])
+def test_steps_of_any_number_of_sequence_heads(rt, store, B, Hq, Hkv, D, T):
+    if store != "plain" and D != 128:
+        pytest.skip("block-quantised steps are of 128 features")
+    rng = np.random.default_rng(B * 100 + T)
+    k, v = (rng.standard_normal((B, Hkv, T, D), dtype=np.float32).astype(np.float16) for _ in range(2))
+    q = (rng.standard_normal((B, Hq, 1, D), dtype=np.float32) / np.float32(np.sqrt(D))).astype(np.float16)
+    fmt = None if store == "plain" else getattr(ta, store)
+    st = ta.InPlaceKvSdpa(axis=2, causal=True, storage_format=fmt).state()
+    st.k.push(k[:, :, :-1]), st.v.push(v[:, :, :-1])
+    got = st.eval([q, np.ascontiguousarray(k[:, :, -1:]), np.ascontiguousarray(v[:, :, -1:])]).to_numpy().astype(np.float64)
+    if fmt is not None:
+        code = {"Q8_0": orc.FMT_Q8_0, "Q4_0": orc.FMT_Q4_0}[store]
+        k, v = (orc.dequant(code, orc.quant(code, x), np.float32).reshape(x.shape) for x in (k, v))
+    want = orc.flash_sdpa(q.astype(np.float32), k.astype(np.float32), v.astype(np.float32), causal=True, threads=8)
+    # probabilities and results are rounded to f16 (2^-11 each): twice 2^-11 of the largest |v|
+    assert np.abs(got - want).max() <= 2 * 2.0 ** -11 * np.abs(v.astype(np.float64)).max()

@@ -407,6 +407,10 @@ int launch_sdpa_decode_ragged_mfma(const DecodeDev &p, int kv_fmt, int gp, int64
 // Partials: at most kMaxSplitRows rows of (D + 2) floats per query head.
 constexpr int64_t kMaxSplitRows = 32768;
 int choose_decode_splits(int64_t BH, int64_t G, int n_tiles, int wg_per_cu);
+// The same for one query per sequence, by what each number of splits is expected to cost; crowd16: sixteenths of its own time
+// that a further workgroup on every compute unit adds.
+constexpr int kCrowdWide = 16, kCrowdCodes = 12, kCrowdNarrow = 8;   // rows of 128 features; block codes; rows of 64
+int choose_step_splits(int64_t BH, int64_t G, int n_tiles, int crowd16);
 // The splits that the caller's workspace has room for (records of BH x splits x G rows of D + 2 floats behind the
 // counter area), at least one: a call with a small or no workspace runs with fewer splits, it does not fail.
 inline int fit_decode_splits(int nsplit, int64_t BH, int64_t G, int64_t D, const void *workspace, size_t workspace_bytes) {

@@ -466,6 +466,33 @@ int choose_decode_splits(int64_t BH, int64_t G, int n_tiles, int wg_per_cu) {
     return (int)ns;
 }
 
+// What a launch of `ns` splits costs, in sixteenths of the time that a wave spends on one tile of its workgroup's group of
+// kWaves: the longest split's groups, times the workgroups that share a compute unit where they stand in each other's way;
+// 1.5 groups for partial records at all, 1 and a sixteenth per split beyond the eight that the narrow merge takes, 3 for a merge
+// launch (more than kWideMergeMax splits), 1 for every further round of workgroups.  One line for all steps: over 650 shapes
+// (batch 1 to 31, 150 to 8000 tokens, f16, f32, Q8_0, Q4_0, 1 to 8 heads per kv head) its choice costs 0.3 to 0.7 % more than the
+// best of 16 split counts in the geometric mean (f32: 1.5 %); a fixed number of workgroups per compute unit, before, cost 4 to 11 %
+// (us, then | now: 24 sequence-heads of 8000 f16 tokens in 11 splits 27.1 | 20.3 in 8, 96 in 3 78.2 | 62.6 in 2, 224 of 300 Q4_0
+// tokens in 2 10.3 | 7.6 in 1).
+int choose_step_splits(int64_t BH, int64_t G, int n_tiles, int crowd16) {
+    static const int forced = getenv("TROCM_DECODE_SPLITS") ? atoi(getenv("TROCM_DECODE_SPLITS")) : 0;
+    const int64_t by_ws = kMaxSplitRows / (BH * G);
+    const int groups = (n_tiles + kWaves - 1) / kWaves, most = by_ws < 1 ? 1 : by_ws < groups ? (int)by_ws : groups;
+    if (forced > 0) return forced < most ? forced : most;
+    const int cus = num_compute_units();
+    int best = 1, best_cost = INT32_MAX;
+    for (int ns = 1; ns <= most && (ns == 1 || (ns <= 256 && BH * ns <= 4 * cus)); ns += ns < kWideMergeMax ? 1 : ns) {
+        const int longest = (groups + ns - 1) / ns, rounds = (int)((BH * ns + cus - 1) / cus);
+        int cost = longest * (rounds * crowd16 > 16 ? rounds * crowd16 : 16) + 16 * (rounds - 1);
+        if (ns > 1) cost += 24;
+        if (ns > kTailMergeMax) cost += 16 + (ns < kWideMergeMax ? ns : kWideMergeMax) - kTailMergeMax;
+        if (ns > kWideMergeMax) cost += 48;
+        if (cost < best_cost) best = ns, best_cost = cost;
+    }
+    const int longest = (groups + best - 1) / best;   // the same critical path with fewer records
+    return (groups + longest - 1) / longest;
+}
+
 int launch_sdpa_decode(const SdpaArgs &a, hipStream_t s) {
     if (a.Sq != 1) return 2;
     {   // grouped heads: the MFMA formulation (it declines f32 and masks over rows whose length is not a multiple of 4)
@@ -489,7 +516,7 @@ int launch_sdpa_decode(const SdpaArgs &a, hipStream_t s) {
     if (BH > (int64_t)(kWsCounterBytes / sizeof(int)) || a.B > 65535 || a.Hkv > 65535) return 2;
 
     int n_tiles = (int)((a.Sk + kTile - 1) / kTile);
-    int nsplit = fit_decode_splits(choose_decode_splits(BH, G, n_tiles, 1), BH, G, a.D, a.workspace, a.workspace_bytes);
+    int nsplit = fit_decode_splits(choose_step_splits(BH, G, n_tiles, a.D == 128 ? kCrowdWide : kCrowdNarrow), BH, G, a.D, a.workspace, a.workspace_bytes);
     int tps = (n_tiles + nsplit - 1) / nsplit;
     nsplit = (n_tiles + tps - 1) / tps;  // no empty split
     DecodeDev p;

@@ -2431,8 +2431,7 @@ int launch_sdpa_decode_quant_mfma(DecodeDev &p, int kv_fmt, int64_t B, void *wor
     if (gp == 0) return 2;
     const int64_t BH = B * p.Hkv;
     const int n_tiles = (p.T + kTile - 1) / kTile;
-    static const int wg_per_cu = getenv("TROCM_DECODE_QUANT_WG_PER_CU") ? atoi(getenv("TROCM_DECODE_QUANT_WG_PER_CU")) : 2;
-    int nsplit = fit_decode_splits(choose_decode_splits(BH, gp, n_tiles, wg_per_cu), BH, gp, 128, workspace, workspace_bytes);
+    int nsplit = fit_decode_splits(choose_step_splits(BH, gp, n_tiles, kCrowdCodes), BH, gp, 128, workspace, workspace_bytes);
     const int tps = (n_tiles + nsplit - 1) / nsplit;
     nsplit = (n_tiles + tps - 1) / tps;
     p.tiles_per_split = tps, p.nsplit = nsplit;
@@ -2458,7 +2457,7 @@ int launch_sdpa_decode_kivi(const KiviSdpaArgs &a, hipStream_t s) {
     if ((uintptr_t)a.k_new % 2 || (uintptr_t)a.v_new % 2 || (uintptr_t)a.k_chan_scale_next % 16 || (uintptr_t)a.k_chan_lo_next % 16) return 2;
     const int64_t BH = a.B * a.Hkv;
     const int n_tiles = (int)((a.T + kTile - 1) / kTile);
-    int nsplit = fit_decode_splits(choose_decode_splits(BH, gp, n_tiles, 2), BH, gp, 128, a.workspace, a.workspace_bytes);
+    int nsplit = fit_decode_splits(choose_step_splits(BH, gp, n_tiles, kCrowdCodes), BH, gp, 128, a.workspace, a.workspace_bytes);
     const int tps = (n_tiles + nsplit - 1) / nsplit;
     nsplit = (n_tiles + tps - 1) / tps;
     DecodeDev p;
@@ -2514,7 +2513,7 @@ int launch_sdpa_decode_mfma(const SdpaArgs &a, hipStream_t s) {
     if (a.B > 65535 || a.Hkv > 65535) return 2;
     const int64_t BH = a.B * a.Hkv;
     const int n_tiles = (int)((a.Sk + kTile - 1) / kTile);
-    int nsplit = fit_decode_splits(choose_decode_splits(BH, gp, n_tiles, 1), BH, gp, a.D, a.workspace, a.workspace_bytes);
+    int nsplit = fit_decode_splits(choose_step_splits(BH, gp, n_tiles, a.D == 128 ? kCrowdWide : kCrowdNarrow), BH, gp, a.D, a.workspace, a.workspace_bytes);
     const int tps = (n_tiles + nsplit - 1) / nsplit;
     nsplit = (n_tiles + tps - 1) / tps;
     DecodeDev p;
