@@ -1414,7 +1414,19 @@ int trocm_inplace_kv_sdpa_eval_rope(const void *q, const void *k_new, const void
                   (long long)cos_sin_batch_stride, (long long)(n_new * kc->D));
     hipStream_t s;
     if (resolve_stream(stream, &s)) return 1;
-    if (n_new == 1 && dtype == TROCM_F16 && (kc->fmt == TROCM_F16 || is_quant(kc->fmt)) && kc->window == 0 && vc->window == 0 && q_heads % kc->H == 0) {
+    // room for rotated copies of q and k_new: asked of every call but the f16 steps that never had a use for it
+    const size_t es = elem_bytes(dtype);
+    const size_t q_bytes = (size_t)kc->B * q_heads * n_new * kc->D * es, k_bytes = (size_t)kc->B * kc->H * n_new * kc->D * es;
+    const size_t q_room = (q_bytes + 255) & ~(size_t)255;
+    auto room_check = [&]() -> int {
+        TROCM_REQUIRE(rot_scratch != nullptr && rot_scratch_bytes >= q_room + k_bytes,
+                      "inplace_kv_sdpa_rope: this call rotates q and k_new into rot_scratch, which must hold %zu bytes (%zu given)",
+                      q_room + k_bytes, rot_scratch_bytes);
+        TROCM_REQUIRE((uintptr_t)rot_scratch % 16 == 0, "rot_scratch must be 16-byte aligned");
+        return 0;
+    };
+    if (dtype == TROCM_F32 && room_check()) return 1;
+    if (n_new == 1 && (is_quant(kc->fmt) ? dtype == TROCM_F16 : dtype == kc->fmt) && kc->window == 0 && vc->window == 0 && q_heads % kc->H == 0) {
         if (equalise_capacities(kc, vc, s)) return 1;
         int64_t dense[4];
         dense[3] = 1, dense[2] = kc->D, dense[1] = kc->D, dense[0] = kc->H * kc->D;
@@ -1434,14 +1446,7 @@ int trocm_inplace_kv_sdpa_eval_rope(const void *q, const void *k_new, const void
             if (rc != 2) return rc;
         }
     }
-    // rotate into the caller's scratch: q first, then k_new
-    const size_t es = elem_bytes(dtype);
-    const size_t q_bytes = (size_t)kc->B * q_heads * n_new * kc->D * es, k_bytes = (size_t)kc->B * kc->H * n_new * kc->D * es;
-    const size_t q_room = (q_bytes + 255) & ~(size_t)255;
-    TROCM_REQUIRE(rot_scratch != nullptr && rot_scratch_bytes >= q_room + k_bytes,
-                  "inplace_kv_sdpa_rope: this call rotates q and k_new into rot_scratch, which must hold %zu bytes (%zu given)",
-                  q_room + k_bytes, rot_scratch_bytes);
-    TROCM_REQUIRE((uintptr_t)rot_scratch % 16 == 0, "rot_scratch must be 16-byte aligned");
+    if (room_check()) return 1;   // rotate into the caller's scratch: q first, then k_new
     void *q_rot = rot_scratch, *k_rot = (char *)rot_scratch + q_room;
     const int64_t cs[4] = {cos_sin_batch_stride, 0, kc->D, 1};
     const int64_t qs[4] = {kc->B, q_heads, n_new, kc->D}, ks[4] = {kc->B, kc->H, n_new, kc->D};

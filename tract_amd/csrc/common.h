@@ -191,6 +191,9 @@ int launch_sdpa_decode(const SdpaArgs &a, hipStream_t s);
 // Split-K decode for 2..32 query heads per kv head (f16): the heads are the rows of MFMA tiles.
 // Returns 2 when not covered (masks, other types).
 int launch_sdpa_decode_mfma(const SdpaArgs &a, hipStream_t s);
+// Split-K decode over f32 rows, up to 16 query heads per kv head, with the rotation of q and k_new (sdpa_decode_f32.hip).
+// Returns 2 when not covered.
+int launch_sdpa_decode_f32(const SdpaArgs &a, hipStream_t s);
 // Split-K decode over Q8_0 / Q4_0 caches with fused dequantisation.  Returns 2 when not covered.
 int launch_sdpa_decode_quant(const SdpaArgs &a, hipStream_t s);
 // Whether a step over a Q8_0 / Q4_0 cache with g_real query heads per kv head can rotate q and the new key (RoPE) inside the
