@@ -23,14 +23,28 @@
 // tile's is used up, V before the scores: each has a phase of 4096 cycles to arrive.  K / V of a kv head stay in one XCD's L2:
 // workgroup ids run over kv heads first.
 //
-// Bound by the f32 matrix rate: 1000 causal queries of 32 heads over 8 kv heads (D = 128) are 8.2 GFLOP, 54 us at the 152
-// TFLOP/s that a large f32 matrix product reaches; a call with its append takes 102.5 us (105.2 while 28 bytes per lane were
-// in scratch memory; the diagonal tiles are computed whole, and the last workgroups leave compute units idle).  The generic
-// kernel, a wave per query with scalar fused multiply-adds and every key row read once per query, took 9040 us.  Error
-// against f64 over the same call 3.3e-7 (generic: 3.8e-7).
+// Bound by the f32 matrix rate (152 TFLOP/s reached by a large product) and, with up to 32 rows, mostly by the chain of a short
+// launch.  The generic kernel, a wave per query with scalar fused multiply-adds, took 9040 us for 1000 queries of 32 heads.
+//
+// More than 32 rows (sdpa_prefill_f32x2_kernel): every f32 is a power of two times the sum of two f16 numbers, and a product is three
+// of v_mfma_f32_32x32x16_f16 (upper by upper, upper by lower, lower by upper; f32 accumulation): three times the f32 instruction's
+// rate, 23 of the 24 bits of every operand, and fewer roundings in the sums.  Error against f64, 1000 causal queries of 32 heads
+// over 8, 2.7e-7, 771 over 451 past tokens 3.9e-7 (the f32 instruction: 3.3e-7, 4.7e-7).
+//  * Two row tiles of 32 per workgroup and two key sets of two waves: a set's waves share the 32-key tiles that its 128 threads turn
+//    into pairs on the way into LDS (K by rows, V transposed into the order in which P comes out of the scores).
+//  * Scales: q's per row, K's and V's from the first tiles of the range with room for 8 times as much.  What does not fit (larger
+//    values later, infinities and NaN, features of V 2^13 weaker than the strongest, scores beyond 2^14) shows as a flag or as a sum
+//    that is no number at the end, and the row tile is done again by the f32 code (attend_tile).
+//  * What bounds it is the issue of instructions: per tile and wave 48 matrix and about 550 vector instructions, whose busy cycles
+//    add up to 97 % of the kernel's (counters; 2000 queries: 33 and 64 %).  Loads have no condition around them, or the waits for
+//    one tile's V would be waits for the next tile's K (71.6 -> 58.2 us).
+// 1000 queries of 32 heads over 8 (D = 128), with the append: 104.7 us on the f32 instruction, 58.0 as pairs; 771 over 451 tokens 132.3,
+// 65.1; 10 queries of 4 x 64 heads over 8, 3629 tokens, 96.0, 51.5.  From 4 tiles on (2 x 70 queries of 32 heads over 32, 3 tiles: 15.3
+// | 17.5; 2 x 116 of 40 over 8 20.0 | 18.0); ranges of keys (us without | with): 49 queries, 32 over 8, 396 tokens 29.7 | 21.5, but
+// 2 x 251, a workgroup per compute unit, 25.0 | 33.7.
 #include <hip/hip_runtime.h>
 #include <string.h>
-#include "common.h"
+#include "decode_common.h"
 
 namespace trocm {
 namespace {
@@ -39,9 +53,9 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kRows = 32, kWaves = 4, kThreads = 64 * kWaves, kMaxSplits = 16;
+constexpr int kRows = 32, kMaxSplits = 64;
+constexpr float kScoreRange = 0x1p14f;
 
 struct PrefillF32 {
     const float *q, *k, *v;
@@ -51,7 +65,8 @@ struct PrefillF32 {
     int64_t kv_stride_b, kv_stride_h;   // elements
     uint32_t kv_row_bytes, kv_bytes;    // bytes between token rows; bytes of one kv head's rows, from the first to the last
     int Hq, Hkv, Sq, Sk, G;
-    int n_bh, n_rt, nsplit;             // batch * kv_heads, row tiles per kv head
+    int n_bh, n_rt, nsplit;             // batch * kv_heads, 32-row tiles per kv head
+    int n_rt2, paired;                  // sdpa_prefill_f32x2_kernel: 64-row tiles per kv head; whether the short ones run beside the long ones
     int causal;
     float scale;
 };
@@ -73,17 +88,24 @@ __device__ __forceinline__ bool finite(float x) { return __builtin_isfinite(x); 
 // the weight exp(m - ref) of a partial result whose maximum is m; nothing seen: m = -inf, weight 0 whatever ref is
 __device__ __forceinline__ float ref_of(float m) { return m == -INFINITY ? 0.0f : m; }
 
+// LDS of a workgroup: q, then the waves' outputs; their maxima and sums
 template <int D>
-__global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32_kernel(PrefillF32 p) {
+struct TileLds {
+    float rows[kWaves * kRows * (D + 4)];
+    float m[kWaves][kRows], l[kWaves][kRows];
+};
+
+// Row tile rt of a (batch, kv head) over the key tiles kt_first .. kt_last - 1 that it sees, by one workgroup.
+template <int D>
+__device__ __forceinline__ void attend_tile(const PrefillF32 &p, TileLds<D> &shared, int bh, int rt, int split, int kt_first, int kt_last) {
     constexpr int T = D / 32, KJ = D / 8, ROW = D + 4;   // (ROW: 16 rows of a 128-bit LDS pass in 16 distinct bank groups)
     typedef typename VecOf<T>::type vec;
-    __shared__ __attribute__((aligned(16))) float lds[kWaves * kRows * ROW];   // q; then the waves' outputs
-    __shared__ float lds_m[kWaves][kRows], lds_l[kWaves][kRows];
+    float *lds = shared.rows;
+    auto &lds_m = shared.m;
+    auto &lds_l = shared.l;
 
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hb = lane >> 5;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int bh = blockIdx.x % p.n_bh, rest = blockIdx.x / p.n_bh;
-    const int split = rest % p.nsplit, rt = p.n_rt - 1 - rest / p.nsplit;
     const int b = bh / p.Hkv, kvh = bh % p.Hkv;
     const int n_rows = p.Sq * p.G, r0 = rt * kRows;
     auto q_row = [&](int r) {   // offset of row r's query (and output) in elements
@@ -93,8 +115,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32_kernel(PrefillF3
     // keys [0, limit) are visible to a row; the tile as a whole sees n_vis
     auto limit_of = [&](int r) { return p.causal ? min(r, n_rows - 1) / p.G + (p.Sk - p.Sq) + 1 : p.Sk; };
     const int limit = limit_of(r0 + l32), limit_first = limit_of(r0), n_vis = limit_of(r0 + kRows - 1);
-    const int tiles = (n_vis + 31) / 32, per_split = (tiles + p.nsplit - 1) / p.nsplit;
-    const int kt_end = min(tiles, (split + 1) * per_split);
+    const int kt_end = min((n_vis + 31) / 32, kt_last);
 
     // rows past the last key read as zeros: the buffer ends with that row
     const float *k_head = p.k + b * p.kv_stride_b + kvh * p.kv_stride_h, *v_head = p.v + b * p.kv_stride_b + kvh * p.kv_stride_h;
@@ -114,7 +135,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32_kernel(PrefillF3
         for (int i = 0; i < 16; i++) vreg[i] = buffer_vec<T>(v_rsrc, off + (uint32_t)(8 * (i / 4) + i % 4) * p.kv_row_bytes);
     };
 
-    int kt = split * per_split + w;
+    int kt = kt_first + w;
     if (kt < kt_end) load_k(kt);
 #pragma unroll
     for (int j = 0; j < kRows * D / 4 / kThreads; j++) {
@@ -263,38 +284,343 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32_kernel(PrefillF3
     }
 }
 
-// The ranges of keys of one row tile per workgroup.
+template <int D>
+__global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32_kernel(PrefillF32 p) {
+    __shared__ __attribute__((aligned(16))) TileLds<D> shared;
+    const int bh = blockIdx.x % p.n_bh, rest = blockIdx.x / p.n_bh;
+    const int split = rest % p.nsplit, rt = p.n_rt - 1 - rest / p.nsplit;
+    const int last = min(rt * kRows + kRows, p.Sq * p.G) - 1, n_vis = p.causal ? last / p.G + (p.Sk - p.Sq) + 1 : p.Sk;
+    const int per_split = ((n_vis + 31) / 32 + p.nsplit - 1) / p.nsplit;
+    attend_tile<D>(p, shared, bh, rt, split, split * per_split, (split + 1) * per_split);
+}
+
+// ---- more than 32 rows: every f32 as a pair of f16 ---------------------------------------------------------------------
+__device__ __forceinline__ int exp_field(float x) { return (int)(__builtin_bit_cast(uint32_t, x) >> 23) & 255; }
+__device__ __forceinline__ float pow2_field(int e) { return __builtin_bit_cast(float, (uint32_t)min(max(e, 0), 254) << 23); }
+// exponent field of the scale that puts `largest` in 2^13 .. 2^14: room for eight times as much (at most 2^55, so that products of
+// two scales and their inverses are normal numbers)
+__device__ __forceinline__ int up_field(float largest) { return min(267 - exp_field(largest), 127 + 55); }
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+// x times a power of two as the sum of two f16 numbers, each rounded once: 23 of its 24 bits.  (Six operations for a pair, all at
+// the full rate: the instructions that multiply, add and round to f16 in one, five for a pair, take two cycles for one.)
+__device__ __forceinline__ void split_pair(float x0, float x1, float scale, uint32_t &hi, uint32_t &lo) {
+    const half2_t h = __builtin_convertvector(f32x2_t{x0 * scale, x1 * scale}, half2_t);
+    const float h0 = (float)h.x, h1 = (float)h.y;
+    hi = __builtin_bit_cast(uint32_t, h);
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{fmaf(x0, scale, -h0), fmaf(x1, scale, -h1)}, half2_t));
+}
+struct Split8 { half8_t hi, lo; };
+template <typename F>
+__device__ __forceinline__ Split8 split8(F x, float scale) {   // x(0) .. x(7)
+    u32x4 h, l;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        uint32_t a, c;
+        split_pair(x(2 * i), x(2 * i + 1), scale, a, c);
+        h[i] = a, l[i] = c;
+    }
+    return Split8{__builtin_bit_cast(half8_t, h), __builtin_bit_cast(half8_t, l)};
+}
+__device__ __forceinline__ f32x16 mfma3(const Split8 &a, const Split8 &b, f32x16 c) {
+    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.lo, b.hi, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.hi, b.lo, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a.hi, b.hi, c, 0, 0, 0);
+}
+template <int D>
+struct PairLds {
+    _Float16 k[2][2][kRows * (D + 8)];          // [key set][upper, lower]: 32 keys of D features
+    _Float16 vt[2][2][D / 32][32 * 40];         // [key set][upper, lower][subtile][feature]: 32 keys in the order of P's registers
+};
+
+template <int D>
+__global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(PrefillF32 p) {
+    constexpr int T = D / 32, C4 = D / 4, NG = 8 * C4 / 128, KROW = D + 8, ROW = D + 4;
+    typedef typename VecOf<T>::type vec;
+    __shared__ __attribute__((aligned(16))) union { PairLds<D> pair; TileLds<D> tile; float rows[2 * kRows * ROW]; } lds;
+    __shared__ float lds_m[kWaves][kRows], lds_l[kWaves][kRows], lds_big[3][kWaves];
+    __shared__ int lds_odd;
+
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hb = lane >> 5;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), rg = w & 1, ks = w >> 1;
+    const int bh = blockIdx.x % p.n_bh, rest = blockIdx.x / p.n_bh, at = rest / p.nsplit, split = rest % p.nsplit;
+    const int half = (p.n_rt2 + 1) / 2, rt2 = p.paired && at >= half ? at - half : p.n_rt2 - 1 - at;
+    const int b = bh / p.Hkv, kvh = bh % p.Hkv;
+    const int n_rows = p.Sq * p.G, r0 = rt2 * 2 * kRows;
+    auto q_row = [&](int r) {
+        const int i = r / p.G, g = r - i * p.G;
+        return (((int64_t)b * p.Hq + kvh * p.G + g) * p.Sq + i) * D;
+    };
+    auto limit_of = [&](int r) { return p.causal ? min(r, n_rows - 1) / p.G + (p.Sk - p.Sq) + 1 : p.Sk; };
+    const int limit = limit_of(r0 + kRows * rg + l32), limit_first = limit_of(r0), n_vis = limit_of(r0 + 2 * kRows - 1);
+    const int tiles = (n_vis + 31) / 32, per_split = (tiles + p.nsplit - 1) / p.nsplit;
+    const int kt_first = split * per_split, kt_last = min(tiles, kt_first + per_split);
+
+    const float *k_head = p.k + b * p.kv_stride_b + kvh * p.kv_stride_h, *v_head = p.v + b * p.kv_stride_b + kvh * p.kv_stride_h;
+    const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(k_head), 0, p.kv_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(v_head), 0, p.kv_bytes, 0x00020000);
+    // a key set's 128 threads: features 4 c4 .. + 3 of the keys 4 (g0 + 4 i) .. + 3
+    const int st = tid & 127, c4 = st % C4, g0 = st / C4;
+    f32x4 kpre[NG][4], vpre[NG][4];
+    auto load_rows = [&](f32x4 (&dst)[NG][4], __amdgpu_buffer_rsrc_t rsrc, int kt) {
+        const uint32_t off = (uint32_t)(32 * kt + 4 * g0) * p.kv_row_bytes + 16 * c4;
+#pragma unroll
+        for (int i = 0; i < NG; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) dst[i][j] = buffer_f32x4(rsrc, off + (uint32_t)(16 * i + j) * p.kv_row_bytes);
+    };
+    int kt = kt_first + ks;
+    load_rows(kpre, k_rsrc, min(kt, tiles)), load_rows(vpre, v_rsrc, min(kt, tiles));   // (past the last tile: zeros)
+
+    // Scales, powers of two: q's per row, K's and V's from the first tiles of the range.
+    Split8 q[D / 16];
+    float c;   // what makes scores of the sums
+    int k_field, v_field;
+    bool odd;
+    {
+        auto largest = [](const f32x4 (&x)[NG][4]) {
+            float big = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NG; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) big = fmaxf(big, fabsf(x[i][j][e]));
+            return wave_max(big);
+        };
+        const float *row = p.q + q_row(min(r0 + kRows * rg + l32, n_rows - 1)) + 8 * hb;
+        f32x4 x[D / 8];
+        float big = 0.0f;
+#pragma unroll
+        for (int j = 0; j < D / 8; j++) {
+            x[j] = *reinterpret_cast<const f32x4 *>(row + 16 * (j / 2) + 4 * (j % 2));
+#pragma unroll
+            for (int e = 0; e < 4; e++) big = fmaxf(big, fabsf(x[j][e]));
+        }
+        big = fmaxf(big, __shfl_xor(big, 32, 64));
+        const int q_field = up_field(big);
+#pragma unroll
+        for (int j = 0; j < D / 16; j++) q[j] = split8([&](int i) { return x[2 * j + i / 4][i % 4]; }, pow2_field(q_field));
+        const float q_big = wave_max(big), k_big = kt < kt_last ? largest(kpre) : 0.0f, v_big = kt < kt_last ? largest(vpre) : 0.0f;
+        auto weak = [](float x, int field) { return x > 0.0f && x * pow2_field(field) < 1.0f; };   // (below 2^-55)
+        const bool weak_q = __any(weak(big, q_field));
+        if (lane == 0) lds_big[0][w] = weak_q ? INFINITY : q_big, lds_big[1][w] = k_big, lds_big[2][w] = v_big;
+        if (tid == 0) lds_odd = 0;
+        __syncthreads();
+        auto of_all = [&](int i) { return fmaxf(fmaxf(lds_big[i][0], lds_big[i][1]), fmaxf(lds_big[i][2], lds_big[i][3])); };
+        k_field = up_field(of_all(1)), v_field = up_field(of_all(2));
+        c = p.scale * pow2_field(254 - q_field) * pow2_field(254 - k_field);
+        // no score is larger than this; what the pairs leave of K, 2^-38 of the first tiles' largest, stays below 2^-24 of a score's unit
+        odd = !(of_all(0) * of_all(1) * p.scale * D < kScoreRange) || weak(of_all(1), k_field);
+        // features of V that are 2^13 times weaker than the strongest: their lower numbers would not be normal
+        if (32 * kt + 32 <= p.Sk && kt < kt_last) {
+            bool bad = false;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float m = 0.0f;
+#pragma unroll
+                for (int i = 0; i < NG; i++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) m = fmaxf(m, fabsf(vpre[i][j][e]));
+                bad = bad || weak(m, v_field);
+            }
+            if (bad) lds_odd = 1;
+        }
+    }
+
+    f32x16 o[T];
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[t][r] = 0.0f;
+    float m_run = -INFINITY, l_run = 0.0f;   // l and P are counted in 2^-14
+    const float k_up = pow2_field(k_field), v_up = pow2_field(v_field);
+    const int steps = (kt_last - kt_first + 1) / 2;
+    for (int it = 0; it < steps; it++, kt += 2) {
+        const bool live = kt < kt_last, edge = 32 * kt + 32 > limit_first;   // edge: some row does not see all of the tile
+        if (live) {
+#pragma unroll
+            for (int i = 0; i < NG; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    uint32_t h0, l0, h1, l1;
+                    split_pair(kpre[i][j][0], kpre[i][j][1], k_up, h0, l0), split_pair(kpre[i][j][2], kpre[i][j][3], k_up, h1, l1);
+                    const int dst = (4 * (g0 + 4 * i) + j) * KROW + 4 * c4;
+                    *reinterpret_cast<u32x2 *>(&lds.pair.k[ks][0][dst]) = u32x2{h0, h1};
+                    *reinterpret_cast<u32x2 *>(&lds.pair.k[ks][1][dst]) = u32x2{l0, l1};
+                }
+        }
+        // (always, a tile again at the end: with a condition around them the wait for V below would be one for these too)
+        load_rows(kpre, k_rsrc, min(kt + 2, kt_last));
+        __syncthreads();   // K is in LDS; every wave is done with the last V
+        f32x16 s;
+        if (live) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) s[r] = 0.0f;
+#pragma unroll
+            for (int j = 0; j < D / 16; j++) {
+                Split8 kf;
+                kf.hi = *reinterpret_cast<const half8_t *>(&lds.pair.k[ks][0][l32 * KROW + 16 * j + 8 * hb]);
+                kf.lo = *reinterpret_cast<const half8_t *>(&lds.pair.k[ks][1][l32 * KROW + 16 * j + 8 * hb]);
+                s = mfma3(kf, q[j], s);
+            }
+#pragma unroll
+            for (int i = 0; i < NG; i++) {
+                const int g = g0 + 4 * i, pos = 16 * (g / 4) + 8 * (g % 2) + 4 * (g % 4 / 2);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    uint32_t h0, l0, h1, l1;
+                    split_pair(vpre[i][0][e], vpre[i][1][e], v_up, h0, l0), split_pair(vpre[i][2][e], vpre[i][3][e], v_up, h1, l1);
+                    const int f = 4 * c4 + e, dst = f / T * 40 + pos;
+                    *reinterpret_cast<u32x2 *>(&lds.pair.vt[ks][0][f % T][dst]) = u32x2{h0, h1};
+                    *reinterpret_cast<u32x2 *>(&lds.pair.vt[ks][1][f % T][dst]) = u32x2{l0, l1};
+                }
+            }
+        }
+        load_rows(vpre, v_rsrc, min(kt + 2, kt_last));
+        __syncthreads();   // V is in LDS; every wave is done with K
+        if (!live) continue;
+
+        if (edge) {
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                if (32 * kt + 8 * (r / 4) + 4 * hb + r % 4 >= limit) s[r] = -INFINITY;
+        }
+        float mx = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; r++) mx = fmaxf(mx, s[r]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c;
+        const float m_new = fmaxf(m_run, mx), ref = ref_of(m_new);
+        if (__any(m_new != m_run)) {
+            const float alpha = expf(m_run - ref);
+            l_run *= alpha;
+#pragma unroll
+            for (int t = 0; t < T; t++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) o[t][r] *= alpha;
+            m_run = m_new;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r++) {   // 2^14 e^(s c - ref)
+            s[r] = fast_exp2(fmaf(fmaf(s[r], c, -ref), 1.4426950408889634f, 14.0f));
+            l_run += s[r];
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const Split8 pf = split8([&](int i) { return s[8 * u + i]; }, 1.0f);
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                Split8 vf;
+                vf.hi = *reinterpret_cast<const half8_t *>(&lds.pair.vt[ks][0][t][l32 * 40 + 16 * u + 8 * hb]);
+                vf.lo = *reinterpret_cast<const half8_t *>(&lds.pair.vt[ks][1][t][l32 * 40 + 16 * u + 8 * hb]);
+                o[t] = mfma3(vf, pf, o[t]);
+            }
+        }
+    }
+    // Infinities, NaN and values that are too large for the scales have left sums that are no numbers.
+    {
+        float probe = l_run * 0.0f;
+#pragma unroll
+        for (int t = 0; t < T; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) probe = fmaf(o[t][r], 0.0f, probe);
+        if (!(probe == 0.0f)) lds_odd = 1;
+        __syncthreads();
+        odd = odd || lds_odd != 0;
+    }
+    if (odd) {   // for this row tile everything again, in f32
+        __syncthreads();
+        for (int i = 0; i < 2 && r0 + kRows * i < n_rows; i++) {
+            attend_tile<D>(p, lds.tile, bh, 2 * rt2 + i, split, kt_first, kt_last);
+            __syncthreads();
+        }
+        return;
+    }
+
+    // ---- the two key sets' results ---------------------------------------------------------------------------------
+    l_run += __shfl_xor(l_run, 32, 64);
+    if (hb == 0) lds_m[w][l32] = m_run, lds_l[w][l32] = l_run * 0x1p-14f;
+    __syncthreads();   // (and every wave is done with V)
+    const float m_all = fmaxf(m_run, lds_m[w ^ 2][l32]);
+    const float wgt = expf(m_run - ref_of(m_all)) * (pow2_field(254 - v_field) * 0x1p-14f);   // o is counted in 1 / (2^14 v_up)
+    float *mine = &lds.rows[(kRows * rg + l32) * ROW];
+#pragma unroll
+    for (int set = 1; set >= 0; set--) {
+        if (ks == set) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                vec *dst = reinterpret_cast<vec *>(mine + T * (8 * (r / 4) + 4 * hb + r % 4));
+                vec x;
+#pragma unroll
+                for (int t = 0; t < T; t++) x[t] = o[t][r] * wgt;
+                if (set == 0) x += *dst;
+                *dst = x;
+            }
+        }
+        __syncthreads();
+    }
+    const int64_t wb0 = (int64_t)bh * p.n_rt + 2 * rt2, n_wb = (int64_t)p.n_bh * p.n_rt;
+#pragma unroll 4
+    for (int j = 0; j < 2 * kRows * C4 / kThreads; j++) {
+        const int f = j * kThreads + tid, r = f / C4, cc = f % C4, r32 = r % kRows, wr = r / kRows;   // waves wr and wr + 2 had the row
+        if (r0 + kRows * wr >= n_rows) continue;
+        f32x4 sum = *reinterpret_cast<const f32x4 *>(&lds.rows[r * ROW + 4 * cc]);
+        const float m0 = lds_m[wr][r32], m1 = lds_m[wr + 2][r32], mm = fmaxf(m0, m1), ref = ref_of(mm);
+        const float l = lds_l[wr][r32] * expf(m0 - ref) + lds_l[wr + 2][r32] * expf(m1 - ref);
+        if (p.nsplit > 1) {
+            const int64_t rec = split * n_wb + wb0 + wr;
+            *reinterpret_cast<f32x4 *>(p.part_o + (rec * kRows + r32) * D + 4 * cc) = sum;
+            if (cc == 0) p.part_ml[rec * 64 + r32] = mm, p.part_ml[rec * 64 + 32 + r32] = l;
+        } else if (r0 + r < n_rows) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) sum[e] = l > 0.0f ? sum[e] / l : 0.0f;
+            *reinterpret_cast<f32x4 *>(p.out + q_row(r0 + r) + 4 * cc) = sum;
+        }
+    }
+}
+
+// The ranges of keys of a row tile: a thread per four features of a row.
 template <int D>
 __global__ __launch_bounds__(kThreads) void sdpa_prefill_f32_merge_kernel(PrefillF32 p) {
-    const int tid = threadIdx.x;
-    const int64_t wb = blockIdx.x, n_wb = (int64_t)p.n_bh * p.n_rt;
-    const int bh = (int)(wb / p.n_rt), rt = (int)(wb % p.n_rt), b = bh / p.Hkv, kvh = bh % p.Hkv;
-    for (int f = tid; f < kRows * D / 4; f += kThreads) {
-        const int r = f / (D / 4), c = f % (D / 4), row = rt * kRows + r;
-        if (row >= p.Sq * p.G) continue;
-        float mm = -INFINITY;
-        for (int s = 0; s < p.nsplit; s++) mm = fmaxf(mm, p.part_ml[(s * n_wb + wb) * 64 + r]);
-        const float ref = ref_of(mm);
-        float l = 0.0f;
-        f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int s = 0; s < p.nsplit; s++) {
-            const float *ml = p.part_ml + (s * n_wb + wb) * 64;
-            const float wgt = expf(ml[r] - ref);
-            l += wgt * ml[32 + r];
-            sum += wgt * *reinterpret_cast<const f32x4 *>(p.part_o + ((s * n_wb + wb) * kRows + r) * D + 4 * c);
-        }
-        const int i = row / p.G, g = row - i * p.G;
+    const int64_t f = (int64_t)blockIdx.x * kThreads + threadIdx.x, n_wb = (int64_t)p.n_bh * p.n_rt, wb = f / (kRows * D / 4);
+    const int r = (int)(f / (D / 4) % kRows), c = (int)(f % (D / 4));
+    const int bh = (int)(wb / p.n_rt), rt = (int)(wb % p.n_rt), b = bh / p.Hkv, kvh = bh % p.Hkv, row = rt * kRows + r;
+    if (row >= p.Sq * p.G) return;
+    const float *ml = p.part_ml + wb * 64 + r, *po = p.part_o + (wb * kRows + r) * D + 4 * c;
+    const int64_t ml_step = n_wb * 64, po_step = n_wb * kRows * D;
+    float mm = -INFINITY, l = 0.0f;
+    f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < p.nsplit; s0 += 8) {   // eight ranges in flight at a time
+        float m8[8], l8[8], top = mm;
+        f32x4 o8[8];
 #pragma unroll
-        for (int e = 0; e < 4; e++) sum[e] = l > 0.0f ? sum[e] / l : 0.0f;
-        *reinterpret_cast<f32x4 *>(p.out + (((int64_t)b * p.Hq + kvh * p.G + g) * p.Sq + i) * D + 4 * c) = sum;
+        for (int i = 0; i < 8; i++) {
+            const int s = min(s0 + i, p.nsplit - 1);
+            m8[i] = ml[s * ml_step], l8[i] = ml[s * ml_step + 32];
+            o8[i] = *reinterpret_cast<const f32x4 *>(po + s * po_step);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) top = fmaxf(top, m8[i]);
+        const float ref = ref_of(top), keep = expf(mm - ref);
+        sum *= keep, l *= keep, mm = top;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float wgt = s0 + i < p.nsplit ? expf(m8[i] - ref) : 0.0f;
+            l += wgt * l8[i];
+            sum += wgt * o8[i];
+        }
     }
+    const int i = row / p.G, g = row - i * p.G;
+#pragma unroll
+    for (int e = 0; e < 4; e++) sum[e] = l > 0.0f ? sum[e] / l : 0.0f;
+    *reinterpret_cast<f32x4 *>(p.out + (((int64_t)b * p.Hq + kvh * p.G + g) * p.Sq + i) * D + 4 * c) = sum;
 }
 
 template <int D>
 int launch(const PrefillF32 &p, hipStream_t s) {
-    const int64_t n_wb = (int64_t)p.n_bh * p.n_rt;
-    hipLaunchKernelGGL((sdpa_prefill_f32_kernel<D>), dim3((unsigned)(n_wb * p.nsplit)), dim3(kThreads), 0, s, p);
-    if (p.nsplit > 1) hipLaunchKernelGGL((sdpa_prefill_f32_merge_kernel<D>), dim3((unsigned)n_wb), dim3(kThreads), 0, s, p);
+    if (p.n_rt2) hipLaunchKernelGGL((sdpa_prefill_f32x2_kernel<D>), dim3((unsigned)(p.n_bh * p.n_rt2 * p.nsplit)), dim3(kThreads), 0, s, p);
+    else hipLaunchKernelGGL((sdpa_prefill_f32_kernel<D>), dim3((unsigned)(p.n_bh * p.n_rt * p.nsplit)), dim3(kThreads), 0, s, p);
+    if (p.nsplit > 1)
+        hipLaunchKernelGGL((sdpa_prefill_f32_merge_kernel<D>), dim3((unsigned)((int64_t)p.n_bh * p.n_rt * (kRows * D / 4 / kThreads))), dim3(kThreads), 0, s, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail("sdpa_prefill_f32 launch failed: %s", hipGetErrorString(e));
     return 0;
@@ -313,7 +639,7 @@ int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
     if ((uintptr_t)a.q % 16 || (uintptr_t)a.k % 16 || (uintptr_t)a.v % 16 || (uintptr_t)a.out % 16) return 2;
     const int64_t G = a.Hq / a.Hkv;
     if (a.Sk >= (1ll << 30) || a.Sq >= (1ll << 30) || a.Sq * G >= (1ll << 30) || a.B * a.Hkv >= (1ll << 30)) return 2;
-    if ((a.Sk + 32) * a.kv_stride_t >= (1ll << 30)) return 2;   // byte offsets of the rows a tile addresses are 32-bit
+    if ((a.Sk + 96) * a.kv_stride_t >= (1ll << 30)) return 2;   // byte offsets of the rows a tile addresses are 32-bit
 
     PrefillF32 p;
     memset(&p, 0, sizeof(p));
@@ -324,11 +650,16 @@ int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
     p.n_bh = (int)(a.B * a.Hkv), p.n_rt = (int)((a.Sq * G + kRows - 1) / kRows);
     p.causal = a.causal, p.scale = a.scale;
 
-    // Two workgroups fit a compute unit.  Fewer than that: ranges of keys, each of at least a tile per wave.
-    const int64_t n_wb = (int64_t)p.n_bh * p.n_rt, want = 2 * (int64_t)num_compute_units(), tiles = (a.Sk + 31) / 32;
-    int64_t ns = n_wb < want ? (want + n_wb - 1) / n_wb : 1;
-    ns = ns < tiles / kWaves ? ns : tiles / kWaves;
+    // Pairs of f16 from 33 rows and 4 tiles on.  Ranges of at least 4 tiles (16 where half the compute units have a workgroup).
+    const int64_t tiles = (a.Sk + 31) / 32, cus = num_compute_units(), want = 2 * cus;
+    const bool pairs = p.n_rt > 1 && tiles >= 4 && a.scale >= 0x1p-16f && a.scale <= 0x1p16f;
+    if (pairs) p.n_rt2 = (int)((a.Sq * G + 2 * kRows - 1) / (2 * kRows));
+    const int64_t n_wb = (int64_t)p.n_bh * p.n_rt, n_wg = pairs ? (int64_t)p.n_bh * p.n_rt2 : n_wb;
+    int64_t ns = pairs ? want / n_wg : n_wg < want ? (want + n_wg - 1) / n_wg : 1;
+    const int64_t most = tiles / (pairs && 2 * n_wg > cus ? 16 : 4);
+    ns = ns < most ? ns : most;
     ns = ns < kMaxSplits ? ns : kMaxSplits;
+    p.paired = pairs && a.causal && n_wg <= want;
     const size_t per_split = (size_t)n_wb * (kRows * a.D + 64) * sizeof(float);
     const size_t avail = a.workspace && a.workspace_bytes > kWsCounterBytes + 256 ? a.workspace_bytes - kWsCounterBytes - 256 : 0;
     if (ns > 1 && (size_t)ns * per_split > avail) ns = (int64_t)(avail / per_split);
@@ -339,7 +670,7 @@ int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
         p.part_o = (float *)base;
         p.part_ml = p.part_o + (size_t)p.nsplit * n_wb * kRows * a.D;
     }
-    if (n_wb * p.nsplit >= (1ll << 31)) return 2;
+    if (n_wb * p.nsplit >= (1ll << 31) || n_wb * (kRows * a.D / 4 / kThreads) >= (1ll << 31)) return 2;
     return a.D == 128 ? launch<128>(p, s) : launch<64>(p, s);
 }
 
