@@ -1,0 +1,27 @@
+"""Q4_0 weights x f16 rows on the tiled matrix-matrix kernel: each of the shapes that its rule chooses, with remainders of rows and of
+weight rows, against the product in 64 bits with the dequantised weights."""
+import numpy as np
+import pytest
+
+import tract_amd as ta
+from oracle import oracle as orc
+from tests.gpu_util import rt  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+# (n, k, m): 32 rows x 32 with k shared by 8 waves, 32 x 64 by 4 sets, 64 x 64 by 4, 64 x 128 by 4 and 2, 64 x 256 by 2, 128 x 256; odd tile
+# counts (k / 128 = 3, 9, 6, 12) that only some of them or none take
+@pytest.mark.parametrize("n,k,m", [(4096, 1024, 49), (2816, 1024, 131), (2832, 1024, 299), (4112, 1024, 321), (5120, 512, 388), (4096, 1024, 1000),
+                                   (14336, 512, 390), (1040, 384, 200), (2064, 1152, 77), (3072, 768, 150), (4096, 1536, 65)])
+def test_shapes_of_the_tiled_product(rt, n, k, m):
+    rng = np.random.default_rng(n + k + m)
+    w = (0.03 * rng.standard_normal((n, k), dtype=np.float32)).astype(np.float32)
+    act = rng.standard_normal((1, m, k), dtype=np.float32).astype(np.float16)
+    blocks = orc.quant(orc.FMT_Q4_0, w)
+    got = ta.GgmlGemm().eval(ta.DeviceTensor.from_numpy(act), ta.Q40Weights(blocks, 1, n, k)).to_numpy().astype(np.float64)[0]
+    want = act[0].astype(np.float64) @ orc.dequant(orc.FMT_Q4_0, blocks, np.float32).reshape(n, k).astype(np.float64).T
+    # every weight and the result are rounded to f16 once: 2^-11 of each at most, about 0.3 of that in the norm
+    assert np.linalg.norm(got - want) <= 2.0 ** -11 * np.linalg.norm(want)
+    # a result is a sum of k products whose weights are off by 2^-11 at most: 6 standard deviations of that, and its own rounding
+    assert np.abs(got - want).max() <= 2.0 ** -11 * (6 * np.sqrt(k) * 0.03 + np.abs(want).max())

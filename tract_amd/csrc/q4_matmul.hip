@@ -378,6 +378,31 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS >= 8 ? 1 : 2) void q4_0_tiled
     }
 }
 
+// The shapes of q4_0_tiled_matmul_kernel that are worth their launch, with what a launch of each takes: `first` us, `tile` us for
+// every tile of k and round of workgroups (one per compute unit; `whole` of it for a round however full it is, the rest by its
+// workgroups), and `round` us for every further round.  Fitted to 200 products (17 to 1024 rows of 1024 x 4096, 2048 x 8192, 2816 x 1024,
+// 4096 x 4096, 4096 x 14336, 5120 x 5120, 8192 x 3072 and 14336 x 4096) within 3 to 7 %; the shape with the least expected time costs
+// 0.6 % more than the best of 26 in the geometric mean, the largest tile that gives three quarters of the compute units a workgroup,
+// before, 12 % (us, then | now: 640 rows of 1024 x 4096 23.7 | 15.2, 288 of 4096 x 14336 85.4 | 56.7, 96 of 5120 x 5120 26.0 | 13.6,
+// 64 of 4096 x 4096 11.7 | 8.3, 160 of 2816 x 1024 10.3 | 5.1).
+struct TiledShape { int bm, ni, ks, nw; float first, tile, whole, round; };
+constexpr TiledShape kTiledShapes[] = {
+    {32, 1, 8, 1, 3.50f, 0.151f, 0.867f, 0.1f}, {32, 1, 4, 2, 3.44f, 0.246f, 0.794f, 0.0f},  {64, 1, 4, 2, 3.77f, 0.397f, 0.737f, 2.2f},
+    {64, 1, 4, 4, 5.32f, 0.602f, 0.536f, 5.4f}, {64, 1, 2, 4, 4.68f, 0.623f, 0.638f, 0.0f},  {64, 2, 2, 4, 7.00f, 1.075f, 0.617f, 7.8f},
+    {128, 2, 1, 4, 9.27f, 1.792f, 0.777f, 0.0f}};
+const TiledShape *best_shape(int64_t n, int64_t m, int64_t act_batch, int64_t tiles, int64_t cus) {
+    const TiledShape *best = nullptr;
+    float best_us = 0.0f;
+    for (const TiledShape &c : kTiledShapes) {
+        if (tiles % c.ks) continue;
+        const int64_t cols = 32 * c.ni * c.nw, wgs = (n + cols - 1) / cols * ((m + c.bm - 1) / c.bm) * act_batch, rounds = (wgs + cus - 1) / cus;
+        const float us = c.first + c.round * (float)(rounds - 1) +
+                         c.tile * (float)tiles * (c.whole * (float)rounds + (1.0f - c.whole) * (float)wgs / (float)cus);
+        if (!best || us < best_us) best = &c, best_us = us;
+    }
+    return best;
+}
+
 }  // namespace
 
 // 2 = not taken (the caller runs the rows in groups on the matrix-vector kernels): f32 activations (their products stay
@@ -396,7 +421,7 @@ int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, i
     if (tiled) {
         // 32-bit byte offsets inside one weight matrix and one batch of activations (rows up to 128 past m are addressed)
         if (n % 16 || k % TK || (n / 16) * (k / TK) * 1152 >= (1ll << 32) || (m + 128) * k >= (1ll << 30)) return 2;
-        // The largest tile of C^T per workgroup -- 256 (n) x 128 (m), 256 x 64, 128 x 64 -- that still gives three
+        // What remains for k that is no multiple of 512 (its sets of waves could not share it): the largest tile of C^T per workgroup -- 256 (n) x 128 (m), 256 x 64, 128 x 64 -- that still gives three
         // quarters of the compute units a workgroup (128 x 128 never has more workgroups than 256 x 64); the smallest
         // when none does, and then (or with 256 x 64) k
         // split over 2 or 4 sets of waves inside the workgroup while the workgroups are fewer than the compute units
@@ -408,13 +433,18 @@ int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, i
         // (up to 32 activation rows: 256 x 32, 128 x 32 -- half the matrix instructions of a tile of 64 rows)
         const int shapes64[3][2] = {{128, 2}, {64, 2}, {64, 1}}, shapes32[3][2] = {{32, 2}, {32, 2}, {32, 1}};
         const int (*shapes)[2] = m <= 32 ? shapes32 : shapes64;
-        int bm = shapes[2][0], ni = 1;
+        int bm = shapes[2][0], ni = 1, pick_nw = 0, pick_ks = 0;
         for (int c = 0; c < 3; c++) {
             const int64_t wgs = ((n + 128 * shapes[c][1] - 1) / (128 * shapes[c][1])) * ((m + shapes[c][0] - 1) / shapes[c][0]) * act_batch;
             if (wgs * 4 >= cus * 3) {
                 bm = shapes[c][0], ni = shapes[c][1];
                 break;
             }
+        }
+        // Otherwise the shape with the least expected time.
+        if (const TiledShape *best = k / TK % 4 == 0 ? best_shape(n, m, act_batch, k / TK, cus) : nullptr) {
+            bm = best->bm, ni = best->ni;
+            pick_nw = best->nw, pick_ks = best->ks;
         }
         if (forced_bm == 32 || forced_bm == 64 || forced_bm == 128) bm = forced_bm;
         if (forced_ni == 1 || forced_ni == 2) ni = forced_ni;
@@ -427,6 +457,7 @@ int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, i
         int nw = 4;
         if (bm <= 64 && ni == 1) {
             while (nw > 1 && ((n + 32 * nw - 1) / (32 * nw)) * ty * act_batch * 4 < cus * 3) nw /= 2;
+            if (pick_nw) nw = pick_nw;
             if (forced_nw == 1 || forced_nw == 2 || forced_nw == 4) nw = forced_nw;
         }
         const int64_t txw = (n + 32 * ni * nw - 1) / (32 * ni * nw);
@@ -437,6 +468,7 @@ int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, i
             else if (ni == 1 && wgs * nw <= cus * 4 && tiles % 4 == 0) ks = 4;       // (16 waves of 128 registers fill a compute unit)
             else if (wgs * nw <= 2 * cus * 4 && tiles % 2 == 0) ks = 2;
         }
+        if (pick_ks) ks = pick_ks;
         if (forced_ks == 1 || ((forced_ks == 2 || ((forced_ks == 4 || (forced_ks == 8 && nw == 1)) && ni == 1)) && bm <= 64 && (k / TK) % forced_ks == 0)) ks = forced_ks;
         const dim3 tgrid((unsigned)txw, (unsigned)ty, (unsigned)act_batch);
         const size_t lds_act = (size_t)ks * 2 * bm * AROW * sizeof(_Float16);
