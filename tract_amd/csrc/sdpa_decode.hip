@@ -468,9 +468,10 @@ int choose_decode_splits(int64_t BH, int64_t G, int n_tiles, int wg_per_cu) {
 
 // What a launch of `ns` splits costs, in sixteenths of the time that a wave spends on one tile of its workgroup's group of
 // kWaves: the longest split's groups, times the workgroups that share a compute unit where they stand in each other's way;
-// 1.5 groups for partial records at all, 1 and a sixteenth per split beyond the eight that the narrow merge takes, 3 for a merge
-// launch (more than kWideMergeMax splits), 1 for every further round of workgroups.  One line for all steps: over 650 shapes
-// (batch 1 to 31, 150 to 8000 tokens, f16, f32, Q8_0, Q4_0, 1 to 8 heads per kv head) its choice costs 0.3 to 0.7 % more than the
+// 1.5 groups for partial records at all, 1.25 and a sixteenth per split beyond the eight that the narrow merge takes and 0.75 where
+// the splits of one sequence-head do not fall on the same XCDs as another's (8192 tokens x 8 sequence-heads: 22 splits 14.4 us, 24
+// 13.6), 3 for a merge launch (more than kWideMergeMax splits), 1 for every further round of workgroups.  One line for all steps: over 650 shapes
+// (batch 1 to 31, 150 to 8000 tokens, f16, f32, Q8_0, Q4_0, 1 to 8 heads per kv head) its choice costs 0.2 to 0.7 % more than the
 // best of 16 split counts in the geometric mean (f32: 1.5 %); a fixed number of workgroups per compute unit, before, cost 4 to 11 %
 // (us, then | now: 24 sequence-heads of 8000 f16 tokens in 11 splits 27.1 | 20.3 in 8, 96 in 3 78.2 | 62.6 in 2, 224 of 300 Q4_0
 // tokens in 2 10.3 | 7.6 in 1).
@@ -485,10 +486,11 @@ int choose_step_splits(int64_t BH, int64_t G, int n_tiles, int crowd16) {
         const int longest = (groups + ns - 1) / ns, rounds = (int)((BH * ns + cus - 1) / cus);
         int cost = longest * (rounds * crowd16 > 16 ? rounds * crowd16 : 16) + 16 * (rounds - 1);
         if (ns > 1) cost += 24;
-        if (ns > kTailMergeMax) cost += 16 + (ns < kWideMergeMax ? ns : kWideMergeMax) - kTailMergeMax;
+        if (ns > kTailMergeMax) cost += 20 + (ns % 8 ? 12 : 0) + (ns < kWideMergeMax ? ns : kWideMergeMax) - kTailMergeMax;
         if (ns > kWideMergeMax) cost += 48;
         if (cost < best_cost) best = ns, best_cost = cost;
     }
+    if (best > kTailMergeMax && best <= kWideMergeMax) return best;
     const int longest = (groups + best - 1) / best;   // the same critical path with fewer records
     return (groups + longest - 1) / longest;
 }
@@ -521,6 +523,10 @@ int launch_sdpa_decode(const SdpaArgs &a, hipStream_t s) {
 
     int n_tiles = (int)((a.Sk + kTile - 1) / kTile);
     int nsplit = fit_decode_splits(choose_step_splits(BH, G, n_tiles, a.D == 128 ? kCrowdWide : kCrowdNarrow), BH, G, a.D, a.workspace, a.workspace_bytes);
+    {   // (more than eight are merged by a launch here, whatever XCD they were on)
+        const int groups = (n_tiles + kWaves - 1) / kWaves, longest = (groups + nsplit - 1) / nsplit;
+        nsplit = (groups + longest - 1) / longest;
+    }
     int tps = (n_tiles + nsplit - 1) / nsplit;
     nsplit = (n_tiles + tps - 1) / tps;  // no empty split
     DecodeDev p;

@@ -2556,7 +2556,9 @@ int launch_sdpa_decode_mfma(const SdpaArgs &a, hipStream_t s) {
     // 32768 tokens or 3 sequences on the two are level or the in-kernel merge wins).  TROCM_DECODE_TAIL_MERGE:
     // 0 = always the launch, 2 = always in the kernel.
     static const int tail = getenv("TROCM_DECODE_TAIL_MERGE") ? atoi(getenv("TROCM_DECODE_TAIL_MERGE")) : 1;
-    const bool short_and_wide = nsplit > kTailMergeMax && a.B <= 2 && a.Sk <= 16384;
+    // (Fewer than 8 sequence-heads, or rows of 64 features up to 10000 tokens: in the kernel; 14 heads over 2, 8192 tokens 13.0 | 12.3,
+    // 2500 10.1 | 9.2; 32 over 8, 64 features, 2500 tokens 9.7 | 7.9, 8192 10.5 | 10.1, 12000 11.3 | 11.8.)
+    const bool short_and_wide = nsplit > kTailMergeMax && a.B <= 2 && a.Sk <= 16384 && BH >= 8 && (a.D == 128 || a.Sk > 10000);
     if (tail && (tail == 2 || !short_and_wide) && gp <= 8 && nsplit > 1 && nsplit <= kWideMergeMax && BH <= (int64_t)(kWsCounterBytes / sizeof(int)))
         p.counters = (int *)a.workspace;
     dim3 grid(nsplit, (unsigned)a.Hkv, (unsigned)a.B);
