@@ -83,7 +83,11 @@ __device__ __forceinline__ typename VecOf<T>::type buffer_vec(__amdgpu_buffer_rs
     if constexpr (T == 4) return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
     else return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
 }
-__device__ __forceinline__ bool finite(float x) { return __builtin_isfinite(x); }
+// all ones if x is finite, else 0.  (Arithmetic: as a condition for each of 32 numbers it takes more scalar registers than there are.)
+__device__ __forceinline__ uint32_t finite_mask(float x) {
+    return (uint32_t)((int)((__builtin_bit_cast(uint32_t, x) & 0x7f800000u) - 0x7f800000u) >> 31);
+}
+__device__ __forceinline__ float masked(float x, uint32_t mask) { return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & mask); }
 
 // the weight exp(m - ref) of a partial result whose maximum is m; nothing seen: m = -inf, weight 0 whatever ref is
 __device__ __forceinline__ float ref_of(float m) { return m == -INFINITY ? 0.0f : m; }
@@ -213,20 +217,20 @@ __device__ __forceinline__ void attend_tile(const PrefillF32 &p, TileLds<D> &sha
                     for (int r = 0; r < 16; r++)
                         if (r == 4 * (kk >> 3) + (kk & 3)) pk = s[r];
                     pk = __shfl(pk, l32 + 32 * ((kk >> 2) & 1), 64);
-                    const bool seen = 32 * kt + kk < limit;
+                    const uint32_t seen = 32 * kt + kk < limit ? ~0u : 0u;
                     const uint32_t off = (uint32_t)(32 * kt + kk) * p.kv_row_bytes;
 #pragma unroll
                     for (int r = 0; r < 16; r++) {
                         const vec x = buffer_vec<T>(v_rsrc, off + 4 * T * (8 * (r / 4) + 4 * hb + r % 4));
 #pragma unroll
                         for (int t = 0; t < T; t++)
-                            o[t][r] = fmaf(pk, seen && !finite(x[t]) ? x[t] : 0.0f, o[t][r]);
+                            o[t][r] = fmaf(pk, masked(x[t], seen & ~finite_mask(x[t])), o[t][r]);
                     }
                 }
 #pragma unroll
                 for (int i = 0; i < 16; i++)
 #pragma unroll
-                    for (int t = 0; t < T; t++) vreg[i][t] = finite(vreg[i][t]) ? vreg[i][t] : 0.0f;
+                    for (int t = 0; t < T; t++) vreg[i][t] = masked(vreg[i][t], finite_mask(vreg[i][t]));
             }
         }
 #pragma unroll
