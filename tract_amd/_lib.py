@@ -130,5 +130,13 @@ def check(rc: int) -> None:
         raise TractRocmError(load().trocm_last_error().decode("utf-8", "replace"))
 
 
+_FUNCTIONS = {}   # name -> the loaded library's function
+
+
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args))
+    fn = _FUNCTIONS.get(name)
+    if fn is None:
+        fn = _FUNCTIONS[name] = getattr(load(), name)
+    rc = fn(*args)
+    if rc:
+        check(rc)

@@ -7,6 +7,7 @@ Mirrors the pieces of tract's device layer that the KV-cache path touches:
 from __future__ import annotations
 
 import ctypes as C
+import functools
 
 import numpy as np
 
@@ -160,6 +161,7 @@ class Workspace:
     scratch, gpu/src/memory/schema.rs:56-128)."""
 
     @staticmethod
+    @functools.lru_cache(maxsize=1024)   # (a function of its arguments alone)
     def bytes_for(batch: int, q_heads: int, q_len: int, head_dim: int) -> int:
         n = C.c_size_t()
         call("trocm_sdpa_workspace_bytes", batch, q_heads, q_len, head_dim, C.byref(n))
