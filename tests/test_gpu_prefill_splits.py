@@ -1,0 +1,62 @@
+"""f16 prompts whose keys are split over workgroups: every way the parts are merged (by the last of up to four, by a launch for up
+to eight and up to sixteen), two workgroups on a compute unit at head size 64, one head per workgroup with few queries, small scratch."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import tract_amd as ta
+from tests.cases import textbook_sdpa
+from tests.gpu_util import rt  # noqa: F401
+from tract_amd._lib import call
+
+pytestmark = pytest.mark.gpu
+
+# q, K and V are exact.  A weight, a part's output and the output are rounded to f16, 2^-11 of each at most, and so is their
+# root mean square over the output; the sum of three, and scores of a few units with 2^-24 each
+TOL = 3 * 2.0 ** -11
+
+
+def _normal(rng, *shape):
+    return rng.standard_normal(shape, dtype=np.float32).astype(np.float16)
+
+
+def _sdpa(q, k, v, causal, ws, size):
+    B, Hq, n, D = q.shape
+    Hkv, T = k.shape[1:3]
+    dq, dk, dv = (ta.DeviceTensor.from_numpy(x) for x in (q, k, v))
+    out = ta.DeviceTensor.from_numpy(np.full(q.shape, 7, np.float16))
+    strides = (C.c_int64 * 3)(Hkv * T * D, T * D, D)
+    call("trocm_sdpa", dq.ptr, dk.ptr, dv.ptr, None, out.ptr, ta.F16, B, Hq, Hkv, n, T, D, strides, 1, 1, C.c_float(float("nan")),
+         int(causal), ws.ptr if size else None, size, None)
+    return out.to_numpy()
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [(1, 8, 2, 128, 3584, 65), (1, 14, 2, 128, 700, 99), (2, 5, 1, 128, 1000, 150),
+                                                (1, 8, 8, 64, 2000, 120), (1, 32, 8, 64, 500, 300), (2, 14, 2, 64, 0, 700),
+                                                (1, 7, 1, 64, 900, 255), (1, 32, 8, 128, 1000, 301), (3, 16, 4, 128, 0, 500),
+                                                (2, 36, 12, 64, 60, 1100), (1, 32, 32, 128, 0, 70), (1, 1, 1, 64, 4000, 190)])
+def test_parts(rt, B, Hq, Hkv, D, past, n):
+    rng = np.random.default_rng(past + n)
+    q, k, v = _normal(rng, B, Hq, n, D), _normal(rng, B, Hkv, past + n, D), _normal(rng, B, Hkv, past + n, D)
+    ws = ta.Workspace(B, Hq, n, D)
+    for causal in (True, False):
+        want = textbook_sdpa(q, k, v, causal=causal).astype(np.float64)
+        for size in ((0, 64 * 1024 + 256, ws.nbytes // 3, ws.nbytes, ws.nbytes) if causal else (ws.nbytes,)):   # (the last again: counters are left as they were)
+            got = _sdpa(q, k, v, causal, ws, size).astype(np.float64)
+            assert np.linalg.norm(got - want) <= TOL * np.linalg.norm(want), (causal, size)
+            rows, err = np.linalg.norm(want, axis=-1), np.linalg.norm(got - want, axis=-1)
+            assert (err <= 2 * TOL * rows + 2.0 ** -20).all(), (causal, size)   # row by row: none is missing or another's
+
+
+@pytest.mark.parametrize("heads,n,past", [(8, 65, 3583), (14, 99, 669)])
+@pytest.mark.parametrize("last", [False, True])
+def test_an_infinite_part(rt, heads, n, past, last):
+    """One part's output is infinite in a feature: so is the result there, and nowhere else, whichever part it is.  (Whole tiles of keys.)"""
+    rng = np.random.default_rng(n)
+    q, k, v = _normal(rng, 1, heads, n, 128), _normal(rng, 1, 2, past + n, 128), _normal(rng, 1, 2, past + n, 128)
+    q *= np.float16(0.125)   # no weight is below f16's smallest
+    v[:, :, past + n - 1 if last else 0, 9] = np.inf
+    ws = ta.Workspace(1, heads, n, 128)
+    got = _sdpa(q, k, v, False, ws, ws.nbytes)
+    assert np.isposinf(got[..., 9]).all() and np.isfinite(np.delete(got, 9, axis=-1)).all()

@@ -16,8 +16,8 @@
 // waves that share queries keep separate online-softmax states and are merged through LDS at
 // the end.  2x2 (64 queries per workgroup) keeps more compute units busy when there are few
 // query tiles, 4x2 (eight waves, 128 queries) halves the K/V staging per query when there are
-// many.  This kernel serves prompts too short for sdpa_prefill_pp.hip, whose grouped-head
-// workgroups are the fast path.
+// many.  sdpa_prefill_pp.hip, whose workgroups share K/V tiles and split the keys, is the fast path; this
+// kernel serves what it does not take: scales that are not positive and outputs aligned to 8 bytes only.
 //
 // K and V tiles: global -> registers (prefetched one tile ahead) -> LDS, both row-major with
 // padded rows, written with 128-bit stores.  K fragments are plain 128-bit LDS reads.  For V

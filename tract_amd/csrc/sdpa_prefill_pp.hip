@@ -16,7 +16,9 @@
 //  * Few workgroups (small batch) are spread over the chip by splitting the key range over
 //    several workgroups.  Each writes its normalised partial output in f16 plus (m, l) to the
 //    workspace, laid out exactly as the accumulator registers are (so every store instruction
-//    covers 512 contiguous bytes), and a small kernel merges them.
+//    covers 512 contiguous bytes), and the last of up to four to arrive, or a small kernel, merges them.
+//  * Head size 64: 128 registers, so that two workgroups fit on a compute unit (129, one, cost 10 to 20 %: 3 x 64 heads x 917
+//    queries behind 3704 261 -> 238 us; a single wave of unequal workgroups gives 3 % of that back: 64 heads x 1761 44.5 -> 46.3).
 //  * The output accumulators are rescaled only when some query's running maximum moved.
 //  * A second tile loop (template argument PING, chosen with TROCM_PREFILL_PING=1, f16 caches without a mask
 //    input) loads K/V tiles straight into LDS (global_load_lds_dwordx4, swizzled rows) and runs waves 0..3 and
@@ -52,6 +54,7 @@ struct PrefillPP {
     int B, Hq, Hkv, Sq, Sk;
     int causal;
     int n_qtiles, nsplit;
+    int paired;         // != 0: how many query tiles make up a first workgroup for every compute unit, where each holds two
     float scale_log2;
     // Partials of key split s and 32-query block wb (= (b * Hq + qh) * n_qb32 + q / 32):
     _Float16 *part_o;   // [nsplit][n_wb][D / 4][32 queries][4 features], normalised by l
@@ -89,6 +92,7 @@ __device__ __attribute__((always_inline)) inline void static_for_impl(F &&f, std
 template <int N, class F>
 __device__ __attribute__((always_inline)) inline void static_for(F &&f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
 constexpr float kLazyMax = 8.0f;
+constexpr int kMaxSplits = 16, kTailSplits = 4;   // key splits; those that the last of them to arrive merges itself
 #ifndef TROCM_PING_PRIO_MFMA
 #define TROCM_PING_PRIO_MFMA 1
 #endif
@@ -118,7 +122,7 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t b0123, uint32_t b4567, half2_
 
 
 template <int D, int HG, bool MASK, int FMT, bool PING = false>
-__global__ __launch_bounds__(kThreadsPP) void sdpa_prefill_pp_kernel(PrefillPP p) {
+__global__ __launch_bounds__(kThreadsPP, D == 64 && !MASK ? 4 : 2) void sdpa_prefill_pp_kernel(PrefillPP p) {
     static_assert(!PING || (!MASK && FMT == TROCM_F16), "the ping-pong loop serves f16 caches without a mask input");
     constexpr int QB = kWavesPP / HG;     // 32-query blocks per workgroup
     constexpr int BLOCK_M = 32 * QB;
@@ -134,15 +138,13 @@ __global__ __launch_bounds__(kThreadsPP) void sdpa_prefill_pp_kernel(PrefillPP p
     constexpr int K_TILE = PING ? kTileN * D : kTileN * KROW;   // halves
     constexpr int V_TILE = PING ? kTileN * D : kTileN * VROW;
     constexpr int TR_HALVES = kWavesPP * 32 * (D / 2 + 8);      // output transposition area of the epilogue
-    constexpr int WTS_HALVES = kWavesPP * 16 * 32 * 2;          // merge weights of the epilogue (floats)
-    constexpr int LDS_HALVES = PING ? (2 * K_TILE + 2 * V_TILE > WTS_HALVES + TR_HALVES ? 2 * K_TILE + 2 * V_TILE : WTS_HALVES + TR_HALVES)
-                                    : 2 * K_TILE + 2 * V_TILE;
+    constexpr int LDS_HALVES = 2 * K_TILE + 2 * V_TILE;
     __shared__ __attribute__((aligned(1024))) _Float16 lds_all[LDS_HALVES];
     _Float16 (*lds_k)[K_TILE] = reinterpret_cast<_Float16 (*)[K_TILE]>(&lds_all[0]);
     _Float16 (*lds_v)[V_TILE] = reinterpret_cast<_Float16 (*)[V_TILE]>(&lds_all[2 * K_TILE]);
 
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int hb = lane >> 5, l32 = lane & 31;
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int lane = tid & 63, hb = lane >> 5, l32 = lane & 31;
 
     // workgroup -> (kv head fastest: consecutive workgroup ids go round-robin to the 8 XCDs, so
     // one kv head's K/V stays in one XCD's L2), head group, key split, query tile (longest first)
@@ -154,8 +156,14 @@ __global__ __launch_bounds__(kThreadsPP) void sdpa_prefill_pp_kernel(PrefillPP p
     id /= (G / HG);
     const int split = id % p.nsplit;
     id /= p.nsplit;
-    const int qt = p.n_qtiles - 1 - (id % p.n_qtiles);
-    const int b = id / p.n_qtiles;
+    int b, qt;
+    if (p.paired) {   // one wave of workgroups over the chip with the longest tiles first, beside them the others, shortest first
+        b = id % p.B, id /= p.B;
+        qt = id < p.paired ? p.n_qtiles - 1 - id : id - p.paired;
+    } else {
+        b = id / p.n_qtiles;
+        qt = p.n_qtiles - 1 - id % p.n_qtiles;
+    }
     const int qh = kvh * G + gg * HG + (w % HG);
 
     const int off = p.Sk - p.Sq;          // query i sees keys j <= i + off when causal
@@ -600,6 +608,10 @@ __global__ __launch_bounds__(kThreadsPP) void sdpa_prefill_pp_kernel(PrefillPP p
         }
         if (grp == 0) half_barrier();   // as many barriers as the second group
     }
+    if constexpr (D == 64) {   // the lane's number taken anew: what the epilogue makes of it would otherwise be kept in registers through the loop
+        asm("" : "+v"(lane));
+        hb = lane >> 5, l32 = lane & 31;
+    }
     l_run += __shfl_xor(l_run, 32, 64);
     // Output rows of this wave (32 queries of one head: one contiguous block of 32 * D halves).  A lane holds
     // 4-feature pieces of its own query's row, which stored as they stand would touch 32 rows per instruction;
@@ -613,8 +625,8 @@ __global__ __launch_bounds__(kThreadsPP) void sdpa_prefill_pp_kernel(PrefillPP p
     };
     auto write_output = [&](float mul) {
         constexpr int FP = D / 2, TROW = FP + 8, CPRW = FP / 8, RPI = 64 / CPRW;   // features per pass, LDS row, 16-byte pieces per row, rows per instruction
-        static_assert(kWavesPP * 32 * TROW == TR_HALVES && (PING || TR_HALVES <= 2 * V_TILE), "transposition area exceeds the V tile buffers");
-        _Float16 *tr = (PING ? &lds_all[WTS_HALVES] : &lds_v[0][0]) + w * (32 * TROW);
+        static_assert(kWavesPP * 32 * TROW == TR_HALVES && TR_HALVES <= (PING ? LDS_HALVES : 2 * V_TILE), "transposition area exceeds the tile buffers");
+        _Float16 *tr = (PING ? &lds_all[0] : &lds_v[0][0]) + w * (32 * TROW);
         _Float16 *obase = p.out + (((int64_t)b * p.Hq + qh) * p.Sq + q0) * D;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
@@ -696,190 +708,138 @@ __global__ __launch_bounds__(kThreadsPP) void sdpa_prefill_pp_kernel(PrefillPP p
     }
     __syncthreads();
     if (!s_last || !wave_has_queries) return;
-    // Every wave merges its own 32-query block: out = sum_s w_s O_s, w_s = l_s 2^(m_s - max m) / sum.
-    // The weights go through a wave-private corner of the (now idle) K tile buffer; the partial
-    // outputs are laid out as the accumulators are, so each lane reads back exactly its own elements,
-    // two splits in flight at a time.
-    constexpr int kMaxSplits = 16;
+    // Every wave merges its own 32-query block: out = sum_s w_s O_s, w_s = l_s 2^(m_s - max m) / sum, over at most
+    // kTailSplits splits.  The partial outputs are laid out as the accumulators are, so each lane reads back exactly
+    // its own elements.
     auto aload_f = [](const float *a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-    static_assert(kWavesPP * kMaxSplits * 32 * sizeof(float) == WTS_HALVES * sizeof(_Float16) && WTS_HALVES <= 2 * K_TILE, "merge weights exceed the K tile buffers");
-    float *wts = reinterpret_cast<float *>(&lds_all[0]) + w * (kMaxSplits * 32);
-    // One merge step for NS splits starting at s0: their outputs and, when WEIGHTS, the (m, l) records of
-    // MAXS splits are requested together; the weights go through LDS (lanes 32..63 need those of lanes 0..31).
-    auto load_outputs = [&](int s0, auto &raw, auto ns_tag) {
-        constexpr int NS = decltype(ns_tag)::value;
-#pragma unroll
-        for (int j = 0; j < NS; j++) {
-            const _Float16 *po = p.part_o + ((int64_t)min(s0 + j, p.nsplit - 1) * p.n_wb + wb) * (32 * D) + l32 * 4;
-#pragma unroll
-            for (int db = 0; db < DB; db++)
-#pragma unroll
-                for (int rq = 0; rq < 4; rq++)
-                    raw[j][db * 4 + rq] = __hip_atomic_load(reinterpret_cast<const uint64_t *>(po + (8 * db + 2 * rq + hb) * 128),
-                                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    };
     // Every lane works out the weights of its query into lv (lanes l and l + 32 the same ones, from the same
     // loads): nothing is handed from lane to lane.
-    auto weights = [&](auto maxs_tag, auto &lv) {
-        constexpr int MAXS = decltype(maxs_tag)::value;
-        float mv[MAXS];
+    auto weights = [&](float (&lv)[kTailSplits]) {
+        float mv[kTailSplits];
 #pragma unroll
-        for (int sp = 0; sp < MAXS; sp++) {
+        for (int sp = 0; sp < kTailSplits; sp++) {
             const float *ml = p.part_ml + ((int64_t)min(sp, p.nsplit - 1) * p.n_wb + wb) * 64;
             mv[sp] = aload_f(ml + l32);
             lv[sp] = aload_f(ml + 32 + l32);
         }
         float mm = -INFINITY;
 #pragma unroll
-        for (int sp = 0; sp < MAXS; sp++) mm = fmaxf(mm, mv[sp]);
+        for (int sp = 0; sp < kTailSplits; sp++) mm = fmaxf(mm, mv[sp]);
         const float m_ref = (mm == -INFINITY) ? 0.0f : mm;
         float total = 0.0f;
 #pragma unroll
-        for (int sp = 0; sp < MAXS; sp++) {
+        for (int sp = 0; sp < kTailSplits; sp++) {
             lv[sp] = sp < p.nsplit ? lv[sp] * fast_exp2(mv[sp] - m_ref) : 0.0f;
             total += lv[sp];
         }
         const float inv_total = total > 0.0f ? 1.0f / total : 0.0f;
 #pragma unroll
-        for (int sp = 0; sp < MAXS; sp++) lv[sp] *= inv_total;
+        for (int sp = 0; sp < kTailSplits; sp++) lv[sp] *= inv_total;
     };
-    auto accumulate = [&](int s0, auto &raw, auto ns_tag) {
-        constexpr int NS = decltype(ns_tag)::value;
+    // Everything in one round trip to the L2, and this workgroup's own partial, still in
+    // its accumulators, is not read back.  Every element is the chain fma(w3, O3, fma(w2, O2, fma(w1, O1,
+    // w0 O0))) over the splits in their order, the own term entering at its place with the f16 value that
+    // was stored: the result does not depend on which split arrived last.
+    uint64_t raw[3][DB * 4];   // the other splits in their order
 #pragma unroll
-        for (int j = 0; j < NS; j++) {
-            const float wgt = s0 + j < p.nsplit ? wts[(s0 + j) * 32 + l32] : 0.0f;
-#pragma unroll
-            for (int db = 0; db < DB; db++)
-#pragma unroll
-                for (int rq = 0; rq < 4; rq++) {
-                    const half4_t h4 = __builtin_bit_cast(half4_t, raw[j][db * 4 + rq]);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) o[db][4 * rq + i] += wgt * (float)h4[i];
-                }
-        }
-    };
-    auto zero_o = [&]() {
+    for (int j = 0; j < 3; j++) {
+        const int sj = min(j + (j >= split), p.nsplit - 1);
+        const _Float16 *po = p.part_o + ((int64_t)sj * p.n_wb + wb) * (32 * D) + l32 * 4;
 #pragma unroll
         for (int db = 0; db < DB; db++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) o[db][r] = 0.0f;
-    };
-    if (p.nsplit <= 4) {
-        // The common case: everything in one round trip to the L2, and this workgroup's own partial, still in
-        // its accumulators, is not read back.  Every element is the chain fma(w3, O3, fma(w2, O2, fma(w1, O1,
-        // w0 O0))) over the splits in their order, the own term entering at its place with the f16 value that
-        // was stored: the result does not depend on which split arrived last.
-        uint64_t raw[3][DB * 4];   // the other splits in their order
+            for (int rq = 0; rq < 4; rq++)
+                raw[j][db * 4 + rq] = __hip_atomic_load(reinterpret_cast<const uint64_t *>(po + (8 * db + 2 * rq + hb) * 128),
+                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    static_assert(kTailSplits == 4, "the chain below is written for four");
+    float wv[kTailSplits];   // 0 past the last split
+    weights(wv);
+    auto chain = [&](auto own_tag) {
+        constexpr int K = decltype(own_tag)::value;
 #pragma unroll
-        for (int j = 0; j < 3; j++) {
-            const int sj = min(j + (j >= split), p.nsplit - 1);
-            const _Float16 *po = p.part_o + ((int64_t)sj * p.n_wb + wb) * (32 * D) + l32 * 4;
+        for (int db = 0; db < DB; db++)
 #pragma unroll
-            for (int db = 0; db < DB; db++)
+            for (int rq = 0; rq < 4; rq++) {
+                half4_t h[3];
 #pragma unroll
-                for (int rq = 0; rq < 4; rq++)
-                    raw[j][db * 4 + rq] = __hip_atomic_load(reinterpret_cast<const uint64_t *>(po + (8 * db + 2 * rq + hb) * 128),
-                                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        float wv[4];   // 0 past the last split
-        weights(std::integral_constant<int, 4>{}, wv);
-        auto chain = [&](auto own_tag) {
-            constexpr int K = decltype(own_tag)::value;
+                for (int j = 0; j < 3; j++) h[j] = __builtin_bit_cast(half4_t, raw[j][db * 4 + rq]);
 #pragma unroll
-            for (int db = 0; db < DB; db++)
+                for (int i = 0; i < 4; i++) {
+                    const float mine = (float)partial_elem(o[db][4 * rq + i]);
+                    float acc = 0.0f;
 #pragma unroll
-                for (int rq = 0; rq < 4; rq++) {
-                    half4_t h[3];
-#pragma unroll
-                    for (int j = 0; j < 3; j++) h[j] = __builtin_bit_cast(half4_t, raw[j][db * 4 + rq]);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float mine = (float)partial_elem(o[db][4 * rq + i]);
-                        float acc = 0.0f;
-#pragma unroll
-                        for (int sp = 0; sp < 4; sp++) {
-                            const float term = sp == K ? mine : (float)h[sp < K ? sp : sp - 1][i];
-                            acc = sp == 0 ? wv[0] * term : __builtin_fmaf(wv[sp], term, acc);
-                        }
-                        o[db][4 * rq + i] = acc;
+                    for (int sp = 0; sp < 4; sp++) {
+                        const float term = sp == K ? mine : (float)h[sp < K ? sp : sp - 1][i];
+                        acc = sp == 0 ? wv[0] * term : __builtin_fmaf(wv[sp], term, acc);
                     }
-                    __builtin_amdgcn_sched_barrier(0);   // piece by piece: hoisting all the own-term products at once spills
+                    o[db][4 * rq + i] = acc;
                 }
-        };
-        switch (split) {
-            case 0: chain(std::integral_constant<int, 0>{}); break;
-            case 1: chain(std::integral_constant<int, 1>{}); break;
-            case 2: chain(std::integral_constant<int, 2>{}); break;
-            default: chain(std::integral_constant<int, 3>{}); break;
-        }
-    } else {
-        float wv[kMaxSplits];
-        weights(std::integral_constant<int, kMaxSplits>{}, wv);
-#pragma unroll
-        for (int sp = 0; sp < kMaxSplits; sp++) wts[sp * 32 + l32] = wv[sp];   // lanes l and l + 32 write the same value and read it back
-        zero_o();
-        for (int s0 = 0; s0 < p.nsplit; s0 += 2) {
-            uint64_t raw[2][DB * 4];
-            load_outputs(s0, raw, std::integral_constant<int, 2>{});
-            accumulate(s0, raw, std::integral_constant<int, 2>{});
-        }
+                __builtin_amdgcn_sched_barrier(0);   // piece by piece: hoisting all the own-term products at once spills
+            }
+    };
+    switch (split) {
+        case 0: chain(std::integral_constant<int, 0>{}); break;
+        case 1: chain(std::integral_constant<int, 1>{}); break;
+        case 2: chain(std::integral_constant<int, 2>{}); break;
+        default: chain(std::integral_constant<int, 3>{}); break;
     }
     write_output(1.0f);
 }
 
-// Merge of the key splits, one workgroup per 32-query block:
+// Merge of the key splits, D / 32 workgroups per 32-query block, 32 features each:
 //   out = sum_s w_s O_s / sum_s w_s,   w_s = l_s 2^(m_s - max m),   O_s normalised partial outputs.
-template <int D>
+// There is little to read (a block of 16 splits 4 KiB each for the 32 features) and all of it is requested before any of it
+// is used: a loop that went to memory split by split, in one workgroup per block, took 14.2 us for 16 splits of 64 blocks
+// where this takes 4.0.
+template <int D, int NS>   // nsplit <= NS
 __global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(PrefillPP p) {
-    constexpr int kMaxSplits = 16;
-    constexpr int OROW = D + 8;
-    __shared__ float wts[kMaxSplits][32];
+    constexpr int OROW = 32 + 8;
+    __shared__ float ms[NS][32], ls[NS][32];
     __shared__ __attribute__((aligned(16))) _Float16 tile[32 * OROW];
-    const int64_t wb = blockIdx.x;
-    const int tid = threadIdx.x;
-    if (tid < 32) {
-        float mm = -INFINITY;
-        for (int sp = 0; sp < p.nsplit; sp++) mm = fmaxf(mm, p.part_ml[((int64_t)sp * p.n_wb + wb) * 64 + tid]);
-        const float m_ref = (mm == -INFINITY) ? 0.0f : mm;
-        float total = 0.0f;
-        for (int sp = 0; sp < p.nsplit; sp++) {
-            const float *ml = p.part_ml + ((int64_t)sp * p.n_wb + wb) * 64;
-            const float wgt = ml[32 + tid] * fast_exp2(ml[tid] - m_ref);
-            wts[sp][tid] = wgt;
-            total += wgt;
-        }
-        const float inv = total > 0.0f ? 1.0f / total : 0.0f;
-        for (int sp = 0; sp < p.nsplit; sp++) wts[sp][tid] *= inv;
+    const int64_t wb = blockIdx.x / (D / 32);
+    const int f0 = 32 * (blockIdx.x % (D / 32));
+    const int tid = threadIdx.x, q = tid & 31, fg = tid >> 5;   // four features f0 + 4 fg .. of query q
+    half4_t h[NS];
+#pragma unroll
+    for (int sp = 0; sp < NS; sp++)
+        h[sp] = *reinterpret_cast<const half4_t *>(p.part_o + ((int64_t)min(sp, p.nsplit - 1) * p.n_wb + wb) * (32 * D) + (f0 / 4 + fg) * 128 + q * 4);
+#pragma unroll
+    for (int j = 0; j < NS * 64 / 256; j++) {
+        const int sp = 4 * j + (tid >> 6), i = tid & 63;   // record i of split sp: 32 maxima, then 32 sums
+        const float x = p.part_ml[((int64_t)min(sp, p.nsplit - 1) * p.n_wb + wb) * 64 + i];
+        (i < 32 ? ms : ls)[sp][i & 31] = x;
     }
     __syncthreads();
+    float mm = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < D / 32; j++) {
-        const int idx = j * 256 + tid;       // (feature group, query) in the partials' order
-        const int fg = idx >> 5, q = idx & 31;
-        float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int sp = 0; sp < p.nsplit; sp++) {
-            const half4_t h = *reinterpret_cast<const half4_t *>(p.part_o + ((int64_t)sp * p.n_wb + wb) * (32 * D) + idx * 4);
-            const float wgt = wts[sp][q];
+    for (int sp = 0; sp < NS; sp++) mm = fmaxf(mm, ms[sp][q]);   // (past the last split: the last one again)
+    const float m_ref = (mm == -INFINITY) ? 0.0f : mm;
+    float wv[NS], total = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc[i] += wgt * (float)h[i];
-        }
-        half4_t h4;
-#pragma unroll
-        for (int i = 0; i < 4; i++) h4[i] = (_Float16)acc[i];
-        *reinterpret_cast<half4_t *>(&tile[q * OROW + fg * 4]) = h4;
+    for (int sp = 0; sp < NS; sp++) {
+        wv[sp] = sp < p.nsplit ? ls[sp][q] * fast_exp2(ms[sp][q] - m_ref) : 0.0f;
+        total += wv[sp];
     }
+    const float inv = total > 0.0f ? 1.0f / total : 0.0f;
+    float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int sp = 0; sp < NS; sp++) {
+        if (sp < p.nsplit) {   // (the weight 0 would make a NaN of an infinity)
+            const float wgt = wv[sp] * inv;
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[i] += wgt * (float)h[sp][i];
+        }
+    }
+    half4_t h4;
+#pragma unroll
+    for (int i = 0; i < 4; i++) h4[i] = (_Float16)acc[i];
+    *reinterpret_cast<half4_t *>(&tile[q * OROW + fg * 4]) = h4;
     __syncthreads();
     const int64_t bh = wb / p.n_qb32;
-    const int q_first = (int)(wb % p.n_qb32) * 32;
-#pragma unroll
-    for (int j = 0; j < D / 64; j++) {
-        const int idx = j * 256 + tid;       // (query, 16-byte segment of its row)
-        const int q = idx / (D / 8), seg = idx % (D / 8);
-        if (q_first + q < p.Sq)
-            *reinterpret_cast<u32x4 *>(p.out + (bh * p.Sq + q_first + q) * D + seg * 8) =
-                *reinterpret_cast<const u32x4 *>(&tile[q * OROW + seg * 8]);
-    }
+    const int row = (int)(wb % p.n_qb32) * 32 + tid / 4, seg = tid % 4;   // (query, 16-byte segment of its 64 bytes)
+    if (tid < 128 && row < p.Sq)
+        *reinterpret_cast<u32x4 *>(p.out + (bh * p.Sq + row) * D + f0 + seg * 8) = *reinterpret_cast<const u32x4 *>(&tile[(tid / 4) * OROW + seg * 8]);
 }
 
 int env_int(const char *name, int dflt) {
@@ -891,6 +851,40 @@ int env_int(const char *name, int dflt) {
 bool ping_enabled() {
     static const int on = env_int("TROCM_PREFILL_PING", 0);
     return on != 0;
+}
+
+// Number of key splits: the one with the least expected time, us, over
+//   * the tile loop: 1.5 us per tile of 64 keys (D = 64: 1.0) for the longest workgroup's share, or for a compute unit's share of all
+//     tiles if that is more; up to half a share again where not all workgroups are resident (one per compute unit, D = 64: two; those
+//     left over are the shortest ones), and, for two on one unit, up to 0.8 of a share that they cost each other;
+//   * the merge: by the last split to arrive (at most kTailSplits) 3.5 + 0.26 per split, by a launch of its own 4 + 0.33 per split,
+//     and 0.5 for every 1024 blocks of 32 x 128 outputs and split.
+// (As many splits as there were workgroups missing for one per compute unit, rounded up, which this replaces, put 257 to 290
+// workgroups on 256 units, and 16 splits before a merge that costs more than the tiles it saves.)  Over 122 prompts of 24 to 1500
+// tokens behind 0 to 4096, each timed at every count: 1.1 % above the best of them on average, 11 % below the old rule.
+// (32 heads in groups of 4: 300 queries behind 3584 49.4 -> 36.7 us, 130 behind 3584 40.2 -> 28, 65 behind 740 21.4 -> 17.6; 2 x 64
+// heads x 415 queries 30.1 -> 21.1.)
+int64_t choose_splits(const PrefillPP &p, int D, int block_m, int64_t wgs1, int64_t cus, int64_t most) {
+    const int64_t longest = (p.Sk + kTileN - 1) / kTileN;   // tiles that the last query sees
+    int64_t all = wgs1 * longest;
+    if (p.causal) {
+        all = 0;
+        for (int qt = 0; qt < p.n_qtiles; qt++) all += (min((qt + 1) * block_m, p.Sq) - 1 + p.Sk - p.Sq) / kTileN + 1;
+        all *= wgs1 / p.n_qtiles;
+    }
+    const float even = p.causal ? (float)((min(block_m, p.Sq) - 1 + p.Sk - p.Sq) / kTileN + 1) / (float)longest : 1.0f;   // first query tile / last
+    const float tile = D == 64 ? 1.0f : 1.5f, slots = (float)(D == 64 ? 2 * cus : cus), busy = (float)all / slots;
+    int64_t best = 1;
+    float best_time = 0.0f;
+    for (int64_t n = 1; n <= kMaxSplits && n <= longest && (n == 1 || n <= most); n++) {
+        const float wgs = (float)(wgs1 * n), share = (float)((longest + n - 1) / n);
+        float time = tile * (share > busy ? share : busy);
+        if (wgs > slots) time += 0.5f * tile * share * (even + (1.0f - even) * fminf(1.0f, 2.5f * (wgs / slots - 1.0f)));
+        if (D == 64 && wgs > (float)cus) time += 0.8f * tile * share * fminf(1.0f, wgs / (float)cus - 1.0f);
+        if (n > 1) time += (n <= kTailSplits ? 3.5f + 0.26f * n : 4.0f + 0.33f * n) + 0.5f / 1024 / 128 * (float)(p.n_wb * D * n);
+        if (n == 1 || time < best_time) best = n, best_time = time;
+    }
+    return best;
 }
 
 template <int D, int HG>
@@ -908,7 +902,11 @@ int launch_cfg(const PrefillPP &p, int fmt, int64_t wgs, hipStream_t s) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail("sdpa_prefill_pp launch failed: %s", hipGetErrorString(e));
     if (p.nsplit > 1 && p.counters == nullptr) {
-        hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D>), dim3((unsigned)p.n_wb), dim3(256), 0, s, p);
+        const dim3 grid((unsigned)(p.n_wb * (D / 32)));
+        if (p.nsplit <= kMaxSplits / 2)
+            hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kMaxSplits / 2>), grid, dim3(256), 0, s, p);
+        else
+            hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kMaxSplits>), grid, dim3(256), 0, s, p);
         e = hipGetLastError();
         if (e != hipSuccess) return fail("sdpa_prefill_merge launch failed: %s", hipGetErrorString(e));
     }
@@ -935,7 +933,7 @@ size_t prefill_workspace_bytes(int64_t B, int64_t Hq, int64_t Sq, int64_t D) {
     const int64_t cus = 256;
     if (wgs1 >= cus) return 0;
     int64_t ns = (cus + wgs1 - 1) / wgs1;
-    if (ns > 16) ns = 16;
+    if (ns > kMaxSplits) ns = kMaxSplits;
     return (size_t)ns * split_bytes(B * Hq * ((Sq + 31) / 32), D) + 256;
 }
 
@@ -969,11 +967,9 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
     const int block_m = 32 * kWavesPP / hg;
     const int64_t n_qtiles = (a.Sq + block_m - 1) / block_m;
     // Waves whose 32-query block lies past q_len idle.  Few queries come here with a mask, from short quantised caches, or
-    // as more groups of 32 rows than pay on the decode tiles (sdpa_decode_rows_fits).  With several heads per workgroup this is
-    // still the better of the two prefill kernels for them: K and V are read once per kv head instead of once per query
-    // head (8 x 32 heads x 4 queries over 8192 tokens: 66 us against 183 us).  With one head per workgroup short prompts
-    // go to the smaller kernel.  (Quantised caches have no smaller kernel: they stay here whatever the prompt length.)
-    if (hg == 1 && !quant && a.Sq * 2 < n_qtiles * block_m) return 2;
+    // as more groups of 32 rows than pay on the decode tiles (sdpa_decode_rows_fits).  That is still the better of the two prefill
+    // kernels for them: K and V are read once per group of heads and the keys are split (8 x 32 heads in groups of 4 x 4 queries over
+    // 8192 tokens: 66 us against 183; 14 heads in groups of 7 x 100 queries behind 4000: 91 against 24, and behind none 10.8 against 10.0).
 
     PrefillPP p;
     memset(&p, 0, sizeof(p));
@@ -1001,16 +997,10 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
 
     const int64_t wgs1 = a.B * (a.Hq / hg) * n_qtiles;
     const int64_t cus = num_compute_units();
-    int64_t ns = 1;
-    if (wgs1 < cus) {
-        ns = (cus + wgs1 - 1) / wgs1;
-        const int64_t tiles = (a.Sk + kTileN - 1) / kTileN;
-        if (ns > tiles / 2) ns = tiles / 2;   // at least two tiles per split
-        if (ns > 16) ns = 16;
-    }
-    if (forced_split > 0) ns = forced_split < 16 ? forced_split : 16;   // the merges handle at most 16 splits
     const size_t per_split = split_bytes(p.n_wb, a.D);
     const size_t avail = a.workspace && a.workspace_bytes > kWsCounterBytes + 256 ? a.workspace_bytes - kWsCounterBytes - 256 : 0;
+    int64_t ns = forced_split < kMaxSplits ? forced_split : kMaxSplits;
+    if (forced_split <= 0) ns = wgs1 < cus ? choose_splits(p, (int)a.D, block_m, wgs1, cus, (int64_t)(avail / per_split)) : 1;
     if (ns > 1 && (size_t)ns * per_split > avail) ns = (int64_t)(avail / per_split);
     if (ns < 1) ns = 1;
     p.nsplit = (int)ns;
@@ -1022,9 +1012,17 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
         // With few enough tiles for the counter area the last split to arrive merges (no second launch);
         // TROCM_PREFILL_TAIL_MERGE=0 keeps the merge launch.
         static const int tail_merge = env_int("TROCM_PREFILL_TAIL_MERGE", 1);
-        if (tail_merge && ns <= 16 && wgs1 <= (int64_t)(kWsCounterBytes / sizeof(int))) p.counters = (int *)a.workspace;
+        if (tail_merge && ns <= kTailSplits && wgs1 <= (int64_t)(kWsCounterBytes / sizeof(int))) p.counters = (int *)a.workspace;
     }
     const int64_t wgs = wgs1 * ns;
+    // Order of the workgroups of a causal prompt.  Where two fit on a compute unit (D = 64) and there are at most so many, all are
+    // resident at once: the shortest tiles go beside the longest (3 x 40 heads x 574 queries behind 1717: 77.7 -> 60.8 us).  Otherwise a
+    // prompt whose tiles differ much runs the longest of all its sequences first (3 x 32 x 1414 at D = 128: 83.9 -> 75.3), and one
+    // behind many tokens one sequence after the other, whose K and V then stay in the L2 (3 x 32 x 1377 behind 752: 128, not 138).
+    if (a.causal && a.D == 64 && wgs > cus && wgs <= 2 * cus)
+        p.paired = (int)((cus + wgs / n_qtiles - 1) / (wgs / n_qtiles));
+    else if (a.causal && a.B > 1 && 5 * a.Sq > 4 * a.Sk)
+        p.paired = (int)n_qtiles;
     if (wgs >= (1ll << 31)) return 2;
     return a.D == 128 ? launch_hg<128>(p, a.kv_fmt, hg, wgs, s) : launch_hg<64>(p, a.kv_fmt, hg, wgs, s);
 }
