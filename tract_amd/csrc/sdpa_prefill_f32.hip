@@ -44,6 +44,7 @@
 // 2 x 251, a workgroup per compute unit, 25.0 | 33.7.
 #include <hip/hip_runtime.h>
 #include <string.h>
+#include <algorithm>
 #include "decode_common.h"
 
 namespace trocm {
@@ -634,6 +635,34 @@ int launch(const PrefillF32 &p, hipStream_t s) {
 
 // 2 = not taken (the generic kernel runs): masks, other types and head sizes, rows that see no key, unaligned rows, a kv
 // head of 4 GB or more.
+// Ranges of keys for sdpa_prefill_f32x2_kernel: the number with the least expected time, in us.  1.5 (D = 64: 1.0) for each pair of
+// tiles of the longest range, or of a compute unit's half of all tiles if that is more; where more than one workgroup shares a compute
+// unit up to 1.9 times that again, and a quarter where not all are resident; 2.5 + 0.12 a range for the merge, and 0.85 for every
+// 1024 blocks of 32 x 128 outputs and range.  55 drawn prompts, each timed at 1 .. 32 ranges: 1.2 % above the best of them on
+// average; ranges of 4 or 16 tiles, as many as two workgroups per compute unit allow, were 2.9 % above (2 x 14 heads x 7 queries
+// behind 401: 20.8 -> 18.7 us; 14 x 143 behind 1750: 30.2 -> 27.9; 3 x 32 x 79 behind 276: 30.9 -> 26.5).
+static int64_t choose_pair_splits(const PrefillF32 &p, int D, int64_t tiles, int64_t n_wg, int64_t cus) {
+    int64_t all = tiles * n_wg;
+    if (p.causal) {
+        all = 0;
+        for (int rt = 0; rt < p.n_rt2; rt++) all += ((std::min(2 * kRows * (rt + 1), p.Sq * p.G) - 1) / p.G + p.Sk - p.Sq + 1 + 31) / 32;
+        all *= p.n_bh;
+    }
+    const float pair = D == 64 ? 1.0f : 1.5f, busy = (float)all / (float)(4 * cus);
+    int64_t best = 1;
+    float best_time = 0.0f;
+    for (int64_t n = 1; n <= kMaxSplits && (n == 1 || 2 * n <= tiles); n++) {
+        const float per_unit = (float)(n_wg * n) / (float)cus, range = (float)(((tiles + n - 1) / n + 1) / 2);
+        float time = range > busy ? range : busy;
+        if (per_unit > 1.0f) time += 1.9f * range * std::min(1.0f, per_unit - 1.0f);
+        if (per_unit > 2.0f) time += 0.25f * range * std::min(1.0f, per_unit / 2.0f - 1.0f);
+        time *= pair;
+        if (n > 1) time += 2.5f + 0.12f * n + 0.85f / 1024 / 128 * (float)((int64_t)p.n_bh * p.n_rt * D * n);
+        if (n == 1 || time < best_time) best = n, best_time = time;
+    }
+    return best;
+}
+
 int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
     if (a.q_dtype != TROCM_F32 || a.kv_fmt != TROCM_F32 || a.mask) return 2;
     if (a.D != 128 && a.D != 64) return 2;
@@ -654,14 +683,19 @@ int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
     p.n_bh = (int)(a.B * a.Hkv), p.n_rt = (int)((a.Sq * G + kRows - 1) / kRows);
     p.causal = a.causal, p.scale = a.scale;
 
-    // Pairs of f16 from 33 rows and 4 tiles on.  Ranges of at least 4 tiles (16 where half the compute units have a workgroup).
-    const int64_t tiles = (a.Sk + 31) / 32, cus = num_compute_units(), want = 2 * cus;
-    const bool pairs = p.n_rt > 1 && tiles >= 4 && a.scale >= 0x1p-16f && a.scale <= 0x1p16f;
-    if (pairs) p.n_rt2 = (int)((a.Sq * G + 2 * kRows - 1) / (2 * kRows));
+    // Pairs of f16 from 33 rows and 5 tiles on; 4 where half the compute units have a workgroup (3 x 32 heads x 117 queries 20.6 -> 18.2
+    // us; but 14 x 107, whose four tiles go to a workgroup's four waves at once on the f32 instruction, 14.0, not 16.8).
+    const int64_t tiles = (a.Sk + 31) / 32, cus = num_compute_units(), want = 2 * cus, n_rt2 = (a.Sq * G + 2 * kRows - 1) / (2 * kRows);
+    const bool pairs = p.n_rt > 1 && (tiles >= 5 || (tiles == 4 && 2 * p.n_bh * n_rt2 > cus)) && a.scale >= 0x1p-16f && a.scale <= 0x1p16f;
+    if (pairs) p.n_rt2 = (int)n_rt2;
     const int64_t n_wb = (int64_t)p.n_bh * p.n_rt, n_wg = pairs ? (int64_t)p.n_bh * p.n_rt2 : n_wb;
-    int64_t ns = pairs ? want / n_wg : n_wg < want ? (want + n_wg - 1) / n_wg : 1;
-    const int64_t most = tiles / (pairs && 2 * n_wg > cus ? 16 : 4);
-    ns = ns < most ? ns : most;
+    int64_t ns;
+    if (pairs) {
+        ns = n_wg < want ? choose_pair_splits(p, (int)a.D, tiles, n_wg, cus) : 1;
+    } else {   // ranges of at least 4 tiles
+        ns = n_wg < want ? (want + n_wg - 1) / n_wg : 1;
+        ns = ns < tiles / 4 ? ns : tiles / 4;
+    }
     ns = ns < kMaxSplits ? ns : kMaxSplits;
     p.paired = pairs && a.causal && n_wg <= want;
     const size_t per_split = (size_t)n_wb * (kRows * a.D + 64) * sizeof(float);
