@@ -2598,7 +2598,8 @@ bool sdpa_decode_rows_fits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64
         // 32 over 8: 2 x 962, 14 queries 37.1 | 33.6, 1 x 906, 16 queries 37.1 | 31.1; 16 over 8, 2 x 6759, 39 queries 65.8 | 70.4
         return BH <= (n_groups < 4 ? 48 : 32) && Sk >= 900;
     }
-    // Odd groups (sdpa_prefill.hip, a workgroup per head and 64 queries): up to a workgroup per compute unit (24 heads over 8,
+    // Odd groups.  The figures are against a prefill kernel of a workgroup per head and 64 queries that did not split the keys; against
+    // the one that does (sdpa_prefill_pp.hip) all lines here together cost 2 % over the faster side of 170 calls.  Up to a workgroup per compute unit (24 heads over 8,
     // 64 queries: 8 x 314 tokens 35.4 | 43.5 with 384, 4 x 1064 55.0 | 46.0 with 192; 32 over 32, 33 queries, 4 x 1033, 256: 65.0 |
     // 54.5); where it needs a second round as many as do not read more (40 over 8, 33 queries: 16 x 283 60.2 | 53.5, 16 x 4445 561 |
     // 487, but one round, 6 x 3389, 38 queries 154 | 194) or two per compute unit (24 over 8, 16 x 283, 33 queries 57.0 | 46.4); rows

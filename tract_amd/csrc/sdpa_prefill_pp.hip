@@ -1,4 +1,4 @@
-// MFMA prefill attention for gfx950, throughput version for q_len >= 32 (GQA heads share K/V tiles).
+// MFMA prefill attention for gfx950, for two and more queries (GQA heads share K/V tiles).
 // f16 in/out, f32 accumulate, causal (bottom-right aligned), unmasked or with an additive mask input, GQA,
 // K/V read in place.
 //
