@@ -54,6 +54,8 @@ struct PrefillPP {
     int B, Hq, Hkv, Sq, Sk;
     int causal;
     int n_qtiles, nsplit;
+    float lazy_max;
+    int part32;         // the partials are f32, merged by a launch
     int paired;         // != 0: how many query tiles make up a first workgroup for every compute unit, where each holds two
     float scale_log2;
     // Partials of key split s and 32-query block wb (= (b * Hq + qh) * n_qb32 + q / 32):
@@ -336,10 +338,10 @@ __global__ __launch_bounds__(kThreadsPP, D == 64 && !MASK ? 4 : 2) void sdpa_pre
             for (int r = 0; r < 16; r++) tmax = fmaxf(tmax, s[kb][r]);
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
         // The reference of the exponentials follows the maximum lazily: it moves only when this tile's maximum exceeds it
-        // by more than kLazyMax (the exponentials then reach 2^kLazyMax at most, far inside f16 and f32 range), so the
+        // by more than lazy_max, at most kLazyMax (the exponentials then reach 2^kLazyMax at most, far inside f16 and f32 range), so the
         // accumulators are rescaled a few times per sequence instead of at most tiles; o / l does not depend on it.
         const float t_scaled = MASK ? tmax : tmax * p.scale_log2;   // scale > 0: the maximum commutes with the scaling
-        const bool moved = t_scaled > m_run + kLazyMax;   // also the first visible key (reference -inf); never for a maximum of -inf
+        const bool moved = t_scaled > m_run + p.lazy_max;   // also the first visible key (reference -inf); never for a maximum of -inf
         const float m_new = moved ? t_scaled : m_run;
         const float m_ref = (m_new == -INFINITY) ? 0.0f : m_new;  // nothing visible yet: keep everything at zero
         float psum = 0.0f;
@@ -683,7 +685,10 @@ __global__ __launch_bounds__(kThreadsPP, D == 64 && !MASK ? 4 : 2) void sdpa_pre
 #pragma unroll
                 for (int i = 0; i < 4; i++) h4[i] = partial_elem(o[db][4 * rq + i]);
                 _Float16 *dst = po + (8 * db + 2 * rq + hb) * 128;
-                if (tail_merge)
+                if (p.part32) {
+                    float *d32 = reinterpret_cast<float *>(p.part_o) + ((int64_t)split * p.n_wb + wb) * (32 * D) + l32 * 4 + (8 * db + 2 * rq + hb) * 128;
+                    *reinterpret_cast<float4_t *>(d32) = float4_t{o[db][4 * rq] * inv, o[db][4 * rq + 1] * inv, o[db][4 * rq + 2] * inv, o[db][4 * rq + 3] * inv};
+                } else if (tail_merge)
                     __hip_atomic_store(reinterpret_cast<uint64_t *>(dst), __builtin_bit_cast(uint64_t, h4), __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
                 else
@@ -792,7 +797,7 @@ __global__ __launch_bounds__(kThreadsPP, D == 64 && !MASK ? 4 : 2) void sdpa_pre
 // There is little to read (a block of 16 splits 4 KiB each for the 32 features) and all of it is requested before any of it
 // is used: a loop that went to memory split by split, in one workgroup per block, took 14.2 us for 16 splits of 64 blocks
 // where this takes 4.0.
-template <int D, int NS>   // nsplit <= NS
+template <int D, int NS, typename T>   // nsplit <= NS
 __global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(PrefillPP p) {
     constexpr int OROW = 32 + 8;
     __shared__ float ms[NS][32], ls[NS][32];
@@ -800,10 +805,11 @@ __global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(PrefillPP p) {
     const int64_t wb = blockIdx.x / (D / 32);
     const int f0 = 32 * (blockIdx.x % (D / 32));
     const int tid = threadIdx.x, q = tid & 31, fg = tid >> 5;   // four features f0 + 4 fg .. of query q
-    half4_t h[NS];
+    typedef T vec4 __attribute__((ext_vector_type(4)));
+    vec4 h[NS];
 #pragma unroll
     for (int sp = 0; sp < NS; sp++)
-        h[sp] = *reinterpret_cast<const half4_t *>(p.part_o + ((int64_t)min(sp, p.nsplit - 1) * p.n_wb + wb) * (32 * D) + (f0 / 4 + fg) * 128 + q * 4);
+        h[sp] = *reinterpret_cast<const vec4 *>(reinterpret_cast<const T *>(p.part_o) + ((int64_t)min(sp, p.nsplit - 1) * p.n_wb + wb) * (32 * D) + (f0 / 4 + fg) * 128 + q * 4);
 #pragma unroll
     for (int j = 0; j < NS * 64 / 256; j++) {
         const int sp = 4 * j + (tid >> 6), i = tid & 63;   // record i of split sp: 32 maxima, then 32 sums
@@ -881,7 +887,7 @@ int64_t choose_splits(const PrefillPP &p, int D, int block_m, int64_t wgs1, int6
         float time = tile * (share > busy ? share : busy);
         if (wgs > slots) time += 0.5f * tile * share * (even + (1.0f - even) * fminf(1.0f, 2.5f * (wgs / slots - 1.0f)));
         if (D == 64 && wgs > (float)cus) time += 0.8f * tile * share * fminf(1.0f, wgs / (float)cus - 1.0f);
-        if (n > 1) time += (n <= kTailSplits ? 3.5f + 0.26f * n : 4.0f + 0.33f * n) + 0.5f / 1024 / 128 * (float)(p.n_wb * D * n);
+        if (n > 1) time += (n <= kTailSplits && !p.part32 ? 3.5f + 0.26f * n : 4.0f + 0.33f * n) + 0.5f / 1024 / 128 * (float)(p.n_wb * D * n);
         if (n == 1 || time < best_time) best = n, best_time = time;
     }
     return best;
@@ -903,10 +909,15 @@ int launch_cfg(const PrefillPP &p, int fmt, int64_t wgs, hipStream_t s) {
     if (e != hipSuccess) return fail("sdpa_prefill_pp launch failed: %s", hipGetErrorString(e));
     if (p.nsplit > 1 && p.counters == nullptr) {
         const dim3 grid((unsigned)(p.n_wb * (D / 32)));
-        if (p.nsplit <= kMaxSplits / 2)
-            hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kMaxSplits / 2>), grid, dim3(256), 0, s, p);
+        const bool few = p.nsplit <= kMaxSplits / 2;
+        if (p.part32 && few)
+            hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kMaxSplits / 2, float>), grid, dim3(256), 0, s, p);
+        else if (p.part32)
+            hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kMaxSplits, float>), grid, dim3(256), 0, s, p);
+        else if (few)
+            hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kMaxSplits / 2, _Float16>), grid, dim3(256), 0, s, p);
         else
-            hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kMaxSplits>), grid, dim3(256), 0, s, p);
+            hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kMaxSplits, _Float16>), grid, dim3(256), 0, s, p);
         e = hipGetLastError();
         if (e != hipSuccess) return fail("sdpa_prefill_merge launch failed: %s", hipGetErrorString(e));
     }
@@ -924,7 +935,7 @@ int launch_hg(const PrefillPP &p, int fmt, int hg, int64_t wgs, hipStream_t s) {
 
 }  // namespace
 
-static size_t split_bytes(int64_t n_wb, int64_t D) { return (size_t)n_wb * (32 * (size_t)D * sizeof(_Float16) + 64 * sizeof(float)); }
+static size_t split_bytes(int64_t n_wb, int64_t D, size_t elem = sizeof(_Float16)) { return (size_t)n_wb * (32 * (size_t)D * elem + 64 * sizeof(float)); }
 
 // Upper bound of the partial-result area the staggered prefill kernel may use for this shape.
 size_t prefill_workspace_bytes(int64_t B, int64_t Hq, int64_t Sq, int64_t D) {
@@ -971,6 +982,9 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
     // kernels for them: K and V are read once per group of heads and the keys are split (8 x 32 heads in groups of 4 x 4 queries over
     // 8192 tokens: 66 us against 183; 14 heads in groups of 7 x 100 queries behind 4000: 91 against 24, and behind none 10.8 against 10.0).
 
+    // (With a mask and one head per workgroup short prompts stay on the generic kernel, whose weights are f32.)
+    if (hg == 1 && a.mask && a.Sq * 2 < n_qtiles * block_m) return 2;
+
     PrefillPP p;
     memset(&p, 0, sizeof(p));
     p.q = (const _Float16 *)a.q;
@@ -988,6 +1002,11 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
     p.n_qtiles = (int)n_qtiles;
     p.n_qb32 = (int)((a.Sq + 31) / 32);
     p.n_wb = a.B * a.Hq * p.n_qb32;
+    // Short prompts of one head per workgroup, f16 caches: partials in f32.  (The smaller kernel, which these came from, held a result
+    // in f32 to its end: f16 partials made the error against 64 bits 1.27 times what it was, 2.7e-4 -> 3.5e-4; f32 ones leave it there.)
+    // (And with the maximum itself as the reference: the largest weight is then 1, without an error; 1.03 to 1.07 times otherwise.)
+    p.part32 = hg == 1 && !quant && a.Sq * 2 < n_qtiles * block_m;
+    p.lazy_max = p.part32 ? 0.0f : kLazyMax;
     if (a.mask) {   // [mask_b, mask_h, Sq, Sk] dense
         p.mask = (const _Float16 *)a.mask;
         p.mask_stride_h = a.mask_h > 1 ? a.Sq * a.Sk : 0;
@@ -997,7 +1016,7 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
 
     const int64_t wgs1 = a.B * (a.Hq / hg) * n_qtiles;
     const int64_t cus = num_compute_units();
-    const size_t per_split = split_bytes(p.n_wb, a.D);
+    const size_t elem = p.part32 ? sizeof(float) : sizeof(_Float16), per_split = split_bytes(p.n_wb, a.D, elem);
     const size_t avail = a.workspace && a.workspace_bytes > kWsCounterBytes + 256 ? a.workspace_bytes - kWsCounterBytes - 256 : 0;
     int64_t ns = forced_split < kMaxSplits ? forced_split : kMaxSplits;
     if (forced_split <= 0) ns = wgs1 < cus ? choose_splits(p, (int)a.D, block_m, wgs1, cus, (int64_t)(avail / per_split)) : 1;
@@ -1008,11 +1027,11 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
         char *base = (char *)a.workspace + kWsCounterBytes;
         base += (256 - ((uintptr_t)base & 255)) & 255;
         p.part_o = (_Float16 *)base;
-        p.part_ml = (float *)(base + (size_t)ns * p.n_wb * 32 * a.D * sizeof(_Float16));
+        p.part_ml = (float *)(base + (size_t)ns * p.n_wb * 32 * a.D * elem);
         // With few enough tiles for the counter area the last split to arrive merges (no second launch);
         // TROCM_PREFILL_TAIL_MERGE=0 keeps the merge launch.
         static const int tail_merge = env_int("TROCM_PREFILL_TAIL_MERGE", 1);
-        if (tail_merge && ns <= kTailSplits && wgs1 <= (int64_t)(kWsCounterBytes / sizeof(int))) p.counters = (int *)a.workspace;
+        if (tail_merge && !p.part32 && ns <= kTailSplits && wgs1 <= (int64_t)(kWsCounterBytes / sizeof(int))) p.counters = (int *)a.workspace;
     }
     const int64_t wgs = wgs1 * ns;
     // Order of the workgroups of a causal prompt.  Where two fit on a compute unit (D = 64) and there are at most so many, all are
