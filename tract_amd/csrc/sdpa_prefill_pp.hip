@@ -864,7 +864,8 @@ bool ping_enabled() {
 //     tiles if that is more; up to half a share again where not all workgroups are resident (one per compute unit, D = 64: two; those
 //     left over are the shortest ones), and, for two on one unit, up to 0.8 of a share that they cost each other;
 //   * the merge: by the last split to arrive (at most kTailSplits) 3.5 + 0.26 per split, by a launch of its own 4 + 0.33 per split,
-//     and 0.5 for every 1024 blocks of 32 x 128 outputs and split.
+//     and 0.5 for every 1024 blocks of 32 x 128 outputs and split; 4 where the partials are f32 (40 heads x 70 queries behind 300: 1 split 14.8
+//     us, 6 17.1; behind 1500 38.8 and 19.8).
 // (As many splits as there were workgroups missing for one per compute unit, rounded up, which this replaces, put 257 to 290
 // workgroups on 256 units, and 16 splits before a merge that costs more than the tiles it saves.)  Over 122 prompts of 24 to 1500
 // tokens behind 0 to 4096, each timed at every count: 1.1 % above the best of them on average, 11 % below the old rule.
@@ -887,7 +888,7 @@ int64_t choose_splits(const PrefillPP &p, int D, int block_m, int64_t wgs1, int6
         float time = tile * (share > busy ? share : busy);
         if (wgs > slots) time += 0.5f * tile * share * (even + (1.0f - even) * fminf(1.0f, 2.5f * (wgs / slots - 1.0f)));
         if (D == 64 && wgs > (float)cus) time += 0.8f * tile * share * fminf(1.0f, wgs / (float)cus - 1.0f);
-        if (n > 1) time += (n <= kTailSplits && !p.part32 ? 3.5f + 0.26f * n : 4.0f + 0.33f * n) + 0.5f / 1024 / 128 * (float)(p.n_wb * D * n);
+        if (n > 1) time += (n <= kTailSplits && !p.part32 ? 3.5f + 0.26f * n : 4.0f + 0.33f * n) + (p.part32 ? 4.0f : 0.5f) / 1024 / 128 * (float)(p.n_wb * D * n);
         if (n == 1 || time < best_time) best = n, best_time = time;
     }
     return best;
