@@ -66,6 +66,56 @@ def test_values_outside_the_pairs(rt, D, what):
         assert np.linalg.norm(got[..., d] - want[..., d]) <= 4e-6 * np.linalg.norm(want[..., d]), d
 
 
+def _late(rng, heads, kv, past, n, D):
+    """Queries that weigh the keys from 64 on only (scores 24 against -24)."""
+    q, k, v = _normal(rng, 1, heads, n, D), _normal(rng, 1, kv, past + n, D), _normal(rng, 1, kv, past + n, D)
+    q[..., 0], k[..., 0] = 4 * np.sqrt(D), 6
+    k[:, :, :64, 0] = -6
+    return q, k, v
+
+
+# what starts beyond the first tiles of a range, where V's scale was taken; 30 queries behind 3000 tokens: many ranges of keys
+@pytest.mark.parametrize("what", ["weak later", "weaker later", "gone later", "feature later", "weaker feature later", "feature of few keys",
+                                  "first row weak", "wide channels", "wide channels later", "zero values", "values later"])
+@pytest.mark.parametrize("D,past,n", [(64, 150, 70), (128, 150, 70), (128, 0, 220), (128, 3000, 30)])
+def test_values_that_change_along_the_keys(rt, D, past, n, what):
+    """Every feature and every row of the result to f32's precision, wherever the magnitudes change."""
+    rng = np.random.default_rng(D + past)
+    heads, kv, T = 4, 2, past + n
+    if what in ("weak later", "weaker later", "gone later"):
+        q, k, v = _late(rng, heads, kv, past, n, D)
+        v[:, :, 64:] *= np.float32({"weak later": 1e-8, "weaker later": 1e-10, "gone later": 1e-16}[what])
+    else:
+        q, k, v = _normal(rng, 1, heads, n, D), _normal(rng, 1, kv, T, D), _normal(rng, 1, kv, T, D)
+    if what in ("feature later", "weaker feature later"):
+        v[:, :, :70, 7] = 0
+        v[:, :, 70:, 7] *= np.float32(2.0 ** (-20 if what == "feature later" else -26))
+    elif what == "feature of few keys":   # strong in the first 64, which these queries hardly weigh
+        q, k, v = _late(rng, heads, kv, past, n, D)
+        v[:, :, 64:, 9] *= np.float32(2.0 ** -24)
+    elif what == "first row weak":
+        v[:, :, 0] *= np.float32(1e-9)
+    elif what == "wide channels":
+        q[..., [3, 11, 40, 41]] *= 20
+        k[..., [3, 11, 40, 41]] *= 20
+    elif what == "wide channels later":
+        k[:, :, 130:, 5] *= 200
+    elif what == "zero values":
+        v[:] = 0
+    elif what == "values later":
+        v[:, :, :130] = 0
+    got, want = _run(q, k, v, past).astype(np.float64), textbook_sdpa(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), causal=True)
+    # A score is a sum of D products of the size |q| |k| scale at most, rounded D times by 2^-25 of that: sqrt(D) of them in each weight
+    # and again in their sum.  Over many rows and keys of scores that are alike this averages out, and a few 2^-24 remain; not in a
+    # single row, nor where one product makes up every score.
+    row = max(4e-6, 2 * np.sqrt(D) * 2.0 ** -25 * np.linalg.norm(q, axis=-1).max() * np.linalg.norm(k, axis=-1).max() / np.sqrt(D))
+    feature = 4e-6 if np.abs(q).max() < 6 and np.abs(k).max() < 6 else row
+    err = got - want
+    for d in range(D):
+        assert np.linalg.norm(err[..., d]) <= feature * np.linalg.norm(want[..., d]), d
+    assert (np.linalg.norm(err, axis=-1) <= row * np.linalg.norm(want, axis=-1)).all()
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_a_later_infinity_stays_out(rt, D):
     rng = np.random.default_rng(D)

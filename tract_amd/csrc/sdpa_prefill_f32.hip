@@ -32,9 +32,13 @@
 // over 8, 2.7e-7, 771 over 451 past tokens 3.9e-7 (the f32 instruction: 3.3e-7, 4.7e-7).
 //  * Two row tiles of 32 per workgroup and two key sets of two waves: a set's waves share the 32-key tiles that its 128 threads turn
 //    into pairs on the way into LDS (K by rows, V transposed into the order in which P comes out of the scores).
-//  * Scales: q's per row, K's and V's from the first tiles of the range with room for 8 times as much.  What does not fit (larger
-//    values later, infinities and NaN, features of V 2^13 weaker than the strongest, scores beyond 2^14) shows as a flag or as a sum
-//    that is no number at the end, and the row tile is done again by the f32 code (attend_tile).
+//  * Scales, powers of two: q's per row, K's and V's from the first two tiles of the range, with room for 16 to 32 (K) and 8 to 16 (V)
+//    times their largest value in what comes later.  A pair is exact to 2^-23 of its number, or to 2^-25 in the scaled unit where
+//    that is more.  What this leaves of K changes a score by at most |q| sqrt(D) scale 2^-25 / k_up, which has to be below 2^-21 (a
+//    few 2^-24 as a rule), and no feature of V may be 2^13 weaker than the strongest in those tiles.
+//  * Otherwise, and where what comes later does not fit, which is seen in the sums, the workgroup starts again with the f32 code (attend_tile): values beyond the room, infinities
+//    and NaN (sums that are no numbers), and V that has become too weak for its unit (a row, or a feature over all the rows, that is
+//    small against what the pairs leave).
 //  * What bounds it is the issue of instructions: per tile and wave 48 matrix and about 550 vector instructions, whose busy cycles
 //    add up to 97 % of the kernel's (counters; 2000 queries: 33 and 64 %).  Loads have no condition around them, or the waits for
 //    one tile's V would be waits for the next tile's K (71.6 -> 58.2 us).
@@ -56,7 +60,11 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kRows = 32, kMaxSplits = 64;
-constexpr float kScoreRange = 0x1p14f;
+// least result, in V's scaled unit: the sum of a row's magnitudes, and the strongest row of a feature.  What the pairs leave, 2^-25 of
+// that unit at most for each number, is then below 2^-22 of a row's norm and 2^-21 of a feature, as much as f32 sums leave.  (A mean of
+// n keys of normal V is about 2^10 / sqrt(n) in that unit: only rows that weigh ten thousands of keys all alike, or features a
+// thousand times weaker than the strongest, fall below these by chance.)
+constexpr float kLeastOfRow = 16.0f, kLeastOfFeature = 0.0625f;
 
 struct PrefillF32 {
     const float *q, *k, *v;
@@ -302,9 +310,9 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32_kernel(PrefillF3
 // ---- more than 32 rows: every f32 as a pair of f16 ---------------------------------------------------------------------
 __device__ __forceinline__ int exp_field(float x) { return (int)(__builtin_bit_cast(uint32_t, x) >> 23) & 255; }
 __device__ __forceinline__ float pow2_field(int e) { return __builtin_bit_cast(float, (uint32_t)min(max(e, 0), 254) << 23); }
-// exponent field of the scale that puts `largest` in 2^13 .. 2^14: room for eight times as much (at most 2^55, so that products of
-// two scales and their inverses are normal numbers)
-__device__ __forceinline__ int up_field(float largest) { return min(267 - exp_field(largest), 127 + 55); }
+// exponent field of the scale that puts `largest` in 2^top .. 2^(top + 1) (at most 2^55, so that products of two scales and their
+// inverses are normal numbers)
+__device__ __forceinline__ int up_field(float largest, int top) { return min(254 + top - exp_field(largest), 127 + 55); }
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 // x times a power of two as the sum of two f16 numbers, each rounded once: 23 of its 24 bits.  (Six operations for a pair, all at
 // the full rate: the instructions that multiply, add and round to f16 in one, five for a pair, take two cycles for one.)
@@ -342,8 +350,10 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
     constexpr int T = D / 32, C4 = D / 4, NG = 8 * C4 / 128, KROW = D + 8, ROW = D + 4;
     typedef typename VecOf<T>::type vec;
     __shared__ __attribute__((aligned(16))) union { PairLds<D> pair; TileLds<D> tile; float rows[2 * kRows * ROW]; } lds;
-    __shared__ float lds_m[kWaves][kRows], lds_l[kWaves][kRows], lds_big[3][kWaves];
+    __shared__ float lds_m[kWaves][kRows], lds_l[kWaves][kRows], lds_big[4][kWaves];
+    __shared__ __attribute__((aligned(16))) float lds_least[2 * kRows];   // by row: what a feature has to reach
     __shared__ int lds_odd;
+    __shared__ uint64_t lds_strong[kWaves];
 
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hb = lane >> 5;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6), rg = w & 1, ks = w >> 1;
@@ -402,23 +412,14 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
             for (int e = 0; e < 4; e++) big = fmaxf(big, fabsf(x[j][e]));
         }
         big = fmaxf(big, __shfl_xor(big, 32, 64));
-        const int q_field = up_field(big);
+        const int q_field = up_field(big, 13);
 #pragma unroll
         for (int j = 0; j < D / 16; j++) q[j] = split8([&](int i) { return x[2 * j + i / 4][i % 4]; }, pow2_field(q_field));
-        const float q_big = wave_max(big), k_big = kt < kt_last ? largest(kpre) : 0.0f, v_big = kt < kt_last ? largest(vpre) : 0.0f;
+        const float q_norm = wave_max(big) * sqrtf(D)   /* at most */, k_big = kt < kt_last ? largest(kpre) : 0.0f, v_big = kt < kt_last ? largest(vpre) : 0.0f;
         auto weak = [](float x, int field) { return x > 0.0f && x * pow2_field(field) < 1.0f; };   // (below 2^-55)
         const bool weak_q = __any(weak(big, q_field));
-        if (lane == 0) lds_big[0][w] = weak_q ? INFINITY : q_big, lds_big[1][w] = k_big, lds_big[2][w] = v_big;
-        if (tid == 0) lds_odd = 0;
-        __syncthreads();
-        auto of_all = [&](int i) { return fmaxf(fmaxf(lds_big[i][0], lds_big[i][1]), fmaxf(lds_big[i][2], lds_big[i][3])); };
-        k_field = up_field(of_all(1)), v_field = up_field(of_all(2));
-        c = p.scale * pow2_field(254 - q_field) * pow2_field(254 - k_field);
-        // no score is larger than this; what the pairs leave of K, 2^-38 of the first tiles' largest, stays below 2^-24 of a score's unit
-        odd = !(of_all(0) * of_all(1) * p.scale * D < kScoreRange) || weak(of_all(1), k_field);
-        // features of V that are 2^13 times weaker than the strongest: their lower numbers would not be normal
+        float v_weak = 0.0f;   // 1 / the largest of eight keys of the weakest feature that has one
         if (32 * kt + 32 <= p.Sk && kt < kt_last) {
-            bool bad = false;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 float m = 0.0f;
@@ -426,10 +427,20 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
                 for (int i = 0; i < NG; i++)
 #pragma unroll
                     for (int j = 0; j < 4; j++) m = fmaxf(m, fabsf(vpre[i][j][e]));
-                bad = bad || weak(m, v_field);
+                v_weak = fmaxf(v_weak, m > 0.0f ? __builtin_amdgcn_rcpf(m) : 0.0f);
             }
-            if (bad) lds_odd = 1;
+            v_weak = wave_max(v_weak);
         }
+        if (lane == 0) lds_big[0][w] = weak_q ? INFINITY : q_norm, lds_big[1][w] = k_big, lds_big[2][w] = v_big, lds_big[3][w] = v_weak;
+        if (tid == 0) lds_odd = 0;
+        __syncthreads();
+        auto of_all = [&](int i) { return fmaxf(fmaxf(lds_big[i][0], lds_big[i][1]), fmaxf(lds_big[i][2], lds_big[i][3])); };
+        k_field = up_field(of_all(1), 11), v_field = up_field(of_all(2), 12);
+        c = p.scale * pow2_field(254 - q_field) * pow2_field(254 - k_field);
+        odd = !(of_all(0) * p.scale * (sqrtf(D) * 0x1p-25f) * pow2_field(254 - k_field) < 0x1p-21f) || weak(of_all(1), k_field);
+        odd = odd || (kt_first < kt_last && of_all(2) == 0.0f);   // (nothing that says what V's unit should be)
+        // features of V that are 2^13 times weaker than the strongest: their lower numbers would lose bits
+        odd = odd || of_all(3) * 0.5f > pow2_field(v_field);
     }
 
     f32x16 o[T];
@@ -521,47 +532,63 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
             }
         }
     }
-    // Infinities, NaN and values that are too large for the scales have left sums that are no numbers.
-    {
-        float probe = l_run * 0.0f;
-#pragma unroll
-        for (int t = 0; t < T; t++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) probe = fmaf(o[t][r], 0.0f, probe);
-        if (!(probe == 0.0f)) lds_odd = 1;
-        __syncthreads();
-        odd = odd || lds_odd != 0;
-    }
-    if (odd) {   // for this row tile everything again, in f32
-        __syncthreads();
-        for (int i = 0; i < 2 && r0 + kRows * i < n_rows; i++) {
-            attend_tile<D>(p, lds.tile, bh, 2 * rt2 + i, split, kt_first, kt_last);
-            __syncthreads();
-        }
-        return;
-    }
-
     // ---- the two key sets' results ---------------------------------------------------------------------------------
     l_run += __shfl_xor(l_run, 32, 64);
     if (hb == 0) lds_m[w][l32] = m_run, lds_l[w][l32] = l_run * 0x1p-14f;
     __syncthreads();   // (and every wave is done with V)
-    const float m_all = fmaxf(m_run, lds_m[w ^ 2][l32]);
-    const float wgt = expf(m_run - ref_of(m_all)) * (pow2_field(254 - v_field) * 0x1p-14f);   // o is counted in 1 / (2^14 v_up)
+    const float m_other = lds_m[w ^ 2][l32], ref_all = ref_of(fmaxf(m_run, m_other)), v_down = pow2_field(254 - v_field);
+    const float f_run = expf(m_run - ref_all), wgt = f_run * (v_down * 0x1p-14f);   // o is counted in 1 / (2^14 v_up)
     float *mine = &lds.rows[(kRows * rg + l32) * ROW];
 #pragma unroll
     for (int set = 1; set >= 0; set--) {
         if (ks == set) {
+            const float l_all = l_run * 0x1p-14f * f_run + lds_l[w ^ 2][l32] * expf(m_other - ref_all), unit = l_all * v_down;
+            float sum = l_all;   // of the row's magnitudes: no number if one is none
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 vec *dst = reinterpret_cast<vec *>(mine + T * (8 * (r / 4) + 4 * hb + r % 4));
                 vec x;
 #pragma unroll
                 for (int t = 0; t < T; t++) x[t] = o[t][r] * wgt;
-                if (set == 0) x += *dst;
+                if (set == 0) {
+                    x += *dst;
+                    if (r == 0) sum *= 0.0f;
+#pragma unroll
+                    for (int t = 0; t < T; t++) sum += fabsf(x[t]);
+                }
                 *dst = x;
+            }
+            if (set == 0) {
+                sum += __shfl_xor(sum, 32, 64);
+                if (!(sum >= unit * kLeastOfRow) || sum == INFINITY) lds_odd = 1;
+                if (hb == 0) lds_least[kRows * rg + l32] = l_all > 0.0f ? unit * kLeastOfFeature : INFINITY;
             }
         }
         __syncthreads();
+    }
+    {   // a thread per feature and part of the rows
+        constexpr int N = 2 * kRows * D / kThreads;
+        const int f = tid % D, first = tid / D * N;
+        float most = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < N; r += 4) {
+            const f32x4 least = *reinterpret_cast<const f32x4 *>(&lds_least[first + r]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) most = fmaxf(most, fabsf(lds.rows[(first + r + i) * ROW + f]) - least[i]);
+        }
+        const uint64_t strong = __ballot(most >= 0.0f || kt_first >= kt_last);
+        if (lane == 0) lds_strong[w] = strong;
+    }
+    __syncthreads();
+    odd = odd || lds_odd != 0;
+    if constexpr (D == 128) odd = odd || ((lds_strong[0] | lds_strong[2]) & (lds_strong[1] | lds_strong[3])) != ~0ull;
+    else odd = odd || (lds_strong[0] | lds_strong[1] | lds_strong[2] | lds_strong[3]) != ~0ull;
+    if (odd) {   // for this row tile everything (again), in f32
+        for (int i = 0; i < 2 && r0 + kRows * i < n_rows; i++) {
+            __syncthreads();
+            attend_tile<D>(p, lds.tile, bh, 2 * rt2 + i, split, kt_first, kt_last);
+        }
+        return;
     }
     const int64_t wb0 = (int64_t)bh * p.n_rt + 2 * rt2, n_wb = (int64_t)p.n_bh * p.n_rt;
 #pragma unroll 4
@@ -633,8 +660,6 @@ int launch(const PrefillF32 &p, hipStream_t s) {
 
 }  // namespace
 
-// 2 = not taken (the generic kernel runs): masks, other types and head sizes, rows that see no key, unaligned rows, a kv
-// head of 4 GB or more.
 // Ranges of keys for sdpa_prefill_f32x2_kernel: the number with the least expected time, in us.  1.5 (D = 64: 1.0) for each pair of
 // tiles of the longest range, or of a compute unit's half of all tiles if that is more; where more than one workgroup shares a compute
 // unit up to 1.9 times that again, and a quarter where not all are resident; 2.5 + 0.12 a range for the merge, and 0.85 for every
@@ -663,6 +688,8 @@ static int64_t choose_pair_splits(const PrefillF32 &p, int D, int64_t tiles, int
     return best;
 }
 
+// 2 = not taken (the generic kernel runs): masks, other types and head sizes, rows that see no key, unaligned rows, a kv
+// head of 4 GB or more.
 int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
     if (a.q_dtype != TROCM_F32 || a.kv_fmt != TROCM_F32 || a.mask) return 2;
     if (a.D != 128 && a.D != 64) return 2;
