@@ -35,17 +35,20 @@
 //  * Scales, powers of two: q's per row, K's and V's from the first two tiles of the range, with room for 16 to 32 (K) and 8 to 16 (V)
 //    times their largest value in what comes later.  A pair is exact to 2^-23 of its number, or to 2^-25 in the scaled unit where
 //    that is more.  What this leaves of K changes a score by at most |q| sqrt(D) scale 2^-25 / k_up, which has to be below 2^-21 (a
-//    few 2^-24 as a rule), and no feature of V may be 2^13 weaker than the strongest in those tiles.
-//  * Otherwise, and where what comes later does not fit, which is seen in the sums, the workgroup starts again with the f32 code (attend_tile): values beyond the room, infinities
+//    few 2^-24 as a rule), and no feature of V may be 2^13 weaker than the strongest in those tiles.  Otherwise the workgroup runs
+//    the f32 code (attend_tile) and nothing else.
+//  * What shows only later is seen in the sums, and the workgroup starts again with the f32 code: values beyond the room, infinities
 //    and NaN (sums that are no numbers), and V that has become too weak for its unit (a row, or a feature over all the rows, that is
 //    small against what the pairs leave).
 //  * What bounds it is the issue of instructions: per tile and wave 48 matrix and about 550 vector instructions, whose busy cycles
 //    add up to 97 % of the kernel's (counters; 2000 queries: 33 and 64 %).  Loads have no condition around them, or the waits for
 //    one tile's V would be waits for the next tile's K (71.6 -> 58.2 us).
-// 1000 queries of 32 heads over 8 (D = 128), with the append: 104.7 us on the f32 instruction, 58.0 as pairs; 771 over 451 tokens 132.3,
-// 65.1; 10 queries of 4 x 64 heads over 8, 3629 tokens, 96.0, 51.5.  From 4 tiles on (2 x 70 queries of 32 heads over 32, 3 tiles: 15.3
-// | 17.5; 2 x 116 of 40 over 8 20.0 | 18.0); ranges of keys (us without | with): 49 queries, 32 over 8, 396 tokens 29.7 | 21.5, but
-// 2 x 251, a workgroup per compute unit, 25.0 | 33.7.
+// us of a call with its append, on the f32 instruction | as pairs | refused: 1000 queries of 32 heads over 8 (D = 128) 104.8 | 60.4 | 106;
+// 771 over 451 tokens 132.3 | 70.1 | 153; 10 queries of 4 x 64 heads over 8, 3629 tokens, 96.3 | 65.3 | 110; 2 x 251 queries 28.6 | 25.9 |
+// 41 (refused tiles cost more where few workgroups of 64 rows take the place of twice as many of 32; 137, 198, 139 and 49 while
+// the pairs' loop ran before them).  What only the sums show: 134, 200, 115 and 50.
+// From 4 tiles on (2 x 70 queries of 32 heads over 32, 3 tiles: 15.3 | 17.5; 2 x 116 of 40 over 8 20.0 | 18.0); ranges of keys (us
+// without | with): 49 queries, 32 over 8, 396 tokens 29.7 | 21.5, but 2 x 251, a workgroup per compute unit, 25.0 | 33.7.
 #include <hip/hip_runtime.h>
 #include <string.h>
 #include <algorithm>
@@ -415,7 +418,16 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
         const int q_field = up_field(big, 13);
 #pragma unroll
         for (int j = 0; j < D / 16; j++) q[j] = split8([&](int i) { return x[2 * j + i / 4][i % 4]; }, pow2_field(q_field));
-        const float q_norm = wave_max(big) * sqrtf(D)   /* at most */, k_big = kt < kt_last ? largest(kpre) : 0.0f, v_big = kt < kt_last ? largest(vpre) : 0.0f;
+        float square = 0.0f;   // of the scaled row, which is neither too large nor too small for it
+#pragma unroll
+        for (int j = 0; j < D / 16; j++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const half2_t h = __builtin_bit_cast(half2_t, __builtin_bit_cast(u32x4, q[j].hi)[i]);
+                square = __builtin_amdgcn_fdot2(h, h, square, false);
+            }
+        square += __shfl_xor(square, 32, 64);
+        const float q_norm = wave_max(sqrtf(square) * pow2_field(254 - q_field)), k_big = kt < kt_last ? largest(kpre) : 0.0f, v_big = kt < kt_last ? largest(vpre) : 0.0f;
         auto weak = [](float x, int field) { return x > 0.0f && x * pow2_field(field) < 1.0f; };   // (below 2^-55)
         const bool weak_q = __any(weak(big, q_field));
         float v_weak = 0.0f;   // 1 / the largest of eight keys of the weakest feature that has one
@@ -450,7 +462,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
         for (int r = 0; r < 16; r++) o[t][r] = 0.0f;
     float m_run = -INFINITY, l_run = 0.0f;   // l and P are counted in 2^-14
     const float k_up = pow2_field(k_field), v_up = pow2_field(v_field);
-    const int steps = (kt_last - kt_first + 1) / 2;
+    const int steps = odd ? 0 : (kt_last - kt_first + 1) / 2;
     for (int it = 0; it < steps; it++, kt += 2) {
         const bool live = kt < kt_last, edge = 32 * kt + 32 > limit_first;   // edge: some row does not see all of the tile
         if (live) {
