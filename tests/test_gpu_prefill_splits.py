@@ -49,12 +49,13 @@ def test_parts(rt, B, Hq, Hkv, D, past, n):
             assert (err <= 2 * TOL * rows + 2.0 ** -20).all(), (causal, size)   # row by row: none is missing or another's
 
 
-@pytest.mark.parametrize("heads,n,past", [(8, 65, 3583), (14, 99, 669)])
+# 15 and 6 parts, merged by a launch; 2, 3 and 4, merged by the last of them
+@pytest.mark.parametrize("heads,kv,n,past", [(8, 2, 65, 3583), (14, 2, 99, 669), (32, 8, 700, 324), (32, 8, 300, 276), (40, 8, 500, 204), (32, 8, 300, 212)])
 @pytest.mark.parametrize("last", [False, True])
-def test_an_infinite_part(rt, heads, n, past, last):
+def test_an_infinite_part(rt, heads, kv, n, past, last):
     """One part's output is infinite in a feature: so is the result there, and nowhere else, whichever part it is.  (Whole tiles of keys.)"""
     rng = np.random.default_rng(n)
-    q, k, v = _normal(rng, 1, heads, n, 128), _normal(rng, 1, 2, past + n, 128), _normal(rng, 1, 2, past + n, 128)
+    q, k, v = _normal(rng, 1, heads, n, 128), _normal(rng, 1, kv, past + n, 128), _normal(rng, 1, kv, past + n, 128)
     q *= np.float16(0.125)   # no weight is below f16's smallest
     v[:, :, past + n - 1 if last else 0, 9] = np.inf
     ws = ta.Workspace(1, heads, n, 128)

@@ -745,10 +745,15 @@ __global__ __launch_bounds__(kThreadsPP, D == 64 && !MASK ? 4 : 2) void sdpa_pre
     // its accumulators, is not read back.  Every element is the chain fma(w3, O3, fma(w2, O2, fma(w1, O1,
     // w0 O0))) over the splits in their order, the own term entering at its place with the f16 value that
     // was stored: the result does not depend on which split arrived last.
-    uint64_t raw[3][DB * 4];   // the other splits in their order
+    uint64_t raw[3][DB * 4];   // the other splits in their order; zeros past the last (a weight of 0 would make a NaN of an infinity)
 #pragma unroll
     for (int j = 0; j < 3; j++) {
-        const int sj = min(j + (j >= split), p.nsplit - 1);
+        const int sj = j + (j >= split);
+        if (sj >= p.nsplit) {
+#pragma unroll
+            for (int i = 0; i < DB * 4; i++) raw[j][i] = 0;
+            continue;
+        }
         const _Float16 *po = p.part_o + ((int64_t)sj * p.n_wb + wb) * (32 * D) + l32 * 4;
 #pragma unroll
         for (int db = 0; db < DB; db++)
