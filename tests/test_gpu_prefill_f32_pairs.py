@@ -131,3 +131,15 @@ def test_a_later_infinity_stays_out(rt, D):
     np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
     fine = np.isfinite(want)
     assert np.abs(got[fine] - want[fine]).max() <= 2e-5 * np.abs(want[fine]).max()
+
+
+# ranges of keys for up to 32 rows and for more of them
+@pytest.mark.parametrize("heads,kv,D,past,n", [(8, 2, 128, 1500, 4), (4, 4, 64, 700, 20), (8, 2, 128, 1500, 20), (14, 2, 64, 1500, 12), (4, 2, 128, 3001, 60)])
+@pytest.mark.parametrize("last", [False, True])
+def test_an_infinite_range(rt, heads, kv, D, past, n, last):
+    """One token's value is infinite in a feature: so is the result there, and nowhere else, whichever range it is in."""
+    rng = np.random.default_rng(past)
+    q, k, v = _normal(rng, 1, heads, n, D) / 10, _normal(rng, 1, kv, past + n, D), _normal(rng, 1, kv, past + n, D)
+    v[:, :, past + n - 1 if last else 0, 9] = np.inf
+    got = _run(q, k, v, past, causal=False)
+    assert np.isposinf(got[..., 9]).all() and np.isfinite(np.delete(got, 9, axis=-1)).all()

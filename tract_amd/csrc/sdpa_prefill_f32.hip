@@ -648,7 +648,8 @@ __global__ __launch_bounds__(kThreads) void sdpa_prefill_f32_merge_kernel(Prefil
         sum *= keep, l *= keep, mm = top;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const float wgt = s0 + i < p.nsplit ? expf(m8[i] - ref) : 0.0f;
+            if (s0 + i >= p.nsplit) break;   // (the weight 0 would make a NaN of an infinity)
+            const float wgt = expf(m8[i] - ref);
             l += wgt * l8[i];
             sum += wgt * o8[i];
         }
