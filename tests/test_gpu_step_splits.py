@@ -29,3 +29,22 @@ def test_steps_of_any_number_of_sequence_heads(rt, store, B, Hq, Hkv, D, T):
     want = orc.flash_sdpa(q.astype(np.float32), k.astype(np.float32), v.astype(np.float32), causal=True, threads=8)
     # probabilities and results are rounded to f16 (2^-11 each): twice 2^-11 of the largest |v|
     assert np.abs(got - want).max() <= 2 * 2.0 ** -11 * np.abs(v.astype(np.float64)).max()
+
+
+# 2 to 8 ranges, up to 32 in the kernel and more by a launch, one to sixteen heads per kv head
+@pytest.mark.parametrize("B,Hq,Hkv,D,T", [(1, 32, 32, 64, 700), (6, 32, 32, 128, 700), (3, 32, 8, 128, 300), (12, 32, 8, 128, 1000), (4, 24, 8, 128, 2000), (1, 14, 2, 128, 3000),
+                                           (2, 16, 1, 128, 900), (1, 8, 1, 128, 5000), (1, 32, 8, 64, 2500), (1, 64, 8, 128, 3500), (5, 14, 2, 64, 1700)])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("where", ["first", "last", "anywhere"])
+def test_an_infinite_range(rt, dtype, B, Hq, Hkv, D, T, where):
+    """One token's value is infinite in a feature: so is the result there, and nowhere else, whichever range it is in."""
+    rng = np.random.default_rng(T)
+    q, k, v = ((0.1 if i == 0 else 1.0) * rng.standard_normal((B, h, n, D), dtype=np.float32) for i, (h, n) in enumerate([(Hq, 1), (Hkv, T), (Hkv, T)]))
+    q, k, v = q.astype(dtype), k.astype(dtype), v.astype(dtype)
+    for b in range(B):
+        for h in range(Hkv):
+            v[b, h, {"first": 0, "last": T - 2, "anywhere": rng.integers(T)}[where], 9] = np.inf
+    st = ta.InPlaceKvSdpa(axis=2, causal=True).state()
+    st.k.push(k[:, :, :-1]), st.v.push(v[:, :, :-1])
+    got = st.eval([q, np.ascontiguousarray(k[:, :, -1:]), np.ascontiguousarray(v[:, :, -1:])]).to_numpy()
+    assert np.isposinf(got[..., 9]).all() and np.isfinite(np.delete(got, 9, axis=-1)).all()

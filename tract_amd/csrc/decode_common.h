@@ -234,7 +234,7 @@ __device__ __forceinline__ void tail_merge(const DecodeDev &p, int *counter, int
         const float *po = p.part_o + first * (G * D) + idx;
 #pragma unroll
         for (int sp = 0; sp < MAXS; sp++) {
-            const int spc = min(sp, nsplit - 1);   // splits past the last repeat it and get weight 0 below
+            const int spc = min(sp, nsplit - 1);   // splits past the last repeat it and are left out below
             mv[e][sp] = aload(ml + spc * ml_step);
             lv[e][sp] = aload(ml + spc * ml_step + G);
             ov[e][sp] = aload(po + spc * po_step);
@@ -250,8 +250,8 @@ __device__ __forceinline__ void tail_merge(const DecodeDev &p, int *counter, int
         float acc = 0.0f, ll = 0.0f;
 #pragma unroll
         for (int sp = 0; sp < MAXS; sp++) {
-            const float f = sp < nsplit ? fast_exp2(mv[e][sp] - mm) : 0.0f;
-            acc += ov[e][sp] * f;
+            const float f = sp < nsplit ? fast_exp2(mv[e][sp] - mm) : 0.0f, x = sp < nsplit ? ov[e][sp] : 0.0f;   // (0 times an infinity is NaN)
+            acc += x * f;
             ll += lv[e][sp] * f;
         }
         if (idx < p.g_real * D) out[idx] = from_f32<T>(ll > 0.0f ? acc / ll : 0.0f);
@@ -290,7 +290,7 @@ __device__ __forceinline__ void tail_merge_pairs(const DecodeDev &p, int *counte
         const float *po = p.part_o + first * (G * D) + idx;
 #pragma unroll
         for (int sp = 0; sp < MAXS; sp++) {
-            const int spc = min(sp, nsplit - 1);   // splits past the last repeat it and get weight 0 below
+            const int spc = min(sp, nsplit - 1);   // splits past the last repeat it and are left out below
             mv[e][sp] = aload(ml + spc * ml_step);
             lv[e][sp] = aload(ml + spc * ml_step + G);
             ov[e][sp] = aload2(po + spc * po_step);
@@ -307,8 +307,9 @@ __device__ __forceinline__ void tail_merge_pairs(const DecodeDev &p, int *counte
 #pragma unroll
         for (int sp = 0; sp < MAXS; sp++) {
             const float f = sp < nsplit ? fast_exp2(mv[e][sp] - mm) : 0.0f;
-            acc0 += __builtin_bit_cast(float, (uint32_t)ov[e][sp]) * f;
-            acc1 += __builtin_bit_cast(float, (uint32_t)(ov[e][sp] >> 32)) * f;
+            const uint64_t x = sp < nsplit ? ov[e][sp] : 0;   // (0 times an infinity is NaN)
+            acc0 += __builtin_bit_cast(float, (uint32_t)x) * f;
+            acc1 += __builtin_bit_cast(float, (uint32_t)(x >> 32)) * f;
             ll += lv[e][sp] * f;
         }
         if (idx < p.g_real * D && idx < LIVE * D) {
@@ -368,7 +369,10 @@ __device__ __forceinline__ void tail_merge_wide(const DecodeDev &p, int *counter
         const float *wh = lds_w + min(idx / D, G - 1) * kWideMergeMax;
         float acc = 0.0f;
 #pragma unroll
-        for (int sp = 0; sp < kWideMergeMax; sp++) acc += ov[e][sp] * wh[sp];
+        for (int sp = 0; sp < kWideMergeMax; sp++) {
+            const float x = sp < nsplit ? ov[e][sp] : 0.0f;   // (0 times an infinity is NaN)
+            acc += x * wh[sp];
+        }
         if (idx < p.g_real * D) out[idx] = from_f32<T>(acc);
     }
 }
