@@ -1,5 +1,9 @@
 """Q4_0 weights x f16 rows on the tiled matrix-matrix kernel: each of the shapes that its rule chooses, with remainders of rows and of
 weight rows, against the product in 64 bits with the dequantised weights."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -25,3 +29,24 @@ def test_shapes_of_the_tiled_product(rt, n, k, m):
     assert np.linalg.norm(got - want) <= 2.0 ** -11 * np.linalg.norm(want)
     # a result is a sum of k products whose weights are off by 2^-11 at most: 6 standard deviations of that, and its own rounding
     assert np.abs(got - want).max() <= 2.0 ** -11 * (6 * np.sqrt(k) * 0.03 + np.abs(want).max())
+
+
+# a tile that is given from outside in one direction only: the rest follows from it, not from the shape that would have been chosen
+@pytest.mark.parametrize("given", ["BM=128", "NI=2", "NW=4", "KS=4"])
+def test_a_tile_given_in_part(rt, given):
+    code = """
+import sys; sys.path.insert(0, %r)
+import numpy as np, tract_amd as ta
+from oracle import oracle as orc
+ta.runtime_for_name("rocm")
+rng = np.random.default_rng(0)
+for n, k, m in [(4096, 1024, 49), (2816, 1024, 131), (4096, 4096, 260)]:   # chosen: 8, 4 and 4 sets of waves
+    blocks = orc.quant(orc.FMT_Q4_0, (0.03 * rng.standard_normal((n, k), dtype=np.float32)).astype(np.float32))
+    act = rng.standard_normal((1, m, k), dtype=np.float32).astype(np.float16)
+    got = ta.GgmlGemm().eval(ta.DeviceTensor.from_numpy(act), ta.Q40Weights(blocks, 1, n, k)).to_numpy().astype(np.float64)[0]
+    want = act[0].astype(np.float64) @ orc.dequant(orc.FMT_Q4_0, blocks, np.float32).reshape(n, k).astype(np.float64).T
+    assert np.linalg.norm(got - want) <= 2.0 ** -11 * np.linalg.norm(want), (n, k, m)
+""" % os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    name, value = given.split("=")
+    p = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, **{"TROCM_Q4_MATMUL_" + name: value}), capture_output=True, text=True, timeout=100)
+    assert p.returncode == 0, p.stderr[-2000:]

@@ -421,14 +421,15 @@ int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, i
     if (tiled) {
         // 32-bit byte offsets inside one weight matrix and one batch of activations (rows up to 128 past m are addressed)
         if (n % 16 || k % TK || (n / 16) * (k / TK) * 1152 >= (1ll << 32) || (m + 128) * k >= (1ll << 30)) return 2;
-        // What remains for k that is no multiple of 512 (its sets of waves could not share it): the largest tile of C^T per workgroup -- 256 (n) x 128 (m), 256 x 64, 128 x 64 -- that still gives three
-        // quarters of the compute units a workgroup (128 x 128 never has more workgroups than 256 x 64); the smallest
-        // when none does, and then (or with 256 x 64) k
-        // split over 2 or 4 sets of waves inside the workgroup while the workgroups are fewer than the compute units
-        // can hold of that size.
+        // k a multiple of 512: the shape with the least expected time.  Other k (which the sets of waves of most shapes could not
+        // share), or a shape that is partly given from outside: the largest tile of C^T per workgroup -- 256 (n) x 128 (m), 256 x 64,
+        // 128 x 64 -- that still gives three quarters of the compute units a workgroup (128 x 128 never has more workgroups than
+        // 256 x 64); the smallest when none does, and then (or with 256 x 64) k split over 2 or 4 sets of waves inside the
+        // workgroup while the workgroups are fewer than the compute units can hold of that size.
         static const int forced_bm = getenv("TROCM_Q4_MATMUL_BM") ? atoi(getenv("TROCM_Q4_MATMUL_BM")) : 0;   // (measurements)
         static const int forced_ni = getenv("TROCM_Q4_MATMUL_NI") ? atoi(getenv("TROCM_Q4_MATMUL_NI")) : 0;
         static const int forced_ks = getenv("TROCM_Q4_MATMUL_KS") ? atoi(getenv("TROCM_Q4_MATMUL_KS")) : 0;
+        static const int forced_nw = getenv("TROCM_Q4_MATMUL_NW") ? atoi(getenv("TROCM_Q4_MATMUL_NW")) : 0;
         const int64_t cus = num_compute_units();
         // (up to 32 activation rows: 256 x 32, 128 x 32 -- half the matrix instructions of a tile of 64 rows)
         const int shapes64[3][2] = {{128, 2}, {64, 2}, {64, 1}}, shapes32[3][2] = {{32, 2}, {32, 2}, {32, 1}};
@@ -441,8 +442,7 @@ int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, i
                 break;
             }
         }
-        // Otherwise the shape with the least expected time.
-        if (const TiledShape *best = k / TK % 4 == 0 ? best_shape(n, m, act_batch, k / TK, cus) : nullptr) {
+        if (const TiledShape *best = k / TK % 4 == 0 && !(forced_bm | forced_ni | forced_ks | forced_nw) ? best_shape(n, m, act_batch, k / TK, cus) : nullptr) {
             bm = best->bm, ni = best->ni;
             pick_nw = best->nw, pick_ks = best->ks;
         }
@@ -453,7 +453,6 @@ int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, i
         if (ty > 65535) return 2;
         // ... and when that smallest tile still leaves compute units idle, sets of 2 waves or 1 (64 or 32 rows of the
         // weights per workgroup)
-        static const int forced_nw = getenv("TROCM_Q4_MATMUL_NW") ? atoi(getenv("TROCM_Q4_MATMUL_NW")) : 0;
         int nw = 4;
         if (bm <= 64 && ni == 1) {
             while (nw > 1 && ((n + 32 * nw - 1) / (32 * nw)) * ty * act_batch * 4 < cus * 3) nw /= 2;
