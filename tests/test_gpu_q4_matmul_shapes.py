@@ -14,9 +14,9 @@ from tests.gpu_util import rt  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 
-# (n, k, m): 32 rows x 32 with k shared by 8 waves, 32 x 64 by 4 sets, 64 x 64 by 4, 64 x 128 by 4 and 2, 64 x 256 by 2, 128 x 256; odd tile
+# (n, k, m): 32 rows x 128 of a tall matrix, 32 rows x 32 with k shared by 8 waves, 32 x 64 by 4 sets, 64 x 64 by 4, 64 x 128 by 4 and 2, 64 x 256 by 2, 128 x 256; odd tile
 # counts (k / 128 = 3, 9, 6, 12) that only some of them or none take
-@pytest.mark.parametrize("n,k,m", [(4096, 1024, 49), (2816, 1024, 131), (2832, 1024, 299), (4112, 1024, 321), (5120, 512, 388), (4096, 1024, 1000),
+@pytest.mark.parametrize("n,k,m", [(65552, 512, 31), (4096, 1024, 49), (2816, 1024, 131), (2832, 1024, 299), (4112, 1024, 321), (5120, 512, 388), (4096, 1024, 1000),
                                    (14336, 512, 390), (1040, 384, 200), (2064, 1152, 77), (3072, 768, 150), (4096, 1536, 65)])
 def test_shapes_of_the_tiled_product(rt, n, k, m):
     rng = np.random.default_rng(n + k + m)

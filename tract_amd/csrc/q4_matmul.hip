@@ -390,7 +390,13 @@ constexpr TiledShape kTiledShapes[] = {
     {32, 1, 8, 1, 3.50f, 0.151f, 0.867f, 0.1f}, {32, 1, 4, 2, 3.44f, 0.246f, 0.794f, 0.0f},  {64, 1, 4, 2, 3.77f, 0.397f, 0.737f, 2.2f},
     {64, 1, 4, 4, 5.32f, 0.602f, 0.536f, 5.4f}, {64, 1, 2, 4, 4.68f, 0.623f, 0.638f, 0.0f},  {64, 2, 2, 4, 7.00f, 1.075f, 0.617f, 7.8f},
     {128, 2, 1, 4, 9.27f, 1.792f, 0.777f, 0.0f}};
+// Taller matrices than those have rounds that run into each other, and few rows on them are faster in larger workgroups with fewer
+// sets: up to 32 rows from two workgroups of 128 weight rows per compute unit on (us, 32 x 64 by 4 sets | 32 x 128 by 2: 17 rows
+// of 128256 x 4096 84.7 | 73.8, 131072 x 2048 42.7 | 37.2, 65536 x 2048 24.3 | 21.1, 65536 x 1024 14.1 | 12.7; below that line 49152 x
+// 8192 54.1 | 57.1, 40960 x 5120 34.8 | 36.2).
+constexpr TiledShape kTallShape = {32, 1, 2, 4, 0.0f, 0.0f, 0.0f, 0.0f};
 const TiledShape *best_shape(int64_t n, int64_t m, int64_t act_batch, int64_t tiles, int64_t cus) {
+    if (m <= 32 && n >= 256 * cus && tiles % kTallShape.ks == 0) return &kTallShape;
     const TiledShape *best = nullptr;
     float best_us = 0.0f;
     for (const TiledShape &c : kTiledShapes) {
