@@ -1,11 +1,14 @@
 """Single tokens over numbers of sequence-heads that do not divide the compute units: one range, a few, more than the narrow
 and the wide merge take."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import tract_amd as ta
 from oracle import oracle as orc
 from tests.gpu_util import rt  # noqa: F401
+from tract_amd._lib import call
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +51,25 @@ def test_an_infinite_range(rt, dtype, B, Hq, Hkv, D, T, where):
     st.k.push(k[:, :, :-1]), st.v.push(v[:, :, :-1])
     got = st.eval([q, np.ascontiguousarray(k[:, :, -1:]), np.ascontiguousarray(v[:, :, -1:])]).to_numpy()
     assert np.isposinf(got[..., 9]).all() and np.isfinite(np.delete(got, 9, axis=-1)).all()
+
+
+@pytest.mark.parametrize("T", [3092, 3701, 6143, 14759, 19764])
+def test_more_than_eight_splits_come_in_eights(rt, T):
+    """Eight sequence-heads of any length: a split's place on the XCDs is every head's.  (Seen in the records that are left in the workspace.)"""
+    B, Hq, Hkv, D = 1, 32, 8, 128
+    rng = np.random.default_rng(T)
+    k, v = (rng.standard_normal((B, Hkv, T, D), dtype=np.float32).astype(np.float16) for _ in range(2))
+    q = (rng.standard_normal((B, Hq, 1, D), dtype=np.float32) / np.float32(np.sqrt(D))).astype(np.float16)
+    ws = ta.Workspace(B, Hq, 1, D)
+    counters = 64 * 1024
+    empty = np.concatenate([np.zeros(counters, np.uint8), np.full(ws.nbytes - counters, 0xFF, np.uint8)])
+    dw = ta.DeviceTensor.from_numpy(empty)
+    dq, dk, dv, out = (ta.DeviceTensor.from_numpy(x) for x in (q, k, v, np.zeros_like(q)))
+    strides = (C.c_int64 * 3)(Hkv * T * D, T * D, D)
+    call("trocm_sdpa", dq.ptr, dk.ptr, dv.ptr, None, out.ptr, ta.F16, B, Hq, Hkv, 1, T, D, strides, 1, 1, C.c_float(float("nan")), 1, dw.ptr, ws.nbytes, None)
+    want = orc.flash_sdpa(q.astype(np.float32), k.astype(np.float32), v.astype(np.float32), causal=True, threads=8)
+    assert np.abs(out.to_numpy().astype(np.float64) - want).max() <= 2 * 2.0 ** -11 * np.abs(v.astype(np.float64)).max()
+    used = np.flatnonzero(dw.to_numpy()[counters:] != 0xFF).max() + 1
+    record = B * Hkv * 8 * (D + 2) * 4   # of one split: rows of eight heads per kv head, their maxima and sums
+    splits = -(-used // record)
+    assert splits > 8 and splits % 8 == 0

@@ -474,7 +474,9 @@ int choose_decode_splits(int64_t BH, int64_t G, int n_tiles, int wg_per_cu) {
 // (batch 1 to 31, 150 to 8000 tokens, f16, f32, Q8_0, Q4_0, 1 to 8 heads per kv head) its choice costs 0.2 to 0.7 % more than the
 // best of 16 split counts in the geometric mean (f32: 1.5 %); a fixed number of workgroups per compute unit, before, cost 4 to 11 %
 // (us, then | now: 24 sequence-heads of 8000 f16 tokens in 11 splits 27.1 | 20.3 in 8, 96 in 3 78.2 | 62.6 in 2, 224 of 300 Q4_0
-// tokens in 2 10.3 | 7.6 in 1).
+// tokens in 2 10.3 | 7.6 in 1).  Those shapes were timed while the matrix-core launchers rounded the number once more to whole tiles
+// per split, 14 or 31 of 16 or 32; as chosen, 44 other shapes are 0.6 % above the best of 18 counts, and 8 sequence-heads of f16 rows
+// gain (us, rounded | as chosen: 3092 tokens 11.7 | 10.3, 4999 12.9 | 11.2, 14759 18.8 | 17.4).
 int choose_step_splits(int64_t BH, int64_t G, int n_tiles, int crowd16) {
     static const int forced = getenv("TROCM_DECODE_SPLITS") ? atoi(getenv("TROCM_DECODE_SPLITS")) : 0;
     const int64_t by_ws = kMaxSplitRows / (BH * G);

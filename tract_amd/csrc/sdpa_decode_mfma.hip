@@ -2426,17 +2426,20 @@ bool decode_quant_appends_in_kernel(int64_t g_real, float scale) {
     return on && gp != 0 && gp <= 16 && use_16_wide(TROCM_Q8_0) && use_block_scaling() && scale > 0.0f;
 }
 
+// Groups of kWaves tiles go to the splits in turn, so that any number of them up to the number of groups leaves none empty.
+// Contiguous ranges (TROCM_DECODE_INTERLEAVE=0) are of whole tiles, and may be fewer.
+static int set_splits(DecodeDev &p, int nsplit, int n_tiles) {
+    static const int interleave = getenv("TROCM_DECODE_INTERLEAVE") ? atoi(getenv("TROCM_DECODE_INTERLEAVE")) : 1;
+    p.interleave = interleave, p.tiles_per_split = (n_tiles + nsplit - 1) / nsplit;
+    return p.nsplit = interleave ? nsplit : (n_tiles + p.tiles_per_split - 1) / p.tiles_per_split;
+}
+
 int launch_sdpa_decode_quant_mfma(DecodeDev &p, int kv_fmt, int64_t B, void *workspace, size_t workspace_bytes, hipStream_t s) {
     const int gp = decode_mfma_group(p.g_real);
     if (gp == 0) return 2;
     const int64_t BH = B * p.Hkv;
     const int n_tiles = (p.T + kTile - 1) / kTile;
-    int nsplit = fit_decode_splits(choose_step_splits(BH, gp, n_tiles, kCrowdCodes), BH, gp, 128, workspace, workspace_bytes);
-    const int tps = (n_tiles + nsplit - 1) / nsplit;
-    nsplit = (n_tiles + tps - 1) / tps;
-    p.tiles_per_split = tps, p.nsplit = nsplit;
-    static const int interleave = getenv("TROCM_DECODE_INTERLEAVE") ? atoi(getenv("TROCM_DECODE_INTERLEAVE")) : 1;
-    p.interleave = interleave;
+    const int nsplit = set_splits(p, fit_decode_splits(choose_step_splits(BH, gp, n_tiles, kCrowdCodes), BH, gp, 128, workspace, workspace_bytes), n_tiles);
     p.live_trim = decode_live_trim();
     p.part_ml = (float *)((char *)workspace + kWsCounterBytes);
     p.part_o = p.part_ml + (size_t)BH * nsplit * 2 * gp;
@@ -2457,11 +2460,9 @@ int launch_sdpa_decode_kivi(const KiviSdpaArgs &a, hipStream_t s) {
     if ((uintptr_t)a.k_new % 2 || (uintptr_t)a.v_new % 2 || (uintptr_t)a.k_chan_scale_next % 16 || (uintptr_t)a.k_chan_lo_next % 16) return 2;
     const int64_t BH = a.B * a.Hkv;
     const int n_tiles = (int)((a.T + kTile - 1) / kTile);
-    int nsplit = fit_decode_splits(choose_step_splits(BH, gp, n_tiles, kCrowdCodes), BH, gp, 128, a.workspace, a.workspace_bytes);
-    const int tps = (n_tiles + nsplit - 1) / nsplit;
-    nsplit = (n_tiles + tps - 1) / tps;
     DecodeDev p;
     memset(&p, 0, sizeof(p));
+    const int nsplit = set_splits(p, fit_decode_splits(choose_step_splits(BH, gp, n_tiles, kCrowdCodes), BH, gp, 128, a.workspace, a.workspace_bytes), n_tiles);
     p.q = (const char *)a.q, p.out = (char *)a.out;
     p.k = (const char *)a.k_codes, p.v = (const char *)a.v_codes;
     if (a.k_cap_rows != a.v_cap_rows) return 2;   // one pair of strides serves both code planes
@@ -2471,12 +2472,9 @@ int launch_sdpa_decode_kivi(const KiviSdpaArgs &a, hipStream_t s) {
     p.chan_scale = a.k_chan_scale, p.chan_lo = a.k_chan_lo, p.chan_scale_next = a.k_chan_scale_next, p.chan_lo_next = a.k_chan_lo_next;
     p.k_new = (const char *)a.k_new, p.v_new = (const char *)a.v_new;
     p.T = (int)a.T;
-    p.tiles_per_split = tps, p.nsplit = nsplit;
     p.Hq = (int)a.Hq, p.Hkv = (int)a.Hkv, p.g_real = (int)g_real;
     p.scale_log2 = a.scale * 1.4426950408889634f;
     p.new_pos = (int)a.T - 1;
-    static const int interleave = getenv("TROCM_DECODE_INTERLEAVE") ? atoi(getenv("TROCM_DECODE_INTERLEAVE")) : 1;
-    p.interleave = interleave;
     p.live_trim = decode_live_trim();
     p.part_ml = (float *)((char *)a.workspace + kWsCounterBytes);
     p.part_o = p.part_ml + (size_t)BH * nsplit * 2 * gp;
@@ -2513,15 +2511,12 @@ int launch_sdpa_decode_mfma(const SdpaArgs &a, hipStream_t s) {
     if (a.B > 65535 || a.Hkv > 65535) return 2;
     const int64_t BH = a.B * a.Hkv;
     const int n_tiles = (int)((a.Sk + kTile - 1) / kTile);
-    int nsplit = fit_decode_splits(choose_step_splits(BH, gp, n_tiles, a.D == 128 ? kCrowdWide : kCrowdNarrow), BH, gp, a.D, a.workspace, a.workspace_bytes);
-    const int tps = (n_tiles + nsplit - 1) / nsplit;
-    nsplit = (n_tiles + tps - 1) / tps;
     DecodeDev p;
     memset(&p, 0, sizeof(p));
+    const int nsplit = set_splits(p, fit_decode_splits(choose_step_splits(BH, gp, n_tiles, a.D == 128 ? kCrowdWide : kCrowdNarrow), BH, gp, a.D, a.workspace, a.workspace_bytes), n_tiles);
     p.q = (const char *)a.q, p.out = (char *)a.out, p.k = (const char *)a.k, p.v = (const char *)a.v;
     p.kv_stride_b = a.kv_stride_b * 2, p.kv_stride_h = a.kv_stride_h * 2, p.kv_stride_t = a.kv_stride_t * 2;
     p.T = (int)a.Sk;
-    p.tiles_per_split = tps, p.nsplit = nsplit;
     p.Hq = (int)a.Hq, p.Hkv = (int)a.Hkv, p.g_real = (int)g_real;
     p.scale_log2 = a.scale * 1.4426950408889634f;
     p.k_new = (const char *)a.k_new, p.v_new = (const char *)a.v_new;
@@ -2534,8 +2529,6 @@ int launch_sdpa_decode_mfma(const SdpaArgs &a, hipStream_t s) {
     }
     p.part_ml = (float *)((char *)a.workspace + kWsCounterBytes);
     p.part_o = p.part_ml + (size_t)BH * nsplit * 2 * gp;
-    static const int interleave = getenv("TROCM_DECODE_INTERLEAVE") ? atoi(getenv("TROCM_DECODE_INTERLEAVE")) : 1;
-    p.interleave = interleave;
     // Workgroups are handed to the 8 XCDs in turn and the odd XCDs stream about a tenth slower than the even ones
     // (time stamps per workgroup: the tile loops of a launch of equal shares end at 33 - 36 us on XCDs 0, 2, 4, 6 and
     // at 37 - 40 us on 1, 3, 5, 7, whatever the shares' addresses): with an even number of splits the odd splits sit
