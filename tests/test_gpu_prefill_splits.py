@@ -61,3 +61,27 @@ def test_an_infinite_part(rt, heads, kv, n, past, last):
     ws = ta.Workspace(1, heads, n, 128)
     got = _sdpa(q, k, v, False, ws, ws.nbytes)
     assert np.isposinf(got[..., 9]).all() and np.isfinite(np.delete(got, 9, axis=-1)).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [120, 200])
+def test_short_prompts_of_odd_groups_sum_their_weights_in_f32(rt, D, T):
+    """One key of weight 1 and value c, T - 1 of weight w and value 0: c / (1 + (T - 1) w), correctly rounded but for f32's own errors.
+    w is half way between two f16 numbers, so that a sum of rounded weights is off by 2^-12 and more, which is another f16 number."""
+    t = np.arange(2048, dtype=np.int64) / 1024 + 1.0   # f16 numbers from 1 to 3
+    w = np.exp(-t)
+    t, w = max(zip(t, w), key=lambda x: abs(float(np.float16(x[1])) - x[1]) / x[1])
+    exact, off = 1 / (1 + (T - 1) * w), 1 / (1 + (T - 1) * float(np.float16(w)))
+    # c such that c * exact lies beside a middle between two f16 numbers, on its side of it, and c * off on the other
+    c = max((np.float64(x) for x in np.arange(1024, 2048) / 1024 if np.float16(x * exact) != np.float16(x * off)),
+            key=lambda x: abs(np.float64(np.float16(x * exact)) - x * off) - abs(np.float64(np.float16(x * exact)) - x * exact))
+    q, k, v = np.zeros((1, 14, 70, D), np.float16), np.zeros((1, 2, T, D), np.float16), np.zeros((1, 2, T, D), np.float16)
+    q[..., 0], k[..., 0] = 1, -t
+    k[:, :, T // 3], v[:, :, T // 3] = 0, c
+    ws = ta.Workspace(1, 14, 70, D)
+    B, Hq, n, _ = q.shape
+    dq, dk, dv = (ta.DeviceTensor.from_numpy(x) for x in (q, k, v))
+    out = ta.DeviceTensor.from_numpy(np.zeros_like(q))
+    strides = (C.c_int64 * 3)(2 * T * D, T * D, D)
+    call("trocm_sdpa", dq.ptr, dk.ptr, dv.ptr, None, out.ptr, ta.F16, B, Hq, 2, n, T, D, strides, 1, 1, C.c_float(1.0), 0, ws.ptr, ws.nbytes, None)
+    np.testing.assert_array_equal(out.to_numpy(), np.full_like(q, np.float16(c * exact)))

@@ -54,8 +54,7 @@ struct PrefillPP {
     int B, Hq, Hkv, Sq, Sk;
     int causal;
     int n_qtiles, nsplit;
-    float lazy_max;
-    int part32;         // the partials are f32, merged by a launch
+    int part32;         // F32 instantiations: sums and partials of f32, merged by a launch
     int paired;         // != 0: how many query tiles make up a first workgroup for every compute unit, where each holds two
     float scale_log2;
     // Partials of key split s and 32-query block wb (= (b * Hq + qh) * n_qb32 + q / 32):
@@ -123,8 +122,11 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t b0123, uint32_t b4567, half2_
 }
 
 
-template <int D, int HG, bool MASK, int FMT, bool PING = false>
+// F32: the row sum takes the weights as they are before they are rounded for the product with V, their reference is the maximum
+// itself, and partials are f32.
+template <int D, int HG, bool MASK, int FMT, bool PING = false, bool F32 = false>
 __global__ __launch_bounds__(kThreadsPP, D == 64 && !MASK ? 4 : 2) void sdpa_prefill_pp_kernel(PrefillPP p) {
+    static_assert(!F32 || (HG == 1 && !MASK && FMT == TROCM_F16 && !PING), "short prompts of one head per workgroup");
     static_assert(!PING || (!MASK && FMT == TROCM_F16), "the ping-pong loop serves f16 caches without a mask input");
     constexpr int QB = kWavesPP / HG;     // 32-query blocks per workgroup
     constexpr int BLOCK_M = 32 * QB;
@@ -338,10 +340,10 @@ __global__ __launch_bounds__(kThreadsPP, D == 64 && !MASK ? 4 : 2) void sdpa_pre
             for (int r = 0; r < 16; r++) tmax = fmaxf(tmax, s[kb][r]);
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
         // The reference of the exponentials follows the maximum lazily: it moves only when this tile's maximum exceeds it
-        // by more than lazy_max, at most kLazyMax (the exponentials then reach 2^kLazyMax at most, far inside f16 and f32 range), so the
+        // by more than kLazyMax (the exponentials then reach 2^kLazyMax at most, far inside f16 and f32 range), so the
         // accumulators are rescaled a few times per sequence instead of at most tiles; o / l does not depend on it.
         const float t_scaled = MASK ? tmax : tmax * p.scale_log2;   // scale > 0: the maximum commutes with the scaling
-        const bool moved = t_scaled > m_run + p.lazy_max;   // also the first visible key (reference -inf); never for a maximum of -inf
+        const bool moved = t_scaled > m_run + (F32 ? 0.0f : kLazyMax);   // also the first visible key (reference -inf); never for a maximum of -inf
         const float m_new = moved ? t_scaled : m_run;
         const float m_ref = (m_new == -INFINITY) ? 0.0f : m_new;  // nothing visible yet: keep everything at zero
         float psum = 0.0f;
@@ -352,7 +354,9 @@ __global__ __launch_bounds__(kThreadsPP, D == 64 && !MASK ? 4 : 2) void sdpa_pre
                 const float sx = s[st >> 1][8 * (st & 1) + i];
                 float pv = fast_exp2(MASK ? sx - m_ref : __builtin_fmaf(sx, p.scale_log2, -m_ref));
                 pf[st][i] = (_Float16)pv;
+                if constexpr (F32) psum += pv;
             }
+            if constexpr (F32) continue;
             // the row sum is taken over the f16 values that enter the product with V (one v_dot2 per pair
             // instead of two additions, and numerator and denominator see the same rounding)
             const half2_t ones = {(_Float16)1.0f, (_Float16)1.0f};
@@ -681,14 +685,16 @@ __global__ __launch_bounds__(kThreadsPP, D == 64 && !MASK ? 4 : 2) void sdpa_pre
         for (int db = 0; db < DB; db++)
 #pragma unroll
             for (int rq = 0; rq < 4; rq++) {
+                if constexpr (F32) {
+                    float *d32 = reinterpret_cast<float *>(p.part_o) + ((int64_t)split * p.n_wb + wb) * (32 * D) + l32 * 4 + (8 * db + 2 * rq + hb) * 128;
+                    *reinterpret_cast<float4_t *>(d32) = float4_t{o[db][4 * rq] * inv, o[db][4 * rq + 1] * inv, o[db][4 * rq + 2] * inv, o[db][4 * rq + 3] * inv};
+                    continue;
+                }
                 half4_t h4;
 #pragma unroll
                 for (int i = 0; i < 4; i++) h4[i] = partial_elem(o[db][4 * rq + i]);
                 _Float16 *dst = po + (8 * db + 2 * rq + hb) * 128;
-                if (p.part32) {
-                    float *d32 = reinterpret_cast<float *>(p.part_o) + ((int64_t)split * p.n_wb + wb) * (32 * D) + l32 * 4 + (8 * db + 2 * rq + hb) * 128;
-                    *reinterpret_cast<float4_t *>(d32) = float4_t{o[db][4 * rq] * inv, o[db][4 * rq + 1] * inv, o[db][4 * rq + 2] * inv, o[db][4 * rq + 3] * inv};
-                } else if (tail_merge)
+                if (tail_merge)
                     __hip_atomic_store(reinterpret_cast<uint64_t *>(dst), __builtin_bit_cast(uint64_t, h4), __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
                 else
@@ -699,7 +705,7 @@ __global__ __launch_bounds__(kThreadsPP, D == 64 && !MASK ? 4 : 2) void sdpa_pre
         else
             *pml = hb ? l_run : m_run;
     }
-    if (!tail_merge) return;
+    if (F32 || !tail_merge) return;
 
     // ---- the last split of this tile to arrive merges all of them ------------------------------------
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this thread's partial stores have completed
@@ -907,6 +913,8 @@ int launch_cfg(const PrefillPP &p, int fmt, int64_t wgs, hipStream_t s) {
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_Q4_0>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     else if (p.mask)
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, true, TROCM_F16>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
+    else if (HG == 1 && p.part32)
+        hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, 1, false, TROCM_F16, false, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     else if (ping_enabled())
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_F16, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     else
@@ -1008,11 +1016,11 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
     p.n_qtiles = (int)n_qtiles;
     p.n_qb32 = (int)((a.Sq + 31) / 32);
     p.n_wb = a.B * a.Hq * p.n_qb32;
-    // Short prompts of one head per workgroup, f16 caches: partials in f32.  (The smaller kernel, which these came from, held a result
-    // in f32 to its end: f16 partials made the error against 64 bits 1.27 times what it was, 2.7e-4 -> 3.5e-4; f32 ones leave it there.)
-    // (And with the maximum itself as the reference: the largest weight is then 1, without an error; 1.03 to 1.07 times otherwise.)
+    // Short prompts of one head per workgroup, f16 caches: row sums of the weights before they are rounded, partials in f32, and the
+    // maximum itself as the reference, as in the smaller kernel that these came from.  (f16 partials made the error against 64 bits
+    // 1.27 times that kernel's, 2.7e-4 -> 3.5e-4, another reference 1.03 to 1.07 times; now 0.99 over 60 prompts.  As an instantiation
+    // of its own it is also 2 to 4 % faster than with conditions in the other one: 40 heads x 70 queries behind 600 17.1 -> 16.6 us.)
     p.part32 = hg == 1 && !quant && a.Sq * 2 < n_qtiles * block_m;
-    p.lazy_max = p.part32 ? 0.0f : kLazyMax;
     if (a.mask) {   // [mask_b, mask_h, Sq, Sk] dense
         p.mask = (const _Float16 *)a.mask;
         p.mask_stride_h = a.mask_h > 1 ? a.Sq * a.Sk : 0;
