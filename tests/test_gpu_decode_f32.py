@@ -76,3 +76,15 @@ def test_f32_steps_over_a_ring_and_an_output_over_the_inputs(rt):
     q = rng.standard_normal((B, Hq, 1, D), dtype=np.float32)
     dq, dk, dv = (ta.DeviceTensor.from_numpy(np.ascontiguousarray(a)) for a in (q, k[:, :, 3000:], v[:, :, 3000:]))
     _check(st.eval_into(dq, dk, dv, dq).to_numpy(), q, k, v)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,T", [(26, 64, 8, 1383), (1, 32, 32, 201), (16, 32, 8, 290)])
+def test_rounding_of_f32_steps(rt, B, Hq, Hkv, T):
+    """Long sums in one range, 64 features: 2.65e-7, 1.96e-7 and 2.0e-7 of the norm is what sixteen sums in several ranges leave (the vector kernel)."""
+    rng = np.random.default_rng(T)
+    q, k, v = (rng.standard_normal((B, h, n, 64), dtype=np.float32) for h, n in ((Hq, 1), (Hkv, T), (Hkv, T)))
+    st = ta.InPlaceKvSdpa(axis=2, causal=True).state()
+    st.k.push(k[:, :, :-1]), st.v.push(v[:, :, :-1])
+    got = st.eval([q, np.ascontiguousarray(k[:, :, -1:]), np.ascontiguousarray(v[:, :, -1:])]).to_numpy()
+    want = textbook_sdpa(q, k, v, causal=True)
+    assert np.linalg.norm(got - want) <= {1383: 2.65e-7, 201: 1.96e-7, 290: 2.0e-7}[T] * np.linalg.norm(want)
