@@ -290,8 +290,9 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_f32_kernel(DecodeF32 
             }
 #pragma unroll
             for (int u = 0; u < 8; u++) {
-                if (s0 + u >= p.nsplit) break;   // (the weight 0 would make a NaN of an infinity)
-                const float f = lds_wt[r][s0 + u];
+                const bool there = s0 + u < p.nsplit;   // (the weight 0 alone would make a NaN of an infinity)
+                const float f = there ? lds_wt[r][s0 + u] : 0.0f;
+                if (!there) x[u][0] = x[u][1] = 0;
                 sum[0] = fmaf(f, lo_of(x[u][0]), sum[0]), sum[1] = fmaf(f, hi_of(x[u][0]), sum[1]);
                 sum[2] = fmaf(f, lo_of(x[u][1]), sum[2]), sum[3] = fmaf(f, hi_of(x[u][1]), sum[3]);
             }

@@ -648,10 +648,11 @@ __global__ __launch_bounds__(kThreads) void sdpa_prefill_f32_merge_kernel(Prefil
         sum *= keep, l *= keep, mm = top;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            if (s0 + i >= p.nsplit) break;   // (the weight 0 would make a NaN of an infinity)
-            const float wgt = expf(m8[i] - ref);
+            const bool there = s0 + i < p.nsplit;   // (the weight 0 alone would make a NaN of an infinity)
+            const float wgt = there ? expf(m8[i] - ref) : 0.0f;
             l += wgt * l8[i];
-            sum += wgt * o8[i];
+#pragma unroll
+            for (int e = 0; e < 4; e++) sum[e] += wgt * (there ? o8[i][e] : 0.0f);
         }
     }
     const int i = row / p.G, g = row - i * p.G;
