@@ -354,7 +354,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
     typedef typename VecOf<T>::type vec;
     __shared__ __attribute__((aligned(16))) union { PairLds<D> pair; TileLds<D> tile; float rows[2 * kRows * ROW]; } lds;
     __shared__ float lds_m[kWaves][kRows], lds_l[kWaves][kRows], lds_big[4][kWaves];
-    __shared__ __attribute__((aligned(16))) float lds_least[2 * kRows];   // by row: what a feature has to reach
+    __shared__ float lds_least[2 * kRows];   // by row: what a feature has to reach
     __shared__ int lds_odd;
     __shared__ uint64_t lds_strong[kWaves];
 
@@ -578,23 +578,23 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
         }
         __syncthreads();
     }
-    {   // a thread per feature and part of the rows
-        constexpr int N = 2 * kRows * D / kThreads;
-        const int f = tid % D, first = tid / D * N;
-        float most = -INFINITY;
-#pragma unroll
-        for (int r = 0; r < N; r += 4) {
-            const f32x4 least = *reinterpret_cast<const f32x4 *>(&lds_least[first + r]);
-#pragma unroll
-            for (int i = 0; i < 4; i++) most = fmaxf(most, fabsf(lds.rows[(first + r + i) * ROW + f]) - least[i]);
-        }
-        const uint64_t strong = __ballot(most >= 0.0f || kt_first >= kt_last);
-        if (lane == 0) lds_strong[w] = strong;
-    }
-    __syncthreads();
     odd = odd || lds_odd != 0;
-    if constexpr (D == 128) odd = odd || ((lds_strong[0] | lds_strong[2]) & (lds_strong[1] | lds_strong[3])) != ~0ull;
-    else odd = odd || (lds_strong[0] | lds_strong[1] | lds_strong[2] | lds_strong[3]) != ~0ull;
+    // A thread per feature and part of the rows: four of them, which is enough for all but a few tiles, then all.
+    constexpr int N = 2 * kRows * D / kThreads;
+    const int feature = tid % D, first = tid / D * N;
+    for (int n = 4; !odd && kt_first < kt_last; n = N) {
+        float most = -INFINITY;
+#pragma unroll 4
+        for (int r = 0; r < n; r++) most = fmaxf(most, fabsf(lds.rows[(first + r) * ROW + feature]) - lds_least[first + r]);
+        const uint64_t strong = __ballot(most >= 0.0f);
+        if (lane == 0) lds_strong[w] = strong;
+        __syncthreads();
+        const bool all = D == 128 ? ((lds_strong[0] | lds_strong[2]) & (lds_strong[1] | lds_strong[3])) == ~0ull
+                                  : (lds_strong[0] | lds_strong[1] | lds_strong[2] | lds_strong[3]) == ~0ull;
+        if (all) break;
+        odd = n == N;
+        __syncthreads();
+    }
     if (odd) {   // for this row tile everything (again), in f32
         for (int i = 0; i < 2 && r0 + kRows * i < n_rows; i++) {
             __syncthreads();
