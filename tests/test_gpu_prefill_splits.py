@@ -49,6 +49,18 @@ def test_parts(rt, B, Hq, Hkv, D, past, n):
             assert (err <= 2 * TOL * rows + 2.0 ** -20).all(), (causal, size)   # row by row: none is missing or another's
 
 
+# head size 64: as many workgroups of 64 queries as compute units (256), more that find place behind each other (320, one or all queries
+# in the last tile), more that share a unit (behind 300 tokens, or of equal length)
+@pytest.mark.parametrize("past,n,causal", [(0, 256, True), (0, 257, True), (0, 320, True), (40, 299, True), (300, 300, True), (0, 300, False)])
+def test_a_compute_unit_alone_and_shared(rt, past, n, causal):
+    rng = np.random.default_rng(past + n)
+    q, k, v = _normal(rng, 4, 64, n, 64), _normal(rng, 4, 8, past + n, 64), _normal(rng, 4, 8, past + n, 64)
+    ws = ta.Workspace(4, 64, n, 64)
+    got, want = _sdpa(q, k, v, causal, ws, ws.nbytes).astype(np.float64), textbook_sdpa(q, k, v, causal=causal)
+    assert np.linalg.norm(got - want) <= TOL * np.linalg.norm(want)
+    assert (np.linalg.norm(got - want, axis=-1) <= 2 * TOL * np.linalg.norm(want, axis=-1) + 2.0 ** -20).all()
+
+
 # 15 and 6 parts, merged by a launch; 2, 3 and 4, merged by the last of them
 @pytest.mark.parametrize("heads,kv,n,past", [(8, 2, 65, 3583), (14, 2, 99, 669), (32, 8, 700, 324), (32, 8, 300, 276), (40, 8, 500, 204), (32, 8, 300, 212)])
 @pytest.mark.parametrize("last", [False, True])

@@ -18,7 +18,9 @@
 //    workspace, laid out exactly as the accumulator registers are (so every store instruction
 //    covers 512 contiguous bytes), and the last of up to four to arrive, or a small kernel, merges them.
 //  * Head size 64: 128 registers, so that two workgroups fit on a compute unit (129, one, cost 10 to 20 %: 3 x 64 heads x 917
-//    queries behind 3704 261 -> 238 us; a single wave of unequal workgroups gives 3 % of that back: 64 heads x 1761 44.5 -> 46.3).
+//    queries behind 3704 261 -> 238 us).  Where one has a unit to itself in any case, or a causal prompt's tiles are so unequal that
+//    the short ones go behind each other, it is an instantiation with 129 (32 heads in groups of 4: 2048 queries, 256 workgroups, 48.4
+//    -> 47.1 us; 2 x 1500, 384, 40.1 -> 37.8; 40 heads x 2048, 320, 50.3 -> 47.9; 3 x 1200, 456, 38.8 -> 36.6).
 //  * The output accumulators are rescaled only when some query's running maximum moved.
 //  * A second tile loop (template argument PING, chosen with TROCM_PREFILL_PING=1, f16 caches without a mask
 //    input) loads K/V tiles straight into LDS (global_load_lds_dwordx4, swizzled rows) and runs waves 0..3 and
@@ -124,8 +126,9 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t b0123, uint32_t b4567, half2_
 
 // F32: the row sum takes the weights as they are before they are rounded for the product with V, their reference is the maximum
 // itself, and partials are f32.
-template <int D, int HG, bool MASK, int FMT, bool PING = false, bool F32 = false>
-__global__ __launch_bounds__(kThreadsPP, D == 64 && !MASK ? 4 : 2) void sdpa_prefill_pp_kernel(PrefillPP p) {
+// ALONE: a workgroup has a compute unit to itself, and as many registers as it likes (D = 64; D = 128 always has).
+template <int D, int HG, bool MASK, int FMT, bool PING = false, bool F32 = false, bool ALONE = D != 64 || MASK>
+__global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_kernel(PrefillPP p) {
     static_assert(!F32 || (HG == 1 && !MASK && FMT == TROCM_F16 && !PING), "short prompts of one head per workgroup");
     static_assert(!PING || (!MASK && FMT == TROCM_F16), "the ping-pong loop serves f16 caches without a mask input");
     constexpr int QB = kWavesPP / HG;     // 32-query blocks per workgroup
@@ -614,7 +617,7 @@ __global__ __launch_bounds__(kThreadsPP, D == 64 && !MASK ? 4 : 2) void sdpa_pre
         }
         if (grp == 0) half_barrier();   // as many barriers as the second group
     }
-    if constexpr (D == 64) {   // the lane's number taken anew: what the epilogue makes of it would otherwise be kept in registers through the loop
+    if constexpr (!ALONE) {   // the lane's number taken anew: what the epilogue makes of it would otherwise be kept in registers through the loop
         asm("" : "+v"(lane));
         hb = lane >> 5, l32 = lane & 31;
     }
@@ -870,6 +873,15 @@ bool ping_enabled() {
     return on != 0;
 }
 
+// tiles of keys that the last query sees, and all workgroups together
+int64_t longest_tiles(const PrefillPP &p) { return (p.Sk + kTileN - 1) / kTileN; }
+int64_t all_tiles(const PrefillPP &p, int block_m, int64_t wgs1) {
+    if (!p.causal) return wgs1 * longest_tiles(p);
+    int64_t all = 0;
+    for (int qt = 0; qt < p.n_qtiles; qt++) all += (min((qt + 1) * block_m, p.Sq) - 1 + p.Sk - p.Sq) / kTileN + 1;
+    return all * (wgs1 / p.n_qtiles);
+}
+
 // Number of key splits: the one with the least expected time, us, over
 //   * the tile loop: 1.5 us per tile of 64 keys (D = 64: 1.0) for the longest workgroup's share, or for a compute unit's share of all
 //     tiles if that is more; up to half a share again where not all workgroups are resident (one per compute unit, D = 64: two; those
@@ -883,13 +895,7 @@ bool ping_enabled() {
 // (32 heads in groups of 4: 300 queries behind 3584 49.4 -> 36.7 us, 130 behind 3584 40.2 -> 28, 65 behind 740 21.4 -> 17.6; 2 x 64
 // heads x 415 queries 30.1 -> 21.1.)
 int64_t choose_splits(const PrefillPP &p, int D, int block_m, int64_t wgs1, int64_t cus, int64_t most) {
-    const int64_t longest = (p.Sk + kTileN - 1) / kTileN;   // tiles that the last query sees
-    int64_t all = wgs1 * longest;
-    if (p.causal) {
-        all = 0;
-        for (int qt = 0; qt < p.n_qtiles; qt++) all += (min((qt + 1) * block_m, p.Sq) - 1 + p.Sk - p.Sq) / kTileN + 1;
-        all *= wgs1 / p.n_qtiles;
-    }
+    const int64_t longest = longest_tiles(p), all = all_tiles(p, block_m, wgs1);
     const float even = p.causal ? (float)((min(block_m, p.Sq) - 1 + p.Sk - p.Sq) / kTileN + 1) / (float)longest : 1.0f;   // first query tile / last
     const float tile = D == 64 ? 1.0f : 1.5f, slots = (float)(D == 64 ? 2 * cus : cus), busy = (float)all / slots;
     int64_t best = 1;
@@ -906,7 +912,7 @@ int64_t choose_splits(const PrefillPP &p, int D, int block_m, int64_t wgs1, int6
 }
 
 template <int D, int HG>
-int launch_cfg(const PrefillPP &p, int fmt, int64_t wgs, hipStream_t s) {
+int launch_cfg(const PrefillPP &p, int fmt, int64_t wgs, bool alone, hipStream_t s) {
     if (fmt == TROCM_Q8_0)
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_Q8_0>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     else if (fmt == TROCM_Q4_0)
@@ -917,6 +923,9 @@ int launch_cfg(const PrefillPP &p, int fmt, int64_t wgs, hipStream_t s) {
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, 1, false, TROCM_F16, false, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     else if (ping_enabled())
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_F16, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
+    else if (D == 64 && alone)   // (the LDS that more workgroups than units ask for is not used: no second one fits beside it)
+        hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_F16, false, false, true>), dim3((unsigned)wgs), dim3(kThreadsPP),
+                           wgs > num_compute_units() ? 48 * 1024 : 0, s, p);
     else
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_F16>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     hipError_t e = hipGetLastError();
@@ -939,11 +948,11 @@ int launch_cfg(const PrefillPP &p, int fmt, int64_t wgs, hipStream_t s) {
 }
 
 template <int D>
-int launch_hg(const PrefillPP &p, int fmt, int hg, int64_t wgs, hipStream_t s) {
+int launch_hg(const PrefillPP &p, int fmt, int hg, int64_t wgs, bool alone, hipStream_t s) {
     switch (hg) {
-        case 4: return launch_cfg<D, 4>(p, fmt, wgs, s);
-        case 2: return launch_cfg<D, 2>(p, fmt, wgs, s);
-        default: return launch_cfg<D, 1>(p, fmt, wgs, s);
+        case 4: return launch_cfg<D, 4>(p, fmt, wgs, alone, s);
+        case 2: return launch_cfg<D, 2>(p, fmt, wgs, alone, s);
+        default: return launch_cfg<D, 1>(p, fmt, wgs, alone, s);
     }
 }
 
@@ -1052,12 +1061,20 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
     // resident at once: the shortest tiles go beside the longest (3 x 40 heads x 574 queries behind 1717: 77.7 -> 60.8 us).  Otherwise a
     // prompt whose tiles differ much runs the longest of all its sequences first (3 x 32 x 1414 at D = 128: 83.9 -> 75.3), and one
     // behind many tokens one sequence after the other, whose K and V then stay in the L2 (3 x 32 x 1377 behind 752: 128, not 138).
-    if (a.causal && a.D == 64 && wgs > cus && wgs <= 2 * cus)
+    // At D = 64 a workgroup has its unit to itself in two cases: there are no more of them than units, or a causal prompt's short tiles
+    // find place behind each other while the longest are at work: all of them, spread over the units, are less than the longest one
+    // by what does not go out evenly (us, two on a unit | alone, by that share: 0.94 38.8 | 36.6, 0.95 49.3 | 46.9, 1.00 52.2 | 52.7,
+    // 1.03 50.6 | 53.2).  The longest of all sequences then go first.
+    const bool fits = a.causal && ns == 1 && 25 * all_tiles(p, block_m, wgs1) <= 24 * cus * longest_tiles(p);
+    const bool alone = a.D == 64 && (wgs <= cus || fits);
+    if (alone && wgs > cus)
+        p.paired = (int)n_qtiles;
+    else if (a.causal && a.D == 64 && wgs > cus && wgs <= 2 * cus)
         p.paired = (int)((cus + wgs / n_qtiles - 1) / (wgs / n_qtiles));
     else if (a.causal && a.B > 1 && 5 * a.Sq > 4 * a.Sk)
         p.paired = (int)n_qtiles;
     if (wgs >= (1ll << 31)) return 2;
-    return a.D == 128 ? launch_hg<128>(p, a.kv_fmt, hg, wgs, s) : launch_hg<64>(p, a.kv_fmt, hg, wgs, s);
+    return a.D == 128 ? launch_hg<128>(p, a.kv_fmt, hg, wgs, true, s) : launch_hg<64>(p, a.kv_fmt, hg, wgs, alone, s);
 }
 
 }  // namespace trocm
