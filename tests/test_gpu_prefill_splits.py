@@ -1,5 +1,6 @@
 """f16 prompts whose keys are split over workgroups: every way the parts are merged (by the last of up to four, by a launch for up
-to eight and up to sixteen), two workgroups on a compute unit at head size 64, one head per workgroup with few queries, small scratch."""
+to eight and up to sixteen), one and two workgroups on a compute unit at head size 64, one head per workgroup with few queries, small
+scratch, and what the kernel without parts takes."""
 import ctypes as C
 
 import numpy as np
@@ -97,3 +98,27 @@ def test_short_prompts_of_odd_groups_sum_their_weights_in_f32(rt, D, T):
     strides = (C.c_int64 * 3)(2 * T * D, T * D, D)
     call("trocm_sdpa", dq.ptr, dk.ptr, dv.ptr, None, out.ptr, ta.F16, B, Hq, 2, n, T, D, strides, 1, 1, C.c_float(1.0), 0, ws.ptr, ws.nbytes, None)
     np.testing.assert_array_equal(out.to_numpy(), np.full_like(q, np.float16(c * exact)))
+
+
+# scales that are not positive, an output that is aligned to 8 bytes only: the smaller kernel (sdpa_prefill.hip), its keys
+# over two sets of waves, 64 or (from 256 workgroups on) 128 queries per workgroup
+@pytest.mark.parametrize("what", ["negative scale", "zero scale", "output"])
+@pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [(1, 6, 2, 128, 31, 65), (1, 5, 5, 64, 0, 130), (2, 64, 8, 64, 70, 129), (1, 3, 1, 128, 300, 64)])
+def test_what_only_the_smaller_kernel_takes(rt, what, B, Hq, Hkv, D, past, n):
+    rng = np.random.default_rng(past + n)
+    T = past + n
+    q, k, v = _normal(rng, B, Hq, n, D), _normal(rng, B, Hkv, T, D), _normal(rng, B, Hkv, T, D)
+    scale = {"negative scale": -0.11, "zero scale": 0.0, "output": 0.11}[what]
+    at = 4 if what == "output" else 0
+    ws = ta.Workspace(B, Hq, n, D)
+    dq, dk, dv = (ta.DeviceTensor.from_numpy(x) for x in (q, k, v))
+    strides = (C.c_int64 * 3)(Hkv * T * D, T * D, D)
+    for causal in (True, False):
+        out = ta.DeviceTensor.from_numpy(np.full(q.size + 8, 7, np.float16))
+        call("trocm_sdpa", dq.ptr, dk.ptr, dv.ptr, None, C.c_void_p(out.ptr.value + 2 * at), ta.F16, B, Hq, Hkv, n, T, D, strides, 1, 1, C.c_float(scale), int(causal),
+             ws.ptr, ws.nbytes, None)
+        flat = out.to_numpy()
+        assert (flat[:at] == 7).all() and (flat[at + q.size :] == 7).all()
+        got, want = flat[at : at + q.size].reshape(q.shape).astype(np.float64), textbook_sdpa(q, k, v, scale=scale, causal=causal)
+        assert np.linalg.norm(got - want) <= TOL * np.linalg.norm(want), causal
+        assert (np.linalg.norm(got - want, axis=-1) <= 2 * TOL * np.linalg.norm(want, axis=-1) + 2.0 ** -20).all(), causal
