@@ -40,13 +40,14 @@
 //  * What shows only later is seen in the sums, and the workgroup starts again with the f32 code: values beyond the room, infinities
 //    and NaN (sums that are no numbers), and V that has become too weak for its unit (a row, or a feature over all the rows, that is
 //    small against what the pairs leave).
-//  * What bounds it is the issue of instructions: per tile and wave 48 matrix and about 550 vector instructions, whose busy cycles
-//    add up to 97 % of the kernel's (counters; 2000 queries: 33 and 64 %).  Loads have no condition around them, or the waits for
-//    one tile's V would be waits for the next tile's K (71.6 -> 58.2 us).
-// us of a call with its append, on the f32 instruction | as pairs | refused: 1000 queries of 32 heads over 8 (D = 128) 104.8 | 60.4 | 106;
-// 771 over 451 tokens 132.3 | 70.1 | 153; 10 queries of 4 x 64 heads over 8, 3629 tokens, 96.3 | 65.3 | 110; 2 x 251 queries 28.6 | 25.9 |
-// 41 (refused tiles cost more where few workgroups of 64 rows take the place of twice as many of 32; 137, 198, 139 and 49 while
-// the pairs' loop ran before them).  What only the sums show: 134, 200, 115 and 50.
+//  * What bounds it is the issue of instructions: per tile and wave 48 matrix and about 550 vector instructions.  1000 queries of 32
+//    heads over 8: matrix units busy 23 % of the kernel's cycles and vector units 44, which do not overlap, and the longest row tiles
+//    run on alone (2000 queries: 33 and 64).  Loads have no condition around them, or the waits for one tile's V would be waits for
+//    the next tile's K (71.6 -> 58.2 us).
+// us of a call with its append, on the f32 instruction | as pairs | refused: 1000 queries of 32 heads over 8 (D = 128) 102.6 | 54.4 | 103;
+// 771 over 451 tokens 130.9 | 63.7 | 152; 10 queries of 4 x 64 heads over 8, 3629 tokens, 96.5 | 65.0 | 114; 2 x 251 queries 28.1 | 24.9 |
+// 41 (refused tiles cost more where few workgroups of 64 rows take the place of twice as many of 32; 135, 197, 141 and 49 while
+// the pairs' loop ran before them).  What only the sums show: 138, 199, 112 and 51.
 // From 4 tiles on (2 x 70 queries of 32 heads over 32, 3 tiles: 15.3 | 17.5; 2 x 116 of 40 over 8 20.0 | 18.0); ranges of keys (us
 // without | with): 49 queries, 32 over 8, 396 tokens 29.7 | 21.5, but 2 x 251, a workgroup per compute unit, 25.0 | 33.7.
 #include <hip/hip_runtime.h>
