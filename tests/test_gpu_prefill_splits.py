@@ -100,6 +100,18 @@ def test_short_prompts_of_odd_groups_sum_their_weights_in_f32(rt, D, T):
     np.testing.assert_array_equal(out.to_numpy(), np.full_like(q, np.float16(c * exact)))
 
 
+@pytest.mark.parametrize("heads,kv,D,n,T", [(40, 8, 128, 70, 370), (14, 2, 64, 70, 970), (5, 5, 128, 100, 100)])
+@pytest.mark.parametrize("size", [500, 20000, 60000])
+def test_a_key_that_is_larger_than_all_others_together(rt, heads, kv, D, n, T, size):
+    """Scores up to 2^36: queries that point along it see that token's value alone."""
+    rng = np.random.default_rng(T)
+    q, k, v = np.full((1, heads, n, D), size, np.float16), _normal(rng, 1, kv, T, D), _normal(rng, 1, kv, T, D)
+    k[:, :, T // 3] = size
+    ws = ta.Workspace(1, heads, n, D)
+    got = _sdpa(q, k, v, False, ws, ws.nbytes)
+    np.testing.assert_array_equal(got, np.broadcast_to(np.repeat(v[:, :, T // 3 : T // 3 + 1], heads // kv, axis=1), q.shape))
+
+
 # scales that are not positive, an output that is aligned to 8 bytes only: the smaller kernel (sdpa_prefill.hip), its keys
 # over two sets of waves, 64 or (from 256 workgroups on) 128 queries per workgroup
 @pytest.mark.parametrize("what", ["negative scale", "zero scale", "output"])

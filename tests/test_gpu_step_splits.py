@@ -7,6 +7,7 @@ import pytest
 
 import tract_amd as ta
 from oracle import oracle as orc
+from tests.cases import textbook_sdpa
 from tests.gpu_util import rt  # noqa: F401
 from tract_amd._lib import call
 
@@ -73,3 +74,29 @@ def test_more_than_eight_splits_come_in_eights(rt, T):
     record = B * Hkv * 8 * (D + 2) * 4   # of one split: rows of eight heads per kv head, their maxima and sums
     splits = -(-used // record)
     assert splits > 8 and splits % 8 == 0
+
+
+# 32 heads over 8 and 64 over 8 with 64 features (f32: the matrix instruction), one head per kv head (vector units)
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,D,T", [(np.float32, 1, 32, 8, 128, 500), (np.float32, 2, 64, 8, 64, 900), (np.float32, 1, 32, 32, 128, 300),
+                                                 (np.float32, 2, 8, 4, 64, 700), (np.float16, 1, 32, 32, 128, 300), (np.float16, 3, 16, 16, 64, 40)])
+@pytest.mark.parametrize("size", [3e4, 6e4, 3e10, 1e20, 1e30])
+def test_a_key_that_is_larger_than_all_others_together(rt, dtype, B, Hq, Hkv, D, T, size):
+    """A query that points along it sees that token's value alone, one that points away from it does not see the token at all."""
+    if dtype is np.float16 and size > 65504:
+        pytest.skip("not an f16 number")
+    rng = np.random.default_rng(T)
+    q, k, v = (rng.standard_normal((B, h, n, D), dtype=np.float32) for h, n in [(Hq, 1), (Hkv, T), (Hkv, T)])
+    first = 8 if dtype is np.float32 else D   # (f16: a score of 2^31 and more takes every feature)
+    k[:, :, T // 3, :first] = size
+    along = rng.integers(2, size=(B, Hq, 1, 1)) > 0
+    if dtype is np.float16:
+        q = np.where(along, np.float32(size), q / 4 - (q / 4).mean(axis=-1, keepdims=True) - np.float32(0.25))
+    else:
+        q[..., :first] = np.where(along, 1, -1) * np.abs(q[..., :first])
+    q, k, v = q.astype(dtype), k.astype(dtype), v.astype(dtype)
+    st = ta.InPlaceKvSdpa(axis=2, causal=True).state()
+    st.k.push(k[:, :, :-1]), st.v.push(v[:, :, :-1])
+    got = st.eval([q, np.ascontiguousarray(k[:, :, -1:]), np.ascontiguousarray(v[:, :, -1:])]).to_numpy().astype(np.float64)
+    want = textbook_sdpa(q, k, v, causal=True)
+    tol = 2 * 2.0 ** -11 if dtype is np.float16 else 2.0 ** -20   # (as above, and as the f32 steps' own tests)
+    assert np.abs(got - want).max() <= tol * np.abs(v.astype(np.float64)).max()

