@@ -79,11 +79,11 @@ def test_more_than_eight_splits_come_in_eights(rt, T):
 # 32 heads over 8 and 64 over 8 with 64 features (f32: the matrix instruction), one head per kv head (vector units)
 @pytest.mark.parametrize("dtype,B,Hq,Hkv,D,T", [(np.float32, 1, 32, 8, 128, 500), (np.float32, 2, 64, 8, 64, 900), (np.float32, 1, 32, 32, 128, 300),
                                                  (np.float32, 2, 8, 4, 64, 700), (np.float16, 1, 32, 32, 128, 300), (np.float16, 3, 16, 16, 64, 40)])
-@pytest.mark.parametrize("size", [3e4, 6e4, 3e10, 1e20, 1e30])
+@pytest.mark.parametrize("size", [6e4, 3e10, 1e30])   # (f16: a tenth of its largest, half of it, its largest)
 def test_a_key_that_is_larger_than_all_others_together(rt, dtype, B, Hq, Hkv, D, T, size):
     """A query that points along it sees that token's value alone, one that points away from it does not see the token at all."""
-    if dtype is np.float16 and size > 65504:
-        pytest.skip("not an f16 number")
+    if dtype is np.float16:
+        size = {6e4: 6550, 3e10: 32752, 1e30: 65504}[size]
     rng = np.random.default_rng(T)
     q, k, v = (rng.standard_normal((B, h, n, D), dtype=np.float32) for h, n in [(Hq, 1), (Hkv, T), (Hkv, T)])
     first = 8 if dtype is np.float32 else D   # (f16: a score of 2^31 and more takes every feature)
