@@ -1,0 +1,68 @@
+"""Prompts and chunks of one whose new rows the attention launch reads from the call's input and stores to the cache itself: bit for
+bit the attention over the same rows in one tensor, and the cache bit for bit the rows."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import tract_amd as ta
+from tests.gpu_util import rt  # noqa: F401
+from tract_amd._lib import call
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(dtype, B, Hq, Hkv, D, past, n):
+    rng = np.random.default_rng(past + n)
+    return tuple(rng.standard_normal((B, h, t, D), dtype=np.float32).astype(dtype) for h, t in ((Hq, n), (Hkv, past + n), (Hkv, past + n)))
+
+
+def _over_one_tensor(q, k, v, causal):
+    B, Hq, n, D = q.shape
+    Hkv, T = k.shape[1:3]
+    dq, dk, dv = (ta.DeviceTensor.from_numpy(x) for x in (q, k, v))
+    out = ta.DeviceTensor(q.shape, q.dtype)
+    ws = ta.Workspace(B, Hq, n, D)
+    call("trocm_sdpa", dq.ptr, dk.ptr, dv.ptr, None, out.ptr, ta.F16 if q.dtype == np.float16 else ta.F32, B, Hq, Hkv, n, T, D,
+         (C.c_int64 * 3)(Hkv * T * D, T * D, D), 1, 1, C.c_float(float("nan")), int(causal), ws.ptr, ws.nbytes, None)
+    return out.to_numpy()
+
+
+def _state(k, v, past, n, causal):
+    """Caches of `past` tokens, in planes longer than they need."""
+    st = ta.InPlaceKvSdpa(axis=2, causal=causal).state()
+    for c, x in ((st.k, k), (st.v, v)):
+        c.reserve(past + n + 37, like=((x.shape[0], x.shape[1], 1, x.shape[3]), x.dtype))
+        if past:
+            c.push(x[:, :, :past])
+    return st
+
+
+# the first new row on a tile's edge, before it and behind it, all of them in one tile; pieces that do not go round; 1 to 8 query heads
+# per kv head, key splits merged by the last of them and by a launch, a workgroup alone on its unit
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,D,past,n", [
+    (np.float16, 1, 8, 2, 128, 640, 150), (np.float16, 2, 8, 2, 128, 639, 99), (np.float16, 1, 16, 4, 128, 65, 301), (np.float16, 1, 14, 2, 128, 700, 99),
+    (np.float16, 2, 4, 4, 128, 0, 700), (np.float16, 1, 32, 32, 64, 30, 1001), (np.float16, 3, 16, 2, 64, 1, 333), (np.float16, 4, 64, 8, 64, 0, 300),
+    (np.float16, 1, 8, 8, 64, 2000, 70), (np.float16, 1, 32, 8, 128, 3000, 41), (np.float16, 1, 2, 1, 128, 5, 65)])
+def test_rows_from_the_call(rt, dtype, B, Hq, Hkv, D, past, n):
+    q, k, v = _inputs(dtype, B, Hq, Hkv, D, past, n)
+    for causal in (True, False):
+        st = _state(k, v, past, n, causal)
+        for _ in range(2):   # again over what the first call left behind
+            if past or _:
+                st.k.truncate(past), st.v.truncate(past)
+            got = st.eval([q, np.ascontiguousarray(k[:, :, past:]), np.ascontiguousarray(v[:, :, past:])]).to_numpy()
+            assert st.k.valid_contiguous().tobytes() == k.tobytes() and st.v.valid_contiguous().tobytes() == v.tobytes()
+            assert got.tobytes() == _over_one_tensor(q, k, v, causal).tobytes(), causal
+
+
+# an output over the new keys or values (as many kv heads as query heads): appended first
+@pytest.mark.parametrize("dtype,past,n", [(np.float16, 100, 200)])
+@pytest.mark.parametrize("over", ["k", "v"])
+def test_results_over_the_new_rows(rt, dtype, past, n, over):
+    q, k, v = _inputs(dtype, 2, 4, 4, 128, past, n)
+    st = _state(k, v, past, n, True)
+    args = {"k": ta.DeviceTensor.from_numpy(np.ascontiguousarray(k[:, :, past:])), "v": ta.DeviceTensor.from_numpy(np.ascontiguousarray(v[:, :, past:]))}
+    got = st.eval_into(ta.DeviceTensor.from_numpy(q), args["k"], args["v"], args[over]).to_numpy()
+    assert st.k.valid_contiguous().tobytes() == k.tobytes() and st.v.valid_contiguous().tobytes() == v.tobytes()
+    assert got.tobytes() == _over_one_tensor(q, k, v, True).tobytes()

@@ -32,6 +32,7 @@
 //
 // Roofline: MFMA-bound.  FLOPs = 4 * B * Hq * D * (visible query-key pairs).
 #include <hip/hip_fp16.h>
+#include <limits.h>
 #include <string.h>
 #include <stdlib.h>
 #include <type_traits>
@@ -75,6 +76,10 @@ struct PrefillPP {
     // k / v, f16 scale planes [B, Hkv, pitch, D/32]; strides in token rows
     const uint16_t *k_scales, *v_scales;
     int64_t row_stride_b, row_stride_h;
+    // Fused append (f16 caches without a mask, registers loop): the last Sq tokens are read from the call's k_new / v_new, dense
+    // [B, Hkv, Sq, D], and stored to the cache (dense token rows) by this launch; NULL: all tokens are in the cache.
+    const _Float16 *k_new, *v_new;
+    int new_from;       // first token that is read from them (INT_MAX: none)
 };
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -217,15 +222,45 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
         ksp = p.k_scales + plane_row * (D / 32);
         vsp = p.v_scales + plane_row * (D / 32);
     }
+    // The append.  A workgroup copies its share of its kv head's new rows (contiguous in both places) on the way in, a 16-byte
+    // piece or two of each tensor per thread beside the loads of the queries and of the first tile; tiles of new rows are read
+    // from the call's input, so no workgroup waits for another.  The one tile that may hold both kinds picks by row.
+    // A call of 512 queries behind 3584 tokens, 32 heads in groups of 4, an append launch and 64-bit addresses per lane before |
+    // now: 45.3 | 43.1 us; behind none 18.4 | 16.2; 2 x 1500 of 32 heads over 32 69.0 | 63.5 (68.3 with all of the share copied on
+    // the way in), at D = 64 44.2 | 38.8; 3 x 917 of 64 over 8 behind 3704, D = 64, 242 | 236.5.
+    constexpr bool APPEND = !QUANT && !MASK && !PING;
+    constexpr int CD = 2;   // pieces of each tensor that a thread copies on the way in
+    const _Float16 *knew = nullptr, *vnew = nullptr;   // where token 0 would be
+    if constexpr (APPEND) {
+        const int64_t first = (((int64_t)b * p.Hkv + kvh) * p.Sq - off) * D;
+        knew = p.k_new + first, vnew = p.v_new + first;
+    }
+    // A tile whose rows are all of one kind and all there is asked for at a wave-uniform address plus one offset per lane.
+    const int key0 = tid / (D / 8), dc0 = tid % (D / 8);
+    constexpr int KEYS = kThreadsPP / (D / 8);   // rows between a thread's pieces
+    const int64_t row_bytes = (APPEND && p.k_new ? D : p.kv_stride_t) * 2;
+    const uint32_t lane_off = QUANT ? 0 : (uint32_t)key0 * (uint32_t)row_bytes + dc0 * 16;   // (rows of less than 2^25 bytes)
     auto prefetch = [&](int kt) {
         if constexpr (!QUANT) {
+            const bool fresh = APPEND && kt * kTileN >= p.new_from;
+            if (kt * kTileN + kTileN <= (fresh || !APPEND ? p.Sk : min(p.Sk, p.new_from))) {
+                const char *tk = reinterpret_cast<const char *>(fresh ? knew : kbase) + (int64_t)kt * kTileN * row_bytes;
+                const char *tv = reinterpret_cast<const char *>(fresh ? vnew : vbase) + (int64_t)kt * kTileN * row_bytes;
+                uint32_t o32 = lane_off;
+                asm volatile("" : "+v"(o32));   // (stays a 32-bit offset up to the loads)
 #pragma unroll
-            for (int j = 0; j < NL; j++) {
-                int c = j * kThreadsPP + tid;
-                int key = c / (D / 8), dc = c % (D / 8);
-                int64_t row = min(kt * kTileN + key, p.Sk - 1);
-                kpre[j] = *reinterpret_cast<const u32x4 *>(kbase + row * p.kv_stride_t + dc * 8);
-                vpre[j] = *reinterpret_cast<const u32x4 *>(vbase + row * p.kv_stride_t + dc * 8);
+                for (int j = 0; j < NL; j++) {
+                    kpre[j] = *reinterpret_cast<const u32x4 *>(tk + j * KEYS * row_bytes + o32);
+                    vpre[j] = *reinterpret_cast<const u32x4 *>(tv + j * KEYS * row_bytes + o32);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < NL; j++) {
+                    const int64_t row = min(kt * kTileN + key0 + j * KEYS, p.Sk - 1);
+                    const bool is_new = APPEND && row >= p.new_from;
+                    kpre[j] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(is_new ? knew : kbase) + row * row_bytes + dc0 * 16);
+                    vpre[j] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(is_new ? vnew : vbase) + row * row_bytes + dc0 * 16);
+                }
             }
         } else if (q_active) {
             const int64_t row = min(kt * kTileN + q_key, p.Sk - 1);
@@ -415,6 +450,23 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
 
     if constexpr (!PING) {
         if (n_it > 0) prefetch(t_begin);   // issued before the Q loads: both latencies overlap
+        u32x4 ck[CD], cv[CD];              // the first of this thread's pieces of the new rows
+        int piece = 0, pieces = 0, hop = 0;
+        const u32x4 *src_k = nullptr, *src_v = nullptr;
+        u32x4 *dst_k = nullptr, *dst_v = nullptr;
+        if constexpr (APPEND) {
+            if (p.k_new) {
+                pieces = p.Sq * (D / 8);
+                piece = (((qt * p.nsplit + split) * (G / HG)) + gg) * kThreadsPP + tid;
+                hop = p.n_qtiles * p.nsplit * (G / HG) * kThreadsPP;
+                src_k = reinterpret_cast<const u32x4 *>(knew + (int64_t)off * D), src_v = reinterpret_cast<const u32x4 *>(vnew + (int64_t)off * D);
+                dst_k = reinterpret_cast<u32x4 *>(const_cast<_Float16 *>(kbase) + (int64_t)off * D);
+                dst_v = reinterpret_cast<u32x4 *>(const_cast<_Float16 *>(vbase) + (int64_t)off * D);
+#pragma unroll
+                for (int j = 0; j < CD; j++)
+                    if (piece + j * hop < pieces) ck[j] = src_k[piece + j * hop], cv[j] = src_v[piece + j * hop];
+            }
+        }
         // Q^T fragments: query = lane % 32, features 16*ks + 8*hb .. +8
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) qf[ks] = *reinterpret_cast<const half8_t *>(qrow + 16 * ks + 8 * hb);
@@ -423,6 +475,13 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
         // for the K/V prefetch issued a few instructions earlier and exposes its whole latency.
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(qf[ks]));
+        if constexpr (APPEND) {
+            if (p.k_new) {
+#pragma unroll
+                for (int j = 0; j < CD; j++)
+                    if (piece + j * hop < pieces) dst_k[piece + j * hop] = ck[j], dst_v[piece + j * hop] = cv[j];
+            }
+        }
 
         if (n_it > 0) {
             stage(0, 0);
@@ -447,6 +506,19 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
             if (it + 1 < n_it) {
                 stage(cur ^ 1, cur ^ 1);
                 if (it + 2 < n_it) prefetch(t_begin + it + 2);
+            }
+        }
+        if constexpr (APPEND) {   // what is left of the share (prompts of few query heads per kv head), four pieces of each tensor at a time
+            for (piece += CD * hop; piece < pieces; piece += 4 * hop) {
+                u32x4 rk[4], rv[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int i = min(piece + j * hop, pieces - 1);
+                    rk[j] = src_k[i], rv[j] = src_v[i];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (piece + j * hop < pieces) dst_k[piece + j * hop] = rk[j], dst_v[piece + j * hop] = rv[j];
             }
         }
     } else {
@@ -997,6 +1069,10 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
     if (!(a.scale > 0.0f)) return 2;       // the running maximum is taken before scaling
     if (a.causal && a.Sk < a.Sq) return 2;  // some queries would see nothing: the generic kernel owns that case
     if (a.Sk >= (1ll << 30) || a.Sq >= (1ll << 30) || a.B >= (1ll << 20)) return 2;
+    if (a.k_new) {   // appended by this launch
+        if (quant || a.mask || ping_enabled() || !a.v_new || a.kv_stride_t != a.D || a.Sk < a.Sq || a.Sq > (1 << 20)) return 2;
+        if ((uintptr_t)a.k_new % 16 || (uintptr_t)a.v_new % 16) return 2;
+    }
     if ((a.kv_stride_b % 8) || (a.kv_stride_h % 8) || (a.kv_stride_t % 8)) return 2;  // 128-bit row loads
     if (a.kv_stride_t >= (1ll << 24)) return 2;  // byte offsets within a tile are 32-bit
     if ((uintptr_t)a.q % 16 || (uintptr_t)a.k % 16 || (uintptr_t)a.v % 16 || (uintptr_t)a.out % 16) return 2;
@@ -1035,6 +1111,8 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
         p.row_stride_b = a.kv_stride_b / a.D, p.row_stride_h = a.kv_stride_h / a.D;
     }
     p.B = (int)a.B, p.Hq = (int)a.Hq, p.Hkv = (int)a.Hkv, p.Sq = (int)a.Sq, p.Sk = (int)a.Sk;
+    p.k_new = (const _Float16 *)a.k_new, p.v_new = (const _Float16 *)a.v_new;
+    p.new_from = a.k_new ? (int)(a.Sk - a.Sq) : INT_MAX;
     p.causal = a.causal;
     p.scale_log2 = a.scale * 1.4426950408889634f;
     p.n_qtiles = (int)n_qtiles;
@@ -1088,7 +1166,7 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
         p.paired = (int)((cus + wgs / n_qtiles - 1) / (wgs / n_qtiles));
     else if (a.causal && a.B > 1 && 5 * a.Sq > 4 * a.Sk)
         p.paired = (int)n_qtiles;
-    if (wgs >= (1ll << 31)) return 2;
+    if (wgs >= (a.k_new ? 1ll << 18 : 1ll << 31)) return 2;   // (the pieces of an append are counted in 32 bits)
     return a.D == 128 ? launch_hg<128>(p, a.kv_fmt, hg, wgs, true, s) : launch_hg<64>(p, a.kv_fmt, hg, wgs, alone, s);
 }
 
