@@ -39,11 +39,14 @@ def _state(k, v, past, n, causal):
 
 
 # the first new row on a tile's edge, before it and behind it, all of them in one tile; pieces that do not go round; 1 to 8 query heads
-# per kv head, key splits merged by the last of them and by a launch, a workgroup alone on its unit
+# per kv head, key splits merged by the last of them and by a launch, a workgroup alone on its unit; f32: none, one and many ranges of
+# keys, one workgroup, shapes that the launch does not take (few tiles, a cache that is not empty)
 @pytest.mark.parametrize("dtype,B,Hq,Hkv,D,past,n", [
     (np.float16, 1, 8, 2, 128, 640, 150), (np.float16, 2, 8, 2, 128, 639, 99), (np.float16, 1, 16, 4, 128, 65, 301), (np.float16, 1, 14, 2, 128, 700, 99),
     (np.float16, 2, 4, 4, 128, 0, 700), (np.float16, 1, 32, 32, 64, 30, 1001), (np.float16, 3, 16, 2, 64, 1, 333), (np.float16, 4, 64, 8, 64, 0, 300),
-    (np.float16, 1, 8, 8, 64, 2000, 70), (np.float16, 1, 32, 8, 128, 3000, 41), (np.float16, 1, 2, 1, 128, 5, 65)])
+    (np.float16, 1, 8, 8, 64, 2000, 70), (np.float16, 1, 32, 8, 128, 3000, 41), (np.float16, 1, 2, 1, 128, 5, 65),
+    (np.float32, 1, 8, 2, 128, 0, 150), (np.float32, 2, 14, 2, 64, 0, 171), (np.float32, 1, 32, 32, 128, 0, 333), (np.float32, 1, 6, 6, 64, 0, 1100),
+    (np.float32, 1, 8, 2, 128, 0, 60), (np.float32, 1, 8, 2, 128, 64, 200)])
 def test_rows_from_the_call(rt, dtype, B, Hq, Hkv, D, past, n):
     q, k, v = _inputs(dtype, B, Hq, Hkv, D, past, n)
     for causal in (True, False):
@@ -57,7 +60,7 @@ def test_rows_from_the_call(rt, dtype, B, Hq, Hkv, D, past, n):
 
 
 # an output over the new keys or values (as many kv heads as query heads): appended first
-@pytest.mark.parametrize("dtype,past,n", [(np.float16, 100, 200)])
+@pytest.mark.parametrize("dtype,past,n", [(np.float16, 100, 200), (np.float32, 0, 200)])
 @pytest.mark.parametrize("over", ["k", "v"])
 def test_results_over_the_new_rows(rt, dtype, past, n, over):
     q, k, v = _inputs(dtype, 2, 4, 4, 128, past, n)
