@@ -134,3 +134,36 @@ def test_what_only_the_smaller_kernel_takes(rt, what, B, Hq, Hkv, D, past, n):
         got, want = flat[at : at + q.size].reshape(q.shape).astype(np.float64), textbook_sdpa(q, k, v, scale=scale, causal=causal)
         assert np.linalg.norm(got - want) <= TOL * np.linalg.norm(want), causal
         assert (np.linalg.norm(got - want, axis=-1) <= 2 * TOL * np.linalg.norm(want, axis=-1) + 2.0 ** -20).all(), causal
+
+
+# more query tiles than whole rounds of compute units take: those left over are cut into 2, 3 and 4 ranges of keys (one head of a
+# group of one, a group of two and of four per workgroup; causal behind past tokens or unmasked; the last tile with few queries)
+@pytest.mark.parametrize("store", [None, ta.Q8_0, ta.Q4_0])
+@pytest.mark.parametrize("B,Hq,Hkv,past,n,causal", [(1, 384, 96, 1100, 130, True), (2, 160, 40, 900, 220, False), (1, 128, 64, 1300, 613, True), (2, 60, 60, 1300, 530, False)])
+def test_tiles_left_for_the_last_round(rt, store, B, Hq, Hkv, past, n, causal):
+    rng = np.random.default_rng(n)
+    T, G = past + n, Hq // Hkv
+    q, k, v = _normal(rng, B, Hq, n, 128), _normal(rng, B, Hkv, T, 128), _normal(rng, B, Hkv, T, 128)
+    if store is None:
+        v[0, 1, 40, 9] = np.inf   # one range's output, in one feature of one kv head
+    kc, vc = ta.InPlaceKvCache(2, store), ta.InPlaceKvCache(2, store)
+    kc.push(k), vc.push(v)
+    dq, out = ta.DeviceTensor.from_numpy(q), ta.DeviceTensor(q.shape, np.float16)
+    ws = ta.Workspace(B, Hq, n, 128)
+    results = []
+    for size in (64 * 1024, ws.nbytes, ws.nbytes):   # whole; cut; the same bits again
+        call("trocm_sdpa_cached", dq.ptr, ta.F16, Hq, n, kc._h, vc._h, out.ptr, C.c_float(float("nan")), int(causal), ws.ptr, size, None)
+        results.append(out.to_numpy())
+    assert results[1].tobytes() == results[2].tobytes()
+    infinite = np.zeros(q.shape, bool)
+    if store is None:
+        infinite[0, G : 2 * G, :, 9] = True
+    for r in results[:2]:
+        np.testing.assert_array_equal(np.isposinf(r), infinite)
+    whole, cut = (np.where(infinite, 0, r).astype(np.float64) for r in results[:2])
+    err, rows = np.linalg.norm(cut - whole, axis=-1), np.linalg.norm(whole, axis=-1)
+    assert (err <= 3 * TOL * rows + 2.0 ** -20).all()   # both round as above
+    if store is None:   # the first and the last heads against f64
+        for b, h in ((0, 0), (B - 1, Hkv - 1)):
+            want = textbook_sdpa(q[b : b + 1, h * G : (h + 1) * G], k[b : b + 1, h : h + 1], v[b : b + 1, h : h + 1], causal=causal)
+            assert np.linalg.norm(cut[b, h * G : (h + 1) * G] - want[0]) <= TOL * np.linalg.norm(want)

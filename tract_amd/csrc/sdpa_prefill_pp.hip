@@ -80,6 +80,9 @@ struct PrefillPP {
     // [B, Hkv, Sq, D], and stored to the cache (dense token rows) by this launch; NULL: all tokens are in the cache.
     const _Float16 *k_new, *v_new;
     int new_from;       // first token that is read from them (INT_MAX: none)
+    // PARTS (choose_parts): so many query tiles, from the last on down, have a workgroup each, the others `nsplit`; partials in f32,
+    // merged by the last range of a tile to arrive.
+    int whole;
 };
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -132,7 +135,9 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t b0123, uint32_t b4567, half2_
 // F32: the row sum takes the weights as they are before they are rounded for the product with V, their reference is the maximum
 // itself, and partials are f32.
 // ALONE: a workgroup has a compute unit to itself, and as many registers as it likes (D = 64; D = 128 always has).
-template <int D, int HG, bool MASK, int FMT, bool PING = false, bool F32 = false, bool ALONE = D != 64 || MASK>
+// PARTS: some query tiles in several key ranges, merged here from f32 partials; an instantiation of its own, since the two
+// ways of merging in one kernel spill registers.
+template <int D, int HG, bool MASK, int FMT, bool PING = false, bool F32 = false, bool ALONE = D != 64 || MASK, bool PARTS = false>
 __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_kernel(PrefillPP p) {
     static_assert(!F32 || (HG == 1 && !MASK && FMT == TROCM_F16 && !PING), "short prompts of one head per workgroup");
     static_assert(!PING || (!MASK && FMT == TROCM_F16), "the ping-pong loop serves f16 caches without a mask input");
@@ -166,10 +171,14 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
     const int G = p.Hq / p.Hkv;
     const int gg = id % (G / HG);
     id /= (G / HG);
-    const int split = id % p.nsplit;
-    id /= p.nsplit;
-    int b, qt;
-    if (p.paired) {   // one wave of workgroups over the chip with the longest tiles first, beside them the others, shortest first
+    int b, qt, split, nsplit = p.nsplit;
+    if constexpr (PARTS) {
+        b = id % p.B, id /= p.B;
+        if (id < p.whole) nsplit = 1;
+        else id -= p.whole;
+        split = id % nsplit;
+        qt = p.n_qtiles - 1 - (nsplit > 1 ? p.whole : 0) - id / nsplit;
+    } else if (split = id % nsplit, id /= nsplit; p.paired) {   // one wave of workgroups over the chip with the longest tiles first, beside them the others, shortest first
         b = id % p.B, id /= p.B;
         qt = id < p.paired ? p.n_qtiles - 1 - id : id - p.paired;
     } else {
@@ -190,7 +199,7 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
     const int wg_q_last = min(qt * BLOCK_M + BLOCK_M, p.Sq) - 1;
     const int last_key = p.causal ? min(p.Sk - 1, wg_q_last + off) : p.Sk - 1;
     const int n_kt = last_key / kTileN + 1;
-    const int per = (n_kt + p.nsplit - 1) / p.nsplit;
+    const int per = (n_kt + nsplit - 1) / nsplit;
     const int t_begin = split * per;
     const int n_it = max(0, min(n_kt, t_begin + per) - t_begin);
     const int wave_q_last = min(q0 + 31, p.Sq - 1);
@@ -457,8 +466,9 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
         if constexpr (APPEND) {
             if (p.k_new) {
                 pieces = p.Sq * (D / 8);
-                piece = (((qt * p.nsplit + split) * (G / HG)) + gg) * kThreadsPP + tid;
-                hop = p.n_qtiles * p.nsplit * (G / HG) * kThreadsPP;
+                // (tiles in unlike numbers of parts: the first range copies for its tile)
+                piece = PARTS ? (split == 0 ? (qt * (G / HG) + gg) * kThreadsPP + tid : pieces) : (((qt * nsplit + split) * (G / HG)) + gg) * kThreadsPP + tid;
+                hop = p.n_qtiles * (PARTS ? 1 : nsplit) * (G / HG) * kThreadsPP;
                 src_k = reinterpret_cast<const u32x4 *>(knew + (int64_t)off * D), src_v = reinterpret_cast<const u32x4 *>(vnew + (int64_t)off * D);
                 dst_k = reinterpret_cast<u32x4 *>(const_cast<_Float16 *>(kbase) + (int64_t)off * D);
                 dst_v = reinterpret_cast<u32x4 *>(const_cast<_Float16 *>(vbase) + (int64_t)off * D);
@@ -745,10 +755,87 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
             wave_sync();   // ... and are done reading before the second half overwrites it
         }
     };
-    if (p.nsplit == 1) {
+    // ---- a tile in a few parts of its own (PARTS): f32 partials, out = sum_s w_s O_s over the parts in their order by the last to
+    // arrive, its own from the registers.  Pieces of 8 bytes, so that a store covers 512 consecutive ones; written through to memory.
+    auto merge_parts = [&]() __attribute__((always_inline)) {
+        const int64_t per_q = (int64_t)p.B * p.Hkv * (G / HG), n_tiles = per_q * (p.n_qtiles - p.whole), tile = qt * per_q + ((int64_t)b * (G / HG) + gg) * p.Hkv + kvh;
+        auto block = [&](int sp) { return ((int64_t)sp * n_tiles + tile) * kWavesPP + w; };
+        float *part_o = reinterpret_cast<float *>(p.part_o) + lane * 2;
+        const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
+        if (wave_has_queries) {
+            float *po = part_o + block(split) * (32 * D);
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    typedef float float2_v __attribute__((ext_vector_type(2)));
+                    o[db][2 * i] *= inv, o[db][2 * i + 1] *= inv;
+                    const float2_v x = {o[db][2 * i], o[db][2 * i + 1]};
+                    __hip_atomic_store(reinterpret_cast<uint64_t *>(po + (db * 8 + i) * 128), __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            __hip_atomic_store(p.part_ml + block(split) * 64 + lane, hb ? l_run : m_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this thread's stores have completed
+        __syncthreads();                                     // ... and so have the whole workgroup's
+        __shared__ int s_arrived;
+        if (tid == 0) {
+            int *counter = p.counters + tile;
+            const int arrived = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (arrived == nsplit - 1) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
+            s_arrived = arrived;
+        }
+        __syncthreads();
+        if (s_arrived != nsplit - 1 || !wave_has_queries) return;
+        float wv[kTailSplits], total = 0.0f, mm = -INFINITY;   // the weights, by every lane from the same records
+#pragma unroll
+        for (int sp = 0; sp < kTailSplits; sp++) {
+            const float *ml = p.part_ml + block(min(sp, nsplit - 1)) * 64 + l32;
+            const float m = __hip_atomic_load(ml, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), l = __hip_atomic_load(ml + 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const float top = fmaxf(mm, m), ref = top == -INFINITY ? 0.0f : top, keep = fast_exp2(mm - ref);
+            wv[sp] = sp < nsplit ? l * fast_exp2(m - ref) : 0.0f;
+#pragma unroll
+            for (int i = 0; i < sp; i++) wv[i] *= keep;
+            total = total * keep + wv[sp], mm = top;
+        }
+        const float inv_total = total > 0.0f ? 1.0f / total : 0.0f;
+#pragma unroll
+        for (int d2 = 0; d2 < DB; d2 += 2) {   // every part's two feature blocks in one trip, the own one's too (kept beside the others it spills)
+            uint64_t raw[kTailSplits][2][8];
+#pragma unroll
+            for (int sp = 0; sp < kTailSplits; sp++) {
+                if (sp >= nsplit) break;
+                const float *po = part_o + block(sp) * (32 * D) + d2 * 1024;
+#pragma unroll
+                for (int db = 0; db < 2; db++)
+#pragma unroll
+                    for (int i = 0; i < 8; i++)
+                        raw[sp][db][i] = __hip_atomic_load(reinterpret_cast<const uint64_t *>(po + (db * 8 + i) * 128), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+#pragma unroll
+            for (int db = 0; db < 2; db++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) o[d2 + db][r] = 0.0f;
+#pragma unroll
+            for (int sp = 0; sp < kTailSplits; sp++) {
+                if (sp >= nsplit) break;
+                const float wgt = wv[sp] * inv_total;
+#pragma unroll
+                for (int db = 0; db < 2; db++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++)
+                        o[d2 + db][r] = __builtin_fmaf(wgt, __builtin_bit_cast(float, (uint32_t)(raw[sp][db][r / 2] >> (32 * (r % 2)))), o[d2 + db][r]);
+            }
+        }
+        write_output(1.0f);
+    };
+    if (nsplit == 1) {
         __syncthreads();   // the V tile buffers are idle from here on
         if (!wave_has_queries) return;
         write_output(l_run > 0.0f ? 1.0f / l_run : 0.0f);
+        return;
+    }
+    if constexpr (PARTS) {
+        merge_parts();
         return;
     }
     // ---- key splits: store this split's normalised partial -----------------------------------------
@@ -998,9 +1085,34 @@ int64_t choose_splits(const PrefillPP &p, int D, int block_m, int64_t wgs1, int6
     return best;
 }
 
+// Query tiles of much the same length (past tokens, no causal mask) take the compute units in whole rounds, and those left for the
+// last round may be few: they are cut into 2 to 4 ranges of keys, so that all units share them.  The number of ranges (1: as it is);
+// `whole` tiles, `per_q` workgroups each, stay whole.  A cut costs about 10 us (f32 partials written through, the arrival, the other
+// parts read back), and units that would idle leave power to the others, so that half of the time it takes off the last round is
+// gained: from 16 us on, at 1.8 us for a tile of 64 keys.  (32 heads over 8, no causal mask, 2 x 1500: 108.7 -> 101 us; behind past
+// tokens 3 x 900 after 2000 152 -> 142, 2 x 1400 after 3000 214 -> 194, 64 over 8, 1300 after 4000 261 -> 224.)  Causal prompts
+// behind little, whose longest tile takes longer than all of them spread over the units, lose what they gain: 2048 queries 63 -> 67,
+// 2 x 1500 55 -> 64 with all tiles longer than that share cut in two.
+int choose_parts(const PrefillPP &p, int block_m, int64_t per_q, int64_t cus, int &whole) {
+    const int64_t wgs1 = per_q * p.n_qtiles;
+    if (wgs1 < cus || wgs1 >= 4 * cus) return 1;
+    auto tiles_of = [&](int qt) { return p.causal ? (min((qt + 1) * block_m, p.Sq) - 1 + p.Sk - p.Sq) / kTileN + 1 : (p.Sk - 1) / kTileN + 1; };
+    if (2 * tiles_of(0) < tiles_of(p.n_qtiles - 1)) return 1;
+    whole = (int)(wgs1 / cus * cus / per_q);
+    const int64_t left = (p.n_qtiles - whole) * per_q;
+    const int parts = left > 0 ? (int)min((int64_t)kTailSplits, cus / left) : 1;
+    return parts > 1 && 1.8f * (float)tiles_of(p.n_qtiles - whole - 1) * (1.0f - 1.0f / (float)parts) >= 16.0f ? parts : 1;
+}
+
 template <int D, int HG>
 int launch_cfg(const PrefillPP &p, int fmt, int64_t wgs, bool alone, hipStream_t s) {
-    if (fmt == TROCM_Q8_0)
+    if (D == 128 && p.whole && fmt == TROCM_Q8_0)
+        hipLaunchKernelGGL((sdpa_prefill_pp_kernel<128, HG, false, TROCM_Q8_0, false, false, true, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
+    else if (D == 128 && p.whole && fmt == TROCM_Q4_0)
+        hipLaunchKernelGGL((sdpa_prefill_pp_kernel<128, HG, false, TROCM_Q4_0, false, false, true, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
+    else if (D == 128 && p.whole)
+        hipLaunchKernelGGL((sdpa_prefill_pp_kernel<128, HG, false, TROCM_F16, false, false, true, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
+    else if (fmt == TROCM_Q8_0)
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_Q8_0>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     else if (fmt == TROCM_Q4_0)
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_Q4_0>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
@@ -1048,11 +1160,12 @@ int launch_hg(const PrefillPP &p, int fmt, int hg, int64_t wgs, bool alone, hipS
 static size_t split_bytes(int64_t n_wb, int64_t D, size_t elem = sizeof(_Float16)) { return (size_t)n_wb * (32 * (size_t)D * elem + 64 * sizeof(float)); }
 
 // Upper bound of the partial-result area the staggered prefill kernel may use for this shape.
-size_t prefill_workspace_bytes(int64_t B, int64_t Hq, int64_t Sq, int64_t D) {
+// least: without what only makes launches of a workgroup per compute unit and more faster (choose_parts).
+size_t prefill_workspace_bytes(int64_t B, int64_t Hq, int64_t Sq, int64_t D, bool least) {
     if (Sq < 2 || (D != 64 && D != 128)) return 0;
     const int64_t wgs1 = B * ((Hq + 3) / 4) * ((Sq + 63) / 64);  // about the fewest workgroups any head grouping gives
     const int64_t cus = 256;
-    if (wgs1 >= cus) return 0;
+    if (wgs1 >= cus) return !least && D == 128 && wgs1 < 5 * cus ? (size_t)cus * kWavesPP * (32 * 128 + 64) * sizeof(float) + 256 : 0;   // a part for each unit
     int64_t ns = (cus + wgs1 - 1) / wgs1;
     if (ns > kMaxSplits) ns = kMaxSplits;
     return (size_t)ns * split_bytes(B * Hq * ((Sq + 31) / 32), D) + 256;
@@ -1149,7 +1262,23 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
         static const int tail_merge = env_int("TROCM_PREFILL_TAIL_MERGE", 1);
         if (tail_merge && !p.part32 && ns <= kTailSplits && wgs1 <= (int64_t)(kWsCounterBytes / sizeof(int))) p.counters = (int *)a.workspace;
     }
-    const int64_t wgs = wgs1 * ns;
+    int64_t wgs = wgs1 * ns;
+    static const int cut_last = env_int("TROCM_PREFILL_PARTS", 1);
+    if (cut_last && ns == 1 && forced_split <= 0 && a.D == 128 && !p.mask && !p.part32 && !ping_enabled()) {
+        const int64_t per_q = wgs1 / n_qtiles;
+        int whole = 0;
+        const int parts = choose_parts(p, block_m, per_q, cus, whole);
+        const int64_t tiles = (n_qtiles - whole) * per_q, blocks = tiles * parts * kWavesPP;
+        if (parts > 1 && (size_t)blocks * (32 * 128 + 64) * sizeof(float) <= avail && tiles <= (int64_t)(kWsCounterBytes / sizeof(int))) {
+            char *base = (char *)a.workspace + kWsCounterBytes;
+            base += (256 - ((uintptr_t)base & 255)) & 255;
+            p.part_o = (_Float16 *)base;
+            p.part_ml = (float *)base + blocks * 32 * 128;
+            p.counters = (int *)a.workspace;
+            p.whole = whole, p.nsplit = parts;
+            wgs = wgs1 + tiles * (parts - 1);
+        }
+    }
     // Order of the workgroups of a causal prompt.  Where two fit on a compute unit (D = 64) and there are at most so many, all are
     // resident at once: the shortest tiles go beside the longest (3 x 40 heads x 574 queries behind 1717: 77.7 -> 60.8 us).  Otherwise a
     // prompt whose tiles differ much runs the longest of all its sequences first (3 x 32 x 1414 at D = 128: 83.9 -> 75.3), and one
