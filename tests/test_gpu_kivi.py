@@ -11,6 +11,7 @@ from tract_amd import kivi
 from oracle import oracle as orc
 from tests.gpu_util import max_abs, rt  # noqa: F401
 from tests.test_oracle_kivi import close_enough_super, lcg, take
+from tract_amd._lib import call
 
 pytestmark = pytest.mark.gpu
 
@@ -479,3 +480,35 @@ def test_quantized_kv_sdpa_over_the_codes_with_small_and_large_magnitudes(rt, k_
             # 8e-3 is what f16 outputs and f16 probabilities leave at unit magnitude; outputs below the halves'
             # normal range (6e-5) are also limited by the output type's own subnormal step (6e-8)
             assert err <= 8e-3 * size + 6e-8, (step, b, h, err, size)
+
+
+# tokens per thread 1 to 8 and one more than they hold, 4, 8 and 16 waves, a few tokens, more than the launch takes; values with
+# zeros of either sign, infinities and NaN among them
+@pytest.mark.parametrize("n", [2, 63, 256, 257, 700, 1024, 1025, 1537, 2049, 3073, 4097, 6145, 8192, 8193])
+@pytest.mark.parametrize("odd", [False, True])
+def test_a_first_prompt_in_one_launch_equals_the_stores_own_passes(rt, n, odd):
+    rng = np.random.default_rng(n)
+    B, Hq, Hkv, D = (2, 4, 2, 128) if n < 2000 else (1, 2, 1, 128)
+    q, k, v = (rng.standard_normal((B, h, n, D)).astype(np.float16) for h in (Hq, Hkv, Hkv))
+    k[..., ::7] *= np.float16(200)   # ranges that move the scale from 1
+    k[:, :, :, 5] = np.linspace(1, -600, n).astype(np.float16)   # a minimum and a scale that move with every token
+    if odd:
+        for x in (k, v):
+            for value in (0.0, -0.0, np.nan, np.inf, -np.inf):
+                x[rng.random(x.shape) < 0.01] = value
+        k[:, :, 0, 9], k[:, :, :, 11] = np.nan, np.nan
+        k[:, :, :, 13] = np.where(rng.random(n) < 0.5, 0.0, -0.0)
+    st = tract_amd.QuantizedKvSdpa(axis=2).state()
+    got = st.eval([q, k, v]).to_numpy()
+    kc, vc = kivi.KiviCache(kivi.KIVI_RUNNING_CHANNEL, 8, 0, B, Hkv, D), kivi.KiviCache(kivi.KIVI_PER_TOKEN, 8, 0, B, Hkv, D)
+    kc.append(k), vc.append(v)
+    for a, b in ((st.k, kc), (st.v, vc)):
+        mine, theirs = a.state(), b.state()
+        assert a.len() == n and mine.keys() == theirs.keys()
+        for part in mine:
+            np.testing.assert_array_equal(mine[part].view(np.uint8), theirs[part].view(np.uint8), err_msg=part)
+    dq, out = tract_amd.DeviceTensor.from_numpy(q), tract_amd.DeviceTensor(q.shape, np.float16)
+    dk, dv, ws = kc.dequantize(np.float16), vc.dequantize(np.float16), tract_amd.Workspace(B, Hq, n, D)
+    call("trocm_sdpa", dq.ptr, dk.ptr, dv.ptr, None, out.ptr, tract_amd.F16, B, Hq, Hkv, n, n, D, (C.c_int64 * 3)(Hkv * n * D, n * D, D), 1, 1,
+         C.c_float(float("nan")), 0, ws.ptr, ws.nbytes, None)
+    np.testing.assert_array_equal(got, out.to_numpy())

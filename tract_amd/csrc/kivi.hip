@@ -879,6 +879,182 @@ __global__ void __launch_bounds__(256) kivi_dequant_vec_kernel(KiviView a, DstT 
     }
 }
 
+// The first prompt of QuantizedKvSdpa in one launch (head_dim 128, u8 codes, f16 rows, empty stores): Keys into the running
+// per-channel store, Values into the per-token store, and both as the attention that follows reads them, dequantised.
+//
+// Keys: a workgroup owns 8 channels of a head row and all its tokens, C consecutive ones per thread, which stay in registers
+// from the first look to the codes.  The parameters at every thread's first token are prefix results, as in
+// kivi_run_scan_both_kernel (the same comparisons in the same order, so the same bits): a scan of the threads' minima, then one of
+// the widest ranges against them, each by DPP moves within a wave and 16 waves' totals through LDS.  The store is empty, so the walk
+// starts from lo = inf, scale = 1.  The 16 workgroups of a head row are BH apart: on one XCD, whose L2 joins their 16-byte pieces
+// of the rows.  Values: 16 lanes per token, as kivi_quant_tokens_vec_kernel.
+//
+// Bound by the chain of its phases, not by bytes (2 x 8 heads x 1500 tokens: 12 MB in, 18 MB out).  Before: three passes over the
+// Keys with a serial walk over the chunks between them, a pass over the Values and two to dequantise, six launches of 49 us.  A
+// session's prompt and 4 steps, before | now: 2 x 1500 tokens 195.5 | 160.6 us, 1000 110.5 | 82.0, 64 66.4 | 49.9, 4 x 700 136.7 | 112.6.
+struct KiviPrompt {
+    const __half *k, *v;
+    int n, BH;
+    uint8_t *k_codes, *v_codes;
+    int64_t k_cap, v_cap;          // rows between head rows of the code planes (and of the Values' parameters)
+    float *k_lo, *k_scale;         // [BH, 128], written
+    float *v_lo, *v_scale;
+    __half *k_deq, *v_deq;         // [BH, n, 128]
+};
+constexpr int kPromptMost = 8192;   // 16 waves of 8 tokens per lane
+
+// inclusive scans over a wave's lanes, earlier lanes first; on equal values (zeros of either sign) the earlier one
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float lanes_before(float x, float none) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, none), __builtin_bit_cast(int, x), CTRL, ROWS, 0xf, false));
+}
+template <typename Op>
+__device__ __forceinline__ float wave_scan(float x, float none, Op op) {   // op(earlier, later)
+    x = op(lanes_before<0x111, 0xf>(x, none), x);   // row_shr:1, 2, 4, 8
+    x = op(lanes_before<0x112, 0xf>(x, none), x);
+    x = op(lanes_before<0x114, 0xf>(x, none), x);
+    x = op(lanes_before<0x118, 0xf>(x, none), x);
+    x = op(lanes_before<0x142, 0xa>(x, none), x);   // row_bcast:15 into rows 1 and 3
+    return op(lanes_before<0x143, 0xc>(x, none), x);   // row_bcast:31 into rows 2 and 3
+}
+// What the threads before this one make of x (`none` for the first), and all of them, for 8 channels
+template <int W, typename Op>
+__device__ __forceinline__ void prompt_scan(float (&x)[8], float (&all)[8], float none, Op op, float (&totals)[W][8]) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const float in = wave_scan(x[e], none, op);
+        if (lane == 63) totals[w][e] = in;
+        x[e] = lanes_before<0x138, 0xf>(in, none);   // wave_shr:1
+        all[e] = none;
+    }
+    __syncthreads();
+    float before[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) before[e] = none;
+#pragma unroll 2
+    for (int i = 0; i < W; i++) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            if (i == w) before[e] = all[e];
+            all[e] = op(all[e], totals[i][e]);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) x[e] = op(before[e], x[e]);
+}
+
+__device__ __forceinline__ F8 affine_values8(uint32_t w0, uint32_t w1, const float (&lo)[8], const float (&scale)[8]) {
+    F8 x;
+#pragma unroll
+    for (int e = 0; e < 8; e++) x.v[e] = __fadd_rn(lo[e], __fmul_rn((float)(((e < 4 ? w0 : w1) >> (8 * (e % 4))) & 255u), scale[e]));
+    return x;
+}
+
+template <int W, int C>   // waves; tokens per thread
+__global__ void __launch_bounds__(64 * W) kivi_prompt_kernel(KiviPrompt p) {
+    __shared__ __attribute__((aligned(16))) float totals[2][W][8];
+    const int tid = threadIdx.x;
+    if ((int)blockIdx.x >= 16 * p.BH) {   // Values
+        const int id = blockIdx.x - 16 * p.BH, bh = id % p.BH, t = id / p.BH * (4 * W) + tid / 16, sub = tid % 16;
+        if (t >= p.n) return;   // whole groups of 16 lanes leave together
+        const int64_t at = ((int64_t)bh * p.n + t) * 128 + sub * 8, row = (int64_t)bh * p.v_cap + t;
+        const F8 x = ld8(p.v + at);
+        float lo = INFINITY, hi = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 8; e++) lo = fminf(lo, quiet(x.v[e])), hi = fmaxf(hi, quiet(x.v[e]));
+        group_min_max<16>(lo, hi);
+        const float scale = affine_scale(lo, hi, 255.0f), inv = affine_inv(scale);
+        uint32_t w0, w1;
+        affine_words8_u8(x.v, lo, scale, inv, w0, w1);
+        *reinterpret_cast<uint2 *>(p.v_codes + row * 128 + sub * 8) = make_uint2(w0, w1);
+        const float los[8] = {lo, lo, lo, lo, lo, lo, lo, lo}, scales[8] = {scale, scale, scale, scale, scale, scale, scale, scale};
+        st8(p.v_deq + at, affine_values8(w0, w1, los, scales));
+        if (sub == 0) p.v_lo[row] = lo, p.v_scale[row] = scale;
+        return;
+    }
+    const int bh = blockIdx.x % p.BH, ch = blockIdx.x / p.BH * 8, t0 = tid * C;
+    const __half *src = p.k + (int64_t)bh * p.n * 128 + ch;
+    uint4 raw[C];
+#pragma unroll
+    for (int u = 0; u < C; u++) raw[u] = ld8raw(src + (int64_t)min(t0 + u, p.n - 1) * 128);
+    float lo[8], most[8], widest[8], lo_all[8], widest_all[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) lo[e] = INFINITY, most[e] = -INFINITY, widest[e] = 0.0f;
+#pragma unroll
+    for (int u = 0; u < C; u++)
+        if (t0 + u < p.n) {
+            const F8 x = cvt8(raw[u]);
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float val = x.v[e];
+                lo[e] = val < lo[e] ? val : lo[e];
+                most[e] = val > most[e] ? val : most[e];
+                const float range = __fsub_rn(val, lo[e]);
+                widest[e] = range > widest[e] ? range : widest[e];   // (a NaN range is never wider)
+            }
+        }
+    prompt_scan<W>(lo, lo_all, INFINITY, [](float a, float b) { return b < a ? b : a; }, totals[0]);
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const float range = __fsub_rn(most[e], lo[e]);   // the thread's largest value against the incoming lo
+        widest[e] = range > widest[e] ? range : widest[e];
+    }
+    prompt_scan<W>(widest, widest_all, 0.0f, [](float a, float b) { return b > a ? b : a; }, totals[1]);
+    auto scale_of = [](float w) {   // the largest quotient is the quotient of the widest range
+        const float ns = w > 0.0f ? __fdiv_rn(w, 255.0f) : 0.0f;
+        return ns > 1.0f ? ns : 1.0f;
+    };
+    // the codes, token by token from the parameters before the thread's first (kivi_run_chunk_vec_kernel)
+    float scale[8], inv[8];
+    bool inv_usable = true;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        scale[e] = scale_of(widest[e]);
+        widest[e] = scale[e] * 254.9f;
+        inv[e] = affine_inv(scale[e]);
+        inv_usable = inv_usable && inv[e] != 0.0f;
+    }
+    uint32_t w0[C], w1[C];
+#pragma unroll
+    for (int u = 0; u < C; u++)
+        if (t0 + u < p.n) {
+            const F8 x = cvt8(raw[u]);
+            bool wider = false;
+            float range[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                lo[e] = x.v[e] < lo[e] ? x.v[e] : lo[e];
+                range[e] = __fsub_rn(x.v[e], lo[e]);
+                wider = wider || range[e] > widest[e];
+            }
+            if (__builtin_amdgcn_ballot_w64(wider) != 0) {
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    if (range[e] > widest[e]) {
+                        widest[e] = range[e];
+                        const float ns = __fdiv_rn(range[e], 255.0f);
+                        if (ns > scale[e]) scale[e] = ns, inv[e] = affine_inv(ns);
+                    }
+                inv_usable = true;
+#pragma unroll
+                for (int e = 0; e < 8; e++) inv_usable = inv_usable && inv[e] != 0.0f;
+            }
+            affine_words8_u8<true>(x.v, lo, scale, inv, w0[u], w1[u], inv_usable);
+        }
+#pragma unroll
+    for (int e = 0; e < 8; e++) scale[e] = scale_of(widest_all[e]);
+#pragma unroll
+    for (int u = 0; u < C; u++)
+        if (t0 + u < p.n) {
+            *reinterpret_cast<uint2 *>(p.k_codes + ((int64_t)bh * p.k_cap + t0 + u) * 128 + ch) = make_uint2(w0[u], w1[u]);
+            st8(p.k_deq + ((int64_t)bh * p.n + t0 + u) * 128 + ch, affine_values8(w0[u], w1[u], lo_all, scale));
+        }
+    if (tid == 0)
+#pragma unroll
+        for (int e = 0; e < 8; e++) p.k_lo[bh * 128 + ch + e] = lo_all[e], p.k_scale[bh * 128 + ch + e] = scale[e];
+}
+
 __global__ void kivi_fill_running_kernel(float *lo, float *scale, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
@@ -1053,8 +1229,8 @@ static int kivi_vec_chunk(int64_t rem) {
 }
 
 // Everything an append of S tokens may have to allocate, before anything is launched or counted: a call that fails here
-// has changed nothing and can be repeated.
-static int kivi_prepare(trocm_kivi_cache *c, int64_t S, hipStream_t s) {
+// has changed nothing and can be repeated.  passes: the Keys' chunk results among it.
+static int kivi_prepare(trocm_kivi_cache *c, int64_t S, hipStream_t s, bool passes = true) {
     if (kivi_alloc_fixed(c, s)) return 1;
     const int64_t ns = c->sink_tokens - c->n_sink < S ? c->sink_tokens - c->n_sink : S;
     const int64_t rem = S - (ns > 0 ? ns : 0);
@@ -1062,7 +1238,7 @@ static int kivi_prepare(trocm_kivi_cache *c, int64_t S, hipStream_t s) {
     int64_t rows = c->n_rows + rem;
     if (c->layout == TROCM_KIVI_BLOCK_CHANNEL) rows = c->n_rows + (c->n_res + rem) / kKeyBlock * kKeyBlock;
     if (rows > c->n_rows && kivi_ensure_rows(c, rows, s)) return 1;
-    if (kivi_prompt_scan(c, rem)) {
+    if (passes && kivi_prompt_scan(c, rem)) {
         const size_t need = (size_t)c->BH * ((rem + kivi_vec_chunk(rem) - 1) / kivi_vec_chunk(rem)) * c->D * 3 * sizeof(float);   // (three results per chunk and channel on the 128-bit path)
         if (kivi_grow_buffer((void **)&c->scan, &c->scan_bytes, need, s, "the chunk results of a prompt")) return 1;
     }
@@ -1222,6 +1398,26 @@ static int kivi_dequantize(const trocm_kivi_cache *c, void *dst, int dst_dtype, 
         if (c->bits == 8) kivi_dequant_kernel<__half, 8><<<grid, 256, 0, s>>>(a, (__half *)dst);
         else kivi_dequant_kernel<__half, 4><<<grid, 256, 0, s>>>(a, (__half *)dst);
     }
+    TROCM_HIP(hipGetLastError());
+    return 0;
+}
+
+// As few waves as hold the prompt, C tokens per lane: their totals are walked one after the other, and a workgroup of many waves has a
+// compute unit to itself (a session's prompt and 4 steps, us, 4 | 8 | 16 waves: 300 tokens 64.6 | 65.8 | 70.0, 1000 82.0 | 82.3 | 87.3,
+// 4 x 700 112.6 | 117.2 | 127.9; 2 x 1500 161.4 | 160.5 | 164.8).
+static int launch_kivi_prompt(const KiviPrompt &p, hipStream_t s) {
+    const int n = p.n, W = n <= 1024 ? 4 : n <= 4096 ? 8 : 16;
+    const dim3 grid((unsigned)(p.BH * (16 + (n + 4 * W - 1) / (4 * W)))), block(64 * W);
+    if (n <= 256) kivi_prompt_kernel<4, 1><<<grid, block, 0, s>>>(p);
+    else if (n <= 512) kivi_prompt_kernel<4, 2><<<grid, block, 0, s>>>(p);
+    else if (n <= 768) kivi_prompt_kernel<4, 3><<<grid, block, 0, s>>>(p);
+    else if (n <= 1024) kivi_prompt_kernel<4, 4><<<grid, block, 0, s>>>(p);
+    else if (n <= 1536) kivi_prompt_kernel<8, 3><<<grid, block, 0, s>>>(p);
+    else if (n <= 2048) kivi_prompt_kernel<8, 4><<<grid, block, 0, s>>>(p);
+    else if (n <= 3072) kivi_prompt_kernel<8, 6><<<grid, block, 0, s>>>(p);
+    else if (n <= 4096) kivi_prompt_kernel<8, 8><<<grid, block, 0, s>>>(p);
+    else if (n <= 6144) kivi_prompt_kernel<16, 6><<<grid, block, 0, s>>>(p);
+    else kivi_prompt_kernel<16, 8><<<grid, block, 0, s>>>(p);
     TROCM_HIP(hipGetLastError());
     return 0;
 }
@@ -1392,6 +1588,12 @@ static bool kivi_fused_step(int dtype, int64_t n_new, const trocm_kivi_cache *k,
            k->n_res == 0 && v->n_res == 0 && k->n_rows == k->len && v->n_rows == v->len;
 }
 
+// A first prompt that kivi_prompt_kernel takes.
+static bool kivi_first_prompt(const void *k_new, const void *v_new, int dtype, int64_t n_new, const trocm_kivi_cache *k, const trocm_kivi_cache *v) {
+    return dtype == TROCM_F16 && n_new > 1 && n_new <= kPromptMost && k->D == 128 && k->len == 0 && k->BH > 0 && k->BH < (1 << 16) &&
+           k->layout == TROCM_KIVI_RUNNING_CHANNEL && v->layout == TROCM_KIVI_PER_TOKEN && k->bits == 8 && v->bits == 8 && k->sink_tokens == 0 &&
+           v->sink_tokens == 0 && !((uintptr_t)k_new & 15) && !((uintptr_t)v_new & 15);
+}
 int trocm_quantized_kv_sdpa_eval(const void *q, const void *k_new, const void *v_new, int dtype, int64_t q_heads,
                                  int64_t n_new, trocm_kivi_cache *k_cache, trocm_kivi_cache *v_cache, void *out,
                                  float scale, void *workspace, size_t workspace_bytes, void *stream) {
@@ -1413,9 +1615,9 @@ int trocm_quantized_kv_sdpa_eval(const void *q, const void *k_new, const void *v
     if (resolve_stream(stream, &s)) return 1;
     // Every allocation of the step, for both stores, before either is touched: a call that fails for want of memory
     // leaves K and V as they were (same length, same counts) and can be repeated.
-    const bool fused_attention = kivi_fused_step(dtype, n_new, k_cache, v_cache);
+    const bool fused_attention = kivi_fused_step(dtype, n_new, k_cache, v_cache), first_prompt = kivi_first_prompt(k_new, v_new, dtype, n_new, k_cache, v_cache);
     for (trocm_kivi_cache *c : {k_cache, v_cache})
-        if (kivi_prepare(c, n_new, s)) return 1;
+        if (kivi_prepare(c, n_new, s, !first_prompt)) return 1;
     if (!(fused_attention && workspace)) {
         const size_t need = (size_t)k_cache->BH * (k_cache->len + n_new) * k_cache->D * elem_bytes(dtype);
         for (trocm_kivi_cache *c : {k_cache, v_cache})
@@ -1482,10 +1684,18 @@ int trocm_quantized_kv_sdpa_eval(const void *q, const void *k_new, const void *v
         for (trocm_kivi_cache *c : {k_cache, v_cache})
             if (kivi_grow_buffer(&c->deq, &c->deq_bytes, need, s, "the dequantised copy of a quantised store")) return 1;
     }
-    if (!pushed && push()) return 1;
+    if (first_prompt) {
+        const RunSets sets = kivi_run_sets(k_cache, n_new);
+        const KiviPrompt prompt{(const __half *)k_new, (const __half *)v_new, (int)n_new, (int)k_cache->BH, k_cache->codes, v_cache->codes, k_cache->cap_rows,
+                                          v_cache->cap_rows, sets.lo_next, sets.scale_next, v_cache->lo, v_cache->scale, (__half *)k_cache->deq, (__half *)v_cache->deq};
+        if (launch_kivi_prompt(prompt, s)) return 1;
+        for (trocm_kivi_cache *c : {k_cache, v_cache}) c->n_rows += n_new, c->len += n_new, kivi_select_set(c);
+    } else {
+        if (!pushed && push()) return 1;
+        for (trocm_kivi_cache *c : {k_cache, v_cache})
+            if (kivi_dequantize(c, c->deq, dtype, s, false)) return 1;
+    }
     const int64_t T = k_cache->len, D = k_cache->D;
-    for (trocm_kivi_cache *c : {k_cache, v_cache})
-        if (kivi_dequantize(c, c->deq, dtype, s, false)) return 1;
     const int64_t strides[3] = {k_cache->H * T * D, T * D, D};
     // kv_quant.rs:326-327: FlashSdpaOp { causal: false, scale }
     return trocm_sdpa(q, k_cache->deq, v_cache->deq, nullptr, out, dtype, k_cache->B, q_heads, k_cache->H, n_new, T, D, strides, 1, 1,
