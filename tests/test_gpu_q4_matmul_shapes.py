@@ -50,3 +50,18 @@ for n, k, m in [(4096, 1024, 49), (2816, 1024, 131), (4096, 4096, 260)]:   # cho
     name, value = given.split("=")
     p = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, **{"TROCM_Q4_MATMUL_" + name: value}), capture_output=True, text=True, timeout=100)
     assert p.returncode == 0, p.stderr[-2000:]
+
+
+# the sets of waves walk 1 to 7 tiles of k each (fewer than, as many as and more than are on their way at a time, and none behind the
+# last): the shapes of 32, 64 and 64 rows in 8 or 4, 4 and 2 sets
+@pytest.mark.parametrize("n,m", [(2816, 49), (2816, 131), (2832, 299), (5136, 388)])
+@pytest.mark.parametrize("tiles", [4, 8, 12, 16, 20, 24, 28])
+def test_short_walks_of_k(rt, n, m, tiles):
+    rng = np.random.default_rng(n + tiles)
+    k = 128 * tiles
+    blocks = orc.quant(orc.FMT_Q4_0, (0.03 * rng.standard_normal((n, k), dtype=np.float32)).astype(np.float32))
+    act = rng.standard_normal((1, m, k), dtype=np.float32).astype(np.float16)
+    got = ta.GgmlGemm().eval(ta.DeviceTensor.from_numpy(act), ta.Q40Weights(blocks, 1, n, k)).to_numpy().astype(np.float64)[0]
+    want = act[0].astype(np.float64) @ orc.dequant(orc.FMT_Q4_0, blocks, np.float32).reshape(n, k).astype(np.float64).T
+    assert np.linalg.norm(got - want) <= 2.0 ** -11 * np.linalg.norm(want)   # (as above)
+    assert np.abs(got - want).max() <= 2.0 ** -11 * (6 * np.sqrt(k) * 0.03 + np.abs(want).max())

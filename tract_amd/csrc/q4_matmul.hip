@@ -195,8 +195,10 @@ constexpr int AROW = HK + 8;                 // halves per activation row in LDS
 // launches with so few workgroups that each compute unit would otherwise hold four waves that walk all of k alone.
 // NW: waves per set (4; 2 or 1 -- 64 or 32 rows of the weights per workgroup -- when even the smallest tile above leaves
 // compute units without a workgroup: the time of such a launch is the work of one compute unit).
-template <int BM, int NI, int KS, int NW>
-__global__ __launch_bounds__(64 * NW * KS, NW * KS >= 8 ? 1 : 2) void q4_0_tiled_matmul_kernel(MatMulDev p) {
+// SHORT: a set has one or two tiles, all asked for at the start (the general loop's code, and its loads past the end, cost 0.05 to 0.1 us
+// of 4 there).
+template <int BM, int NI, int KS, int NW, bool SHORT = false>
+__global__ __launch_bounds__(64 * NW * KS, BM == 32 && NW * KS >= 8 && NI == 1 ? 4 : NW * KS >= 8 ? 1 : 2) void q4_0_tiled_matmul_kernel(MatMulDev p) {
     constexpr int MS = BM / 32;                  // 32-row subtiles of m
     constexpr int TS = 64 * NW;                  // threads of a set
     constexpr int TN = 32 * NI * NW;             // rows of the weights per workgroup
@@ -204,7 +206,7 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS >= 8 ? 1 : 2) void q4_0_tiled
     // for launches in which a workgroup walks k alone, and a half tile's arithmetic is shorter than a trip to the L2.
     constexpr int PA = BM == 128 ? 1 : 2;
     // Tiles of the weights on their way from HBM, likewise: one tile's arithmetic of a small shape is about half of that trip.
-    constexpr int PW = BM == 128 ? 1 : 3;
+    constexpr int PW = SHORT ? 2 : BM == 128 ? 1 : (BM == 64 && NW == 4) || KS == 8 ? 2 : 3;
     constexpr int AP = BM * 8 / TS;              // 16-byte activation pieces per thread and half tile
     constexpr int RPP = TS / 8;                  // activation rows that the set's threads stage in one pass
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];   // [KS][2][BM AROW] halves; then the sums
@@ -245,17 +247,24 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS >= 8 ? 1 : 2) void q4_0_tiled
 
     struct Weights { u32x4 c[NI][2]; u32x2 s[NI]; };   // a tile's slots g = hb, 2 + hb and scales, for each 32 rows of the wave
     u32x4 apre[PA][AP];
+    // STEADY: no load of the loop is behind a branch, or the waits for older ones would be waits for all of them; past
+    // the set's share nothing is read (an offset beyond the buffer), but the load is issued, and the last tile,
+    // which fetches and stages nothing, is written out on its own.  us before | now: 100 rows of 4096 x 14336 31.0 | 28.1, 150 41.7 |
+    // 37.1, 512 72.7 | 70.5; 20 of 14336 x 4096 13.0 | 11.6; 400 of 2048 x 8192 26.5 | 24.6.  Not with 128 rows, which fetch one half tile
+    // ahead only and wait for it in any case (1000 rows of 14336 x 4096 114.3 | 116.8).
+    constexpr bool STEADY = BM != 128;
+    constexpr uint32_t kNowhere = 0xFFFFFC00u;
     auto prefetch_w = [&](Weights &wt, int t) {
 #pragma unroll
         for (int i = 0; i < NI; i++) {
-            wt.c[i][0] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_slot[i], (tile0 + t) * 1152, 0);
-            wt.c[i][1] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_slot[i] + 512, (tile0 + t) * 1152, 0);
-            wt.s[i] = __builtin_amdgcn_raw_buffer_load_b64(w_rsrc, w_scale[i], (tile0 + t) * 1152, 0);
+            wt.c[i][0] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, t < Tg || !STEADY ? w_slot[i] : kNowhere, (tile0 + t) * 1152, 0);
+            wt.c[i][1] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, (t < Tg || !STEADY ? w_slot[i] : kNowhere) + 512, (tile0 + t) * 1152, 0);
+            wt.s[i] = __builtin_amdgcn_raw_buffer_load_b64(w_rsrc, t < Tg || !STEADY ? w_scale[i] : kNowhere, (tile0 + t) * 1152, 0);
         }
     };
     auto prefetch_a = [&](int set, int it) {   // half tile `it` of this set's share of k
 #pragma unroll
-        for (int j = 0; j < AP; j++) apre[set][j] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_src[j], (2 * tile0 + it) * HK * 2, 0);
+        for (int j = 0; j < AP; j++) apre[set][j] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, it < 2 * Tg || !STEADY ? a_src[j] : kNowhere, (2 * tile0 + it) * HK * 2, 0);
     };
     auto stage_a = [&](int set, int buf) {
 #pragma unroll
@@ -280,18 +289,21 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS >= 8 ? 1 : 2) void q4_0_tiled
         if (u < Tg) prefetch_w(ring[u], u);
     prefetch_a(0, 0);
     stage_a(0, 0);
-    if (PA == 2 && Tg * 2 > 1) prefetch_a(1, 1);
+    if (PA == 2) prefetch_a(1, 1);
     const int a_frag = l32 * AROW + 8 * hb;
-    auto tile = [&](int t, const Weights &wt, Weights &refill) {
-        if (t + PW < Tg) prefetch_w(refill, t + PW);
+    // `last` (STEADY): the set's last tile
+    auto tile = [&](auto last, int t, const Weights &wt, Weights &refill) {
+        constexpr bool LAST = decltype(last)::value;
+        if (STEADY ? !LAST && !SHORT : t + PW < Tg) prefetch_w(refill, t + PW);
 #pragma unroll
         for (int hh = 0; hh < 2; hh++) {
             // Half tile it = 2 t + hh of the activations is in buffer hh; every wave is done with the other buffer.  Half
             // it + PA is requested now (into the registers that held half it, PA = 2, or it + 1 just staged), and half
             // it + 1 is written into the other buffer after this half's arithmetic.
             __syncthreads();
-            const bool more = 2 * t + hh + 1 < 2 * Tg;
-            if (2 * t + hh + PA < 2 * Tg) prefetch_a(PA == 2 ? hh : 0, 2 * t + hh + PA);
+            if (STEADY ? !LAST || hh + PA < 2 : 2 * t + hh + PA < 2 * Tg) prefetch_a(PA == 2 ? hh : 0, 2 * t + hh + PA);
+            // asked for here, not where it is used (but in sets of two waves, 64 rows: 40 rows of 4096 x 4096 8.5 us with this, 8.2 without)
+            if constexpr (STEADY && (BM != 64 || NI * NW != 2)) __builtin_amdgcn_sched_barrier(0);
             const _Float16 *at = &lds_a[hh * BM * AROW + a_frag];
             half8_t bf[2][MS];   // the activation fragments of a step are read during the step before
 #pragma unroll
@@ -315,16 +327,39 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS >= 8 ? 1 : 2) void q4_0_tiled
                     for (int mm = 0; mm < MS; mm++) acc[i][mm] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf[step & 1][mm], acc[i][mm], 0, 0, 0);
                 }
             }
-            if (more) stage_a(PA == 2 ? hh ^ 1 : 0, hh ^ 1);
+            if (STEADY ? !LAST || hh == 0 : 2 * t + hh + 1 < 2 * Tg) stage_a(PA == 2 ? hh ^ 1 : 0, hh ^ 1);
         }
     };
-    for (int t0 = 0; t0 < Tg; t0 += PW) {
+    if constexpr (SHORT) {
+        if (Tg > 1) {
+            tile(std::false_type{}, 0, ring[0], ring[0]);
+            tile(std::true_type{}, 1, ring[1], ring[1]);
+        } else {
+            tile(std::true_type{}, 0, ring[0], ring[0]);
+        }
+    } else if constexpr (!STEADY) {
+        for (int t = 0; t < Tg; t++) {   // (PW = 1)
+            const Weights cur = ring[0];
+            tile(std::false_type{}, t, cur, ring[0]);
+        }
+    } else {
+        int t0 = 0;
+        for (; t0 + PW < Tg; t0 += PW) {
 #pragma unroll
-        for (int u = 0; u < PW; u++)
-            if (t0 + u < Tg) {
+            for (int u = 0; u < PW; u++) {
                 const Weights cur = ring[u];
-                tile(t0 + u, cur, ring[u]);
+                tile(std::false_type{}, t0 + u, cur, ring[u]);
             }
+        }
+#pragma unroll
+        for (int u = 0; u < PW; u++) {
+            const Weights cur = ring[u];
+            if (t0 + u + 1 < Tg) {
+                tile(std::false_type{}, t0 + u, cur, ring[u]);
+            } else if (t0 + u + 1 == Tg) {
+                tile(std::true_type{}, t0 + u, cur, ring[u]);
+            }
+        }
     }
 
     if constexpr (KS > 1) {
@@ -489,8 +524,11 @@ int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, i
         };
         auto launch_small = [&](auto bm_tag, auto nw_tag) -> int {   // 64 or 32 activation rows, 32 rows of the weights per wave
             constexpr int BMc = decltype(bm_tag)::value, NWc = decltype(nw_tag)::value;
+            const bool few = k / TK <= 2 * ks;   // tiles of a set
             if constexpr (NWc == 1)
-                if (ks == 8) return launch(q4_0_tiled_matmul_kernel<BMc, 1, 8, 1>);
+                if (ks == 8) return few ? launch(q4_0_tiled_matmul_kernel<BMc, 1, 8, 1, true>) : launch(q4_0_tiled_matmul_kernel<BMc, 1, 8, 1>);
+            if constexpr (NWc == 2)
+                if (ks == 4 && few) return launch(q4_0_tiled_matmul_kernel<BMc, 1, 4, 2, true>);
             return ks == 4 ? launch(q4_0_tiled_matmul_kernel<BMc, 1, 4, NWc>) : ks == 2 ? launch(q4_0_tiled_matmul_kernel<BMc, 1, 2, NWc>)
                                                                                         : launch(q4_0_tiled_matmul_kernel<BMc, 1, 1, NWc>);
         };
