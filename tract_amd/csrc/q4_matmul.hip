@@ -253,7 +253,7 @@ __global__ __launch_bounds__(64 * NW * KS, BM == 32 && NW * KS >= 8 && NI == 1 ?
     // 37.1, 512 72.7 | 70.5; 20 of 14336 x 4096 13.0 | 11.6; 400 of 2048 x 8192 26.5 | 24.6.  Not with 128 rows, which fetch one half tile
     // ahead only and wait for it in any case (1000 rows of 14336 x 4096 114.3 | 116.8).
     constexpr bool STEADY = BM != 128;
-    constexpr uint32_t kNowhere = 0xFFFFFC00u;
+    constexpr uint32_t kNowhere = 0xFFFFFC00u;   // (no buffer is longer: the launcher)
     auto prefetch_w = [&](Weights &wt, int t) {
 #pragma unroll
         for (int i = 0; i < NI; i++) {
@@ -461,7 +461,7 @@ int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, i
     p.n = (int)n, p.k = (int)k, p.m = (int)m, p.ratio = (int)(act_batch / w_batch);
     if (tiled) {
         // 32-bit byte offsets inside one weight matrix and one batch of activations (rows up to 128 past m are addressed)
-        if (n % 16 || k % TK || (n / 16) * (k / TK) * 1152 >= (1ll << 32) || (m + 128) * k >= (1ll << 30)) return 2;
+        if (n % 16 || k % TK || (n / 16) * (k / TK) * 1152 > 0xFFFFFC00ll || (m + 128) * k >= (1ll << 30)) return 2;
         // k a multiple of 512: the shape with the least expected time.  Other k (which the sets of waves of most shapes could not
         // share), or a shape that is partly given from outside: the largest tile of C^T per workgroup -- 256 (n) x 128 (m), 256 x 64,
         // 128 x 64 -- that still gives three quarters of the compute units a workgroup (128 x 128 never has more workgroups than
