@@ -65,3 +65,22 @@ def test_short_walks_of_k(rt, n, m, tiles):
     want = act[0].astype(np.float64) @ orc.dequant(orc.FMT_Q4_0, blocks, np.float32).reshape(n, k).astype(np.float64).T
     assert np.linalg.norm(got - want) <= 2.0 ** -11 * np.linalg.norm(want)   # (as above)
     assert np.abs(got - want).max() <= 2.0 ** -11 * (6 * np.sqrt(k) * 0.03 + np.abs(want).max())
+
+
+# f32 rows: 16 x 32, 16 x 48, 16 x 64, 32 x 64, 32 x 96 and 32 x 128 (activation rows x weight rows), each as planes and as tiles, with
+# remainders of both; one row's values are so large that its blocks are done in f32, for every part of the workgroup's weight rows
+@pytest.mark.parametrize("m,n,k", [(16, 4130, 160), (16, 4112, 256), (64, 2817, 1056), (64, 2064, 1152), (33, 4130, 160), (33, 4112, 384), (150, 2063, 1024),
+                                   (150, 2064, 1152), (150, 4100, 1056), (150, 4112, 1152), (200, 4130, 160), (200, 4112, 256)])
+def test_shapes_of_the_f32_product(rt, m, n, k):
+    rng = np.random.default_rng(n + k + m)
+    blocks = orc.quant(orc.FMT_Q4_0, (0.05 * rng.standard_normal((n, k), dtype=np.float32)).astype(np.float32))
+    act = rng.standard_normal((1, m, k), dtype=np.float32)
+    act[0, m // 2] *= np.float32(1e36)
+    got = ta.GgmlGemm().eval(ta.DeviceTensor.from_numpy(act), ta.Q40Weights(blocks, 1, n, k)).to_numpy().astype(np.float64)[0]
+    wd = orc.dequant(orc.FMT_Q4_0, blocks, np.float32).reshape(n, k).astype(np.float64)
+    want, size = act[0].astype(np.float64) @ wd.T, np.abs(act[0].astype(np.float64)) @ np.abs(wd).T
+    # as in test_gpu_matvec.py: products are exact and at most k / 32 / 8 + 15 additions stand one after the other, each rounding by 2^-24 of a
+    # partial sum that is no larger than the sum of the magnitudes; in f32 products round too and a block's are added one by one, k / 8 per wave
+    steps = np.full((m, 1), k / 256 + 15)
+    steps[m // 2 // 32 * 32 : m // 2 // 32 * 32 + 32] = k / 4 + 15   # (the rows that share blocks with the large one)
+    assert np.all(np.abs(got - want) <= size * steps * 2.0 ** -24)
