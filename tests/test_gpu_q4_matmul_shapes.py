@@ -84,3 +84,16 @@ def test_shapes_of_the_f32_product(rt, m, n, k):
     steps = np.full((m, 1), k / 256 + 15)
     steps[m // 2 // 32 * 32 : m // 2 // 32 * 32 + 32] = k / 4 + 15   # (the rows that share blocks with the large one)
     assert np.all(np.abs(got - want) <= size * steps * 2.0 ** -24)
+
+
+# f16 rows with k shared among waves: 32 x 16, 48 x 32 and 64 x 32 (planes), and 6 to 8 rows of tiles
+@pytest.mark.parametrize("m,n,k", [(90, 1010, 1056), (290, 1010, 160), (290, 1001, 2080), (450, 1010, 1056), (470, 1001, 96), (6, 4112, 1152), (7, 5136, 384), (8, 272, 2176)])
+def test_shapes_with_k_shared_among_waves(rt, m, n, k):
+    rng = np.random.default_rng(n + k + m)
+    blocks = orc.quant(orc.FMT_Q4_0, (0.05 * rng.standard_normal((n, k), dtype=np.float32)).astype(np.float32))
+    act = rng.standard_normal((1, m, k), dtype=np.float32).astype(np.float16)
+    got = ta.GgmlGemm().eval(ta.DeviceTensor.from_numpy(act), ta.Q40Weights(blocks, 1, n, k)).to_numpy().astype(np.float64)[0]
+    wd = orc.dequant(orc.FMT_Q4_0, blocks, np.float32).reshape(n, k).astype(np.float64)   # (not rounded to f16)
+    want, size = act[0].astype(np.float64) @ wd.T, np.abs(act[0].astype(np.float64)) @ np.abs(wd).T
+    # products are exact; at most k / 32 / 8 + 10 f32 additions stand one after the other, and the result is rounded to f16
+    assert np.all(np.abs(got - want) <= size * (k / 256 + 11) * 2.0 ** -24 + np.abs(want) * 2.0 ** -11 + 2.0 ** -25)

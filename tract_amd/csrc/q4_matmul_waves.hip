@@ -16,7 +16,7 @@
 // the end.  A launch is bound by a wave's own chain (first loads, one load latency per unit, the sums) while there is no
 // more than a workgroup per compute unit, and by the conversions (11 operations per 8 codes, one per result and block) and
 // the activations' way through the L2 beyond that, where q4_matmul.hip, which shares both in LDS, is the better one.
-// Measured (us, before | now): 476 rows of 1000 x 2080 (planes, in groups of 8 rows) 444.6 | 20.2, 64 rows 51.2 | 7.9, 9 rows
+// Measured (us, before | now): 476 rows of 1000 x 2080 (planes, in groups of 8 rows) 444.6 | 15.4, 64 rows 51.2 | 7.5, 9 rows
 // 10.3 | 7.2; tiles, q4_matmul.hip: 64 rows of 1024 x 4096 12.3 | 7.8, 128 rows 12.9 | 8.8; q4_tiled.hip: 9 rows of
 // 4096 x 14336 18.4 | 13.6, 16 rows 23.1 | 18.3.
 #include <hip/hip_runtime.h>
@@ -223,9 +223,13 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_waves_kernel(MatMulWav
     }
 }
 
-struct Shape { int ms, ni, us; };
-// us: a round of workgroups, one per compute unit, at 4096 features when there are several rounds
-constexpr Shape kShapes[] = {{1, 1, 5}, {1, 2, 6}, {2, 2, 10}, {2, 4, 13}, {4, 4, 20}};
+struct Shape { int ms, ni; float tiled, first, later; };
+// us of a round of workgroups, one per compute unit: tiles at 4096 features when there are several rounds; planes at 2080 features, the first
+// and later ones.  32 x 16, 48 x 32 and 64 x 32 are for planes, whose codes come in words of 4 bytes, so that a weight row costs more there:
+// 100 rows of 1000 x 2080 10.9 (16 x 32) -> 9.3 (32 x 16), 300 19.7 (32 x 64) -> 14.5 (48 x 32), 500 19.9 -> 15.4 (64 x 32).
+constexpr float kNever = 1e9f;
+constexpr Shape kShapes[] = {{1, 1, 5.0f, 7.3f, 5.0f},    {1, 2, 6.0f, 10.6f, 8.5f},    {2, 2, 10.0f, 12.4f, 10.5f},  {2, 4, 13.0f, kNever, kNever},
+                             {4, 4, 20.0f, 23.0f, 20.0f}, {2, 1, kNever, 9.2f, 6.7f},   {3, 2, kNever, 14.5f, 12.5f}, {4, 2, kNever, 15.2f, 14.0f}};
 int64_t workgroups(const Shape &c, int64_t n, int64_t m, int64_t act_batch) {
     return (n + 16 * c.ni - 1) / (16 * c.ni) * ((m + 16 * c.ms - 1) / (16 * c.ms)) * act_batch;
 }
@@ -248,34 +252,43 @@ int launch_q4_0_matmul_waves(const void *codes, const void *scales, int64_t w_ba
     p.codes = (const uint8_t *)codes, p.scales = (const uint16_t *)scales;
     p.act = (const _Float16 *)act, p.out = (_Float16 *)out;
     p.n = (int)n, p.k = (int)k, p.m = (int)m, p.ratio = (int)(act_batch / w_batch);
-    // The shape that takes the least time: rounds of workgroups times the time of a round (1000 x 2080: 64 rows 16 x 16 7.9 us,
-    // 16 x 32 11.2; 200 rows 32 x 32 13.1, 16 x 32 19.7; 476 rows 32 x 64 20.2, 32 x 32 23.7, 64 x 64 23.5).  Below 1024 features,
-    // where some waves have no unit (before | here: 9 rows of 4096 x 512 4.9 | 4.4, 128 rows 4.6 | 4.5, 16 rows of 320 x 992 8.3 | 5.0).
+    // The shape that takes the least time (1000 x 2080: 64 rows 16 x 16 7.9 us, 16 x 32 11.2; 200 rows 32 x 32 13.1, 16 x 32 19.7).  Below
+    // 1024 features, where some waves have no unit (before | here: 9 rows of 4096 x 512 4.9 | 4.4, 128 rows 4.6 | 4.5, 16 rows of 320 x 992
+    // 8.3 | 5.0).
     int best = 0;
-    int64_t best_cost = 0;
-    for (int c = 0; c < 5; c++) {
-        const int64_t cost = (workgroups(kShapes[c], n, m, act_batch) + num_compute_units() - 1) / num_compute_units() * kShapes[c].us;
-        if (c == 0 || cost < best_cost) best = c, best_cost = cost;
+    float best_us = 0.0f;
+    for (int c = 0; c < 8; c++) {
+        const Shape &x = kShapes[c];
+        const float rounds = (float)((workgroups(x, n, m, act_batch) + num_compute_units() - 1) / num_compute_units());
+        const float us = tiled ? rounds * x.tiled : x.first + (rounds - 1.0f) * x.later;
+        if (c == 0 || us < best_us) best = c, best_us = us;
     }
     auto go = [&](auto ms, auto ni) -> int {
         constexpr int MS = decltype(ms)::value, NI = decltype(ni)::value, DB = MS < 4 ? 4 : 2;
         const dim3 grid((unsigned)((n + 16 * NI - 1) / (16 * NI)), (unsigned)((m + 16 * MS - 1) / (16 * MS)), (unsigned)act_batch);
         if (grid.y > 65535) return 2;
-        if (tiled) hipLaunchKernelGGL((q4_0_matmul_waves_kernel<MS, NI, DB, true>), grid, dim3(64 * kW), 0, s, p);
-        else hipLaunchKernelGGL((q4_0_matmul_waves_kernel<MS, NI, DB, false>), grid, dim3(64 * kW), 0, s, p);
+        constexpr bool TILES = !(NI == 1 && MS == 2) && !(NI == 2 && MS > 2), PLANES = !(MS == 2 && NI == 4);   // (the other's never chosen)
+        if constexpr (TILES)
+            if (tiled) hipLaunchKernelGGL((q4_0_matmul_waves_kernel<MS, NI, DB, true>), grid, dim3(64 * kW), 0, s, p);
+        if constexpr (PLANES)
+            if (!tiled) hipLaunchKernelGGL((q4_0_matmul_waves_kernel<MS, NI, DB, false>), grid, dim3(64 * kW), 0, s, p);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return fail("q4_0_matmul (shared k) launch failed: %s", hipGetErrorString(e));
         return 0;
     };
     typedef std::integral_constant<int, 1> I1;
     typedef std::integral_constant<int, 2> I2;
+    typedef std::integral_constant<int, 3> I3;
     typedef std::integral_constant<int, 4> I4;
     switch (best) {
         case 0: return go(I1(), I1());
         case 1: return go(I1(), I2());
         case 2: return go(I2(), I2());
         case 3: return go(I2(), I4());
-        default: return go(I4(), I4());
+        case 4: return go(I4(), I4());
+        case 5: return go(I2(), I1());
+        case 6: return go(I3(), I2());
+        default: return go(I4(), I2());
     }
 }
 

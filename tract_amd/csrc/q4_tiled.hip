@@ -537,9 +537,10 @@ int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int6
     if (n >= (1ll << 30) || k >= (1ll << 30) || act_batch > 65535) return fail("q4_0_matvec: shape too large");
     // (a row group's records are addressed through one buffer descriptor: 32-bit offsets)
     if ((k / 128) * kTile >= (1ll << 31)) return fail("q4_0_matvec: rows of %lld features are too long for the tiled layout", (long long)k);
-    // 9 f16 rows and more with few tiles (us, the kernel above | there: 5 rows of 4096 x 14336 12.2 | 12.5; 9 rows 18.4 | 13.6,
-    // 16 rows 23.1 | 18.3, of 4096 x 4096 8.3 | 8.0)
-    if (act_dtype == TROCM_F16 && m >= 9 && q4_0_matmul_waves_fits(n, m, act_batch)) {
+    // 6 f16 rows and more with few tiles (us, the kernel above | there: 5 rows of 4096 x 14336 11.5 | 11.9, of 1024 x 14336 10.9 | 11.4; 6 rows
+    // 14.4 | 12.2, 13.4 | 11.9, of 5120 x 5120 8.7 | 7.0, of 8192 x 8192 11.5 | 10.7, of 4096 x 4096 5.6 | 5.4; 8 rows of 4096 x 14336 15.3 |
+    // 12.7, of 1024 x 4096 5.4 | 5.5; 16 rows 23.1 | 18.3, of 4096 x 4096 8.3 | 8.0)
+    if (act_dtype == TROCM_F16 && m >= 6 && q4_0_matmul_waves_fits(n, m, act_batch)) {
         const int rc = launch_q4_0_matmul_waves(tiles, nullptr, w_batch, n, k, act, act_batch, m, out, s, 1);
         if (rc != 2) return rc;
     }
