@@ -70,6 +70,17 @@ struct RaggedItem {
 struct RaggedSeqSlots {
     int slot0, nsplit;
 };
+// The same plan as a kernel argument, for few sequences: no upload before the launch.  A sequence's items are consecutive.
+constexpr int kPlanSeqs = 64, kPlanItems = 640;
+struct RaggedPlan {
+    struct Seq {
+        const char *k, *v, *ks, *vs;
+        int cap, T;                  // token rows between kv heads, tokens
+        uint16_t first, nsplit;      // its items
+        uint16_t slot0, seq;
+    } seqs[kPlanSeqs];
+    uint32_t seq_of[kPlanItems / 4];   // a byte per item: its place in `seqs`
+};
 
 namespace {
 
@@ -412,7 +423,7 @@ int decode_mfma_group(int64_t g_real);   // 0: not taken by the MFMA formulation
 int launch_sdpa_decode_quant_mfma(DecodeDev &p, int kv_fmt, int64_t B, void *workspace, size_t workspace_bytes, hipStream_t s);
 bool decode_quant_appends_in_kernel(int64_t g_real, float scale);
 bool decode_quant_rotates_in_kernel(int64_t g_real);
-int launch_sdpa_decode_ragged_mfma(const DecodeDev &p, int kv_fmt, int gp, int64_t D, const RaggedItem *items, int n_items,
+int launch_sdpa_decode_ragged_mfma(const DecodeDev &p, int kv_fmt, int gp, int64_t D, const RaggedItem *items, const RaggedPlan &plan, int n_items,
                                    const RaggedSeqSlots *seqs, int n_seq, bool any_split, hipStream_t s);
 
 // Partials: at most kMaxSplitRows rows of (D + 2) floats per query head.
@@ -432,3 +443,4 @@ inline int fit_decode_splits(int nsplit, int64_t BH, int64_t G, int64_t D, const
 }
 
 }  // namespace trocm
+static_assert(sizeof(trocm::RaggedPlan) + sizeof(trocm::DecodeDev) + 8 <= 4096, "kernel arguments");

@@ -690,8 +690,60 @@ int ragged_per_sequence(const void *q, void *out, int q_dtype, int kv_fmt, int64
 
 }  // namespace
 
+namespace {
+// Tiles per item of a ragged launch on the matrix cores.  A workgroup takes groups of kWaves tiles one after the other, `step_bytes`
+// each; what it takes is modelled (us) as the larger of all groups at the rate of the memory (or of the arithmetic, for codes), the
+// longest item's chain of groups alone on its compute unit, and that chain where two share one, plus a third of the longest chain, which
+// some unit may end with; more than two per unit do not run at once, and each costs its prologue.  Tried are the smallest items that give up to one and up
+// to two workgroups per unit, and items for 4 and 8 per unit.  Fitted to 23 batches (3 to 64 sequences of 20 to 32768 tokens, f16, Q8_0
+// and Q4_0, 64 and 128 features) at up to 18 item sizes each: 3 % above the best size in the geometric mean, an item per unit (8
+// workgroups per unit with 8 kv heads), before, 27 %.  us of a call before (with its upload, see below) | now: 16 sequences of 91 to 1828
+// tokens, f16, 32.0 | 18.1, 5 of 500 to 10000 47.3 | 29.1, 40 of 100 to 6000, Q4_0, 64.4 | 46.6, 6 of 3000 to 9000, Q4_0, 33.7 | 20.8, 64 of 512
+// to 32768 717 | 710.
+int64_t choose_item_tiles(const RaggedSeq *seqs, int64_t n_seq, int64_t Hkv, int64_t total_tiles, int64_t step_bytes) {
+    const int64_t cus = num_compute_units();
+    std::vector<uint32_t> tiles((size_t)n_seq);
+    uint32_t most = 1;
+    for (int64_t i = 0; i < n_seq; i++) tiles[i] = (uint32_t)((seqs[i].len + kTile - 1) / kTile), most = std::max(most, tiles[i]);
+    const float rate = std::max((float)step_bytes / 6.84e6f, 0.0035f) * 256.0f / (float)cus, chain = 0.54f + 9.6e-6f * (float)step_bytes,
+                shared = 2.0f * std::max(0.85f * chain, (float)step_bytes / 46e3f);
+    uint32_t best = kWaves;
+    float best_us = INFINITY;
+    auto weigh = [&](uint32_t t) {
+        int64_t items = 0, groups = 0;
+        uint32_t longest = 0, splits = 1;
+        for (uint32_t x : tiles) {
+            uint32_t ns = (x + t - 1) / t;
+            const uint32_t per = (x + ns - 1) / ns, steps = (per + kWaves - 1) / kWaves;
+            ns = (x + per - 1) / per;
+            items += ns, groups += ns * steps, longest = std::max(longest, steps), splits = std::max(splits, ns);
+        }
+        const int64_t wgs = items * Hkv;
+        const float alone = chain * (float)longest;
+        float us = std::max((float)(groups * Hkv) * rate, wgs > cus ? std::max(alone, shared * (float)longest) : alone);
+        us += 0.3f * alone + (wgs <= cus ? 0.0f : wgs <= 2 * cus ? 1.5f : 2.0f + 0.004f * (float)wgs);
+        us += splits > kWideMergeMax ? 16.0f : splits > kTailMergeMax ? 2.0f : splits > 1 ? 0.5f : 0.0f;   // (the most: a merge launch, and its table)
+        if (us < best_us) best = t, best_us = us;
+    };
+    auto whole_groups = [&](int64_t wgs) { return (uint32_t)std::max<int64_t>(kWaves, (total_tiles * Hkv / wgs + kWaves - 1) / kWaves * kWaves); };
+    for (int64_t wgs : {cus, 2 * cus}) {
+        if (n_seq * Hkv > wgs) continue;
+        uint32_t t = whole_groups(wgs);
+        for (; t < most; t += std::max<uint32_t>(kWaves, t / 12 / kWaves * kWaves)) {
+            int64_t items = 0;
+            for (uint32_t x : tiles) items += (x + t - 1) / t;
+            if (items * Hkv <= wgs) break;
+        }
+        weigh(t);
+    }
+    weigh(whole_groups(4 * cus)), weigh(whole_groups(8 * cus));
+    return best;
+}
+
+}  // namespace
+
 // Ragged decode: one launch for all sequences.  The host cuts the sequences into work items
-// of about equal tile counts, uploads the plan (items + per-sequence slot ranges) into the
+// of about equal tile counts; the plan (items + per-sequence slot ranges) travels as a kernel argument, or is uploaded into the
 // head of the workspace, and the kernels index it by blockIdx.
 int launch_sdpa_decode_ragged(const void *q, void *out, int q_dtype, int kv_fmt, int64_t n_seq, int64_t Hq, int64_t Hkv,
                               int64_t D, const RaggedSeq *seqs, float scale, void *workspace, size_t workspace_bytes,
@@ -741,13 +793,13 @@ int launch_sdpa_decode_ragged(const void *q, void *out, int q_dtype, int kv_fmt,
         ((int64_t)kWsPlanBytes - n_seq * (int64_t)sizeof(RaggedSeqSlots)) / (int64_t)sizeof(RaggedItem);
     TROCM_REQUIRE(max_items_tbl >= n_seq, "ragged decode: the plan area holds %lld work items, fewer than the %lld sequences",
                   (long long)max_items_tbl, (long long)n_seq);
-    // Workgroups (items x kv heads) per compute unit: two are resident at a time, and the last round of
-    // them is only partly full, so more and smaller items shorten the tail at the cost of partial records.
+    // The matrix-core kernels with records of 8 rows: choose_item_tiles.  Others: an item per compute unit.
     static const int wg_per_cu = getenv("TROCM_RAGGED_WG_PER_CU") ? atoi(getenv("TROCM_RAGGED_WG_PER_CU")) : 0;
     int64_t want_items = wg_per_cu > 0 ? ((int64_t)num_compute_units() * wg_per_cu + Hkv - 1) / Hkv : num_compute_units();
     if (want_items < 1) want_items = 1;
     int64_t tiles_per_item = (total_tiles + want_items - 1) / want_items;
     if (tiles_per_item < kWaves) tiles_per_item = kWaves;
+    if (mfma_gp == 8 && wg_per_cu <= 0) tiles_per_item = choose_item_tiles(seqs, n_seq, Hkv, total_tiles, 4 * kTile * 2 * (rb + (quant ? D / 16 : 0)));
     int64_t n_items = 0, n_slots = 0;
     for (;;) {   // ends at the latest when no sequence is cut: n_seq items, no records
         n_items = n_slots = 0;
@@ -760,54 +812,95 @@ int launch_sdpa_decode_ragged(const void *q, void *out, int q_dtype, int kv_fmt,
         if (n_items <= max_items_tbl && n_slots <= max_slots_ws) break;
         tiles_per_item += (tiles_per_item + 3) / 4;
     }
-    StageSlot *stage;
-    if (acquire_stage(&stage)) return 1;
-    RaggedItem *items = (RaggedItem *)stage->host;
-    RaggedSeqSlots *slots = (RaggedSeqSlots *)(items + n_items);
-    int64_t it = 0, slot_it = 0;
-    bool any_split = false;
-    int64_t max_split = 1;
-    for (int64_t i = 0; i < n_seq; i++) {
-        int64_t tiles = (seqs[i].len + kTile - 1) / kTile;
+    // Each sequence's cut: ns[i] items of tps tiles (no empty one)
+    auto cut = [&](int64_t i, int64_t &tps) {
+        const int64_t tiles = (seqs[i].len + kTile - 1) / kTile;
         int64_t ns = (tiles + tiles_per_item - 1) / tiles_per_item;
-        int64_t tps = (tiles + ns - 1) / ns;
-        ns = (tiles + tps - 1) / tps;
-        slots[i].slot0 = (int)slot_it;   // first partial record of the sequence (unused when it is not cut)
-        slots[i].nsplit = (int)ns;
-        if (ns > 1) slot_it += ns;
-        any_split |= ns > 1;
+        tps = (tiles + ns - 1) / ns;
+        return (tiles + tps - 1) / tps;
+    };
+    int64_t it = 0, slot_it = 0, max_split = 1;
+    bool any_split = false, short_rows = true;
+    for (int64_t i = 0; i < n_seq; i++) {
+        int64_t tps;
+        const int64_t ns = cut(i, tps);
+        it += ns;
+        if (ns > 1) slot_it += ns, any_split = true;
         if (ns > max_split) max_split = ns;
-        for (int64_t sp = 0; sp < ns; sp++, it++) {
-            RaggedItem &r = items[it];
-            r.k = (const char *)seqs[i].k;
-            r.v = (const char *)seqs[i].v;
-            r.stride_h = seqs[i].cap * rb;
-            r.ks = (const char *)seqs[i].k_scales, r.vs = (const char *)seqs[i].v_scales;
-            r.sc_stride_h = seqs[i].cap * (D / 32) * 2;
-            r.T = (int)seqs[i].len;
-            r.tile_begin = (int)(sp * tps);
-            r.tile_end = (int)((sp + 1) * tps < tiles ? (sp + 1) * tps : tiles);
-            r.seq = (int)i, r.split = (int)sp, r.nsplit = (int)ns, r.slot0 = slots[i].slot0;
-        }
+        short_rows = short_rows && seqs[i].cap < (1ll << 31);
     }
     n_items = it;
-    // Longest items first: the workgroups that start last, when the device is no longer full, are the short ones.
-    // (An item carries its own partial slot, so the order is free.)
-    std::stable_sort(items, items + n_items, [](const RaggedItem &a, const RaggedItem &b) {
-        return a.tile_end - a.tile_begin > b.tile_end - b.tile_begin;
-    });
-    // the seq table sits right after the items actually emitted
-    RaggedSeqSlots *slots_packed = (RaggedSeqSlots *)(items + n_items);
-    if (slots_packed != slots) memmove(slots_packed, slots, (size_t)n_seq * sizeof(RaggedSeqSlots));
-    size_t plan_bytes = (size_t)n_items * sizeof(RaggedItem) + (size_t)n_seq * sizeof(RaggedSeqSlots);
-    {
-        const int n16 = (int)((plan_bytes + 15) / 16);   // the slot and the plan area are both kWsPlanBytes long
-        hipLaunchKernelGGL(plan_upload_kernel, dim3((n16 + 255) / 256), dim3(256), 0, s, (const uint4 *)stage->host_dev,
-                           (uint4 *)((char *)workspace + kWsCounterBytes), n16);
-        TROCM_HIP(hipGetLastError());
+    // The MFMA kernel merges the splits of a sequence-head itself when none has more than it can hold in registers.
+    static const int tail = getenv("TROCM_DECODE_TAIL_MERGE") ? atoi(getenv("TROCM_DECODE_TAIL_MERGE")) : 1;
+    const bool in_kernel = tail && mfma_gp && mfma_gp <= 8 && any_split && max_split <= kWideMergeMax && n_seq * Hkv <= (int64_t)(kWsCounterBytes / sizeof(int));
+    // A plan of few sequences travels as a kernel argument: the launch that brought it into device memory and the event behind it
+    // held the device for 5 to 10 us of every call (4 us and a gap of 5.5 in a trace; 11 sequences of 368 to 1104 Q4_0
+    // tokens 18.5 -> 13.8 with the same items, 3 of 400 to 1200, f16, 15.8 -> 11.2).
+    // (The merge launch reads a table in device memory.)
+    const bool by_value = mfma_gp && (in_kernel || !any_split) && n_seq <= kPlanSeqs && n_items <= kPlanItems && short_rows;
+    RaggedPlan plan;
+    if (by_value) {
+        int order[kPlanSeqs];
+        int64_t per[kPlanSeqs];
+        for (int i = 0; i < (int)n_seq; i++) order[i] = i, cut(i, per[i]);
+        std::stable_sort(order, order + n_seq, [&](int x, int y) { return per[x] > per[y]; });   // longest items first (as below)
+        int first = 0, slot = 0;
+        for (int j = 0; j < (int)n_seq; j++) {
+            const RaggedSeq &src = seqs[order[j]];
+            RaggedPlan::Seq &d = plan.seqs[j];
+            int64_t tps;
+            const int ns = (int)cut(order[j], tps);
+            d.k = (const char *)src.k, d.v = (const char *)src.v, d.ks = (const char *)src.k_scales, d.vs = (const char *)src.v_scales;
+            d.cap = (int)src.cap, d.T = (int)src.len;
+            d.first = (uint16_t)first, d.nsplit = (uint16_t)ns, d.slot0 = (uint16_t)slot, d.seq = (uint16_t)order[j];
+            for (int sp = 0; sp < ns; sp++) reinterpret_cast<uint8_t *>(plan.seq_of)[first + sp] = (uint8_t)j;
+            first += ns;
+            if (ns > 1) slot += ns;
+        }
     }
-    TROCM_HIP(hipEventRecord(stage->done, s));
-    stage->in_flight = true;
+    if (!by_value) {
+        StageSlot *stage;
+        if (acquire_stage(&stage)) return 1;
+        RaggedItem *items = (RaggedItem *)stage->host;
+        RaggedSeqSlots *slots = (RaggedSeqSlots *)(items + n_items);
+        it = slot_it = 0;
+        for (int64_t i = 0; i < n_seq; i++) {
+            int64_t tps;
+            const int64_t tiles = (seqs[i].len + kTile - 1) / kTile, ns = cut(i, tps);
+            slots[i].slot0 = (int)slot_it;   // first partial record of the sequence (unused when it is not cut)
+            slots[i].nsplit = (int)ns;
+            if (ns > 1) slot_it += ns;
+            for (int64_t sp = 0; sp < ns; sp++, it++) {
+                RaggedItem &r = items[it];
+                r.k = (const char *)seqs[i].k;
+                r.v = (const char *)seqs[i].v;
+                r.stride_h = seqs[i].cap * rb;
+                r.ks = (const char *)seqs[i].k_scales, r.vs = (const char *)seqs[i].v_scales;
+                r.sc_stride_h = seqs[i].cap * (D / 32) * 2;
+                r.T = (int)seqs[i].len;
+                r.tile_begin = (int)(sp * tps);
+                r.tile_end = (int)((sp + 1) * tps < tiles ? (sp + 1) * tps : tiles);
+                r.seq = (int)i, r.split = (int)sp, r.nsplit = (int)ns, r.slot0 = slots[i].slot0;
+            }
+        }
+        // Longest items first: the workgroups that start last, when the device is no longer full, are the short ones.
+        // (An item carries its own partial slot, so the order is free.)
+        std::stable_sort(items, items + n_items, [](const RaggedItem &a, const RaggedItem &b) {
+            return a.tile_end - a.tile_begin > b.tile_end - b.tile_begin;
+        });
+        // the seq table sits right after the items actually emitted
+        RaggedSeqSlots *slots_packed = (RaggedSeqSlots *)(items + n_items);
+        if (slots_packed != slots) memmove(slots_packed, slots, (size_t)n_seq * sizeof(RaggedSeqSlots));
+        size_t plan_bytes = (size_t)n_items * sizeof(RaggedItem) + (size_t)n_seq * sizeof(RaggedSeqSlots);
+        {
+            const int n16 = (int)((plan_bytes + 15) / 16);   // the slot and the plan area are both kWsPlanBytes long
+            hipLaunchKernelGGL(plan_upload_kernel, dim3((n16 + 255) / 256), dim3(256), 0, s, (const uint4 *)stage->host_dev,
+                               (uint4 *)((char *)workspace + kWsCounterBytes), n16);
+            TROCM_HIP(hipGetLastError());
+        }
+        TROCM_HIP(hipEventRecord(stage->done, s));
+        stage->in_flight = true;
+    }
 
     DecodeDev p;
     memset(&p, 0, sizeof(p));
@@ -826,12 +919,8 @@ int launch_sdpa_decode_ragged(const void *q, void *out, int q_dtype, int kv_fmt,
     p.part_o = p.part_ml + (size_t)slot_it * Hkv * 2 * G;
     const RaggedItem *d_items = (const RaggedItem *)((char *)workspace + kWsCounterBytes);
     const RaggedSeqSlots *d_slots = (const RaggedSeqSlots *)(d_items + n_items);
-    // The MFMA kernel merges the splits of a sequence-head itself when none has more than it can hold in registers.
-    static const int tail = getenv("TROCM_DECODE_TAIL_MERGE") ? atoi(getenv("TROCM_DECODE_TAIL_MERGE")) : 1;
-    if (tail && mfma_gp && mfma_gp <= 8 && any_split && max_split <= kWideMergeMax &&
-        n_seq * Hkv <= (int64_t)(kWsCounterBytes / sizeof(int)))
-        p.counters = (int *)workspace;
-    if (mfma_gp) return launch_sdpa_decode_ragged_mfma(p, kv_fmt, mfma_gp, D, d_items, (int)n_items, d_slots, (int)n_seq, any_split, s);
+    if (in_kernel) p.counters = (int *)workspace;
+    if (mfma_gp) return launch_sdpa_decode_ragged_mfma(p, kv_fmt, mfma_gp, D, by_value ? nullptr : d_items, plan, (int)n_items, d_slots, (int)n_seq, any_split, s);
     if (kv_fmt == TROCM_F16)
         return D == 128 ? launch_ragged_g<__half, 128>(p, (int)G, d_items, (int)n_items, d_slots, (int)n_seq, any_split, s)
                         : launch_ragged_g<__half, 64>(p, (int)G, d_items, (int)n_items, d_slots, (int)n_seq, any_split, s);
