@@ -283,9 +283,9 @@ int launch_q4_0_matvec(const void *codes, const void *scales, int64_t w_batch, i
         const int rc = launch_q4_0_matmul(codes, scales, w_batch, n, k, act, act_dtype, act_batch, m, out, s);
         if (rc != 2) return rc;
     }
-    // f32 rows from 7 on: one pass over the weights for all of them (us for 1000 x 2080, here | there: 5 rows 7.2 | 7.3, 6 rows
-    // 8.0 | 7.3, 8 rows 11.6 | 7.4)
-    if (act_dtype == TROCM_F32 && m >= 7) {
+    // f32 rows from 6 on, and 5 of a large matrix: one pass over the weights for all of them (us, here | there: 5 rows of 1000 x 2080 6.6 |
+    // 6.8, of 4090 x 4096 20.9 | 14.4; 6 rows 7.3 | 6.8, 26.4 | 14.5; 8 rows of 1000 x 2080 11.6 | 7.0)
+    if (act_dtype == TROCM_F32 && (m >= 6 || (m == 5 && n > 2048))) {
         const int rc = launch_q4_0_matmul_f32(codes, scales, w_batch, n, k, act, act_batch, m, out, s, 0);
         if (rc != 2) return rc;
     }

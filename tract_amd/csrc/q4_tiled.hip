@@ -530,7 +530,7 @@ int launch_q4_0_tiled_export(const void *tiles, void *blocks, int64_t rows, int6
 }
 
 // Tiled weights x activations for any m: f16 rows in groups of up to 16 (more than 16 rows go to the matrix-matrix
-// kernel first, which reads the same tiles, when it takes the call), up to 6 f32 rows (more go to q4_matmul_f32.hip; in
+// kernel first, which reads the same tiles, when it takes the call), up to 5 f32 rows (more go to q4_matmul_f32.hip; in
 // groups of 8 what that refuses, and few rows of tall matrices).
 int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int64_t k, const void *act, int act_dtype,
                              int64_t act_batch, int64_t m, void *out, hipStream_t s) {
@@ -552,17 +552,15 @@ int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int6
         const int rc = launch_q4_0_matmul(tiles, nullptr, w_batch, n, k, act, act_dtype, act_batch, m, out, s, 1);
         if (rc != 2) return rc;
     }
-    // f32 rows from 7 on: one pass over the weights for all of them (us, here | there, 6 rows and 7: 4096 x 4096 9.5 | 8.7 and 13.0 |
-    // 8.8, 4096 x 14336 31.2 | 24.8 and 34.4 | 25.1).  Its workgroups of 16 activation rows take 16 or 32 weight rows each, one workgroup
-    // per compute unit: few rows of a tall matrix need several rounds of them, while a pass of 8 rows here streams the weights at
-    // the memory's rate.
-    // 7 and 8 rows: 32768 x 4096 27.6 | 40.3, 32768 x 128 4.8 | 7.2, 24576 x 4096 28.9 | 22.3, 14336 x 1024 7.0 | 6.4 (14336 x 4096
-    // 16.5 | 19.3 goes there for its smaller error against 64 bits, 1.5e-7 | 9.9e-8); 12 rows, two passes: 128256 x 512 24.6 | 31.2, 128256 x 4096 165 | 153, 65536 x
-    // 2048 40.9 | 45.0, 65536 x 1024 23.6 | 24.1, 65536 x 128 12.9 | 13.7; 17 rows: 128256 x 128 26.0 | 28.1, 128256 x 512 48.0 | 32.2.
-    const bool stream = m <= 8 ? n > 24576
-                      : m <= 16 ? n >= 57344 && k < 4096 && (n > 98304 || k < 256 || k >= 2048)
-                                : m <= 24 && n > 98304 && k < 256;
-    if (act_dtype == TROCM_F32 && m >= 7 && !stream) {
+    // f32 rows from 7 on, and 5 and 6 of a small matrix: one pass over the weights for all of them (us, here | there: 5 rows of 5120 x 5120 17.9 |
+    // 11.8, 4096 x 4096 8.5 | 8.3, 1024 x 4096 8.0 | 7.3, 14336 x 4096 14.9 | 15.7, 4096 x 14336 22.7 | 23.8; 6 rows 4096 x 14336 30.5 | 24.0,
+    // 8192 x 8192 25.1 | 18.7, 4096 x 4096 8.8 | 8.4, 14336 x 4096 15.5 | 15.8; 4 rows of 4096 x 4096 6.6 | 8.2).  Its workgroups of 16 rows
+    // take up to 64 weight rows each, one workgroup per compute unit: 6 to 8 rows of a tall matrix need several rounds of them, while a pass
+    // of 8 rows here streams the weights at the memory's rate (8 rows: 65536 x 128 6.2 | 7.0, x 2048 24.9 | 28.3, x 4096 52.7 | 51.3; 32768 x
+    // 512 6.7 | 5.9, x 2048 14.2 | 15.7, x 4096 27.6 | 26.9; 128256 x 1024 25.5 | 27.8, x 4096 98.9 | 95.3, 6 rows of it 82.0 | 93.7); 9 and
+    // more need two passes (12 rows of 65536 x 128 12.9 | 6.8, of 128256 x 1024 39.9 | 28.8, x 4096 equal).
+    const bool stream = m <= 8 && n > 24576 && (m > 6 ? k < 4096 && (k >= 2048 || n >= 57344) : k >= 2048 || n >= 57344);
+    if (act_dtype == TROCM_F32 && (m >= 7 || (m == 6 && (n <= 8192 || n > 24576)) || (m == 5 && n <= 8192 && k <= 5120)) && !stream) {
         const int rc = launch_q4_0_matmul_f32(tiles, nullptr, w_batch, n, k, act, act_batch, m, out, s, 1);
         if (rc != 2) return rc;
     }
