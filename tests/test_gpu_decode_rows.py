@@ -183,3 +183,33 @@ def test_scratch_limits_and_strided_rows(rt, dtype, Hq, n, causal):
         # f16: as above; f32: sums of D products and 2600 weights, 2^-24 of the score in the exponent
         tol = 2 * 2.0 ** -11 * np.abs(v.astype(np.float64)).max() if dtype == np.float16 else 2e-5 * np.abs(want).max()
         assert np.abs(got - want).max() <= tol, size
+
+
+# 9 to 32 rows per kv head in 2, 3 and 4 ranges of keys, which the last workgroup to arrive merges (and 5 and more: the launch), a last
+# group of fewer rows, 64 features; an infinity of V in a range of its own stays one, calls repeated on the same counters
+@pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [(8, 32, 8, 128, 2200, 8), (8, 24, 8, 128, 2300, 5), (10, 32, 8, 128, 2600, 3), (16, 32, 8, 64, 2700, 4), (4, 10, 2, 128, 2100, 9),
+                                               (11, 32, 8, 128, 2400, 3), (5, 32, 32, 64, 1900, 11)])
+def test_ranges_merged_by_the_last_workgroup(rt, B, Hq, Hkv, D, past, n):
+    rng = np.random.default_rng(past + n)
+    k, v = (rng.standard_normal((B, Hkv, past + n, D), dtype=np.float32).astype(np.float16) for _ in range(2))
+    q = rng.standard_normal((B, Hq, n, D), dtype=np.float32).astype(np.float16)
+    v[0, 0, 7, 3] = np.inf
+    st = ta.InPlaceKvSdpa(axis=2, causal=True).state()
+    st.k.push(k[:, :, :past]), st.v.push(v[:, :, :past])
+    kn, vn = np.ascontiguousarray(k[:, :, past:]), np.ascontiguousarray(v[:, :, past:])
+    G = Hq // Hkv
+    for turn in range(3):
+        st.k.truncate(past), st.v.truncate(past)
+        out = st.eval([q, kn, vn]).to_numpy().astype(np.float64)
+        for b in (0, B - 1):
+            for h in (0, Hq - 1):
+                kh, vh = k[b, h // G].astype(np.float64), v[b, h // G].astype(np.float64)
+                s = q[b, h].astype(np.float64) @ kh.T / np.sqrt(D)
+                s[np.arange(past + n)[None, :] > past + np.arange(n)[:, None]] = -np.inf
+                p = np.exp(s - s.max(axis=1, keepdims=True))
+                p /= p.sum(axis=1, keepdims=True)
+                if b == 0 and h // G == 0:
+                    assert np.all(np.isposinf(out[b, h, :, 3])), turn
+                    vh[7, 3], out[b, h, :, 3] = 0.0, (p @ np.where(np.isfinite(vh), vh, 0.0))[:, 3]
+                # weights and results rounded to f16; f32 sums of D products in the scores (7 at most), of the tokens in the result
+                assert np.all(np.abs(out[b, h] - p @ vh) <= 2.0 ** -9 * (p @ np.abs(vh)) + 2.0 ** -24), (turn, b, h)

@@ -337,6 +337,64 @@ __device__ __forceinline__ void tail_merge_pairs(const DecodeDev &p, int *counte
     }
 }
 
+constexpr int kRowsMergeMax = 4;
+// The same for records of 16 or 32 rows, `rows` of them real: a thread weighs one (row, split), the weights go through `lds_w` (two
+// floats a row and one a row and split, of LDS that nothing else uses any more), and every split's elements are asked for before that.
+template <typename T, int D, int G, int MAXS>
+__device__ __forceinline__ void tail_merge_rows(const DecodeDev &p, int *counter, int nsplit, int64_t first, T *out, int rows, int tid, float *lds_w) {
+    static_assert(G * MAXS <= kThreads && (MAXS & (MAXS - 1)) == 0, "a thread per (row, split)");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this thread's partial stores have completed
+    __syncthreads();                                     // ... and so have the whole workgroup's
+    __shared__ int s_last_rows;
+    if (tid == 0) {
+        const int arrived = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last_rows = arrived == nsplit - 1;
+        if (s_last_rows) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!s_last_rows) return;
+    auto aload = [](const float *a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    const int h = min(tid / MAXS, G - 1), sp_w = tid % MAXS;
+    const float *ml = p.part_ml + (first + min(sp_w, nsplit - 1)) * (2 * G) + h;
+    const float m = aload(ml), l = aload(ml + G);
+    constexpr int NE = G * D / (2 * kThreads);
+    uint64_t ov[NE][MAXS];
+#pragma unroll
+    for (int e = 0; e < NE; e++)
+#pragma unroll
+        for (int sp = 0; sp < MAXS; sp++)   // splits past the last repeat it and are left out below, rows past the last likewise
+            ov[e][sp] = __hip_atomic_load(reinterpret_cast<const uint64_t *>(p.part_o + (first + min(sp, nsplit - 1)) * (G * D) + min(2 * (tid + e * kThreads), rows * D - 2)),
+                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    float mm = m;
+#pragma unroll
+    for (int d = 1; d < MAXS; d <<= 1) mm = fmaxf(mm, __shfl_xor(mm, d, 64));
+    const float f = sp_w < nsplit ? fast_exp2(m - (mm == -INFINITY ? 0.0f : mm)) : 0.0f;
+    float ll = sp_w < nsplit ? l * f : 0.0f;
+#pragma unroll
+    for (int d = 1; d < MAXS; d <<= 1) ll += __shfl_xor(ll, d, 64);
+    if (tid < G * MAXS) {
+        lds_w[h * MAXS + sp_w] = f;
+        if (sp_w == 0) lds_w[G * MAXS + h] = ll;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < NE; e++) {
+        const int idx = 2 * (tid + e * kThreads), row = idx / D;
+        if (row >= rows) continue;
+        float acc0 = 0.0f, acc1 = 0.0f;
+#pragma unroll
+        for (int sp = 0; sp < MAXS; sp++) {
+            const float w = lds_w[row * MAXS + sp];
+            const uint64_t x = sp < nsplit ? ov[e][sp] : 0;   // (0 times an infinity is NaN)
+            acc0 += __builtin_bit_cast(float, (uint32_t)x) * w;
+            acc1 += __builtin_bit_cast(float, (uint32_t)(x >> 32)) * w;
+        }
+        const float total = lds_w[G * MAXS + row];
+        out[idx] = from_f32<T>(total > 0.0f ? acc0 / total : 0.0f);
+        out[idx + 1] = from_f32<T>(total > 0.0f ? acc1 / total : 0.0f);
+    }
+}
+
 // The same for up to kWideMergeMax splits (small batches: 32 splits at batch 1), with G * kWideMergeMax <=
 // kThreads: thread (h, sp) loads the (m, l) record of head h in split sp and the 32 threads of a head reduce
 // them to weights, which go through `lds_w` (G * kWideMergeMax floats of LDS that nothing else uses any more);

@@ -93,7 +93,7 @@ struct MfmaWork {
 // The tail every formulation shares: the four waves' records (O[GP][D], m[GP], l[GP], in `lds_raw`, kCombStride floats
 // each) become the output rows (one split), or this workgroup's partial record, merged by the last workgroup to
 // arrive or by the merge launch.
-template <int D, int GP>
+template <int D, int GP, bool ROWS = false>
 __device__ __forceinline__ void wave_records_to_output(const DecodeDev &p, const MfmaWork &wk, unsigned char *lds_raw, int64_t head0,
                                                        int g, int tid) {
     constexpr int kCombStride = GP * D + 2 * GP;
@@ -143,7 +143,13 @@ __device__ __forceinline__ void wave_records_to_output(const DecodeDev &p, const
             }
         }
     }
-    if constexpr (GP <= 8) {   // (larger groups: the merge launch; the in-kernel merge would need too many registers)
+    if constexpr (ROWS && GP > 8) {
+        if (wk.nsplit > 1 && wk.counter != nullptr) {
+            __syncthreads();   // (the weights go where the waves' records were)
+            tail_merge_rows<__half, D, GP, kRowsMergeMax>(p, wk.counter, wk.nsplit, wk.part_first, out, g, tid, comb);
+        }
+    }
+    if constexpr (GP <= 8) {   // (larger groups of heads: the merge launch; the in-kernel merge would need too many registers)
         if (wk.nsplit > kTailMergeMax && wk.counter != nullptr)
             tail_merge_wide<__half, D, GP>(p, wk.counter, wk.nsplit, wk.part_first, wk.part_stride, out, tid, reinterpret_cast<float *>(lds_raw));
         else if (wk.nsplit > 1 && wk.nsplit <= 4 && wk.counter != nullptr && half_live)   // (cfg2's shape: 4 splits of 4 heads)
@@ -745,7 +751,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
             cw[GP * D + GP + l32_end] = l_run;
         }
     }
-    wave_records_to_output<D, GP>(p, wk, lds_raw, head0, g, tid);
+    wave_records_to_output<D, GP, ROWS>(p, wk, lds_raw, head0, g, tid);
 }
 
 // Transposing 64-bit LDS load of 8-bit elements: in each block of 16 lanes, lane i receives byte i%8 of the eight
@@ -2696,8 +2702,8 @@ int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s) {
     // 8, 12 x 5549 tokens, 10 queries, two layers 63.4 us in 2 ranges, 56.9 in 3; 32 over 32, 6 x 2610 55.1 in 1, 48.9 in 2; no
     // difference below 64 workgroups per range); two with several groups and more than 8 tiles per wave (40 heads over 8,
     // 4 x 5000 tokens, 8 queries 38.7 -> 33.4 us), 32 where one range of keys fills the chip (32 over 32, 4 x 1064, 64 queries 83.0
-    // split, 58.5 not).  Records of more than 8 rows are merged by a second launch, the dearer the more of them there are:
-    // below these lengths it costs more than the split gives (us of two layers, split | not: BH 128, 10 tiles 38.5 | 27.3, 20 tiles
+    // split, 58.5 not).  Records of more than 8 rows in more than kRowsMergeMax ranges are merged by a second launch, the dearer the more of them there are:
+    // below these lengths it costs more than the split gives (us of two layers, split | not, with the launch for any number of ranges: BH 128, 10 tiles 38.5 | 27.3, 20 tiles
     // 39.2 | 33.5, 33 tiles equal; BH 64, 9 tiles 26.9 | 23.2, 20 tiles equal; BH 32, 9 tiles 24.4 | 22.9, 16 tiles 26.5 | 29.5;
     // quantised caches, whose waves take longer for a tile: BH 64, 16 tiles 27.1 | 28.9).
     int64_t resident = num_compute_units();
@@ -2710,7 +2716,10 @@ int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s) {
     p.live_trim = decode_live_trim();
     p.part_ml = (float *)((char *)a.workspace + kWsCounterBytes);
     p.part_o = p.part_ml + (size_t)BH * p.nsplit * 2 * gp;
-    if (gp <= 8 && p.nsplit > 1 && p.nsplit <= kWideMergeMax && BH <= (int64_t)(kWsCounterBytes / sizeof(int))) p.counters = (int *)a.workspace;
+    // Up to 4 ranges of more than 8 rows are merged by the last workgroup to arrive; more cost that one more than the launch takes (us, merge
+    // launch | here: 8 x 3000 tokens, 8 queries, 4 ranges 26.8 | 25.5, 8 x 1500, Q8_0, 6 queries 22.4 | 21.1, 5 x 1244, 11 queries of 32 heads over
+    // 32 15.9 | 14.8; 8 ranges: 4 x 5000, 6 queries 22.6 | 23.6, Q4_0, 5 queries 22.4 | 22.9).
+    if (p.nsplit > 1 && p.nsplit <= (gp <= 8 ? kWideMergeMax : kRowsMergeMax) && BH <= (int64_t)(kWsCounterBytes / sizeof(int))) p.counters = (int *)a.workspace;
     const dim3 grid((unsigned)p.nsplit, (unsigned)(a.Hkv * n_groups), (unsigned)a.B);
     if (a.kv_fmt == TROCM_Q8_0) return launch_rows_gp<128, TROCM_Q8_0>(p, gp, grid, s);
     if (a.kv_fmt == TROCM_Q4_0) return launch_rows_gp<128, TROCM_Q4_0>(p, gp, grid, s);
