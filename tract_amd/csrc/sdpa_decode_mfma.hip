@@ -2711,7 +2711,10 @@ int launch_sdpa_decode_rows(const SdpaArgs &a, hipStream_t s) {
     if (n_groups > 1 && n_tiles >= (nsplit == 1 ? 128 : 32 * nsplit)) nsplit = choose_decode_splits(BH, gp, n_tiles, 2), resident *= 2;
     const bool light = a.D == 64 && gp <= 16 && BH >= 64 && n_tiles >= 32;
     if (nsplit > 1 && BH * nsplit > resident && resident >= BH && !light) nsplit = (int)(resident / BH);
-    if (gp > 8 && nsplit > 1 && n_tiles <= 8 + (quant ? 16 : 48) / nsplit) nsplit = 1;
+    // (merged by the last workgroup: us a layer, split in 3 or 4 | not: BH 64, 16 rows, 23 tiles 11.5 | 14.1; BH 48, 32 rows, 13 tiles 13.6 | 14.1;
+    // BH 16, 13 tiles of 64 features 8.0 | 8.6; 10 tiles 12.6 | 12.1)
+    const bool tail = nsplit <= kRowsMergeMax;
+    if (gp > 8 && nsplit > 1 && n_tiles <= (quant ? 8 + 16 / nsplit : tail ? 6 + 24 / nsplit : 8 + 48 / nsplit)) nsplit = 1;
     p.nsplit = fit_decode_splits(nsplit, BH, gp, a.D, a.workspace, a.workspace_bytes);
     p.live_trim = decode_live_trim();
     p.part_ml = (float *)((char *)a.workspace + kWsCounterBytes);
