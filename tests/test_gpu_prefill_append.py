@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import tract_amd as ta
+from tests.cases import textbook_sdpa
 from tests.gpu_util import rt  # noqa: F401
 from tract_amd._lib import call
 
@@ -69,3 +70,29 @@ def test_results_over_the_new_rows(rt, dtype, past, n, over):
     got = st.eval_into(ta.DeviceTensor.from_numpy(q), args["k"], args["v"], args[over]).to_numpy()
     assert st.k.valid_contiguous().tobytes() == k.tobytes() and st.v.valid_contiguous().tobytes() == v.tobytes()
     assert got.tobytes() == _over_one_tensor(q, k, v, True).tobytes()
+
+
+# f32 rows behind a cache whose last tile of keys is not full (the call's rows begin a tile of their own): one row and all but one of a tile,
+# up to 32 rows per kv head and more, ranges of keys, 1 to 8 query heads per kv head
+@pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [(1, 8, 2, 128, 1, 3), (2, 4, 4, 64, 31, 2), (1, 14, 2, 128, 348, 10), (3, 32, 8, 64, 801, 11), (6, 32, 8, 128, 910, 3), (1, 8, 2, 128, 33, 200),
+                                               (1, 32, 8, 128, 225, 373), (2, 6, 2, 64, 1999, 65), (1, 16, 16, 128, 500, 97), (1, 64, 8, 64, 95, 33)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_f32_rows_behind_a_cache(rt, B, Hq, Hkv, D, past, n, causal):
+    q, k, v = _inputs(np.float32, B, Hq, Hkv, D, past, n)
+    want = textbook_sdpa(q, k, v, causal=causal)
+    for poisoned in (False, True):
+        if poisoned:   # a value that only the last query sees (all of them without a causal mask), and one in the cache's last row
+            v[0, 0, past + n - 1, 2], v[B - 1, Hkv - 1, past - 1, 1] = np.inf, -np.inf
+        st = _state(k, v, past, n, causal)
+        got = st.eval([q, np.ascontiguousarray(k[:, :, past:]), np.ascontiguousarray(v[:, :, past:])]).to_numpy().astype(np.float64)
+        assert st.k.valid_contiguous().tobytes() == k.tobytes() and st.v.valid_contiguous().tobytes() == v.tobytes()
+        if poisoned:
+            G = Hq // Hkv
+            seen = got[0, :G, :, 2] if not causal else got[0, :G, -1:, 2]
+            assert np.all(np.isposinf(seen)) and np.all(np.isneginf(got[B - 1, Hq - G :, :, 1]))
+            if causal:
+                assert np.all(np.isfinite(got[0, :G, :-1, 2]))
+            got = np.where(np.isfinite(got), got, want)
+        # as many f32 roundings as additions stand one after the other, of a mean of values of about 1; measured 2e-7 of the norm
+        assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+        assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max()

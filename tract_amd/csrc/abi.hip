@@ -1373,11 +1373,11 @@ int trocm_inplace_kv_sdpa_eval(const void *q, const void *k_new, const void *v_n
             if (rc != 2) return rc;
         }
     }
-    // Several tokens at once on an f16 cache: likewise, by the decode tiles (4 x 5000 tokens, 8 new ones, 32 heads over 8: 26.4 us
-    // with an append launch, 24.8 without; 1 x 229: 14.9, 12.6) or the prefill kernel; an f32 prompt into an empty cache.  Not where
-    // the output lies over the new rows: one workgroup stores results while another still reads them.
+    // Several tokens at once on a plain cache: likewise, by the decode tiles (4 x 5000 tokens, 8 new ones, 32 heads over 8: 26.4 us
+    // with an append launch, 24.8 without; 1 x 229: 14.9, 12.6) or the prefill kernels.  Not where the output lies over the new rows: one
+    // workgroup stores results while another still reads them.
     const size_t es = elem_bytes(dtype), new_bytes = (size_t)kc->B * kc->H * n_new * kc->D * es, out_bytes = (size_t)kc->B * q_heads * n_new * kc->D * es;
-    if (n_new > 1 && is_dense && kc->B > 0 && kc->fmt == dtype && (dtype == TROCM_F16 || kc->len == 0) && kc->window == 0 && vc->window == 0 &&
+    if (n_new > 1 && is_dense && kc->B > 0 && kc->fmt == dtype && kc->window == 0 && vc->window == 0 &&
         !ranges_meet(out, out_bytes, k_new, new_bytes) && !ranges_meet(out, out_bytes, v_new, new_bytes)) {
         hipStream_t s;
         if (resolve_stream(stream, &s)) return 1;

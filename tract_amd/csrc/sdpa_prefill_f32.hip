@@ -51,6 +51,7 @@
 // From 4 tiles on (2 x 70 queries of 32 heads over 32, 3 tiles: 15.3 | 17.5; 2 x 116 of 40 over 8 20.0 | 18.0); ranges of keys (us
 // without | with): 49 queries, 32 over 8, 396 tokens 29.7 | 21.5, but 2 x 251, a workgroup per compute unit, 25.0 | 33.7.
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <string.h>
 #include <algorithm>
 #include "decode_common.h"
@@ -82,11 +83,12 @@ struct PrefillF32 {
     int n_rt2, paired;                  // sdpa_prefill_f32x2_kernel: 64-row tiles per kv head; whether the short ones run beside the long ones
     int causal;
     float scale;
-    // Fused append of a first prompt (sdpa_prefill_f32x2_kernel): k and v are then the call's own dense rows, and their copies
-    // go here, one kv head's rows `kv_dst_stride_h` elements after the last one's.  NULL: nothing to store.
-    float *k_dst, *v_dst;
-    int64_t kv_dst_stride_h;
+    // Fused append (dense token rows): the tokens from `past` on are read from the call's own dense rows, [B, Hkv, Sq, D], and copied to
+    // the cache by this launch; kv_bytes are then those of the tokens before.  NULL: all Sk = `past` are in the cache.
+    const float *k_new, *v_new;
+    int past;
 };
+
 
 template <int T> struct VecOf;
 template <> struct VecOf<2> { typedef f32x2 type; };
@@ -105,6 +107,27 @@ __device__ __forceinline__ uint32_t finite_mask(float x) {
     return (uint32_t)((int)((__builtin_bit_cast(uint32_t, x) & 0x7f800000u) - 0x7f800000u) >> 31);
 }
 __device__ __forceinline__ float masked(float x, uint32_t mask) { return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & mask); }
+
+// Tiles of 32 keys: those of the cache, the last of them with fewer rows, then those of the call's rows.
+struct KeyTiles {
+    int past, old;   // tokens and tiles in the cache
+    __device__ __forceinline__ int first_key(int kt) const { return kt < old ? 32 * kt : past + 32 * (kt - old); }
+    __device__ __forceinline__ int end(int kt) const { return kt < old ? min(32 * kt + 32, past) : INT_MAX; }   // keys from here on are not its own
+    __device__ __forceinline__ int count(int n_vis) const { return n_vis <= past ? (n_vis + 31) / 32 : old + (n_vis - past + 31) / 32; }
+};
+// The rows of one kv head of K or V: rows after the last one of a buffer read as zeros.
+struct Rows {
+    const float *head, *head_new;
+    uint32_t bytes, bytes_new, row_bytes;
+    int old;
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(int kt) const {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(kt < old ? head : head_new), 0, kt < old ? bytes : bytes_new, 0x00020000);
+    }
+    __device__ __forceinline__ uint32_t off(int kt, int row) const { return (uint32_t)(32 * (kt < old ? kt : kt - old) + row) * row_bytes; }   // row of tile kt
+};
+__device__ __forceinline__ Rows rows_of(const PrefillF32 &p, const float *cache, const float *call, int b, int kvh, int D) {
+    return Rows{cache + b * p.kv_stride_b + kvh * p.kv_stride_h, call + (call ? ((int64_t)b * p.Hkv + kvh) * p.Sq * D : 0), p.kv_bytes, call ? (uint32_t)p.Sq * D * 4 : 0, p.kv_row_bytes, (p.past + 31) / 32};
+}
 
 // the weight exp(m - ref) of a partial result whose maximum is m; nothing seen: m = -inf, weight 0 whatever ref is
 __device__ __forceinline__ float ref_of(float m) { return m == -INFINITY ? 0.0f : m; }
@@ -136,24 +159,25 @@ __device__ __forceinline__ void attend_tile(const PrefillF32 &p, TileLds<D> &sha
     // keys [0, limit) are visible to a row; the tile as a whole sees n_vis
     auto limit_of = [&](int r) { return p.causal ? min(r, n_rows - 1) / p.G + (p.Sk - p.Sq) + 1 : p.Sk; };
     const int limit = limit_of(r0 + l32), limit_first = limit_of(r0), n_vis = limit_of(r0 + kRows - 1);
-    const int kt_end = min((n_vis + 31) / 32, kt_last);
+    const KeyTiles keys{p.past, (p.past + 31) / 32};
+    const int kt_end = min(keys.count(n_vis), kt_last);
 
     // rows past the last key read as zeros: the buffer ends with that row
-    const float *k_head = p.k + b * p.kv_stride_b + kvh * p.kv_stride_h, *v_head = p.v + b * p.kv_stride_b + kvh * p.kv_stride_h;
-    const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(k_head), 0, p.kv_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(v_head), 0, p.kv_bytes, 0x00020000);
+    const Rows k_rows = rows_of(p, p.k, p.k_new, b, kvh, D), v_rows = rows_of(p, p.v, p.v_new, b, kvh, D);
 
     f32x4 kreg[KJ];
     vec vreg[16];
     auto load_k = [&](int kt) {
-        const uint32_t off = (uint32_t)(32 * kt + l32) * p.kv_row_bytes + 16 * hb;
+        const __amdgpu_buffer_rsrc_t rsrc = k_rows.rsrc(kt);
+        const uint32_t off = k_rows.off(kt, l32) + 16 * hb;
 #pragma unroll
-        for (int j = 0; j < KJ; j++) kreg[j] = buffer_f32x4(k_rsrc, off + 32 * j);
+        for (int j = 0; j < KJ; j++) kreg[j] = buffer_f32x4(rsrc, off + 32 * j);
     };
     auto load_v = [&](int kt) {
-        const uint32_t off = (uint32_t)(32 * kt + 4 * hb) * p.kv_row_bytes + 4 * T * l32;
+        const __amdgpu_buffer_rsrc_t rsrc = v_rows.rsrc(kt);
+        const uint32_t off = v_rows.off(kt, 4 * hb) + 4 * T * l32;
 #pragma unroll
-        for (int i = 0; i < 16; i++) vreg[i] = buffer_vec<T>(v_rsrc, off + (uint32_t)(8 * (i / 4) + i % 4) * p.kv_row_bytes);
+        for (int i = 0; i < 16; i++) vreg[i] = buffer_vec<T>(rsrc, off + (uint32_t)(8 * (i / 4) + i % 4) * p.kv_row_bytes);
     };
 
     int kt = kt_first + w;
@@ -189,13 +213,14 @@ __device__ __forceinline__ void attend_tile(const PrefillF32 &p, TileLds<D> &sha
         if (kt + kWaves < kt_end) load_k(kt + kWaves);
         __builtin_amdgcn_sched_barrier(0);
 
-        const bool edge = 32 * kt + 32 > limit_first;   // some row does not see all of the tile
+        const int key0 = keys.first_key(kt), own = min(limit, keys.end(kt));
+        const bool edge = key0 + 32 > min(limit_first, keys.end(kt));   // some row does not see all of the tile
 #pragma unroll
         for (int r = 0; r < 16; r++) s[r] *= p.scale;
         if (edge) {
 #pragma unroll
             for (int r = 0; r < 16; r++)
-                if (32 * kt + 8 * (r / 4) + 4 * hb + r % 4 >= limit) s[r] = -INFINITY;
+                if (key0 + 8 * (r / 4) + 4 * hb + r % 4 >= own) s[r] = -INFINITY;
         }
         float mx = s[0];
 #pragma unroll
@@ -234,11 +259,12 @@ __device__ __forceinline__ void attend_tile(const PrefillF32 &p, TileLds<D> &sha
                     for (int r = 0; r < 16; r++)
                         if (r == 4 * (kk >> 3) + (kk & 3)) pk = s[r];
                     pk = __shfl(pk, l32 + 32 * ((kk >> 2) & 1), 64);
-                    const uint32_t seen = 32 * kt + kk < limit ? ~0u : 0u;
-                    const uint32_t off = (uint32_t)(32 * kt + kk) * p.kv_row_bytes;
+                    const uint32_t seen = key0 + kk < own ? ~0u : 0u;
+                    const __amdgpu_buffer_rsrc_t rsrc = v_rows.rsrc(kt);
+                    const uint32_t off = v_rows.off(kt, kk);
 #pragma unroll
                     for (int r = 0; r < 16; r++) {
-                        const vec x = buffer_vec<T>(v_rsrc, off + 4 * T * (8 * (r / 4) + 4 * hb + r % 4));
+                        const vec x = buffer_vec<T>(rsrc, off + 4 * T * (8 * (r / 4) + 4 * hb + r % 4));
 #pragma unroll
                         for (int t = 0; t < T; t++)
                             o[t][r] = fmaf(pk, masked(x[t], seen & ~finite_mask(x[t])), o[t][r]);
@@ -311,8 +337,17 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32_kernel(PrefillF3
     const int bh = blockIdx.x % p.n_bh, rest = blockIdx.x / p.n_bh;
     const int split = rest % p.nsplit, rt = p.n_rt - 1 - rest / p.nsplit;
     const int last = min(rt * kRows + kRows, p.Sq * p.G) - 1, n_vis = p.causal ? last / p.G + (p.Sk - p.Sq) + 1 : p.Sk;
-    const int per_split = ((n_vis + 31) / 32 + p.nsplit - 1) / p.nsplit;
+    const int per_split = (KeyTiles{p.past, (p.past + 31) / 32}.count(n_vis) + p.nsplit - 1) / p.nsplit;
     attend_tile<D>(p, shared, bh, rt, split, split * per_split, (split + 1) * per_split);
+    // The append: this workgroup's share of its kv head's rows (contiguous in both places).  With an append launch | now: 69 rows of 32 heads
+    // over 8 14.3 | 12.2 us, 10 of 14 over 2 behind 348 18.8 | 16.4.
+    if (p.k_new) {
+        const int64_t from = (int64_t)bh * p.Sq * D, to = (bh / p.Hkv) * p.kv_stride_b + (bh % p.Hkv) * p.kv_stride_h + (int64_t)p.past * D;
+        for (int i = rest * kThreads + threadIdx.x; i < p.Sq * (D / 4); i += p.n_rt * p.nsplit * kThreads) {
+            reinterpret_cast<f32x4 *>(const_cast<float *>(p.k) + to)[i] = reinterpret_cast<const f32x4 *>(p.k_new + from)[i];
+            reinterpret_cast<f32x4 *>(const_cast<float *>(p.v) + to)[i] = reinterpret_cast<const f32x4 *>(p.v_new + from)[i];
+        }
+    }
 }
 
 // ---- more than 32 rows: every f32 as a pair of f16 ---------------------------------------------------------------------
@@ -375,37 +410,37 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
     };
     auto limit_of = [&](int r) { return p.causal ? min(r, n_rows - 1) / p.G + (p.Sk - p.Sq) + 1 : p.Sk; };
     const int limit = limit_of(r0 + kRows * rg + l32), limit_first = limit_of(r0), n_vis = limit_of(r0 + 2 * kRows - 1);
-    const int tiles = (n_vis + 31) / 32, per_split = (tiles + p.nsplit - 1) / p.nsplit;
+    const KeyTiles keys{p.past, (p.past + 31) / 32};
+    const int tiles = keys.count(n_vis), per_split = (tiles + p.nsplit - 1) / p.nsplit;
     const int kt_first = split * per_split, kt_last = min(tiles, kt_first + per_split);
 
-    const float *k_head = p.k + b * p.kv_stride_b + kvh * p.kv_stride_h, *v_head = p.v + b * p.kv_stride_b + kvh * p.kv_stride_h;
-    const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(k_head), 0, p.kv_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(v_head), 0, p.kv_bytes, 0x00020000);
+    const Rows k_rows = rows_of(p, p.k, p.k_new, b, kvh, D), v_rows = rows_of(p, p.v, p.v_new, b, kvh, D);
     // a key set's 128 threads: features 4 c4 .. + 3 of the keys 4 (g0 + 4 i) .. + 3
     const int st = tid & 127, c4 = st % C4, g0 = st / C4;
     f32x4 kpre[NG][4], vpre[NG][4];
-    auto load_rows = [&](f32x4 (&dst)[NG][4], __amdgpu_buffer_rsrc_t rsrc, int kt) {
-        const uint32_t off = (uint32_t)(32 * kt + 4 * g0) * p.kv_row_bytes + 16 * c4;
+    auto load_rows = [&](f32x4 (&dst)[NG][4], const Rows &rows, int kt) {
+        const __amdgpu_buffer_rsrc_t rsrc = rows.rsrc(kt);
+        const uint32_t off = rows.off(kt, 4 * g0) + 16 * c4;
 #pragma unroll
         for (int i = 0; i < NG; i++)
 #pragma unroll
             for (int j = 0; j < 4; j++) dst[i][j] = buffer_f32x4(rsrc, off + (uint32_t)(16 * i + j) * p.kv_row_bytes);
     };
     int kt = kt_first + ks;
-    load_rows(kpre, k_rsrc, min(kt, tiles)), load_rows(vpre, v_rsrc, min(kt, tiles));   // (past the last tile: zeros)
+    load_rows(kpre, k_rows, min(kt, tiles)), load_rows(vpre, v_rows, min(kt, tiles));   // (past the last tile: zeros)
 
     // The append.  A workgroup copies its share of its kv head's rows (contiguous in both places), the first two 16-byte pieces of
-    // each tensor per thread beside the loads above and of q, the others after the loop; nobody waits for another's copy, K and V
-    // are read from the call's input.  1000 queries of 32 heads over 8, with an append launch | now: 57.3 | 51.8 us; 900 of 32 over
-    // 32 59.1 | 51.5.
+    // each tensor per thread beside the loads above and of q, the others after the loop; nobody waits for another's copy, the new rows
+    // of K and V are read from the call's input.  1000 queries of 32 heads over 8, with an append launch | now: 57.3 | 51.8 us; 900 of 32 over
+    // 32 59.1 | 51.5; behind a cache 2 x 3 rows of 40 heads over 2579 tokens, 64 features, 19.5 | 17.8, 373 of 32 heads over 224 49.2 | 46.7.
     const f32x4 *src_k = nullptr, *src_v = nullptr;
     f32x4 *dst_k = nullptr, *dst_v = nullptr;
     int piece = 0, pieces = 0;   // this thread's next one, and how many there are
     const int hop = p.n_rt2 * p.nsplit * kThreads;
-    if (p.k_dst) {
-        src_k = reinterpret_cast<const f32x4 *>(k_head), src_v = reinterpret_cast<const f32x4 *>(v_head);
-        dst_k = reinterpret_cast<f32x4 *>(p.k_dst + bh * p.kv_dst_stride_h), dst_v = reinterpret_cast<f32x4 *>(p.v_dst + bh * p.kv_dst_stride_h);
-        piece = rest * kThreads + tid, pieces = p.Sk * C4;
+    if (p.k_new) {
+        src_k = reinterpret_cast<const f32x4 *>(k_rows.head_new), src_v = reinterpret_cast<const f32x4 *>(v_rows.head_new);
+        dst_k = reinterpret_cast<f32x4 *>(const_cast<float *>(k_rows.head) + (int64_t)p.past * D), dst_v = reinterpret_cast<f32x4 *>(const_cast<float *>(v_rows.head) + (int64_t)p.past * D);
+        piece = rest * kThreads + tid, pieces = p.Sq * C4;
     }
     f32x4 ck[2], cv[2];
 #pragma unroll
@@ -454,7 +489,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
         auto weak = [](float x, int field) { return x > 0.0f && x * pow2_field(field) < 1.0f; };   // (below 2^-55)
         const bool weak_q = __any(weak(big, q_field));
         float v_weak = 0.0f;   // 1 / the largest of eight keys of the weakest feature that has one
-        if (32 * kt + 32 <= p.Sk && kt < kt_last) {
+        if (keys.first_key(kt) + 32 <= min(p.Sk, keys.end(kt)) && kt < kt_last) {
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 float m = 0.0f;
@@ -490,7 +525,8 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
     const float k_up = pow2_field(k_field), v_up = pow2_field(v_field);
     const int steps = odd ? 0 : (kt_last - kt_first + 1) / 2;
     for (int it = 0; it < steps; it++, kt += 2) {
-        const bool live = kt < kt_last, edge = 32 * kt + 32 > limit_first;   // edge: some row does not see all of the tile
+        const int key0 = keys.first_key(kt);
+        const bool live = kt < kt_last, edge = key0 + 32 > min(limit_first, keys.end(kt));   // edge: some row does not see all of the tile
         if (live) {
 #pragma unroll
             for (int i = 0; i < NG; i++)
@@ -504,7 +540,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
                 }
         }
         // (always, a tile again at the end: with a condition around them the wait for V below would be one for these too)
-        load_rows(kpre, k_rsrc, min(kt + 2, kt_last));
+        load_rows(kpre, k_rows, min(kt + 2, kt_last));
         __syncthreads();   // K is in LDS; every wave is done with the last V
         f32x16 s;
         if (live) {
@@ -530,14 +566,14 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
                 }
             }
         }
-        load_rows(vpre, v_rsrc, min(kt + 2, kt_last));
+        load_rows(vpre, v_rows, min(kt + 2, kt_last));
         __syncthreads();   // V is in LDS; every wave is done with K
         if (!live) continue;
 
         if (edge) {
 #pragma unroll
             for (int r = 0; r < 16; r++)
-                if (32 * kt + 8 * (r / 4) + 4 * hb + r % 4 >= limit) s[r] = -INFINITY;
+                if (key0 + 8 * (r / 4) + 4 * hb + r % 4 >= min(limit, keys.end(kt))) s[r] = -INFINITY;
         }
         float mx = s[0];
 #pragma unroll
@@ -766,12 +802,12 @@ int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
     const int64_t tiles = (a.Sk + 31) / 32, cus = num_compute_units(), want = 2 * cus, n_rt2 = (a.Sq * G + 2 * kRows - 1) / (2 * kRows);
     const bool pairs = p.n_rt > 1 && (tiles >= 5 || (tiles == 4 && 2 * p.n_bh * n_rt2 > cus)) && a.scale >= 0x1p-16f && a.scale <= 0x1p16f;
     if (pairs) p.n_rt2 = (int)n_rt2;
-    if (a.k_new) {   // a first prompt, stored to the cache by this launch
-        if (!pairs || a.Sk != a.Sq || a.kv_stride_t != a.D || a.kv_stride_b != a.Hkv * a.kv_stride_h || !a.v_new) return 2;
-        if ((uintptr_t)a.k_new % 16 || (uintptr_t)a.v_new % 16 || a.Sq > (1 << 20) || (int64_t)n_rt2 * kMaxSplits >= (1 << 18)) return 2;
-        p.k_dst = (float *)a.k, p.v_dst = (float *)a.v, p.kv_dst_stride_h = a.kv_stride_h;
-        p.k = (const float *)a.k_new, p.v = (const float *)a.v_new;
-        p.kv_stride_h = a.Sk * a.D, p.kv_stride_b = a.Hkv * p.kv_stride_h, p.kv_bytes = (uint32_t)(a.Sk * a.D * 4);
+    p.past = (int)a.Sk;
+    if (a.k_new) {   // the last Sq tokens, stored to the cache by this launch
+        if (a.kv_stride_t != a.D || a.Sk < a.Sq || !a.v_new) return 2;
+        if ((uintptr_t)a.k_new % 16 || (uintptr_t)a.v_new % 16 || a.Sq > (1 << 20) || (int64_t)p.n_rt * kMaxSplits >= (1 << 18)) return 2;
+        p.k_new = (const float *)a.k_new, p.v_new = (const float *)a.v_new;
+        p.past = (int)(a.Sk - a.Sq), p.kv_bytes = (uint32_t)p.past * p.kv_row_bytes;
     }
     const int64_t n_wb = (int64_t)p.n_bh * p.n_rt, n_wg = pairs ? (int64_t)p.n_bh * p.n_rt2 : n_wb;
     int64_t ns;
