@@ -901,7 +901,7 @@ struct KiviPrompt {
     float *v_lo, *v_scale;
     __half *k_deq, *v_deq;         // [BH, n, 128]
 };
-constexpr int kPromptMost = 8192;   // 16 waves of 8 tokens per lane
+constexpr int kPromptMost = 6144;   // 16 waves of 6 tokens per lane (8 do not fit their registers)
 
 // inclusive scans over a wave's lanes, earlier lanes first; on equal values (zeros of either sign) the earlier one
 template <int CTRL, int ROWS>
@@ -1416,8 +1416,7 @@ static int launch_kivi_prompt(const KiviPrompt &p, hipStream_t s) {
     else if (n <= 2048) kivi_prompt_kernel<8, 4><<<grid, block, 0, s>>>(p);
     else if (n <= 3072) kivi_prompt_kernel<8, 6><<<grid, block, 0, s>>>(p);
     else if (n <= 4096) kivi_prompt_kernel<8, 8><<<grid, block, 0, s>>>(p);
-    else if (n <= 6144) kivi_prompt_kernel<16, 6><<<grid, block, 0, s>>>(p);
-    else kivi_prompt_kernel<16, 8><<<grid, block, 0, s>>>(p);
+    else kivi_prompt_kernel<16, 6><<<grid, block, 0, s>>>(p);
     TROCM_HIP(hipGetLastError());
     return 0;
 }

@@ -303,7 +303,7 @@ __global__ __launch_bounds__(64 * NW * KS, BM == 32 && NW * KS >= 8 && NI == 1 ?
             __syncthreads();
             if (STEADY ? !LAST || hh + PA < 2 : 2 * t + hh + PA < 2 * Tg) prefetch_a(PA == 2 ? hh : 0, 2 * t + hh + PA);
             // asked for here, not where it is used (but in sets of two waves, 64 rows: 40 rows of 4096 x 4096 8.5 us with this, 8.2 without)
-            if constexpr (STEADY && (BM != 64 || NI * NW != 2)) __builtin_amdgcn_sched_barrier(0);
+            if constexpr (STEADY && (BM != 64 || NI * NW != 2) && (BM != 32 || KS != 8)) __builtin_amdgcn_sched_barrier(0);
             const _Float16 *at = &lds_a[hh * BM * AROW + a_frag];
             half8_t bf[2][MS];   // the activation fragments of a step are read during the step before
 #pragma unroll
