@@ -77,16 +77,16 @@ struct PrefillF32 {
     float *part_o;    // [nsplit][n_wg][32][D], not normalised
     float *part_ml;   // [nsplit][n_wg][64]: maxima, then sums
     int64_t kv_stride_b, kv_stride_h;   // elements
-    uint32_t kv_row_bytes, kv_bytes;    // bytes between token rows; bytes of one kv head's rows, from the first to the last
+    uint32_t kv_row_bytes;              // bytes between token rows
     int Hq, Hkv, Sq, Sk, G;
     int n_bh, n_rt, nsplit;             // batch * kv_heads, 32-row tiles per kv head
     int n_rt2, paired;                  // sdpa_prefill_f32x2_kernel: 64-row tiles per kv head; whether the short ones run beside the long ones
     int causal;
     float scale;
     // Fused append (dense token rows): the tokens from `past` on are read from the call's own dense rows, [B, Hkv, Sq, D], and copied to
-    // the cache by this launch; kv_bytes are then those of the tokens before.  NULL: all Sk = `past` are in the cache.
+    // the cache by this launch.  NULL: all Sk = `past` are in the cache, n_new is 0.
     const float *k_new, *v_new;
-    int past;
+    int past, n_new;
 };
 
 
@@ -118,15 +118,16 @@ struct KeyTiles {
 // The rows of one kv head of K or V: rows after the last one of a buffer read as zeros.
 struct Rows {
     const float *head, *head_new;
-    uint32_t bytes, bytes_new, row_bytes;
-    int old;
+    int past, n_new;
+    uint32_t row_bytes;
     __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(int kt) const {
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(kt < old ? head : head_new), 0, kt < old ? bytes : bytes_new, 0x00020000);
+        const bool old = 32 * kt < past;
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(old ? head : head_new), 0, (uint32_t)(old ? past : n_new) * row_bytes, 0x00020000);
     }
-    __device__ __forceinline__ uint32_t off(int kt, int row) const { return (uint32_t)(32 * (kt < old ? kt : kt - old) + row) * row_bytes; }   // row of tile kt
+    __device__ __forceinline__ uint32_t off(int kt, int row) const { return (uint32_t)(32 * (32 * kt < past ? kt : kt - (past + 31) / 32) + row) * row_bytes; }   // row of tile kt
 };
 __device__ __forceinline__ Rows rows_of(const PrefillF32 &p, const float *cache, const float *call, int b, int kvh, int D) {
-    return Rows{cache + b * p.kv_stride_b + kvh * p.kv_stride_h, call + (call ? ((int64_t)b * p.Hkv + kvh) * p.Sq * D : 0), p.kv_bytes, call ? (uint32_t)p.Sq * D * 4 : 0, p.kv_row_bytes, (p.past + 31) / 32};
+    return Rows{cache + b * p.kv_stride_b + kvh * p.kv_stride_h, call + ((int64_t)b * p.Hkv + kvh) * p.Sq * D, p.past, p.n_new, p.kv_row_bytes};
 }
 
 // the weight exp(m - ref) of a partial result whose maximum is m; nothing seen: m = -inf, weight 0 whatever ref is
@@ -338,8 +339,8 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32_kernel(PrefillF3
     const int split = rest % p.nsplit, rt = p.n_rt - 1 - rest / p.nsplit;
     const int last = min(rt * kRows + kRows, p.Sq * p.G) - 1, n_vis = p.causal ? last / p.G + (p.Sk - p.Sq) + 1 : p.Sk;
     const int per_split = (KeyTiles{p.past, (p.past + 31) / 32}.count(n_vis) + p.nsplit - 1) / p.nsplit;
-    attend_tile<D>(p, shared, bh, rt, split, split * per_split, (split + 1) * per_split);
-    // The append: this workgroup's share of its kv head's rows (contiguous in both places).  With an append launch | now: 69 rows of 32 heads
+    // The append: this workgroup's share of its kv head's rows (contiguous in both places; ahead of the attention, through which the
+    // addresses would be kept in more scalar registers than there are).  With an append launch | now: 69 rows of 32 heads
     // over 8 14.3 | 12.2 us, 10 of 14 over 2 behind 348 18.8 | 16.4.
     if (p.k_new) {
         const int64_t from = (int64_t)bh * p.Sq * D, to = (bh / p.Hkv) * p.kv_stride_b + (bh % p.Hkv) * p.kv_stride_h + (int64_t)p.past * D;
@@ -348,6 +349,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32_kernel(PrefillF3
             reinterpret_cast<f32x4 *>(const_cast<float *>(p.v) + to)[i] = reinterpret_cast<const f32x4 *>(p.v_new + from)[i];
         }
     }
+    attend_tile<D>(p, shared, bh, rt, split, split * per_split, (split + 1) * per_split);
 }
 
 // ---- more than 32 rows: every f32 as a pair of f16 ---------------------------------------------------------------------
@@ -792,7 +794,7 @@ int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
     memset(&p, 0, sizeof(p));
     p.q = (const float *)a.q, p.k = (const float *)a.k, p.v = (const float *)a.v, p.out = (float *)a.out;
     p.kv_stride_b = a.kv_stride_b, p.kv_stride_h = a.kv_stride_h;
-    p.kv_row_bytes = (uint32_t)(a.kv_stride_t * 4), p.kv_bytes = (uint32_t)(((a.Sk - 1) * a.kv_stride_t + a.D) * 4);
+    p.kv_row_bytes = (uint32_t)(a.kv_stride_t * 4);
     p.Hq = (int)a.Hq, p.Hkv = (int)a.Hkv, p.Sq = (int)a.Sq, p.Sk = (int)a.Sk, p.G = (int)G;
     p.n_bh = (int)(a.B * a.Hkv), p.n_rt = (int)((a.Sq * G + kRows - 1) / kRows);
     p.causal = a.causal, p.scale = a.scale;
@@ -807,7 +809,7 @@ int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
         if (a.kv_stride_t != a.D || a.Sk < a.Sq || !a.v_new) return 2;
         if ((uintptr_t)a.k_new % 16 || (uintptr_t)a.v_new % 16 || a.Sq > (1 << 20) || (int64_t)p.n_rt * kMaxSplits >= (1 << 18)) return 2;
         p.k_new = (const float *)a.k_new, p.v_new = (const float *)a.v_new;
-        p.past = (int)(a.Sk - a.Sq), p.kv_bytes = (uint32_t)p.past * p.kv_row_bytes;
+        p.past = (int)(a.Sk - a.Sq), p.n_new = (int)a.Sq;
     }
     const int64_t n_wb = (int64_t)p.n_bh * p.n_rt, n_wg = pairs ? (int64_t)p.n_bh * p.n_rt2 : n_wb;
     int64_t ns;
