@@ -834,8 +834,8 @@ def sdpa_decode_ragged(q: DeviceTensor, k_caches, v_caches, scale=None, workspac
     if out is None:
         out = DeviceTensor(q.shape, q.dtype)
     ws = workspace or Workspace(n, Hq, 1, D, stream)
-    ks = (C.c_void_p * n)(*[c.handle for c in k_caches])
-    vs = (C.c_void_p * n)(*[c.handle for c in v_caches])
+    ks = (C.c_void_p * n)(*[c._h for c in k_caches])
+    vs = (C.c_void_p * n)(*[c._h for c in v_caches])
     call("trocm_sdpa_decode_ragged", q.ptr, dtype_code(q.dtype), Hq, n, ks, vs, out.ptr, _scale_arg(scale),
          ws.ptr, ws.nbytes, _sh(stream))
     return out
@@ -854,8 +854,8 @@ def inplace_kv_sdpa_eval_ragged(q: DeviceTensor, k_new: DeviceTensor, v_new: Dev
     if out is None:
         out = DeviceTensor(q.shape, q.dtype)
     ws = workspace or Workspace(n, Hq, 1, D, stream)
-    ks = (C.c_void_p * n)(*[c.handle for c in k_caches])
-    vs = (C.c_void_p * n)(*[c.handle for c in v_caches])
+    ks = (C.c_void_p * n)(*[c._h for c in k_caches])
+    vs = (C.c_void_p * n)(*[c._h for c in v_caches])
     call("trocm_inplace_kv_sdpa_eval_ragged", q.ptr, k_new.ptr, v_new.ptr, dtype_code(q.dtype), Hq, n, ks, vs,
          out.ptr, _scale_arg(scale), ws.ptr, ws.nbytes, _sh(stream))
     return out
@@ -882,8 +882,8 @@ def inplace_kv_sdpa_eval_ragged_rope(q: DeviceTensor, k_new: DeviceTensor, v_new
     need = ((n * Hq * D * es + 255) & ~255) + n * k_new.shape[1] * D * es
     if rot_scratch is None:
         rot_scratch = DeviceTensor((need,), np.uint8)
-    ks = (C.c_void_p * n)(*[c.handle for c in k_caches])
-    vs = (C.c_void_p * n)(*[c.handle for c in v_caches])
+    ks = (C.c_void_p * n)(*[c._h for c in k_caches])
+    vs = (C.c_void_p * n)(*[c._h for c in v_caches])
     call("trocm_inplace_kv_sdpa_eval_ragged_rope", q.ptr, k_new.ptr, v_new.ptr, cos.ptr, sin.ptr, dtype_code(q.dtype), Hq, n, ks, vs,
          out.ptr, _scale_arg(scale), ws.ptr, ws.nbytes, rot_scratch.ptr, rot_scratch.nbytes, _sh(stream))
     return out
