@@ -100,3 +100,10 @@ def test_a_key_that_is_larger_than_all_others_together(rt, dtype, B, Hq, Hkv, D,
     want = textbook_sdpa(q, k, v, causal=True)
     tol = 2 * 2.0 ** -11 if dtype is np.float16 else 2.0 ** -20   # (as above, and as the f32 steps' own tests)
     assert np.abs(got - want).max() <= tol * np.abs(v.astype(np.float64)).max()
+
+
+# eight splits of which some have a group of tiles more than others
+@pytest.mark.parametrize("store", ["plain", "Q8_0", "Q4_0"])
+@pytest.mark.parametrize("B,Hq,Hkv,T", [(2, 32, 8, 1030), (2, 32, 8, 1500), (3, 14, 2, 2049), (2, 40, 8, 2500)])
+def test_eight_unequal_splits(rt, store, B, Hq, Hkv, T):
+    test_steps_of_any_number_of_sequence_heads(rt, store, B, Hq, Hkv, 128, T)

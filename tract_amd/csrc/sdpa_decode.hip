@@ -491,6 +491,10 @@ int choose_step_splits(int64_t BH, int64_t G, int n_tiles, int crowd16) {
     const int groups = (n_tiles + kWaves - 1) / kWaves, most = by_ws < 1 ? 1 : by_ws < groups ? (int)by_ws : groups;
     if (forced > 0) return forced < most ? forced : most;
     const int cus = num_compute_units();
+    // Of split counts of the same longest run, 8, which puts a split of every sequence-head on the same XCD: 56 drawn steps 0.99 of the
+    // time with the fewest (2 x 1500 tokens, f16 9.4 -> 9.0 us, Q4_0 8.3 -> 7.9; 2513, Q4_0, 9.0 -> 8.5), but for 8 or fewer sequence-heads of wide
+    // rows (1246 tokens of 40 heads over 8 8.8 -> 9.0).
+    const int even = BH > 8 || crowd16 != kCrowdWide ? kTailMergeMax : 0;
     int best = 1, best_cost = INT32_MAX;
     for (int ns = 1; ns <= most && (ns == 1 || (ns <= 256 && BH * ns <= 4 * cus)); ns += ns < kWideMergeMax ? 1 : ns) {
         const int longest = (groups + ns - 1) / ns, rounds = (int)((BH * ns + cus - 1) / cus);
@@ -498,9 +502,9 @@ int choose_step_splits(int64_t BH, int64_t G, int n_tiles, int crowd16) {
         if (ns > 1) cost += 24;
         if (ns > kTailMergeMax) cost += 20 + (ns % 8 ? 12 : 0) + (ns < kWideMergeMax ? ns : kWideMergeMax) - kTailMergeMax;
         if (ns > kWideMergeMax) cost += 48;
-        if (cost < best_cost) best = ns, best_cost = cost;
+        if (cost < best_cost || (cost == best_cost && ns == even)) best = ns, best_cost = cost;
     }
-    if (best > kTailMergeMax && best <= kWideMergeMax) return best;
+    if ((best > kTailMergeMax && best <= kWideMergeMax) || best == even) return best;
     const int longest = (groups + best - 1) / best;   // the same critical path with fewer records
     return (groups + longest - 1) / longest;
 }
