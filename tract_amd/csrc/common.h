@@ -146,10 +146,10 @@ int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, i
 int launch_q4_0_matmul_f32(const void *codes, const void *scales, int64_t w_batch, int64_t n, int64_t k, const void *act,
                            int64_t act_batch, int64_t m, void *out, hipStream_t s, int tiled);
 // The same for f16 activations with k shared among the waves of a workgroup (q4_matmul_waves.hip), any m and k of whole blocks;
-// returns 2 when not covered.  q4_0_matmul_waves_fits: few enough tiles for it to be the faster one from 9 rows on.
+// returns 2 when not covered.  q4_0_matmul_waves_fits: few enough tiles for it to be the faster one from 6 f16 rows on.
 int launch_q4_0_matmul_waves(const void *codes, const void *scales, int64_t w_batch, int64_t n, int64_t k, const void *act, int64_t act_batch,
                              int64_t m, void *out, hipStream_t s, int tiled);
-bool q4_0_matmul_waves_fits(int64_t n, int64_t m, int64_t act_batch);
+bool q4_0_matmul_waves_fits(int64_t n, int64_t m, int64_t act_batch, bool tiled);
 // Q4_0 weights tiled by 16 rows x 128 features (n a multiple of 16, k of 128): the layout, its inverse, and the product
 // with m rows of f16 or f32 activations (q4_tiled.hip).
 bool q4_0_tiled_layout_fits(int64_t n, int64_t k);

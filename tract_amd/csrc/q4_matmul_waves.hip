@@ -225,11 +225,12 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_waves_kernel(MatMulWav
 
 struct Shape { int ms, ni; float tiled, first, later; };
 // us of a round of workgroups, one per compute unit: tiles at 4096 features when there are several rounds; planes at 2080 features, the first
-// and later ones.  32 x 16, 48 x 32 and 64 x 32 are for planes, whose codes come in words of 4 bytes, so that a weight row costs more there:
+// and later ones.  16 x 64 is for tiles where it saves a second round.  32 x 16, 48 x 32 and 64 x 32 are for planes, whose codes come in words of 4 bytes, so that a weight row costs more there:
 // 100 rows of 1000 x 2080 10.9 (16 x 32) -> 9.3 (32 x 16), 300 19.7 (32 x 64) -> 14.5 (48 x 32), 500 19.9 -> 15.4 (64 x 32).
 constexpr float kNever = 1e9f;
 constexpr Shape kShapes[] = {{1, 1, 5.0f, 7.3f, 5.0f},    {1, 2, 6.0f, 10.6f, 8.5f},    {2, 2, 10.0f, 12.4f, 10.5f},  {2, 4, 13.0f, kNever, kNever},
-                             {4, 4, 20.0f, 23.0f, 20.0f}, {2, 1, kNever, 9.2f, 6.7f},   {3, 2, kNever, 14.5f, 12.5f}, {4, 2, kNever, 15.2f, 14.0f}};
+                             {4, 4, 20.0f, 23.0f, 20.0f}, {2, 1, kNever, 9.2f, 6.7f},   {3, 2, kNever, 14.5f, 12.5f}, {4, 2, kNever, 15.2f, 14.0f},
+                             {1, 4, 9.0f, kNever, kNever}};
 int64_t workgroups(const Shape &c, int64_t n, int64_t m, int64_t act_batch) {
     return (n + 16 * c.ni - 1) / (16 * c.ni) * ((m + 16 * c.ms - 1) / (16 * c.ms)) * act_batch;
 }
@@ -239,7 +240,13 @@ int64_t workgroups(const Shape &c, int64_t n, int64_t m, int64_t act_batch) {
 // Whether a product has so few tiles that this kernel's smallest shapes need no more than a workgroup per compute unit (us,
 // q4_matmul.hip | here; inside the line: 128 rows of 1024 x 4096 12.9 | 8.8, 32 of 4096 x 4096 9.3 | 8.7; outside: 64 of
 // 4096 x 4096 13.1 | 12.9, 200 of 1024 x 4096 13.2 | 13.1, 32 of 14336 x 4096 14.1 | 15.0).
-bool q4_0_matmul_waves_fits(int64_t n, int64_t m, int64_t act_batch) { return workgroups(kShapes[1], n, m, act_batch) <= num_compute_units(); }
+// Tiles, up to 16 rows: also those of 16 x 64 (us, q4_tiled.hip | here: 9 rows of 14336 x 4096 10.8 | 10.1, 16 rows 11.7 | 10.8, of 9216 x 5120
+// 21.2 | 11.5, of 14336 x 8192 22.9 | 18.6; 8 rows of 12288 x 4096 11.3 | 9.7, 10240 x 4096 11.2 | 9.2, 14336 x 4096 10.4 | 10.2, x 8192
+// 16.7 | 17.2).
+bool q4_0_matmul_waves_fits(int64_t n, int64_t m, int64_t act_batch, bool tiled) {
+    const int64_t cus = num_compute_units();
+    return workgroups(kShapes[1], n, m, act_batch) <= cus || (tiled && m <= 16 && workgroups(kShapes[8], n, m, act_batch) <= (m > 8 ? cus : 3 * cus / 4));
+}
 
 // 2 = not taken: operands beyond 32-bit offsets, misaligned ones.
 int launch_q4_0_matmul_waves(const void *codes, const void *scales, int64_t w_batch, int64_t n, int64_t k, const void *act, int64_t act_batch,
@@ -257,7 +264,7 @@ int launch_q4_0_matmul_waves(const void *codes, const void *scales, int64_t w_ba
     // 8.3 | 5.0).
     int best = 0;
     float best_us = 0.0f;
-    for (int c = 0; c < 8; c++) {
+    for (int c = 0; c < 9; c++) {
         const Shape &x = kShapes[c];
         const float rounds = (float)((workgroups(x, n, m, act_batch) + num_compute_units() - 1) / num_compute_units());
         const float us = tiled ? rounds * x.tiled : x.first + (rounds - 1.0f) * x.later;
@@ -267,7 +274,7 @@ int launch_q4_0_matmul_waves(const void *codes, const void *scales, int64_t w_ba
         constexpr int MS = decltype(ms)::value, NI = decltype(ni)::value, DB = MS < 4 ? 4 : 2;
         const dim3 grid((unsigned)((n + 16 * NI - 1) / (16 * NI)), (unsigned)((m + 16 * MS - 1) / (16 * MS)), (unsigned)act_batch);
         if (grid.y > 65535) return 2;
-        constexpr bool TILES = !(NI == 1 && MS == 2) && !(NI == 2 && MS > 2), PLANES = !(MS == 2 && NI == 4);   // (the other's never chosen)
+        constexpr bool TILES = !(NI == 1 && MS == 2) && !(NI == 2 && MS > 2), PLANES = !(MS <= 2 && NI == 4);   // (the other's never chosen)
         if constexpr (TILES)
             if (tiled) hipLaunchKernelGGL((q4_0_matmul_waves_kernel<MS, NI, DB, true>), grid, dim3(64 * kW), 0, s, p);
         if constexpr (PLANES)
@@ -288,7 +295,8 @@ int launch_q4_0_matmul_waves(const void *codes, const void *scales, int64_t w_ba
         case 4: return go(I4(), I4());
         case 5: return go(I2(), I1());
         case 6: return go(I3(), I2());
-        default: return go(I4(), I2());
+        case 7: return go(I4(), I2());
+        default: return go(I1(), I4());
     }
 }
 

@@ -275,7 +275,7 @@ int launch_q4_0_matvec(const void *codes, const void *scales, int64_t w_batch, i
         if (rc != 2) return rc;
     }
     // the matrix-matrix arms for f16 activations: k shared among waves for few tiles and for a k that q4_matmul.hip does not take
-    if (m > 8 && act_dtype == TROCM_F16 && (k % 64 || q4_0_matmul_waves_fits(n, m, act_batch))) {
+    if (m > 8 && act_dtype == TROCM_F16 && (k % 64 || q4_0_matmul_waves_fits(n, m, act_batch, false))) {
         const int rc = launch_q4_0_matmul_waves(codes, scales, w_batch, n, k, act, act_batch, m, out, s, 0);
         if (rc != 2) return rc;
     }

@@ -540,7 +540,7 @@ int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int6
     // 6 f16 rows and more with few tiles (us, the kernel above | there: 5 rows of 4096 x 14336 11.5 | 11.9, of 1024 x 14336 10.9 | 11.4; 6 rows
     // 14.4 | 12.2, 13.4 | 11.9, of 5120 x 5120 8.7 | 7.0, of 8192 x 8192 11.5 | 10.7, of 4096 x 4096 5.6 | 5.4; 8 rows of 4096 x 14336 15.3 |
     // 12.7, of 1024 x 4096 5.4 | 5.5; 16 rows 23.1 | 18.3, of 4096 x 4096 8.3 | 8.0)
-    if (act_dtype == TROCM_F16 && m >= 6 && q4_0_matmul_waves_fits(n, m, act_batch)) {
+    if (act_dtype == TROCM_F16 && m >= 6 && q4_0_matmul_waves_fits(n, m, act_batch, true)) {
         const int rc = launch_q4_0_matmul_waves(tiles, nullptr, w_batch, n, k, act, act_batch, m, out, s, 1);
         if (rc != 2) return rc;
     }
