@@ -146,3 +146,22 @@ def test_no_kernel_spills_registers():
     for name, v in usage.items():
         if "sdpa_prefill_pp_kernel" in name:
             assert v["Occupancy [waves/SIMD]"] >= 2, (name, v)
+
+
+def test_prompts_of_a_workgroup_per_unit_need_a_steps_workspace():
+    """From 256 workgroups of a prompt on no scratch is asked for beyond what a decode step of the same heads has, so that these prompts also
+    fit the static scratch of trocm_sdpa_cached_noalloc, whose header refuses what asks for more."""
+    import ctypes as C
+
+    from tract_amd import _lib
+    lib = _lib.load()
+    static = int(re.search(r"TROCM_STATIC_SCRATCH_BYTES \((\d+)u << 20\)", open(os.path.join(ROOT, "include", "tract_rocm.h")).read()).group(1)) << 20
+
+    def need(*shape):
+        n = C.c_size_t()
+        assert lib.trocm_sdpa_workspace_bytes(*shape, C.byref(n)) == 0
+        return n.value
+
+    for batch, heads, queries in ((1, 32, 2048), (3, 32, 900), (2, 32, 2048), (1, 40, 1664), (1, 384, 192), (4, 32, 2048), (8, 64, 4096)):
+        for dim in (64, 128):
+            assert need(batch, heads, queries, dim) == need(batch, heads, 1, dim) <= static

@@ -138,9 +138,13 @@ def test_what_only_the_smaller_kernel_takes(rt, what, B, Hq, Hkv, D, past, n):
 
 # more query tiles than whole rounds of compute units take: those left over are cut into 2, 3 and 4 ranges of keys (one head of a
 # group of one, a group of two and of four per workgroup; causal behind past tokens or unmasked; the last tile with few queries)
+CUT = [(1, 384, 96, 1100, 130, True, 96, 2), (2, 160, 40, 900, 220, False, 80, 2), (1, 128, 64, 1300, 613, True, 64, 3), (2, 60, 60, 1300, 530, False, 120, 2),
+       (1, 168, 42, 1000, 400, True, 42, 4)]
+
+
 @pytest.mark.parametrize("store", [None, ta.Q8_0, ta.Q4_0])
-@pytest.mark.parametrize("B,Hq,Hkv,past,n,causal", [(1, 384, 96, 1100, 130, True), (2, 160, 40, 900, 220, False), (1, 128, 64, 1300, 613, True), (2, 60, 60, 1300, 530, False)])
-def test_tiles_left_for_the_last_round(rt, store, B, Hq, Hkv, past, n, causal):
+@pytest.mark.parametrize("B,Hq,Hkv,past,n,causal,left,parts", CUT)
+def test_tiles_left_for_the_last_round(rt, store, B, Hq, Hkv, past, n, causal, left, parts):
     rng = np.random.default_rng(n)
     T, G = past + n, Hq // Hkv
     q, k, v = _normal(rng, B, Hq, n, 128), _normal(rng, B, Hkv, T, 128), _normal(rng, B, Hkv, T, 128)
@@ -151,10 +155,16 @@ def test_tiles_left_for_the_last_round(rt, store, B, Hq, Hkv, past, n, causal):
     dq, out = ta.DeviceTensor.from_numpy(q), ta.DeviceTensor(q.shape, np.float16)
     ws = ta.Workspace(B, Hq, n, 128)
     results = []
+    call("trocm_memset", C.c_void_p(ws.ptr.value + 64 * 1024), 0xA5, ws.nbytes - 64 * 1024, None)
     for size in (64 * 1024, ws.nbytes, ws.nbytes):   # whole; cut; the same bits again
         call("trocm_sdpa_cached", dq.ptr, ta.F16, Hq, n, kc._h, vc._h, out.ptr, C.c_float(float("nan")), int(causal), ws.ptr, size, None)
         results.append(out.to_numpy())
     assert results[1].tobytes() == results[2].tobytes()
+    # all but one part of a tile have been stored, 8 waves' 32 x 128 sums each: the first of every tile's places, and none behind the last
+    kept = ws.buf.to_numpy()[64 * 1024 :][: 16 * 1024 * 8 * left * (parts - 1)].reshape(parts - 1, left, 8, 16 * 1024)
+    assert (kept[:, :, 0] != 0xA5).any(axis=-1).all()
+    behind = ws.buf.to_numpy()[64 * 1024 + (parts - 1) * left * 8 * (16 * 1024 + 256) :]
+    assert behind.size and (behind == 0xA5).all()
     infinite = np.zeros(q.shape, bool)
     if store is None:
         infinite[0, G : 2 * G, :, 9] = True

@@ -49,10 +49,12 @@ PAIRS = [
     [(ta.Q8_0, np.float16, 4, 32, 8, 1, 4096, 128, True), (ta.Q4_0, np.float16, 1, 32, 8, 1, 1000, 128, True)],
     # prefill with the key range split over workgroups (f16 partials in the scratch), then a short one
     [(None, np.float16, 1, 32, 8, 256, 2048, 128, True), (None, np.float16, 1, 8, 2, 64, 192, 64, True)],
+    # 120 and 80 query tiles left for a last round, cut into two ranges of keys
+    [(None, np.float16, 3, 32, 8, 900, 2900, 128, True), (ta.Q8_0, np.float16, 2, 160, 40, 220, 1120, 128, False)],
 ]
 
 
-@pytest.mark.parametrize("pair", PAIRS, ids=["decode_f16", "decode_g16_then_f32", "decode_quant", "prefill"])
+@pytest.mark.parametrize("pair", PAIRS, ids=["decode_f16", "decode_g16_then_f32", "decode_quant", "prefill", "prefill_last_round"])
 def test_noalloc_matches_the_workspace_entry_point(rt, pair):
     rng = np.random.default_rng(77)
     stream = Stream()

@@ -1152,17 +1152,12 @@ int trocm_rotate_half(const void *input, void *out, int dtype, int rank, const i
 }
 
 // ---- attention -----------------------------------------------------------------------------------
-// least: what the static scratch has to hold, without what only makes launches that fill the chip faster
-static size_t sdpa_scratch(int64_t batch, int64_t q_heads, int64_t q_len, int64_t head_dim, bool least) {
-    const size_t need = decode_workspace_bytes(batch, q_heads, head_dim);
-    const size_t prefill = kWsCounterBytes + prefill_workspace_bytes(batch, q_heads, q_len, head_dim, least);
-    return need > prefill ? need : prefill;
-}
-
 int trocm_sdpa_workspace_bytes(int64_t batch, int64_t q_heads, int64_t q_len, int64_t head_dim, size_t *bytes) {
     TROCM_NOT_NULL(bytes);
     TROCM_REQUIRE(batch >= 0 && q_heads >= 0 && q_len >= 0 && head_dim >= 0, "workspace_bytes: negative dimension");
-    *bytes = sdpa_scratch(batch, q_heads, q_len, head_dim, false);
+    size_t need = decode_workspace_bytes(batch, q_heads, head_dim);
+    size_t prefill = kWsCounterBytes + prefill_workspace_bytes(batch, q_heads, q_len, head_dim);
+    *bytes = need > prefill ? need : prefill;
     return 0;
 }
 
@@ -1283,7 +1278,8 @@ int trocm_sdpa_cached_noalloc(const void *q, int q_dtype, int64_t q_heads, int64
     TROCM_REQUIRE(stream != nullptr, "sdpa_cached_noalloc: a stream is required (the library's per-thread stream would be created here)");
     if (sdpa_cached_check(q, q_dtype, q_heads, kc, vc, out)) return 1;
     TROCM_REQUIRE(q_len >= 0, "sdpa: negative dimension");
-    const size_t need = sdpa_scratch(kc->B, q_heads, q_len, kc->D, true);
+    size_t need = 0;
+    if (trocm_sdpa_workspace_bytes(kc->B, q_heads, q_len, kc->D, &need)) return 1;
     TROCM_REQUIRE(need <= (size_t)TROCM_STATIC_SCRATCH_BYTES,
                   "sdpa_cached_noalloc: batch %lld x %lld query heads x %lld queries at head_dim %lld asks for %zu bytes of split-K "
                   "scratch, the static buffer holds %zu; call trocm_sdpa_cached with a workspace of that size instead",

@@ -228,7 +228,7 @@ bool sdpa_decode_rows_fits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64
 int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s);
 // The same for f32 q, K and V (2..: any number of queries), on the f32 matrix instruction.  Returns 2 when not covered.
 int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s);
-size_t prefill_workspace_bytes(int64_t B, int64_t Hq, int64_t Sq, int64_t D, bool least);
+size_t prefill_workspace_bytes(int64_t B, int64_t Hq, int64_t Sq, int64_t D);
 
 // Ragged decode: per-sequence descriptors live in pinned host memory owned by the library.
 struct RaggedSeq {

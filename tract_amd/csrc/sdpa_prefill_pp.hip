@@ -80,8 +80,8 @@ struct PrefillPP {
     // [B, Hkv, Sq, D], and stored to the cache (dense token rows) by this launch; NULL: all tokens are in the cache.
     const _Float16 *k_new, *v_new;
     int new_from;       // first token that is read from them (INT_MAX: none)
-    // PARTS (choose_parts): so many query tiles, from the last on down, have a workgroup each, the others `nsplit`; partials in f32,
-    // merged by the last range of a tile to arrive.
+    // PARTS (choose_parts): so many query tiles, from the last on down, have a workgroup each, the others `nsplit`, merged by the last of
+    // a tile's to arrive from its own and the others' stored results, in f32.
     int whole;
 };
 
@@ -755,76 +755,111 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
             wave_sync();   // ... and are done reading before the second half overwrites it
         }
     };
-    // ---- a tile in a few parts of its own (PARTS): f32 partials, out = sum_s w_s O_s over the parts in their order by the last to
-    // arrive, its own from the registers.  Pieces of 8 bytes, so that a store covers 512 consecutive ones; written through to memory.
+    // ---- a tile in a few parts of its own (PARTS): out = sum_s w_s O_s over the parts in their order, O_s f32 and normalised, by the last
+    // to arrive, whose own part never leaves its registers: the others, a part per place, store theirs and then say so.  The last waits
+    // for that; they have arrived, so all that is left for them to do is to store.  Two parts of a tile take one place: the
+    // 120 tiles of 3 x 900 queries of 32 heads over 8 behind 2000 tokens 16 MB, not 32, which every workspace has (a decode step's).
+    // A tile's counter: how many have arrived (bits 0 to 7) and stored (8 to 15), and which part the one of place i is (two bits from
+    // 16 + 2 i on).  Stores in pieces of 8 bytes, so that each covers 512 consecutive ones; written through to memory.
     auto merge_parts = [&]() __attribute__((always_inline)) {
         const int64_t per_q = (int64_t)p.B * p.Hkv * (G / HG), n_tiles = per_q * (p.n_qtiles - p.whole), tile = qt * per_q + ((int64_t)b * (G / HG) + gg) * p.Hkv + kvh;
-        auto block = [&](int sp) { return ((int64_t)sp * n_tiles + tile) * kWavesPP + w; };
+        auto block = [&](int place) { return ((int64_t)place * n_tiles + tile) * kWavesPP + w; };
         float *part_o = reinterpret_cast<float *>(p.part_o) + lane * 2;
+        int *counter = p.counters + tile;
+        __shared__ int s_word;
+        __syncthreads();   // (every wave is past the tile loop, whose V buffers the output goes through)
+        if (tid == 0) s_word = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 255;
+        __syncthreads();
+        const int place = __builtin_amdgcn_readfirstlane(s_word);
         const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
-        if (wave_has_queries) {
-            float *po = part_o + block(split) * (32 * D);
 #pragma unroll
-            for (int db = 0; db < DB; db++)
+        for (int db = 0; db < DB; db++)
 #pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    typedef float float2_v __attribute__((ext_vector_type(2)));
-                    o[db][2 * i] *= inv, o[db][2 * i + 1] *= inv;
-                    const float2_v x = {o[db][2 * i], o[db][2 * i + 1]};
-                    __hip_atomic_store(reinterpret_cast<uint64_t *>(po + (db * 8 + i) * 128), __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-            __hip_atomic_store(p.part_ml + block(split) * 64 + lane, hb ? l_run : m_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int r = 0; r < 16; r++) o[db][r] *= inv;
+        if (place < nsplit - 1) {
+            if (wave_has_queries) {
+                float *po = part_o + block(place) * (32 * D);
+#pragma unroll
+                for (int db = 0; db < DB; db++)
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        typedef float float2_v __attribute__((ext_vector_type(2)));
+                        const float2_v x = {o[db][2 * i], o[db][2 * i + 1]};
+                        __hip_atomic_store(reinterpret_cast<uint64_t *>(po + (db * 8 + i) * 128), __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                __hip_atomic_store(p.part_ml + block(place) * 64 + lane, hb ? l_run : m_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this thread's stores have completed
+            __syncthreads();                                     // ... and so have the whole workgroup's
+            if (tid == 0) __hip_atomic_fetch_add(counter, (1 << 8) + (split << (16 + 2 * place)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this thread's stores have completed
-        __syncthreads();                                     // ... and so have the whole workgroup's
-        __shared__ int s_arrived;
+        __syncthreads();   // (s_word has been read)
         if (tid == 0) {
-            int *counter = p.counters + tile;
-            const int arrived = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (arrived == nsplit - 1) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
-            s_arrived = arrived;
+            int word;
+            while ((((word = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 8) & 255) != nsplit - 1) __builtin_amdgcn_s_sleep(1);
+            __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
+            s_word = word;
         }
         __syncthreads();
-        if (s_arrived != nsplit - 1 || !wave_has_queries) return;
-        float wv[kTailSplits], total = 0.0f, mm = -INFINITY;   // the weights, by every lane from the same records
+        if (!wave_has_queries) return;
+        const int word = __builtin_amdgcn_readfirstlane(s_word);
+        // the other parts in their order: the places they stored to
+        int place_of[kTailSplits - 1];
 #pragma unroll
-        for (int sp = 0; sp < kTailSplits; sp++) {
-            const float *ml = p.part_ml + block(min(sp, nsplit - 1)) * 64 + l32;
-            const float m = __hip_atomic_load(ml, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), l = __hip_atomic_load(ml + 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const float top = fmaxf(mm, m), ref = top == -INFINITY ? 0.0f : top, keep = fast_exp2(mm - ref);
-            wv[sp] = sp < nsplit ? l * fast_exp2(m - ref) : 0.0f;
+        for (int j = 0; j < kTailSplits - 1; j++) {
+            const int sp = j + (j >= split);   // (past the last part: whatever was found first, weighed 0)
+            place_of[j] = 0;
 #pragma unroll
-            for (int i = 0; i < sp; i++) wv[i] *= keep;
-            total = total * keep + wv[sp], mm = top;
+            for (int i = 0; i < kTailSplits - 1; i++)
+                if (i < nsplit - 1 && ((word >> (16 + 2 * i)) & 3) == sp) place_of[j] = i;
         }
+        // The weights, by every lane from the same records (both halves of a wave hold a query's own).
+        float m_part[kTailSplits - 1], w_part[kTailSplits - 1], mm = m_run;
+#pragma unroll
+        for (int j = 0; j < kTailSplits - 1; j++) {
+            const float *ml = p.part_ml + block(place_of[j]) * 64 + l32;
+            m_part[j] = __hip_atomic_load(ml, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), w_part[j] = __hip_atomic_load(ml + 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            mm = fmaxf(mm, m_part[j]);
+        }
+        const float ref = mm == -INFINITY ? 0.0f : mm;
+        float w_own = l_run * fast_exp2(m_run - ref), total = 0.0f;
+#pragma unroll
+        for (int j = 0; j < kTailSplits - 1; j++) {
+            if (j == split) total += w_own;
+            w_part[j] *= fast_exp2(m_part[j] - ref);
+            if (j < nsplit - 1) total += w_part[j];
+        }
+        if (split == kTailSplits - 1) total += w_own;
         const float inv_total = total > 0.0f ? 1.0f / total : 0.0f;
+        w_own *= inv_total;
 #pragma unroll
-        for (int d2 = 0; d2 < DB; d2 += 2) {   // every part's two feature blocks in one trip, the own one's too (kept beside the others it spills)
-            uint64_t raw[kTailSplits][2][8];
+        for (int db = 0; db < DB; db++) {   // a feature block of the other parts in one trip (two of them spill)
+            uint64_t raw[kTailSplits - 1][8];
 #pragma unroll
-            for (int sp = 0; sp < kTailSplits; sp++) {
-                if (sp >= nsplit) break;
-                const float *po = part_o + block(sp) * (32 * D) + d2 * 1024;
+            for (int j = 0; j < kTailSplits - 1; j++) {
+                if (j >= nsplit - 1) break;
+                const float *po = part_o + block(place_of[j]) * (32 * D) + db * 1024;
 #pragma unroll
-                for (int db = 0; db < 2; db++)
-#pragma unroll
-                    for (int i = 0; i < 8; i++)
-                        raw[sp][db][i] = __hip_atomic_load(reinterpret_cast<const uint64_t *>(po + (db * 8 + i) * 128), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (int i = 0; i < 8; i++) raw[j][i] = __hip_atomic_load(reinterpret_cast<const uint64_t *>(po + i * 128), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
+            float16_t sum;
 #pragma unroll
-            for (int db = 0; db < 2; db++)
+            for (int r = 0; r < 16; r++) sum[r] = 0.0f;
+            auto add_own = [&]() __attribute__((always_inline)) {
 #pragma unroll
-                for (int r = 0; r < 16; r++) o[d2 + db][r] = 0.0f;
+                for (int r = 0; r < 16; r++) sum[r] = __builtin_fmaf(w_own, o[db][r], sum[r]);
+            };
 #pragma unroll
-            for (int sp = 0; sp < kTailSplits; sp++) {
-                if (sp >= nsplit) break;
-                const float wgt = wv[sp] * inv_total;
+            for (int j = 0; j < kTailSplits - 1; j++) {
+                if (j == split) add_own();
+                if (j >= nsplit - 1) break;
+                const float wgt = w_part[j] * inv_total;
 #pragma unroll
-                for (int db = 0; db < 2; db++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++)
-                        o[d2 + db][r] = __builtin_fmaf(wgt, __builtin_bit_cast(float, (uint32_t)(raw[sp][db][r / 2] >> (32 * (r % 2)))), o[d2 + db][r]);
+                for (int r = 0; r < 16; r++) sum[r] = __builtin_fmaf(wgt, __builtin_bit_cast(float, (uint32_t)(raw[j][r / 2] >> (32 * (r % 2)))), sum[r]);
             }
+            if (split == kTailSplits - 1) add_own();
+            o[db] = sum;
         }
         write_output(1.0f);
     };
@@ -1093,6 +1128,9 @@ int64_t choose_splits(const PrefillPP &p, int D, int block_m, int64_t wgs1, int6
 // tokens 3 x 900 after 2000 152 -> 142, 2 x 1400 after 3000 214 -> 194, 64 over 8, 1300 after 4000 261 -> 224.)  Causal prompts
 // behind little, whose longest tile takes longer than all of them spread over the units, lose what they gain: 2048 queries 63 -> 67,
 // 2 x 1500 55 -> 64 with all tiles longer than that share cut in two.
+// All but one of a tile's parts are stored (merge_parts): at most kCutPlaces of them, which a decode step's workspace of the same heads
+// holds, so that no workspace is larger for the cut and the scratch of trocm_sdpa_cached_noalloc is large enough too.
+constexpr int64_t kCutPlaces = 128;
 int choose_parts(const PrefillPP &p, int block_m, int64_t per_q, int64_t cus, int &whole) {
     const int64_t wgs1 = per_q * p.n_qtiles;
     if (wgs1 < cus || wgs1 >= 4 * cus) return 1;
@@ -1100,7 +1138,8 @@ int choose_parts(const PrefillPP &p, int block_m, int64_t per_q, int64_t cus, in
     if (2 * tiles_of(0) < tiles_of(p.n_qtiles - 1)) return 1;
     whole = (int)(wgs1 / cus * cus / per_q);
     const int64_t left = (p.n_qtiles - whole) * per_q;
-    const int parts = left > 0 ? (int)min((int64_t)kTailSplits, cus / left) : 1;
+    int parts = left > 0 ? (int)min((int64_t)kTailSplits, cus / left) : 1;
+    if (parts > 1) parts = (int)min((int64_t)parts, 1 + kCutPlaces / left);
     return parts > 1 && 1.8f * (float)tiles_of(p.n_qtiles - whole - 1) * (1.0f - 1.0f / (float)parts) >= 16.0f ? parts : 1;
 }
 
@@ -1160,12 +1199,12 @@ int launch_hg(const PrefillPP &p, int fmt, int hg, int64_t wgs, bool alone, hipS
 static size_t split_bytes(int64_t n_wb, int64_t D, size_t elem = sizeof(_Float16)) { return (size_t)n_wb * (32 * (size_t)D * elem + 64 * sizeof(float)); }
 
 // Upper bound of the partial-result area the staggered prefill kernel may use for this shape.
-// least: without what only makes launches of a workgroup per compute unit and more faster (choose_parts).
-size_t prefill_workspace_bytes(int64_t B, int64_t Hq, int64_t Sq, int64_t D, bool least) {
+// (The parts of a last round that is cut, choose_parts, have room in a decode step's.)
+size_t prefill_workspace_bytes(int64_t B, int64_t Hq, int64_t Sq, int64_t D) {
     if (Sq < 2 || (D != 64 && D != 128)) return 0;
     const int64_t wgs1 = B * ((Hq + 3) / 4) * ((Sq + 63) / 64);  // about the fewest workgroups any head grouping gives
     const int64_t cus = 256;
-    if (wgs1 >= cus) return !least && D == 128 && wgs1 < 5 * cus ? (size_t)cus * kWavesPP * (32 * 128 + 64) * sizeof(float) + 256 : 0;   // a part for each unit
+    if (wgs1 >= cus) return 0;
     int64_t ns = (cus + wgs1 - 1) / wgs1;
     if (ns > kMaxSplits) ns = kMaxSplits;
     return (size_t)ns * split_bytes(B * Hq * ((Sq + 31) / 32), D) + 256;
@@ -1268,8 +1307,8 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
         const int64_t per_q = wgs1 / n_qtiles;
         int whole = 0;
         const int parts = choose_parts(p, block_m, per_q, cus, whole);
-        const int64_t tiles = (n_qtiles - whole) * per_q, blocks = tiles * parts * kWavesPP;
-        if (parts > 1 && (size_t)blocks * (32 * 128 + 64) * sizeof(float) <= avail && tiles <= (int64_t)(kWsCounterBytes / sizeof(int))) {
+        const int64_t tiles = (n_qtiles - whole) * per_q, blocks = tiles * (parts - 1) * kWavesPP;
+        if (parts > 1 && (size_t)blocks * split_bytes(1, 128, sizeof(float)) <= avail) {
             char *base = (char *)a.workspace + kWsCounterBytes;
             base += (256 - ((uintptr_t)base & 255)) & 255;
             p.part_o = (_Float16 *)base;
