@@ -96,3 +96,21 @@ def test_f32_rows_behind_a_cache(rt, B, Hq, Hkv, D, past, n, causal):
         # as many f32 roundings as additions stand one after the other, of a mean of values of about 1; measured 2e-7 of the norm
         assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
         assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max()
+
+
+# the call's rows begin a tile of keys of their own: 21 and 61 tiles for 620 and 1915 tokens, in 6 and 16 ranges of four, one for each wave (in 5
+# and 15 ranges one wave would take two); 45 tiles of 24 kv heads in 9 ranges of five (12 of four would be more workgroups than compute units)
+@pytest.mark.parametrize("B,Hq,Hkv,past,n,ranges", [(2, 32, 8, 618, 2, 6), (1, 32, 8, 1910, 5, 16), (3, 64, 8, 1405, 4, 9)])
+def test_f32_ranges_count_the_tile_that_is_not_full(rt, B, Hq, Hkv, past, n, ranges):
+    q, k, v = _inputs(np.float32, B, Hq, Hkv, 128, past, n)
+    st = _state(k, v, past, n, True)
+    new = [ta.DeviceTensor.from_numpy(np.ascontiguousarray(x)) for x in (q, k[:, :, past:], v[:, :, past:])]
+    st.eval_into(*new)   # (makes the state's workspace)
+    st.k.truncate(past), st.v.truncate(past)
+    call("trocm_memset", C.c_void_p(st._ws.ptr.value + 64 * 1024), 0xA5, st._ws.nbytes - 64 * 1024, None)
+    got = st.eval_into(*new).to_numpy()
+    kept = st._ws.buf.to_numpy()[64 * 1024 :]
+    stored = ranges * B * Hkv * (32 * 128 + 64) * 4   # a range's results of up to 32 rows per kv head, their maxima and sums
+    assert (kept[:stored].reshape(-1, 256) != 0xA5).any(axis=-1).all() and (kept[stored:] == 0xA5).all()
+    want = textbook_sdpa(q, k, v, causal=True)
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)   # (as above)

@@ -811,13 +811,23 @@ int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
         p.k_new = (const float *)a.k_new, p.v_new = (const float *)a.v_new;
         p.past = (int)(a.Sk - a.Sq), p.n_new = (int)a.Sq;
     }
+    // (as the launch counts them: the call's rows begin a tile of their own)
+    const int64_t cut_tiles = (p.past + 31) / 32 + (p.n_new + 31) / 32;
     const int64_t n_wb = (int64_t)p.n_bh * p.n_rt, n_wg = pairs ? (int64_t)p.n_bh * p.n_rt2 : n_wb;
     int64_t ns;
     if (pairs) {
-        ns = n_wg < want ? choose_pair_splits(p, (int)a.D, tiles, n_wg, cus) : 1;
-    } else {   // ranges of at least 4 tiles
-        ns = n_wg < want ? (want + n_wg - 1) / n_wg : 1;
-        ns = ns < tiles / 4 ? ns : tiles / 4;
+        ns = n_wg < want ? choose_pair_splits(p, (int)a.D, cut_tiles, n_wg, cus) : 1;
+    } else {
+        // Ranges of four tiles, one for each wave, where all of them are at work at once or there are few; otherwise the next longer ones.
+        // (A call with its append, us, ranges of five | of four: 2 x 32 heads over 8, 2 queries behind 618 tokens 19.7 | 15.2, 1 x 5 behind
+        // 1910 21.4 | 17.0, 4 x 32 over 32, 6 behind 395 27.1 | 24.0; of four, more than a workgroup per unit, | of five: 3 x 64 over 8, 4 behind
+        // 1405 24.8 | 22.8; a merge for two ranges | none: 6 x 4 over 184 tokens of 64 features 10.9 | 10.3.)
+        auto not_empty = [&](int64_t n) {
+            const int64_t longest = (cut_tiles + n - 1) / n;
+            return (cut_tiles + longest - 1) / longest;
+        };
+        const int64_t most = n_wg < want ? (want + n_wg - 1) / n_wg : 1, fours = cut_tiles < 8 ? 1 : (cut_tiles + 3) / 4;
+        ns = not_empty(std::min(most, n_wg * fours <= cus || (fours <= 4 && n_wg * fours <= want) ? fours : cut_tiles / 4));
     }
     ns = ns < kMaxSplits ? ns : kMaxSplits;
     p.paired = pairs && a.causal && n_wg <= want;
