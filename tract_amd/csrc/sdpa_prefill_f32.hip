@@ -108,26 +108,30 @@ __device__ __forceinline__ uint32_t finite_mask(float x) {
 }
 __device__ __forceinline__ float masked(float x, uint32_t mask) { return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & mask); }
 
-// Tiles of 32 keys: those of the cache, the last of them with fewer rows, then those of the call's rows.
+// Tiles of 32 keys: those of the cache, the last of them with fewer rows, then those of the call's rows.  NEW: the launch has such rows (what
+// picks between the two costs calls over a cache alone 1.4 % on average and 4 % of the shortest).
+template <bool NEW>
 struct KeyTiles {
     int past, old;   // tokens and tiles in the cache
-    __device__ __forceinline__ int first_key(int kt) const { return kt < old ? 32 * kt : past + 32 * (kt - old); }
-    __device__ __forceinline__ int end(int kt) const { return kt < old ? min(32 * kt + 32, past) : INT_MAX; }   // keys from here on are not its own
-    __device__ __forceinline__ int count(int n_vis) const { return n_vis <= past ? (n_vis + 31) / 32 : old + (n_vis - past + 31) / 32; }
+    __device__ __forceinline__ int first_key(int kt) const { return !NEW || kt < old ? 32 * kt : past + 32 * (kt - old); }
+    __device__ __forceinline__ int end(int kt) const { return NEW && kt < old ? min(32 * kt + 32, past) : INT_MAX; }   // keys from here on are not its own
+    __device__ __forceinline__ int count(int n_vis) const { return !NEW || n_vis <= past ? (n_vis + 31) / 32 : old + (n_vis - past + 31) / 32; }
 };
 // The rows of one kv head of K or V: rows after the last one of a buffer read as zeros.
+template <bool NEW>
 struct Rows {
     const float *head, *head_new;
     int past, n_new;
     uint32_t row_bytes;
     __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(int kt) const {
-        const bool old = 32 * kt < past;
+        const bool old = !NEW || 32 * kt < past;
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(old ? head : head_new), 0, (uint32_t)(old ? past : n_new) * row_bytes, 0x00020000);
     }
-    __device__ __forceinline__ uint32_t off(int kt, int row) const { return (uint32_t)(32 * (32 * kt < past ? kt : kt - (past + 31) / 32) + row) * row_bytes; }   // row of tile kt
+    __device__ __forceinline__ uint32_t off(int kt, int row) const { return (uint32_t)(32 * (!NEW || 32 * kt < past ? kt : kt - (past + 31) / 32) + row) * row_bytes; }   // row of tile kt
 };
-__device__ __forceinline__ Rows rows_of(const PrefillF32 &p, const float *cache, const float *call, int b, int kvh, int D) {
-    return Rows{cache + b * p.kv_stride_b + kvh * p.kv_stride_h, call + ((int64_t)b * p.Hkv + kvh) * p.Sq * D, p.past, p.n_new, p.kv_row_bytes};
+template <bool NEW>
+__device__ __forceinline__ Rows<NEW> rows_of(const PrefillF32 &p, const float *cache, const float *call, int b, int kvh, int D) {
+    return Rows<NEW>{cache + b * p.kv_stride_b + kvh * p.kv_stride_h, call + ((int64_t)b * p.Hkv + kvh) * p.Sq * D, p.past, p.n_new, p.kv_row_bytes};
 }
 
 // the weight exp(m - ref) of a partial result whose maximum is m; nothing seen: m = -inf, weight 0 whatever ref is
@@ -141,7 +145,7 @@ struct TileLds {
 };
 
 // Row tile rt of a (batch, kv head) over the key tiles kt_first .. kt_last - 1 that it sees, by one workgroup.
-template <int D>
+template <int D, bool NEW>
 __device__ __forceinline__ void attend_tile(const PrefillF32 &p, TileLds<D> &shared, int bh, int rt, int split, int kt_first, int kt_last) {
     constexpr int T = D / 32, KJ = D / 8, ROW = D + 4;   // (ROW: 16 rows of a 128-bit LDS pass in 16 distinct bank groups)
     typedef typename VecOf<T>::type vec;
@@ -160,11 +164,11 @@ __device__ __forceinline__ void attend_tile(const PrefillF32 &p, TileLds<D> &sha
     // keys [0, limit) are visible to a row; the tile as a whole sees n_vis
     auto limit_of = [&](int r) { return p.causal ? min(r, n_rows - 1) / p.G + (p.Sk - p.Sq) + 1 : p.Sk; };
     const int limit = limit_of(r0 + l32), limit_first = limit_of(r0), n_vis = limit_of(r0 + kRows - 1);
-    const KeyTiles keys{p.past, (p.past + 31) / 32};
+    const KeyTiles<NEW> keys{p.past, (p.past + 31) / 32};
     const int kt_end = min(keys.count(n_vis), kt_last);
 
     // rows past the last key read as zeros: the buffer ends with that row
-    const Rows k_rows = rows_of(p, p.k, p.k_new, b, kvh, D), v_rows = rows_of(p, p.v, p.v_new, b, kvh, D);
+    const Rows<NEW> k_rows = rows_of<NEW>(p, p.k, p.k_new, b, kvh, D), v_rows = rows_of<NEW>(p, p.v, p.v_new, b, kvh, D);
 
     f32x4 kreg[KJ];
     vec vreg[16];
@@ -332,24 +336,24 @@ __device__ __forceinline__ void attend_tile(const PrefillF32 &p, TileLds<D> &sha
     }
 }
 
-template <int D>
+template <int D, bool NEW>
 __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32_kernel(PrefillF32 p) {
     __shared__ __attribute__((aligned(16))) TileLds<D> shared;
     const int bh = blockIdx.x % p.n_bh, rest = blockIdx.x / p.n_bh;
     const int split = rest % p.nsplit, rt = p.n_rt - 1 - rest / p.nsplit;
     const int last = min(rt * kRows + kRows, p.Sq * p.G) - 1, n_vis = p.causal ? last / p.G + (p.Sk - p.Sq) + 1 : p.Sk;
-    const int per_split = (KeyTiles{p.past, (p.past + 31) / 32}.count(n_vis) + p.nsplit - 1) / p.nsplit;
+    const int per_split = (KeyTiles<NEW>{p.past, (p.past + 31) / 32}.count(n_vis) + p.nsplit - 1) / p.nsplit;
     // The append: this workgroup's share of its kv head's rows (contiguous in both places; ahead of the attention, through which the
     // addresses would be kept in more scalar registers than there are).  With an append launch | now: 69 rows of 32 heads
     // over 8 14.3 | 12.2 us, 10 of 14 over 2 behind 348 18.8 | 16.4.
-    if (p.k_new) {
+    if constexpr (NEW) {
         const int64_t from = (int64_t)bh * p.Sq * D, to = (bh / p.Hkv) * p.kv_stride_b + (bh % p.Hkv) * p.kv_stride_h + (int64_t)p.past * D;
         for (int i = rest * kThreads + threadIdx.x; i < p.Sq * (D / 4); i += p.n_rt * p.nsplit * kThreads) {
             reinterpret_cast<f32x4 *>(const_cast<float *>(p.k) + to)[i] = reinterpret_cast<const f32x4 *>(p.k_new + from)[i];
             reinterpret_cast<f32x4 *>(const_cast<float *>(p.v) + to)[i] = reinterpret_cast<const f32x4 *>(p.v_new + from)[i];
         }
     }
-    attend_tile<D>(p, shared, bh, rt, split, split * per_split, (split + 1) * per_split);
+    attend_tile<D, NEW>(p, shared, bh, rt, split, split * per_split, (split + 1) * per_split);
 }
 
 // ---- more than 32 rows: every f32 as a pair of f16 ---------------------------------------------------------------------
@@ -390,7 +394,7 @@ struct PairLds {
     _Float16 vt[2][2][D / 32][32 * 40];         // [key set][upper, lower][subtile][feature]: 32 keys in the order of P's registers
 };
 
-template <int D>
+template <int D, bool NEW>
 __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(PrefillF32 p) {
     constexpr int T = D / 32, C4 = D / 4, NG = 8 * C4 / 128, KROW = D + 8, ROW = D + 4;
     typedef typename VecOf<T>::type vec;
@@ -412,15 +416,15 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
     };
     auto limit_of = [&](int r) { return p.causal ? min(r, n_rows - 1) / p.G + (p.Sk - p.Sq) + 1 : p.Sk; };
     const int limit = limit_of(r0 + kRows * rg + l32), limit_first = limit_of(r0), n_vis = limit_of(r0 + 2 * kRows - 1);
-    const KeyTiles keys{p.past, (p.past + 31) / 32};
+    const KeyTiles<NEW> keys{p.past, (p.past + 31) / 32};
     const int tiles = keys.count(n_vis), per_split = (tiles + p.nsplit - 1) / p.nsplit;
     const int kt_first = split * per_split, kt_last = min(tiles, kt_first + per_split);
 
-    const Rows k_rows = rows_of(p, p.k, p.k_new, b, kvh, D), v_rows = rows_of(p, p.v, p.v_new, b, kvh, D);
+    const Rows<NEW> k_rows = rows_of<NEW>(p, p.k, p.k_new, b, kvh, D), v_rows = rows_of<NEW>(p, p.v, p.v_new, b, kvh, D);
     // a key set's 128 threads: features 4 c4 .. + 3 of the keys 4 (g0 + 4 i) .. + 3
     const int st = tid & 127, c4 = st % C4, g0 = st / C4;
     f32x4 kpre[NG][4], vpre[NG][4];
-    auto load_rows = [&](f32x4 (&dst)[NG][4], const Rows &rows, int kt) {
+    auto load_rows = [&](f32x4 (&dst)[NG][4], const Rows<NEW> &rows, int kt) {
         const __amdgpu_buffer_rsrc_t rsrc = rows.rsrc(kt);
         const uint32_t off = rows.off(kt, 4 * g0) + 16 * c4;
 #pragma unroll
@@ -439,7 +443,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
     f32x4 *dst_k = nullptr, *dst_v = nullptr;
     int piece = 0, pieces = 0;   // this thread's next one, and how many there are
     const int hop = p.n_rt2 * p.nsplit * kThreads;
-    if (p.k_new) {
+    if constexpr (NEW) {
         src_k = reinterpret_cast<const f32x4 *>(k_rows.head_new), src_v = reinterpret_cast<const f32x4 *>(v_rows.head_new);
         dst_k = reinterpret_cast<f32x4 *>(const_cast<float *>(k_rows.head) + (int64_t)p.past * D), dst_v = reinterpret_cast<f32x4 *>(const_cast<float *>(v_rows.head) + (int64_t)p.past * D);
         piece = rest * kThreads + tid, pieces = p.Sq * C4;
@@ -447,7 +451,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
     f32x4 ck[2], cv[2];
 #pragma unroll
     for (int j = 0; j < 2; j++)
-        if (piece + j * hop < pieces) ck[j] = src_k[piece + j * hop], cv[j] = src_v[piece + j * hop];
+        if (NEW && piece + j * hop < pieces) ck[j] = src_k[piece + j * hop], cv[j] = src_v[piece + j * hop];
 
     // Scales, powers of two: q's per row, K's and V's from the first tiles of the range.
     Split8 q[D / 16];
@@ -505,7 +509,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
         }
 #pragma unroll
         for (int j = 0; j < 2; j++)
-            if (piece + j * hop < pieces) dst_k[piece + j * hop] = ck[j], dst_v[piece + j * hop] = cv[j];
+            if (NEW && piece + j * hop < pieces) dst_k[piece + j * hop] = ck[j], dst_v[piece + j * hop] = cv[j];
         if (lane == 0) lds_big[0][w] = weak_q ? INFINITY : q_norm, lds_big[1][w] = k_big, lds_big[2][w] = v_big, lds_big[3][w] = v_weak;
         if (tid == 0) lds_odd = 0;
         __syncthreads();
@@ -608,7 +612,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
             }
         }
     }
-    for (piece += 2 * hop; piece < pieces; piece += 4 * hop) {   // what is left of the append
+    for (piece += 2 * hop; NEW && piece < pieces; piece += 4 * hop) {   // what is left of the append
         f32x4 rk[4], rv[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -673,7 +677,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_prefill_f32x2_kernel(Prefill
     if (odd) {   // for this row tile everything (again), in f32
         for (int i = 0; i < 2 && r0 + kRows * i < n_rows; i++) {
             __syncthreads();
-            attend_tile<D>(p, lds.tile, bh, 2 * rt2 + i, split, kt_first, kt_last);
+            attend_tile<D, NEW>(p, lds.tile, bh, 2 * rt2 + i, split, kt_first, kt_last);
         }
         return;
     }
@@ -736,10 +740,10 @@ __global__ __launch_bounds__(kThreads) void sdpa_prefill_f32_merge_kernel(Prefil
     *reinterpret_cast<f32x4 *>(p.out + (((int64_t)b * p.Hq + kvh * p.G + g) * p.Sq + i) * D + 4 * c) = sum;
 }
 
-template <int D>
+template <int D, bool NEW>
 int launch(const PrefillF32 &p, hipStream_t s) {
-    if (p.n_rt2) hipLaunchKernelGGL((sdpa_prefill_f32x2_kernel<D>), dim3((unsigned)(p.n_bh * p.n_rt2 * p.nsplit)), dim3(kThreads), 0, s, p);
-    else hipLaunchKernelGGL((sdpa_prefill_f32_kernel<D>), dim3((unsigned)(p.n_bh * p.n_rt * p.nsplit)), dim3(kThreads), 0, s, p);
+    if (p.n_rt2) hipLaunchKernelGGL((sdpa_prefill_f32x2_kernel<D, NEW>), dim3((unsigned)(p.n_bh * p.n_rt2 * p.nsplit)), dim3(kThreads), 0, s, p);
+    else hipLaunchKernelGGL((sdpa_prefill_f32_kernel<D, NEW>), dim3((unsigned)(p.n_bh * p.n_rt * p.nsplit)), dim3(kThreads), 0, s, p);
     if (p.nsplit > 1)
         hipLaunchKernelGGL((sdpa_prefill_f32_merge_kernel<D>), dim3((unsigned)((int64_t)p.n_bh * p.n_rt * (kRows * D / 4 / kThreads))), dim3(kThreads), 0, s, p);
     hipError_t e = hipGetLastError();
@@ -842,7 +846,8 @@ int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
         p.part_ml = p.part_o + (size_t)p.nsplit * n_wb * kRows * a.D;
     }
     if (n_wb * p.nsplit >= (1ll << 31) || n_wb * (kRows * a.D / 4 / kThreads) >= (1ll << 31)) return 2;
-    return a.D == 128 ? launch<128>(p, s) : launch<64>(p, s);
+    if (a.k_new) return a.D == 128 ? launch<128, true>(p, s) : launch<64, true>(p, s);
+    return a.D == 128 ? launch<128, false>(p, s) : launch<64, false>(p, s);
 }
 
 }  // namespace trocm
