@@ -137,7 +137,9 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t b0123, uint32_t b4567, half2_
 // ALONE: a workgroup has a compute unit to itself, and as many registers as it likes (D = 64; D = 128 always has).
 // PARTS: some query tiles in several key ranges, merged here from f32 partials; an instantiation of its own, since the two
 // ways of merging in one kernel spill registers.
-template <int D, int HG, bool MASK, int FMT, bool PING = false, bool F32 = false, bool ALONE = D != 64 || MASK, bool PARTS = false>
+// APPEND: the last Sq tokens are the call's rows, which this launch stores to the cache; an instantiation of its own as well: picking
+// between the two kinds of rows takes prompts of 10 to 20 us that bring none 4 to 6 % longer.
+template <int D, int HG, bool MASK, int FMT, bool PING = false, bool F32 = false, bool ALONE = D != 64 || MASK, bool PARTS = false, bool APPEND = false>
 __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_kernel(PrefillPP p) {
     static_assert(!F32 || (HG == 1 && !MASK && FMT == TROCM_F16 && !PING), "short prompts of one head per workgroup");
     static_assert(!PING || (!MASK && FMT == TROCM_F16), "the ping-pong loop serves f16 caches without a mask input");
@@ -237,7 +239,7 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
     // A call of 512 queries behind 3584 tokens, 32 heads in groups of 4, an append launch and 64-bit addresses per lane before |
     // now: 45.3 | 43.1 us; behind none 18.4 | 16.2; 2 x 1500 of 32 heads over 32 69.0 | 63.5 (68.3 with all of the share copied on
     // the way in), at D = 64 44.2 | 38.8; 3 x 917 of 64 over 8 behind 3704, D = 64, 242 | 236.5.
-    constexpr bool APPEND = !QUANT && !MASK && !PING;
+    static_assert(!APPEND || (!QUANT && !MASK && !PING), "f16 caches without a mask, registers loop");
     constexpr int CD = 2;   // pieces of each tensor that a thread copies on the way in
     const _Float16 *knew = nullptr, *vnew = nullptr;   // where token 0 would be
     if constexpr (APPEND) {
@@ -247,7 +249,7 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
     // A tile whose rows are all of one kind and all there is asked for at a wave-uniform address plus one offset per lane.
     const int key0 = tid / (D / 8), dc0 = tid % (D / 8);
     constexpr int KEYS = kThreadsPP / (D / 8);   // rows between a thread's pieces
-    const int64_t row_bytes = (APPEND && p.k_new ? D : p.kv_stride_t) * 2;
+    const int64_t row_bytes = (APPEND ? D : p.kv_stride_t) * 2;
     const uint32_t lane_off = QUANT ? 0 : (uint32_t)key0 * (uint32_t)row_bytes + dc0 * 16;   // (rows of less than 2^25 bytes)
     auto prefetch = [&](int kt) {
         if constexpr (!QUANT) {
@@ -464,18 +466,16 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
         const u32x4 *src_k = nullptr, *src_v = nullptr;
         u32x4 *dst_k = nullptr, *dst_v = nullptr;
         if constexpr (APPEND) {
-            if (p.k_new) {
-                pieces = p.Sq * (D / 8);
-                // (tiles in unlike numbers of parts: the first range copies for its tile)
-                piece = PARTS ? (split == 0 ? (qt * (G / HG) + gg) * kThreadsPP + tid : pieces) : (((qt * nsplit + split) * (G / HG)) + gg) * kThreadsPP + tid;
-                hop = p.n_qtiles * (PARTS ? 1 : nsplit) * (G / HG) * kThreadsPP;
-                src_k = reinterpret_cast<const u32x4 *>(knew + (int64_t)off * D), src_v = reinterpret_cast<const u32x4 *>(vnew + (int64_t)off * D);
-                dst_k = reinterpret_cast<u32x4 *>(const_cast<_Float16 *>(kbase) + (int64_t)off * D);
-                dst_v = reinterpret_cast<u32x4 *>(const_cast<_Float16 *>(vbase) + (int64_t)off * D);
+            pieces = p.Sq * (D / 8);
+            // (tiles in unlike numbers of parts: the first range copies for its tile)
+            piece = PARTS ? (split == 0 ? (qt * (G / HG) + gg) * kThreadsPP + tid : pieces) : (((qt * nsplit + split) * (G / HG)) + gg) * kThreadsPP + tid;
+            hop = p.n_qtiles * (PARTS ? 1 : nsplit) * (G / HG) * kThreadsPP;
+            src_k = reinterpret_cast<const u32x4 *>(knew + (int64_t)off * D), src_v = reinterpret_cast<const u32x4 *>(vnew + (int64_t)off * D);
+            dst_k = reinterpret_cast<u32x4 *>(const_cast<_Float16 *>(kbase) + (int64_t)off * D);
+            dst_v = reinterpret_cast<u32x4 *>(const_cast<_Float16 *>(vbase) + (int64_t)off * D);
 #pragma unroll
-                for (int j = 0; j < CD; j++)
-                    if (piece + j * hop < pieces) ck[j] = src_k[piece + j * hop], cv[j] = src_v[piece + j * hop];
-            }
+            for (int j = 0; j < CD; j++)
+                if (piece + j * hop < pieces) ck[j] = src_k[piece + j * hop], cv[j] = src_v[piece + j * hop];
         }
         // Q^T fragments: query = lane % 32, features 16*ks + 8*hb .. +8
 #pragma unroll
@@ -486,11 +486,9 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(qf[ks]));
         if constexpr (APPEND) {
-            if (p.k_new) {
 #pragma unroll
-                for (int j = 0; j < CD; j++)
-                    if (piece + j * hop < pieces) dst_k[piece + j * hop] = ck[j], dst_v[piece + j * hop] = cv[j];
-            }
+            for (int j = 0; j < CD; j++)
+                if (piece + j * hop < pieces) dst_k[piece + j * hop] = ck[j], dst_v[piece + j * hop] = cv[j];
         }
 
         if (n_it > 0) {
@@ -1149,6 +1147,8 @@ int launch_cfg(const PrefillPP &p, int fmt, int64_t wgs, bool alone, hipStream_t
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<128, HG, false, TROCM_Q8_0, false, false, true, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     else if (D == 128 && p.whole && fmt == TROCM_Q4_0)
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<128, HG, false, TROCM_Q4_0, false, false, true, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
+    else if (D == 128 && p.whole && p.k_new)
+        hipLaunchKernelGGL((sdpa_prefill_pp_kernel<128, HG, false, TROCM_F16, false, false, true, true, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     else if (D == 128 && p.whole)
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<128, HG, false, TROCM_F16, false, false, true, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     else if (fmt == TROCM_Q8_0)
@@ -1157,15 +1157,21 @@ int launch_cfg(const PrefillPP &p, int fmt, int64_t wgs, bool alone, hipStream_t
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_Q4_0>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     else if (p.mask)
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, true, TROCM_F16>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
+    else if (HG == 1 && p.part32 && p.k_new)
+        hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, 1, false, TROCM_F16, false, true, D != 64, false, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     else if (HG == 1 && p.part32)
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, 1, false, TROCM_F16, false, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
     else if (ping_enabled())
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_F16, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
-    else if (D == 64 && alone)   // (the LDS that more workgroups than units ask for is not used: no second one fits beside it)
-        hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_F16, false, false, true>), dim3((unsigned)wgs), dim3(kThreadsPP),
-                           wgs > num_compute_units() ? 48 * 1024 : 0, s, p);
-    else
+    else if (D == 64 && !alone && p.k_new)
+        hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_F16, false, false, D != 64, false, true>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
+    else if (D == 64 && !alone)
         hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_F16>), dim3((unsigned)wgs), dim3(kThreadsPP), 0, s, p);
+    else {   // (the LDS that more workgroups than units ask for at 64 features is not used: no second one fits beside it)
+        const size_t lds = D == 64 && wgs > num_compute_units() ? 48 * 1024 : 0;
+        if (p.k_new) hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_F16, false, false, true, false, true>), dim3((unsigned)wgs), dim3(kThreadsPP), lds, s, p);
+        else hipLaunchKernelGGL((sdpa_prefill_pp_kernel<D, HG, false, TROCM_F16, false, false, true>), dim3((unsigned)wgs), dim3(kThreadsPP), lds, s, p);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail("sdpa_prefill_pp launch failed: %s", hipGetErrorString(e));
     if (p.nsplit > 1 && p.counters == nullptr) {
