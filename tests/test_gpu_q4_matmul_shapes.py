@@ -99,3 +99,21 @@ def test_shapes_with_k_shared_among_waves(rt, m, n, k):
     want, size = act[0].astype(np.float64) @ wd.T, np.abs(act[0].astype(np.float64)) @ np.abs(wd).T
     # products are exact; at most k / 32 / 8 + 10 f32 additions stand one after the other, and the result is rounded to f16
     assert np.all(np.abs(got - want) <= size * (k / 256 + 11) * 2.0 ** -24 + np.abs(want) * 2.0 ** -11 + 2.0 ** -25)
+
+
+# more activation rows than a grid has tiles of: the bits of the same rows in calls that fit (one pass over the weights in every case)
+@pytest.mark.parametrize("m,n", [(65535 * 32 + 33, 33), (65535 * 16 + 5, 16)])
+def test_more_f32_rows_than_a_grid_holds(rt, m, n):
+    rng = np.random.default_rng(n)
+    k, part = 32, 999_968   # (whole tiles of 16 and of 32 rows)
+    blocks = orc.quant(orc.FMT_Q4_0, (0.05 * rng.standard_normal((n, k), dtype=np.float32)).astype(np.float32))
+    w, op = ta.Q40Weights(blocks, 1, n, k), ta.GgmlGemm()
+    act = rng.standard_normal((1, m, k), dtype=np.float32)
+    got = op.eval(ta.DeviceTensor.from_numpy(act), w).to_numpy()[0]
+    for at in range(0, m, part):
+        want = op.eval(ta.DeviceTensor.from_numpy(np.ascontiguousarray(act[:, at : at + part])), w).to_numpy()[0]
+        whole = min(part, m - at) // 32 * 32   # (the few rows left of a call may be given a tile of another shape)
+        if whole > 512:
+            np.testing.assert_array_equal(got[at : at + whole], want[:whole])
+    tail = act[0, -40:].astype(np.float64) @ orc.dequant(orc.FMT_Q4_0, blocks, np.float32).reshape(n, k).astype(np.float64).T
+    assert np.abs(got[-40:] - tail).max() <= 1e-5

@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 #include <string.h>
 #include <type_traits>
+#include <algorithm>
 #include "common.h"
 
 namespace trocm {
@@ -48,6 +49,7 @@ struct MatMulF32 {
     const float *act;         // [act_batch, m, k]
     float *out;               // [act_batch, m, n]
     int n, k, m, ratio;       // ratio = act_batch / w_batch
+    int tile0;                // tiles of activation rows ahead of this launch's
 };
 
 template <int SUB> struct AccOf;
@@ -97,7 +99,7 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
 
     const int tid = threadIdx.x, lane = tid & 63, row = lane % SUB, grp = lane / SUB;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n0 = blockIdx.x * SUB * NI, m0 = blockIdx.y * SUB, b = blockIdx.z, wb = b / p.ratio;
+    const int n0 = blockIdx.x * SUB * NI, m0 = (p.tile0 + blockIdx.y) * SUB, b = blockIdx.z, wb = b / p.ratio;
     const int nb = p.k / 32, units = (nb + 3) / 4;
     // slot g of a block: its features 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3.  Instruction st of a block contracts slots
     // 2 st + grp (SUB 32) or all four (SUB 16).
@@ -324,10 +326,13 @@ int launch_q4_0_matmul_f32(const void *codes, const void *scales, int64_t w_batc
     const int64_t cus = num_compute_units();
     auto launch = [&](auto sub, auto ni) -> int {
         constexpr int SUB = decltype(sub)::value, NI = decltype(ni)::value;
-        const dim3 grid((unsigned)((n + SUB * NI - 1) / (SUB * NI)), (unsigned)((m + SUB - 1) / SUB), (unsigned)act_batch);
-        if (grid.y > 65535) return 2;
-        if (tiled) hipLaunchKernelGGL((q4_0_matmul_f32_kernel<SUB, NI, true>), grid, dim3(64 * kW), 0, s, p);
-        else hipLaunchKernelGGL((q4_0_matmul_f32_kernel<SUB, NI, false>), grid, dim3(64 * kW), 0, s, p);
+        const int64_t row_tiles = (m + SUB - 1) / SUB;
+        for (int64_t t = 0; t < row_tiles; t += 65535) {   // (a launch: as many as its grid holds)
+            const dim3 grid((unsigned)((n + SUB * NI - 1) / (SUB * NI)), (unsigned)std::min<int64_t>(65535, row_tiles - t), (unsigned)act_batch);
+            p.tile0 = (int)t;
+            if (tiled) hipLaunchKernelGGL((q4_0_matmul_f32_kernel<SUB, NI, true>), grid, dim3(64 * kW), 0, s, p);
+            else hipLaunchKernelGGL((q4_0_matmul_f32_kernel<SUB, NI, false>), grid, dim3(64 * kW), 0, s, p);
+        }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return fail("q4_0_matmul (f32) launch failed: %s", hipGetErrorString(e));
         return 0;
