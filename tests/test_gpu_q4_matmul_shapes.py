@@ -67,10 +67,12 @@ def test_short_walks_of_k(rt, n, m, tiles):
     assert np.abs(got - want).max() <= 2.0 ** -11 * (6 * np.sqrt(k) * 0.03 + np.abs(want).max())
 
 
-# f32 rows: 16 x 32, 16 x 48, 16 x 64, 32 x 64, 32 x 96 and 32 x 128 (activation rows x weight rows), each as planes and as tiles, with
-# remainders of both; one row's values are so large that its blocks are done in f32, for every part of the workgroup's weight rows
+# f32 rows: 16 x 32, 16 x 48, 16 x 64, 32 x 64, 32 x 96 and 32 x 128 (activation rows x weight rows) of tiles, 16 x 16, 16 x 32, 32 x 32, 32 x
+# 64, 32 x 96 and 64 x 64 of planes, with remainders of both; one row's values are so large that its blocks are done in f32, for every part
+# of the workgroup's weight rows
 @pytest.mark.parametrize("m,n,k", [(16, 4130, 160), (16, 4112, 256), (64, 2817, 1056), (64, 2064, 1152), (33, 4130, 160), (33, 4112, 384), (150, 2063, 1024),
                                    (150, 2064, 1152), (150, 4100, 1056), (150, 4112, 1152), (200, 4130, 160), (200, 4112, 256),
+                                   (40, 1001, 96), (130, 1001, 1056), (250, 1001, 160), (210, 4090, 544), (97, 8210, 1120),
                                    # ... and the fewest rows it takes, of small and tall matrices
                                    (5, 4112, 384), (5, 2065, 160), (6, 1040, 2176), (6, 30000, 128), (7, 57360, 128), (8, 32784, 512), (12, 65552, 256)])
 def test_shapes_of_the_f32_product(rt, m, n, k):

@@ -10,7 +10,7 @@
 // f32; planes' blocks also where a lane's values are so small that 2^-133 counts among them (tiled weights are split the same way
 // by the kernel for few rows, q4_tiled.hip; the test costs 2 % of 150 rows of 4096 x 4096).
 //
-// A workgroup of 8 waves owns SUB (activation rows) x SUB NI (weight rows) of the result.  Its waves share k, not the
+// A workgroup of 8 waves owns SUB MS (activation rows) x SUB NI (weight rows) of the result.  Its waves share k, not the
 // tile: wave w takes units (4 blocks, a record of tiled weights) w, w + 8, ..  Both operands then go from memory straight
 // into the registers that feed the instruction, without LDS and without a barrier; the eight sums are added through LDS at
 // the end.  Eight short sums are also more exact than one long one (error against f64, 150 rows of 4096 features: 9.5e-8;
@@ -88,18 +88,18 @@ __device__ __forceinline__ bf16x8_t codes_bf16(uint32_t word) {
     return __builtin_bit_cast(bf16x8_t, o);
 }
 
-template <int SUB, int NI, bool TILED>
+template <int SUB, int MS, int NI, bool TILED>
 __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p) {
     typedef typename AccOf<SUB>::type acc_t;
     constexpr int R = SUB == 32 ? 16 : 4;        // results per lane and subtile
     constexpr int KST = SUB == 32 ? 2 : 1;       // instructions per block
-    constexpr int PER_WAVE = NI * R * 64;        // results of a wave
+    constexpr int PER_WAVE = MS * NI * R * 64;   // results of a wave
     constexpr int COPIES = PER_WAVE * kW * 4 <= 65536 ? kW : kW / 2;   // the waves' sums that LDS holds at once
     __shared__ __attribute__((aligned(16))) float lds[COPIES * PER_WAVE];
 
     const int tid = threadIdx.x, lane = tid & 63, row = lane % SUB, grp = lane / SUB;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n0 = blockIdx.x * SUB * NI, m0 = (p.tile0 + blockIdx.y) * SUB, b = blockIdx.z, wb = b / p.ratio;
+    const int n0 = blockIdx.x * SUB * NI, m0 = (p.tile0 + blockIdx.y) * SUB * MS, b = blockIdx.z, wb = b / p.ratio;
     const int nb = p.k / 32, units = (nb + 3) / 4;
     // slot g of a block: its features 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3.  Instruction st of a block contracts slots
     // 2 st + grp (SUB 32) or all four (SUB 16).
@@ -114,8 +114,9 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
         const_cast<uint8_t *>(p.codes + wb * w_bytes), 0, (uint32_t)w_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t *>(TILED ? nullptr : p.scales + (int64_t)wb * p.n * nb), 0, TILED ? 0u : (uint32_t)((int64_t)p.n * nb * 2), 0x00020000);
-    const uint32_t a_off = (uint32_t)(m0 + row) * (uint32_t)p.k * 4u + 16u * slot(0);
-    uint32_t w_off[NI], s_off[NI];
+    uint32_t a_off[MS], w_off[NI], s_off[NI];
+#pragma unroll
+    for (int i = 0; i < MS; i++) a_off[i] = (uint32_t)(m0 + SUB * i + row) * (uint32_t)p.k * 4u + 16u * slot(0);
 #pragma unroll
     for (int i = 0; i < NI; i++) {
         const int j = min(n0 + SUB * i + row, p.n - 1);
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
     }
 
     struct Weights { uint32_t c[NI][KST][4]; uint32_t s[NI][2]; };   // a unit: words per (instruction, block), scales of its blocks
-    struct Act { f32x4 x[KST][2]; };                                 // a block: features 4 g .., 16 + 4 g ..
+    struct Act { f32x4 x[MS][KST][2]; };                             // a block: features 4 g .., 16 + 4 g ..
     auto load_w = [&](Weights &d, int u) {
 #pragma unroll
         for (int i = 0; i < NI; i++) {
@@ -158,28 +159,38 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
     };
     auto load_a = [&](Act &d, int blk) {
 #pragma unroll
-        for (int st = 0; st < KST; st++)
+        for (int i = 0; i < MS; i++)
 #pragma unroll
-            for (int h = 0; h < 2; h++) d.x[st][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_off + 32 * st + 64 * h, blk * 128, 0));
+            for (int st = 0; st < KST; st++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    d.x[i][st][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_off[i] + 32 * st + 64 * h, blk * 128, 0));
     };
 
-    acc_t acc[NI];
+    acc_t acc[MS][NI];
 #pragma unroll
-    for (int j = 0; j < NI; j++)
+    for (int i = 0; i < MS; i++)
 #pragma unroll
-        for (int r = 0; r < R; r++) acc[j][r] = 0.0f;
+        for (int j = 0; j < NI; j++)
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[i][j][r] = 0.0f;
 
-    // result register r of a lane: activation row out_row(r) of the workgroup's, weight row SUB j + lane % SUB
+    // result register r of a lane: activation row SUB i + out_row(r) of the workgroup's, weight row SUB j + lane % SUB
     auto out_row = [&](int r) { return SUB == 32 ? 8 * (r / 4) + 4 * grp + r % 4 : 4 * grp + r; };
 
-    // Whether a block is one of those, by the largest magnitude among a lane's values.
-    auto needs_f32 = [](float big) { return __any(big >= kBig || (!TILED && big < kSmall && big > 0.0f)); };
+    // Whether a block is one of those, by the largest magnitude among a lane's 8 values of each of its activation rows.
+    auto needs_f32 = [](const float (&big)[MS]) {
+        bool any = false;
+#pragma unroll
+        for (int i = 0; i < MS; i++) any = any || big[i] >= kBig || (!TILED && big[i] < kSmall && big[i] > 0.0f);
+        return __any(any);
+    };
     // Products with the dequantised weights, one after the other.
     auto slow_block = [&](int blk) {
         const float *act = p.act + (int64_t)b * p.m * p.k + blk * 32;
 #pragma unroll 1
-        for (int jj = 0; jj < NI; jj++) {
-            const int j = min(n0 + SUB * jj + row, p.n - 1);
+        for (int ij = 0; ij < MS * NI; ij++) {
+            const int i = ij / NI, jj = ij % NI, j = min(n0 + SUB * jj + row, p.n - 1);
             acc_t sum;
 #pragma unroll
             for (int r = 0; r < R; r++) sum[r] = 0.0f;
@@ -198,11 +209,13 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
                 const float wt = ((float)(e < 16 ? c & 15 : c >> 4) - 8.0f) * f16_to_f32(d);
 #pragma unroll
                 for (int r = 0; r < R; r++)
-                    sum[r] = fmaf(act[(int64_t)min(m0 + out_row(r), p.m - 1) * p.k + e], wt, sum[r]);
+                    sum[r] = fmaf(act[(int64_t)min(m0 + SUB * i + out_row(r), p.m - 1) * p.k + e], wt, sum[r]);
             }
 #pragma unroll
-            for (int y = 0; y < NI; y++)
-                if (y == jj) acc[y] += sum;
+            for (int x = 0; x < MS; x++)
+#pragma unroll
+                for (int y = 0; y < NI; y++)
+                    if (x * NI + y == ij) acc[x][y] += sum;
         }
     };
 
@@ -224,22 +237,26 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
                 if (next < nb) load_a(nxt, next);
             }
             __builtin_amdgcn_sched_barrier(0);   // (a block's fragments live only as long as the block)
-            bf16x8_t part[3][KST];   // the smallest first
-            float big = 0.0f;
+            bf16x8_t part[3][MS][KST];   // the smallest first
+            float big[MS];
 #pragma unroll
-            for (int st = 0; st < KST; st++) {
-                u32x4 b1, b2, b3;
+            for (int i = 0; i < MS; i++) big[i] = 0.0f;
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float x0 = cur.x[st][e >> 1][2 * (e & 1)], x1 = cur.x[st][e >> 1][2 * (e & 1) + 1];
-                    big = fmaxf(fmaxf(fabsf(x0), fabsf(x1)), big);
-                    const float r0 = rest(x0), r1 = rest(x1);
-                    b1[e] = upper2(x0, x1), b2[e] = upper2(r0, r1), b3[e] = upper2(rest(r0), rest(r1));
+            for (int i = 0; i < MS; i++)
+#pragma unroll
+                for (int st = 0; st < KST; st++) {
+                    u32x4 b1, b2, b3;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const float x0 = cur.x[i][st][e >> 1][2 * (e & 1)], x1 = cur.x[i][st][e >> 1][2 * (e & 1) + 1];
+                        big[i] = fmaxf(fmaxf(fabsf(x0), fabsf(x1)), big[i]);
+                        const float r0 = rest(x0), r1 = rest(x1);
+                        b1[e] = upper2(x0, x1), b2[e] = upper2(r0, r1), b3[e] = upper2(rest(r0), rest(r1));
+                    }
+                    part[0][i][st] = __builtin_bit_cast(bf16x8_t, b3);
+                    part[1][i][st] = __builtin_bit_cast(bf16x8_t, b2);
+                    part[2][i][st] = __builtin_bit_cast(bf16x8_t, b1);
                 }
-                part[0][st] = __builtin_bit_cast(bf16x8_t, b3);
-                part[1][st] = __builtin_bit_cast(bf16x8_t, b2);
-                part[2][st] = __builtin_bit_cast(bf16x8_t, b1);
-            }
             if (needs_f32(big)) {   // after the loop
                 skipped = true;
                 continue;
@@ -250,15 +267,21 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
 #pragma unroll
                 for (int st = 0; st < KST; st++) cf[st] = codes_bf16(wt.c[jj][st][j]);
                 const float d = f16_to_f32(wt.s[jj][j >> 1] >> (16 * (j & 1)));
-                acc_t sum;
+                acc_t sum[MS];
 #pragma unroll
-                for (int r = 0; r < R; r++) sum[r] = 0.0f;
+                for (int i = 0; i < MS; i++)
+#pragma unroll
+                    for (int r = 0; r < R; r++) sum[i][r] = 0.0f;
 #pragma unroll
                 for (int q = 0; q < 3; q++)
 #pragma unroll
-                    for (int st = 0; st < KST; st++) sum = mfma<SUB>(part[q][st], cf[st], sum);
+                    for (int st = 0; st < KST; st++)
 #pragma unroll
-                for (int r = 0; r < R; r++) acc[jj][r] = fmaf(sum[r], d, acc[jj][r]);
+                        for (int i = 0; i < MS; i++) sum[i] = mfma<SUB>(part[q][i][st], cf[st], sum[i]);
+#pragma unroll
+                for (int i = 0; i < MS; i++)
+#pragma unroll
+                    for (int r = 0; r < R; r++) acc[i][jj][r] = fmaf(sum[i][r], d, acc[i][jj][r]);
             }
         }
     }
@@ -266,12 +289,16 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
     if (skipped) {
         for (u = w; u < units; u += kW)
             for (int blk = 4 * u; blk < min(4 * u + 4, nb); blk++) {
-                float big = 0.0f;
+                float big[MS];
                 load_a(cur, blk);
 #pragma unroll
-                for (int st = 0; st < KST; st++)
+                for (int i = 0; i < MS; i++) big[i] = 0.0f;
 #pragma unroll
-                    for (int e = 0; e < 8; e++) big = fmaxf(big, fabsf(cur.x[st][e >> 2][e & 3]));
+                for (int i = 0; i < MS; i++)
+#pragma unroll
+                    for (int st = 0; st < KST; st++)
+#pragma unroll
+                        for (int e = 0; e < 8; e++) big[i] = fmaxf(big[i], fabsf(cur.x[i][st][e >> 2][e & 3]));
                 if (needs_f32(big)) slow_block(blk);
             }
     }
@@ -279,18 +306,22 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
     // ---- the eight sums, [wave][subtile][register][lane] in LDS, added in the order of the waves ---------------------
     auto write = [&](int at) {
 #pragma unroll
-        for (int j = 0; j < NI; j++)
+        for (int i = 0; i < MS; i++)
 #pragma unroll
-            for (int r = 0; r < R; r++) lds[at * PER_WAVE + (j * R + r) * 64 + lane] = acc[j][r];
+            for (int j = 0; j < NI; j++)
+#pragma unroll
+                for (int r = 0; r < R; r++) lds[at * PER_WAVE + ((i * NI + j) * R + r) * 64 + lane] = acc[i][j][r];
     };
     if constexpr (COPIES < kW) {
         if (w >= COPIES) write(w - COPIES);
         __syncthreads();
         if (w < COPIES) {
 #pragma unroll
-            for (int j = 0; j < NI; j++)
+            for (int i = 0; i < MS; i++)
 #pragma unroll
-                for (int r = 0; r < R; r++) acc[j][r] += lds[w * PER_WAVE + (j * R + r) * 64 + lane];
+                for (int j = 0; j < NI; j++)
+#pragma unroll
+                    for (int r = 0; r < R; r++) acc[i][j][r] += lds[w * PER_WAVE + ((i * NI + j) * R + r) * 64 + lane];
             write(w);   // (read and written by the same thread)
         }
     } else {
@@ -303,8 +334,8 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
 #pragma unroll
         for (int c = 1; c < COPIES; c++) sum += lds[c * PER_WAVE + e];
         // (an element's lane is its thread's: 64 divides the workgroup)
-        const int r = (e >> 6) % R, j = (e >> 6) / R;
-        const int mi = m0 + out_row(r), ni = n0 + SUB * j + row;
+        const int r = (e >> 6) % R, j = (e >> 6) / R % NI, i = (e >> 6) / (R * NI);
+        const int mi = m0 + SUB * i + out_row(r), ni = n0 + SUB * j + row;
         if (mi < p.m && ni < p.n) out[(int64_t)mi * p.n + ni] = sum;
     }
 }
@@ -324,14 +355,17 @@ int launch_q4_0_matmul_f32(const void *codes, const void *scales, int64_t w_batc
     p.n = (int)n, p.k = (int)k, p.m = (int)m, p.ratio = (int)(act_batch / w_batch);
 
     const int64_t cus = num_compute_units();
-    auto launch = [&](auto sub, auto ni) -> int {
-        constexpr int SUB = decltype(sub)::value, NI = decltype(ni)::value;
-        const int64_t row_tiles = (m + SUB - 1) / SUB;
+    auto launch = [&](auto sub, auto ms, auto ni) -> int {
+        constexpr int SUB = decltype(sub)::value, MS = decltype(ms)::value, NI = decltype(ni)::value;
+        const int64_t row_tiles = (m + SUB * MS - 1) / (SUB * MS);
         for (int64_t t = 0; t < row_tiles; t += 65535) {   // (a launch: as many as its grid holds)
             const dim3 grid((unsigned)((n + SUB * NI - 1) / (SUB * NI)), (unsigned)std::min<int64_t>(65535, row_tiles - t), (unsigned)act_batch);
             p.tile0 = (int)t;
-            if (tiled) hipLaunchKernelGGL((q4_0_matmul_f32_kernel<SUB, NI, true>), grid, dim3(64 * kW), 0, s, p);
-            else hipLaunchKernelGGL((q4_0_matmul_f32_kernel<SUB, NI, false>), grid, dim3(64 * kW), 0, s, p);
+            constexpr bool TILES = !(SUB == 32 && (MS == 2 || NI == 1)), PLANES = SUB == 16 ? NI <= 2 : NI <= 3;   // (the other's never chosen)
+            if constexpr (TILES)
+                if (tiled) hipLaunchKernelGGL((q4_0_matmul_f32_kernel<SUB, MS, NI, true>), grid, dim3(64 * kW), 0, s, p);
+            if constexpr (PLANES)
+                if (!tiled) hipLaunchKernelGGL((q4_0_matmul_f32_kernel<SUB, MS, NI, false>), grid, dim3(64 * kW), 0, s, p);
         }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return fail("q4_0_matmul (f32) launch failed: %s", hipGetErrorString(e));
@@ -343,33 +377,45 @@ int launch_q4_0_matmul_f32(const void *codes, const void *scales, int64_t w_batc
     std::integral_constant<int, 4> four;
     std::integral_constant<int, 16> sub16;
     std::integral_constant<int, 32> sub32;
-    // The shape that takes the least time: rounds of workgroups, one per compute unit, the first and the later ones as measured with 1024,
-    // 4096 and 14336 features (us, straight lines in the units of a wave).  Against squares of 32 and 64 and oblongs of 16 x 16, 16 x 32
-    // and 32 x 64 only: 150 rows of 4096 x 4096 36.7 -> 26.4 (32 x 96; 32 x 128 29.2), 40 17.8 -> 14.1 (16 x 64), 512 74.5 -> 62.3
-    // (32 x 128), 16 of 14336 x 4096 20.0 -> 15.0, 500 252 -> 216.  Squares share more of the split of the activations, oblongs of the
-    // same size have half the registers for it: 64 x 64 is 250 there.  Below 1024 features, where some waves have no unit, a launch takes its
+    // The shape that takes the least time: rounds of workgroups, one per compute unit, the first and the later ones as measured (us, straight
+    // lines in the units of the busiest wave), tiles with 1024, 4096 and 14336 features, planes at 12 matrices of 512 to 14336 and 8 to 500
+    // rows.  Against squares of 32 and 64 and oblongs of 16 x 16, 16 x 32 and 32 x 64 by one number each: tiles, 150 rows of 4096 x 4096 36.7
+    // -> 26.4 (32 x 96; 32 x 128 29.2), 40 17.8 -> 14.1 (16 x 64), 512 74.5 -> 62.3 (32 x 128), 16 of 14336 x 4096 20.0 -> 15.0, 500 252
+    // -> 216.  Squares share more of the split of the activations, oblongs of the same size have half the registers for it: 64 x 64 is
+    // 250 there.  The codes of planes come in words of 4 bytes, so that a weight row costs more and squares stay the better ones (us, as
+    // for tiles | as here: 40 rows of 4090 x 4096 39.3 | 27.1 (32 x 32), 500 127 | 111 (64 x 64), 200 of 1000 x 2080 16.2 | 13.1); 0.984 of
+    // the time by one number each over those 144 products, none longer.  Below 1024 features, where some waves have no unit, a launch takes its
     // 4 to 5 us and is still the faster side (groups of 8 rows | here: 7 rows of 4096 x 32 7.1 | 4.1, of 4096 x 512 5.4 | 4.2; 40 rows of
     // 16384 x 128 23.7 | 7.7, of 1000 x 96 24.7 | 4.5).
-    struct Shape { int sub, ni; float first, first_k, later, later_k; };
-    const Shape shapes[] = {{16, 1, 1.3f, 1.75f, 0.4f, 1.75f}, {16, 2, 1.4f, 2.27f, 0.2f, 1.93f}, {16, 3, 2.6f, 2.45f, 0.25f, 2.17f}, {16, 4, 2.3f, 2.93f, 0.3f, 2.45f},
-                            {32, 2, 2.6f, 4.08f, 1.9f, 4.1f},  {32, 3, 3.6f, 5.05f, 3.0f, 5.45f}, {32, 4, 4.3f, 6.1f, 4.2f, 6.4f}};
-    const float per_wave = (float)((k + 128 * kW - 1) / (128 * kW));
+    struct Times { float first, first_k, later, later_k; };
+    constexpr float kNever = 1e9f;
+    struct Shape { int sub, ms, ni; Times tiles, planes; };
+    const Shape shapes[] = {{16, 1, 1, {1.3f, 1.75f, 0.4f, 1.75f}, {1.24f, 2.92f, -0.74f, 2.57f}}, {16, 1, 2, {1.4f, 2.27f, 0.2f, 1.93f}, {0.89f, 4.37f, -1.35f, 3.75f}},
+                            {16, 1, 3, {2.6f, 2.45f, 0.25f, 2.17f}, {kNever}},                     {16, 1, 4, {2.3f, 2.93f, 0.3f, 2.45f}, {kNever}},
+                            {32, 1, 1, {kNever}, {0.78f, 5.04f, -1.76f, 5.06f}},                   {32, 1, 2, {2.6f, 4.08f, 1.9f, 4.1f}, {0.68f, 7.33f, -0.06f, 7.24f}},
+                            {32, 1, 3, {3.6f, 5.05f, 3.0f, 5.45f}, {0.92f, 9.86f, 1.87f, 9.37f}},  {32, 1, 4, {4.3f, 6.1f, 4.2f, 6.4f}, {kNever}},
+                            {32, 2, 2, {kNever}, {1.64f, 10.62f, 2.59f, 10.83f}}};
+    const int64_t units = (k + 127) / 128, last = k / 32 - 4 * (units - 1);   // blocks of the last unit, which is a wave's last if no other one has as many
+    const float per_wave = (float)((units - 1) / 8 * 4 + ((units - 1) % 8 ? 4 : last)) / 4.0f;
     int best = 0;
     float best_us = 0.0f;
-    for (int c = 0; c < 7; c++) {
+    for (int c = 0; c < 9; c++) {
         const Shape &x = shapes[c];
-        const int64_t wgs = (n + x.sub * x.ni - 1) / (x.sub * x.ni) * ((m + x.sub - 1) / x.sub) * act_batch, rounds = (wgs + cus - 1) / cus;
-        const float us = x.first + x.first_k * per_wave + (x.later + x.later_k * per_wave) * (float)(rounds - 1);
+        const Times &t = tiled ? x.tiles : x.planes;
+        const int64_t bm = x.sub * x.ms, bn = x.sub * x.ni, rounds = ((n + bn - 1) / bn * ((m + bm - 1) / bm) * act_batch + cus - 1) / cus;
+        const float us = t.first + t.first_k * per_wave + (t.later + t.later_k * per_wave) * (float)(rounds - 1);
         if (c == 0 || us < best_us) best = c, best_us = us;
     }
     switch (best) {
-        case 0: return launch(sub16, one);
-        case 1: return launch(sub16, two);
-        case 2: return launch(sub16, three);
-        case 3: return launch(sub16, four);
-        case 4: return launch(sub32, two);
-        case 5: return launch(sub32, three);
-        default: return launch(sub32, four);
+        case 0: return launch(sub16, one, one);
+        case 1: return launch(sub16, one, two);
+        case 2: return launch(sub16, one, three);
+        case 3: return launch(sub16, one, four);
+        case 4: return launch(sub32, one, one);
+        case 5: return launch(sub32, one, two);
+        case 6: return launch(sub32, one, three);
+        case 7: return launch(sub32, one, four);
+        default: return launch(sub32, two, two);
     }
 }
 

@@ -283,9 +283,12 @@ int launch_q4_0_matvec(const void *codes, const void *scales, int64_t w_batch, i
         const int rc = launch_q4_0_matmul(codes, scales, w_batch, n, k, act, act_dtype, act_batch, m, out, s);
         if (rc != 2) return rc;
     }
-    // f32 rows from 6 on, and 5 of a large matrix: one pass over the weights for all of them (us, here | there: 5 rows of 1000 x 2080 6.6 |
-    // 6.8, of 4090 x 4096 20.9 | 14.4; 6 rows 7.3 | 6.8, 26.4 | 14.5; 8 rows of 1000 x 2080 11.6 | 7.0)
-    if (act_dtype == TROCM_F32 && (m >= 6 || (m == 5 && n > 2048))) {
+    // f32 rows from 7 on: one pass over the weights for all of them; 5 and 6 of matrices that keep this kernel busy for more than a round, and
+    // 6 of smaller ones whose chain along k, which one round of that kernel takes, is not the longer (us, here | there: 5 rows of 1000 x 2080
+    // 6.6 | 6.8, of 3000 x 4128 12.0 | 11.4, of 4090 x 4096 18.6 | 14.3; 6 rows of 1000 x 2080 7.3 | 6.8, of 2010 x 8224 21.2 | 20.4, x 10272
+    // 24.9 | 26.0, of 3000 x 10272 30.5 | 26.1, of 500 x 14336 32.1 | 40.0; 8 rows of 1000 x 2080 11.6 | 7.0)
+    const bool one_pass = m >= 7 || (m >= 5 && n > 2048) || (m == 6 && k <= 9216);
+    if (act_dtype == TROCM_F32 && one_pass) {
         const int rc = launch_q4_0_matmul_f32(codes, scales, w_batch, n, k, act, act_batch, m, out, s, 0);
         if (rc != 2) return rc;
     }
