@@ -226,9 +226,11 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_waves_kernel(MatMulWav
 struct Shape { int ms, ni; float tiled, first, later; };
 // us of a round of workgroups, one per compute unit: tiles at 4096 features when there are several rounds; planes at 2080 features, the first
 // and later ones.  16 x 64 is for tiles where it saves a second round.  32 x 16, 48 x 32 and 64 x 32 are for planes, whose codes come in words of 4 bytes, so that a weight row costs more there:
-// 100 rows of 1000 x 2080 10.9 (16 x 32) -> 9.3 (32 x 16), 300 19.7 (32 x 64) -> 14.5 (48 x 32), 500 19.9 -> 15.4 (64 x 32).
+// 100 rows of 1000 x 2080 10.9 (16 x 32) -> 9.3 (32 x 16), 300 19.7 (32 x 64) -> 14.5 (48 x 32), 500 19.9 -> 15.4 (64 x 32).  32 x 64 is still
+// the best where the others need one more round (150 rows of 3000 x 3104 25.8, 64 x 64 30.3).  144 products with planes, 9 to 500 rows, 250
+// to 8200 weight rows, 544 to 14368 features: 0.93 of the time without these three, none longer.
 constexpr float kNever = 1e9f;
-constexpr Shape kShapes[] = {{1, 1, 5.0f, 7.3f, 5.0f},    {1, 2, 6.0f, 10.6f, 8.5f},    {2, 2, 10.0f, 12.4f, 10.5f},  {2, 4, 13.0f, kNever, kNever},
+constexpr Shape kShapes[] = {{1, 1, 5.0f, 7.3f, 6.0f},    {1, 2, 6.0f, 10.6f, 8.5f},    {2, 2, 10.0f, 12.4f, 10.5f},  {2, 4, 13.0f, 22.7f, 16.5f},
                              {4, 4, 20.0f, 23.0f, 20.0f}, {2, 1, kNever, 9.2f, 6.7f},   {3, 2, kNever, 14.5f, 12.5f}, {4, 2, kNever, 15.2f, 14.0f},
                              {1, 4, 9.0f, kNever, kNever}};
 int64_t workgroups(const Shape &c, int64_t n, int64_t m, int64_t act_batch) {
@@ -274,7 +276,7 @@ int launch_q4_0_matmul_waves(const void *codes, const void *scales, int64_t w_ba
         constexpr int MS = decltype(ms)::value, NI = decltype(ni)::value, DB = MS < 4 ? 4 : 2;
         const dim3 grid((unsigned)((n + 16 * NI - 1) / (16 * NI)), (unsigned)((m + 16 * MS - 1) / (16 * MS)), (unsigned)act_batch);
         if (grid.y > 65535) return 2;
-        constexpr bool TILES = !(NI == 1 && MS == 2) && !(NI == 2 && MS > 2), PLANES = !(MS <= 2 && NI == 4);   // (the other's never chosen)
+        constexpr bool TILES = !(NI == 1 && MS == 2) && !(NI == 2 && MS > 2), PLANES = !(MS == 1 && NI == 4);   // (the other's never chosen)
         if constexpr (TILES)
             if (tiled) hipLaunchKernelGGL((q4_0_matmul_waves_kernel<MS, NI, DB, true>), grid, dim3(64 * kW), 0, s, p);
         if constexpr (PLANES)
