@@ -302,8 +302,9 @@ __global__ __launch_bounds__(64 * NW * KS, BM == 32 && NW * KS >= 8 && NI == 1 ?
             // it + 1 is written into the other buffer after this half's arithmetic.
             __syncthreads();
             if (STEADY ? !LAST || hh + PA < 2 : 2 * t + hh + PA < 2 * Tg) prefetch_a(PA == 2 ? hh : 0, 2 * t + hh + PA);
-            // asked for here, not where it is used (but in sets of two waves, 64 rows: 40 rows of 4096 x 4096 8.5 us with this, 8.2 without)
-            if constexpr (STEADY && (BM != 64 || NI * NW != 2) && (BM != 32 || KS != 8)) __builtin_amdgcn_sched_barrier(0);
+            // asked for here, not where it is used (but in sets of two waves, 64 rows: 40 rows of 4096 x 4096 8.5 us with this, 8.2 without; and
+            // of one wave, one or two sets: 48 rows of 9216 x 2304 14.2 | 13.6, 17 10.8 | 10.6, 128 of 2560 x 6912 25.9 | 24.8)
+            if constexpr (STEADY && (BM != 64 || NI * NW != 2) && (BM != 32 || KS != 8) && (KS > 2 || NW > 1)) __builtin_amdgcn_sched_barrier(0);
             const _Float16 *at = &lds_a[hh * BM * AROW + a_frag];
             half8_t bf[2][MS];   // the activation fragments of a step are read during the step before
 #pragma unroll
