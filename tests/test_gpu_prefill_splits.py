@@ -2,6 +2,9 @@
 to eight and up to sixteen), one and two workgroups on a compute unit at head size 64, one head per workgroup with few queries, small
 scratch, and what the kernel without parts takes."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -177,3 +180,24 @@ def test_tiles_left_for_the_last_round(rt, store, B, Hq, Hkv, past, n, causal, l
         for b, h in ((0, 0), (B - 1, Hkv - 1)):
             want = textbook_sdpa(q[b : b + 1, h * G : (h + 1) * G], k[b : b + 1, h : h + 1], v[b : b + 1, h : h + 1], causal=causal)
             assert np.linalg.norm(cut[b, h * G : (h + 1) * G] - want[0]) <= TOL * np.linalg.norm(want)
+
+
+def test_no_merge_by_the_last_to_arrive_means_no_cut():
+    """TROCM_PREFILL_TAIL_MERGE=0 (no workgroup waits for or merges another's results) leaves a last round as whole as
+    TROCM_PREFILL_PARTS=0 does: the same bits, others than those of the cut."""
+    code = """
+import sys; sys.path.insert(0, %r)
+import numpy as np, tract_amd as ta
+ta.runtime_for_name("rocm")
+rng = np.random.default_rng(5)
+q, k, v = (rng.standard_normal((1, h, n, 128), dtype=np.float32).astype(np.float16) for h, n in ((168, 400), (42, 1400), (42, 1400)))
+sys.stdout.buffer.write(ta.Sdpa(datum_type=np.float16, is_causal=True).eval(q, k, v).to_numpy().tobytes())
+""" % os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+    def run(**env):
+        p = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, **env), capture_output=True, timeout=100)
+        assert p.returncode == 0, p.stderr[-2000:]
+        return p.stdout[-168 * 400 * 128 * 2 :]
+
+    cut, whole = run(), run(TROCM_PREFILL_PARTS="0")
+    assert run(TROCM_PREFILL_TAIL_MERGE="0") == whole != cut

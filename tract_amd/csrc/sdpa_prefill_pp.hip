@@ -1292,6 +1292,8 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
     const int64_t cus = num_compute_units();
     const size_t elem = p.part32 ? sizeof(float) : sizeof(_Float16), per_split = split_bytes(p.n_wb, a.D, elem);
     const size_t avail = a.workspace && a.workspace_bytes > kWsCounterBytes + 256 ? a.workspace_bytes - kWsCounterBytes - 256 : 0;
+    // TROCM_PREFILL_TAIL_MERGE=0: nothing is merged by the last workgroup to arrive (a merge launch, or no cut of the last round)
+    static const int tail_merge = env_int("TROCM_PREFILL_TAIL_MERGE", 1);
     int64_t ns = forced_split < kMaxSplits ? forced_split : kMaxSplits;
     if (forced_split <= 0) ns = wgs1 < cus ? choose_splits(p, (int)a.D, block_m, wgs1, cus, (int64_t)(avail / per_split)) : 1;
     if (ns > 1 && (size_t)ns * per_split > avail) ns = (int64_t)(avail / per_split);
@@ -1302,14 +1304,12 @@ int launch_sdpa_prefill_pp(const SdpaArgs &a, hipStream_t s) {
         base += (256 - ((uintptr_t)base & 255)) & 255;
         p.part_o = (_Float16 *)base;
         p.part_ml = (float *)(base + (size_t)ns * p.n_wb * 32 * a.D * elem);
-        // With few enough tiles for the counter area the last split to arrive merges (no second launch);
-        // TROCM_PREFILL_TAIL_MERGE=0 keeps the merge launch.
-        static const int tail_merge = env_int("TROCM_PREFILL_TAIL_MERGE", 1);
+        // with few enough tiles for the counter area the last split to arrive merges (no second launch)
         if (tail_merge && !p.part32 && ns <= kTailSplits && wgs1 <= (int64_t)(kWsCounterBytes / sizeof(int))) p.counters = (int *)a.workspace;
     }
     int64_t wgs = wgs1 * ns;
     static const int cut_last = env_int("TROCM_PREFILL_PARTS", 1);
-    if (cut_last && ns == 1 && forced_split <= 0 && a.D == 128 && !p.mask && !p.part32 && !ping_enabled()) {
+    if (cut_last && tail_merge && ns == 1 && forced_split <= 0 && a.D == 128 && !p.mask && !p.part32 && !ping_enabled()) {
         const int64_t per_q = wgs1 / n_qtiles;
         int whole = 0;
         const int parts = choose_parts(p, block_m, per_q, cus, whole);
