@@ -40,12 +40,14 @@ def _state(k, v, past, n, causal):
 
 
 # the first new row on a tile's edge, before it and behind it, all of them in one tile; pieces that do not go round; 1 to 8 query heads
-# per kv head, key splits merged by the last of them and by a launch, a workgroup alone on its unit; f32: none, one and many ranges of
-# keys, one workgroup, shapes that the launch does not take (few tiles, a cache that is not empty)
+# per kv head, key splits merged by the last of them and by a launch, a workgroup alone on its unit, a last round cut into 2, 3 and 4
+# ranges of keys (1, 2 and 4 query heads per workgroup); f32: none, one and many ranges of keys, one workgroup, behind whole tiles of keys
+# (behind others the sums are taken in another order: below)
 @pytest.mark.parametrize("dtype,B,Hq,Hkv,D,past,n", [
     (np.float16, 1, 8, 2, 128, 640, 150), (np.float16, 2, 8, 2, 128, 639, 99), (np.float16, 1, 16, 4, 128, 65, 301), (np.float16, 1, 14, 2, 128, 700, 99),
     (np.float16, 2, 4, 4, 128, 0, 700), (np.float16, 1, 32, 32, 64, 30, 1001), (np.float16, 3, 16, 2, 64, 1, 333), (np.float16, 4, 64, 8, 64, 0, 300),
     (np.float16, 1, 8, 8, 64, 2000, 70), (np.float16, 1, 32, 8, 128, 3000, 41), (np.float16, 1, 2, 1, 128, 5, 65),
+    (np.float16, 2, 60, 60, 128, 1300, 530), (np.float16, 1, 128, 64, 128, 1300, 613), (np.float16, 1, 168, 42, 128, 1001, 400),
     (np.float32, 1, 8, 2, 128, 0, 150), (np.float32, 2, 14, 2, 64, 0, 171), (np.float32, 1, 32, 32, 128, 0, 333), (np.float32, 1, 6, 6, 64, 0, 1100),
     (np.float32, 1, 8, 2, 128, 0, 60), (np.float32, 1, 8, 2, 128, 64, 200)])
 def test_rows_from_the_call(rt, dtype, B, Hq, Hkv, D, past, n):
@@ -70,6 +72,26 @@ def test_results_over_the_new_rows(rt, dtype, past, n, over):
     got = st.eval_into(ta.DeviceTensor.from_numpy(q), args["k"], args["v"], args[over]).to_numpy()
     assert st.k.valid_contiguous().tobytes() == k.tobytes() and st.v.valid_contiguous().tobytes() == v.tobytes()
     assert got.tobytes() == _over_one_tensor(q, k, v, True).tobytes()
+
+
+# new rows that do not begin on a 16-byte boundary: an append launch, then the attention (a few queries on the decode tiles, a prompt, f32)
+@pytest.mark.parametrize("dtype,Hq,past,n", [(np.float16, 8, 300, 3), (np.float16, 8, 300, 150), (np.float16, 8, 0, 70), (np.float32, 8, 300, 3), (np.float32, 8, 65, 150), (np.float32, 8, 0, 70)])
+def test_rows_that_the_launch_does_not_take(rt, dtype, Hq, past, n):
+    q, k, v = _inputs(dtype, 2, Hq, 2, 128, past, n)
+    st = _state(k, v, past, n, True)
+
+    def shifted(x):
+        x = np.ascontiguousarray(x)
+        whole = ta.DeviceTensor.from_numpy(np.concatenate([np.zeros(1, dtype), x.ravel()]))
+        return ta.DeviceTensor(x.shape, dtype, ptr=whole.ptr.value + whole.dtype.itemsize, owner=whole)
+
+    for _ in range(2):
+        if past or _:
+            st.k.truncate(past), st.v.truncate(past)
+        got = st.eval_into(ta.DeviceTensor.from_numpy(q), shifted(k[:, :, past:]), shifted(v[:, :, past:])).to_numpy()
+        assert st.k.len() == st.v.len() == past + n
+        assert st.k.valid_contiguous().tobytes() == k.tobytes() and st.v.valid_contiguous().tobytes() == v.tobytes()
+        assert got.tobytes() == _over_one_tensor(q, k, v, True).tobytes()
 
 
 # f32 rows behind a cache whose last tile of keys is not full (the call's rows begin a tile of their own): one row and all but one of a tile,
