@@ -530,8 +530,8 @@ int launch_q4_0_tiled_export(const void *tiles, void *blocks, int64_t rows, int6
 }
 
 // Tiled weights x activations for any m: f16 rows in groups of up to 16 (more than 16 rows go to the matrix-matrix
-// kernel first, which reads the same tiles, when it takes the call), up to 5 f32 rows (more go to q4_matmul_f32.hip; in
-// groups of 8 what that refuses, and few rows of tall matrices).
+// kernel first, which reads the same tiles, when it takes the call), f32 rows in groups of 8: up to 4, up to 6 where the line below
+// leaves them here, up to 8 of tall matrices, and what q4_matmul_f32.hip, which takes the others, refuses.
 int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int64_t k, const void *act, int act_dtype,
                              int64_t act_batch, int64_t m, void *out, hipStream_t s) {
     if (n >= (1ll << 30) || k >= (1ll << 30) || act_batch > 65535) return fail("q4_0_matvec: shape too large");
@@ -552,7 +552,8 @@ int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int6
         const int rc = launch_q4_0_matmul(tiles, nullptr, w_batch, n, k, act, act_dtype, act_batch, m, out, s, 1);
         if (rc != 2) return rc;
     }
-    // f32 rows from 7 on, and 5 and 6 of a small matrix: one pass over the weights for all of them (us, here | there: 5 rows of 5120 x 5120 17.9 |
+    // f32 rows from 7 on, and 5 and 6 of a matrix that one round of that kernel takes (up to 8192 weight rows: 16 x 32 to a workgroup): one
+    // pass over the weights for all of them.  Between 8193 and 24576 weight rows 5 and 6 stay here (us, here | there: 5 rows of 5120 x 5120 17.9 |
     // 11.8, 4096 x 4096 8.5 | 8.3, 1024 x 4096 8.0 | 7.3, 14336 x 4096 14.9 | 15.7, 4096 x 14336 22.7 | 23.8; 6 rows 4096 x 14336 30.5 | 24.0,
     // 8192 x 8192 25.1 | 18.7, 4096 x 4096 8.8 | 8.4, 14336 x 4096 15.5 | 15.8; 4 rows of 4096 x 4096 6.6 | 8.2).  Its workgroups of 16 rows
     // take up to 64 weight rows each, one workgroup per compute unit: 6 to 8 rows of a tall matrix need several rounds of them, while a pass
