@@ -104,18 +104,34 @@ def test_shapes_with_k_shared_among_waves(rt, m, n, k):
 
 
 # more activation rows than a grid has tiles of: the bits of the same rows in calls that fit (one pass over the weights in every case)
-@pytest.mark.parametrize("m,n", [(65535 * 32 + 33, 33), (65535 * 16 + 5, 16)])
-def test_more_f32_rows_than_a_grid_holds(rt, m, n):
+@pytest.mark.parametrize("m,n,k", [(65535 * 64 + 33, 33, 32), (65535 * 16 + 5, 16, 32), (65535 * 16 + 5, 16, 128)])
+def test_more_f32_rows_than_a_grid_holds(rt, m, n, k):
     rng = np.random.default_rng(n)
-    k, part = 32, 999_968   # (whole tiles of 16 and of 32 rows)
+    part = 999_936   # (whole tiles of every shape)
     blocks = orc.quant(orc.FMT_Q4_0, (0.05 * rng.standard_normal((n, k), dtype=np.float32)).astype(np.float32))
     w, op = ta.Q40Weights(blocks, 1, n, k), ta.GgmlGemm()
     act = rng.standard_normal((1, m, k), dtype=np.float32)
     got = op.eval(ta.DeviceTensor.from_numpy(act), w).to_numpy()[0]
     for at in range(0, m, part):
         want = op.eval(ta.DeviceTensor.from_numpy(np.ascontiguousarray(act[:, at : at + part])), w).to_numpy()[0]
-        whole = min(part, m - at) // 32 * 32   # (the few rows left of a call may be given a tile of another shape)
+        whole = min(part, m - at) // 64 * 64   # (the few rows left of a call may be given a tile of another shape)
         if whole > 512:
             np.testing.assert_array_equal(got[at : at + whole], want[:whole])
     tail = act[0, -40:].astype(np.float64) @ orc.dequant(orc.FMT_Q4_0, blocks, np.float32).reshape(n, k).astype(np.float64).T
     assert np.abs(got[-40:] - tail).max() <= 1e-5
+
+
+# ... of several batches, over their own weights and over shared ones: planes and tiles
+@pytest.mark.parametrize("batches,w_batches,n,k", [(2, 2, 16, 96), (2, 1, 16, 128), (4, 2, 15, 32)])
+def test_more_f32_rows_than_a_grid_holds_in_batches(rt, batches, w_batches, n, k):
+    rng = np.random.default_rng(n + batches)
+    m = 65535 * 16 + 21
+    blocks = [orc.quant(orc.FMT_Q4_0, (0.05 * rng.standard_normal((n, k), dtype=np.float32)).astype(np.float32)) for _ in range(w_batches)]
+    act = np.zeros((batches, m, k), np.float32)
+    rows = np.concatenate([[0, 1, 65535 * 16 - 1, 65535 * 16, m - 1], rng.integers(0, m, 30)])   # (the others are zeros)
+    act[:, rows] = rng.standard_normal((batches, len(rows), k), dtype=np.float32)
+    got = ta.GgmlGemm().eval(ta.DeviceTensor.from_numpy(act), ta.Q40Weights(np.concatenate([np.asarray(x).reshape(-1) for x in blocks]), w_batches, n, k)).to_numpy()
+    for b in range(batches):
+        w = orc.dequant(orc.FMT_Q4_0, blocks[b * w_batches // batches], np.float32).reshape(n, k).astype(np.float64)
+        assert np.abs(got[b, rows] - act[b, rows].astype(np.float64) @ w.T).max() <= 1e-5
+        assert np.count_nonzero(np.delete(got[b], rows, axis=0)) == 0

@@ -49,7 +49,6 @@ struct MatMulF32 {
     const float *act;         // [act_batch, m, k]
     float *out;               // [act_batch, m, n]
     int n, k, m, ratio;       // ratio = act_batch / w_batch
-    int tile0;                // tiles of activation rows ahead of this launch's
 };
 
 template <int SUB> struct AccOf;
@@ -99,7 +98,7 @@ __global__ __launch_bounds__(64 * kW, 2) void q4_0_matmul_f32_kernel(MatMulF32 p
 
     const int tid = threadIdx.x, lane = tid & 63, row = lane % SUB, grp = lane / SUB;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n0 = blockIdx.x * SUB * NI, m0 = (p.tile0 + blockIdx.y) * SUB * MS, b = blockIdx.z, wb = b / p.ratio;
+    const int n0 = blockIdx.x * SUB * NI, m0 = blockIdx.y * SUB * MS, b = blockIdx.z, wb = b / p.ratio;
     const int nb = p.k / 32, units = (nb + 3) / 4;
     // slot g of a block: its features 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3.  Instruction st of a block contracts slots
     // 2 st + grp (SUB 32) or all four (SUB 16).
@@ -357,16 +356,25 @@ int launch_q4_0_matmul_f32(const void *codes, const void *scales, int64_t w_batc
     const int64_t cus = num_compute_units();
     auto launch = [&](auto sub, auto ms, auto ni) -> int {
         constexpr int SUB = decltype(sub)::value, MS = decltype(ms)::value, NI = decltype(ni)::value;
-        const int64_t row_tiles = (m + SUB * MS - 1) / (SUB * MS);
-        for (int64_t t = 0; t < row_tiles; t += 65535) {   // (a launch: as many as its grid holds)
-            const dim3 grid((unsigned)((n + SUB * NI - 1) / (SUB * NI)), (unsigned)std::min<int64_t>(65535, row_tiles - t), (unsigned)act_batch);
-            p.tile0 = (int)t;
-            constexpr bool TILES = !(SUB == 32 && (MS == 2 || NI == 1)), PLANES = SUB == 16 ? NI <= 2 : NI <= 3;   // (the other's never chosen)
+        constexpr bool TILES = !(SUB == 32 && (MS == 2 || NI == 1)), PLANES = SUB == 16 ? NI <= 2 : NI <= 3;   // (the other's never chosen)
+        auto grid_of = [&](const MatMulF32 &part, int64_t batches) {
+            const dim3 grid((unsigned)((n + SUB * NI - 1) / (SUB * NI)), (unsigned)((part.m + SUB * MS - 1) / (SUB * MS)), (unsigned)batches);
             if constexpr (TILES)
-                if (tiled) hipLaunchKernelGGL((q4_0_matmul_f32_kernel<SUB, MS, NI, true>), grid, dim3(64 * kW), 0, s, p);
+                if (tiled) hipLaunchKernelGGL((q4_0_matmul_f32_kernel<SUB, MS, NI, true>), grid, dim3(64 * kW), 0, s, part);
             if constexpr (PLANES)
-                if (!tiled) hipLaunchKernelGGL((q4_0_matmul_f32_kernel<SUB, MS, NI, false>), grid, dim3(64 * kW), 0, s, p);
-        }
+                if (!tiled) hipLaunchKernelGGL((q4_0_matmul_f32_kernel<SUB, MS, NI, false>), grid, dim3(64 * kW), 0, s, part);
+        };
+        const int64_t most = 65535ll * SUB * MS;   // rows that a grid has tiles for
+        if (m <= most) grid_of(p, act_batch);
+        for (int64_t b = 0; m > most && b < act_batch; b++)
+            for (int64_t row = 0; row < m; row += most) {
+                MatMulF32 part = p;
+                part.codes += b / p.ratio * (tiled ? n / 16 * (k / 128) * kTile : n * (k / 2));
+                if (!tiled) part.scales += b / p.ratio * n * (k / 32);
+                part.act += (b * m + row) * k, part.out += (b * m + row) * n;
+                part.m = (int)std::min(most, m - row), part.ratio = 1;
+                grid_of(part, 1);
+            }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return fail("q4_0_matmul (f32) launch failed: %s", hipGetErrorString(e));
         return 0;
@@ -384,7 +392,8 @@ int launch_q4_0_matmul_f32(const void *codes, const void *scales, int64_t w_batc
     // -> 216.  Squares share more of the split of the activations, oblongs of the same size have half the registers for it: 64 x 64 is
     // 250 there.  The codes of planes come in words of 4 bytes, so that a weight row costs more and squares stay the better ones (us, as
     // for tiles | as here: 40 rows of 4090 x 4096 39.3 | 27.1 (32 x 32), 500 127 | 111 (64 x 64), 200 of 1000 x 2080 16.2 | 13.1); 0.984 of
-    // the time by one number each over those 144 products, none longer.  Below 1024 features, where some waves have no unit, a launch takes its
+    // the time by one number each over those 144 products, none longer, and 0.96 over 539 of up to 50000 x 4128 and 2000 rows (at most
+    // 1.07, but for 8 and 16 rows of 16390 x 2080, one tile more than two rounds, 1.18 and 1.10).  Below 1024 features, where some waves have no unit, a launch takes its
     // 4 to 5 us and is still the faster side (groups of 8 rows | here: 7 rows of 4096 x 32 7.1 | 4.1, of 4096 x 512 5.4 | 4.2; 40 rows of
     // 16384 x 128 23.7 | 7.7, of 1000 x 96 24.7 | 4.5).
     struct Times { float first, first_k, later, later_k; };
@@ -394,9 +403,9 @@ int launch_q4_0_matmul_f32(const void *codes, const void *scales, int64_t w_batc
                             {16, 1, 3, {2.6f, 2.45f, 0.25f, 2.17f}, {kNever}},                     {16, 1, 4, {2.3f, 2.93f, 0.3f, 2.45f}, {kNever}},
                             {32, 1, 1, {kNever}, {0.78f, 5.04f, -1.76f, 5.06f}},                   {32, 1, 2, {2.6f, 4.08f, 1.9f, 4.1f}, {0.68f, 7.33f, -0.06f, 7.24f}},
                             {32, 1, 3, {3.6f, 5.05f, 3.0f, 5.45f}, {0.92f, 9.86f, 1.87f, 9.37f}},  {32, 1, 4, {4.3f, 6.1f, 4.2f, 6.4f}, {kNever}},
-                            {32, 2, 2, {kNever}, {1.64f, 10.62f, 2.59f, 10.83f}}};
+                            {32, 2, 2, {kNever}, {1.64f, 10.62f, 2.59f, 10.0f}}};
     const int64_t units = (k + 127) / 128, last = k / 32 - 4 * (units - 1);   // blocks of the last unit, which is a wave's last if no other one has as many
-    const float per_wave = (float)((units - 1) / 8 * 4 + ((units - 1) % 8 ? 4 : last)) / 4.0f;
+    const float per_wave = std::max(0.5f, (float)((units - 1) / 8 * 4 + ((units - 1) % 8 ? 4 : last)) / 4.0f);   // (the lines end there)
     int best = 0;
     float best_us = 0.0f;
     for (int c = 0; c < 9; c++) {
