@@ -182,6 +182,27 @@ def test_tiles_left_for_the_last_round(rt, store, B, Hq, Hkv, past, n, causal, l
             assert np.linalg.norm(cut[b, h * G : (h + 1) * G] - want[0]) <= TOL * np.linalg.norm(want)
 
 
+def test_a_cut_over_counters_that_are_not_zero_ends(rt):
+    """A workspace whose header is not what trocm_sdpa_workspace_init left: no part of a tile is the first to arrive, nothing is stored, and all
+    of them stop waiting for it.  After another init the workspace serves again."""
+    B, Hq, Hkv, past, n, causal, _, _ = CUT[0]
+    rng = np.random.default_rng(1)
+    q, k, v = _normal(rng, B, Hq, n, 128), _normal(rng, B, Hkv, past + n, 128), _normal(rng, B, Hkv, past + n, 128)
+    kc, vc = ta.InPlaceKvCache(2), ta.InPlaceKvCache(2)
+    kc.push(k), vc.push(v)
+    dq, out, ws = ta.DeviceTensor.from_numpy(q), ta.DeviceTensor(q.shape, np.float16), ta.Workspace(B, Hq, n, 128)
+
+    def run():
+        call("trocm_sdpa_cached", dq.ptr, ta.F16, Hq, n, kc._h, vc._h, out.ptr, C.c_float(float("nan")), int(causal), ws.ptr, ws.nbytes, None)
+        return out.to_numpy().tobytes()
+
+    want = run()
+    call("trocm_memset", ws.ptr, 0x40, 64 * 1024, None)
+    run()
+    call("trocm_sdpa_workspace_init", ws.ptr, ws.nbytes, None)
+    assert run() == want
+
+
 def test_no_merge_by_the_last_to_arrive_means_no_cut():
     """TROCM_PREFILL_TAIL_MERGE=0 (no workgroup waits for or merges another's results) leaves a last round as whole as
     TROCM_PREFILL_PARTS=0 does: the same bits, others than those of the cut."""

@@ -104,6 +104,7 @@ template <int N, class F>
 __device__ __attribute__((always_inline)) inline void static_for(F &&f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
 constexpr float kLazyMax = 8.0f;
 constexpr int kMaxSplits = 16, kTailSplits = 4;   // key splits; those that the last of them to arrive merges itself
+constexpr int kMostLooks = 1 << 17;   // of a workgroup at a counter that others have yet to add to (a look is most of a microsecond)
 #ifndef TROCM_PING_PRIO_MFMA
 #define TROCM_PING_PRIO_MFMA 1
 #endif
@@ -794,8 +795,12 @@ __global__ __launch_bounds__(kThreadsPP, ALONE ? 2 : 4) void sdpa_prefill_pp_ker
         }
         __syncthreads();   // (s_word has been read)
         if (tid == 0) {
-            int word;
-            while ((((word = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 8) & 255) != nsplit - 1) __builtin_amdgcn_s_sleep(1);
+            int word = 0;   // (a counter that was not zero before the launch never gets there: looked at so often, about a tenth of a second)
+            for (int looks = 0; looks < kMostLooks; looks++) {
+                word = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (((word >> 8) & 255) == nsplit - 1) break;
+                __builtin_amdgcn_s_sleep(1);
+            }
             __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
             s_word = word;
         }
