@@ -93,7 +93,7 @@ struct MfmaWork {
 // The tail every formulation shares: the four waves' records (O[GP][D], m[GP], l[GP], in `lds_raw`, kCombStride floats
 // each) become the output rows (one split), or this workgroup's partial record, merged by the last workgroup to
 // arrive or by the merge launch.
-template <int D, int GP, bool ROWS = false>
+template <int D, int GP, bool TAIL_ROWS = false>
 __device__ __forceinline__ void wave_records_to_output(const DecodeDev &p, const MfmaWork &wk, unsigned char *lds_raw, int64_t head0,
                                                        int g, int tid) {
     constexpr int kCombStride = GP * D + 2 * GP;
@@ -143,11 +143,9 @@ __device__ __forceinline__ void wave_records_to_output(const DecodeDev &p, const
             }
         }
     }
-    if constexpr (ROWS && GP > 8) {
-        if (wk.nsplit > 1 && wk.counter != nullptr) {
-            __syncthreads();   // (the weights go where the waves' records were)
-            tail_merge_rows<__half, D, GP, kRowsMergeMax>(p, wk.counter, wk.nsplit, wk.part_first, out, g, tid, comb);
-        }
+    if constexpr (TAIL_ROWS) {
+        __syncthreads();   // (the weights go where the waves' records were)
+        tail_merge_rows<__half, D, GP, kRowsMergeMax>(p, wk.counter, wk.nsplit, wk.part_first, out, g, tid, comb);
     }
     if constexpr (GP <= 8) {   // (larger groups of heads: the merge launch; the in-kernel merge would need too many registers)
         if (wk.nsplit > kTailMergeMax && wk.counter != nullptr)
@@ -223,7 +221,7 @@ __device__ __forceinline__ uint32_t not_finite(uint32_t pair) { return ((((pair 
 // tile.  Error against 64 bits over 24 drawn batches: 0.98 of that of items of a few tiles, rounded against the wave's largest; 1.03
 // (1.11 at most) with the longer items rounded so.  f16 batches take 0 to 1 % longer for it, Q4_0 ones up to 14 % (42.2 -> 48.1 us, 59.0
 // with the short items).
-template <int D, int GP, int FMT, bool MASK = false, bool W16 = false, bool ROPE = false, bool ROWS = false, bool FINE = false>
+template <int D, int GP, int FMT, bool MASK = false, bool W16 = false, bool ROPE = false, bool ROWS = false, bool FINE = false, bool TAIL_ROWS = false>
 __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaWork &wk) {
     static_assert(!W16 || GP <= 16, "the 16-wide layout: at most 16 heads");
     static_assert(!FINE || (W16 && !MASK && !ROWS), "ragged batches on the 16-wide tiles");
@@ -751,7 +749,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeDev &p, const MfmaW
             cw[GP * D + GP + l32_end] = l_run;
         }
     }
-    wave_records_to_output<D, GP, ROWS>(p, wk, lds_raw, head0, g, tid);
+    wave_records_to_output<D, GP, TAIL_ROWS>(p, wk, lds_raw, head0, g, tid);
 }
 
 // Transposing 64-bit LDS load of 8-bit elements: in each block of 16 lanes, lane i receives byte i%8 of the eight
@@ -2179,7 +2177,9 @@ __global__ __launch_bounds__(kThreads, (QB ? QB % 10 : 2)) void sdpa_decode_mfma
 // Several queries per sequence: grid (splits, kv_heads * row groups, batch).  Row r = head r / q_len, query r % q_len of a
 // kv head's G q_len rows (consecutive in q and in the output); group i takes up to g_real of them from i g_real on.  (Not one
 // of them twice: the output may lie over q, whose rows must not be read once another group has stored its results.)
-template <int D, int GP, int FMT, bool W16>
+// TAIL: records of more than 8 rows, merged by the last workgroup to arrive (an instantiation of its own: calls of one range of keys
+// over a few hundred tokens took 0.25 us of 9 to 12 longer with that merge behind a condition).
+template <int D, int GP, int FMT, bool W16, bool TAIL = false>
 __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_rows_kernel(DecodeDev p) {
     const int split = blockIdx.x, kvh = blockIdx.y / p.n_groups, group = blockIdx.y % p.n_groups, b = blockIdx.z;
     MfmaWork wk;
@@ -2202,7 +2202,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_rows_kernel(DecodeDev
     wk.mask = nullptr;
     wk.row_in_head0 = group * p.g_real, wk.rows = min(p.g_real, p.n_rows - wk.row_in_head0);
     wk.row0 = ((int64_t)b * p.Hkv + kvh) * p.n_rows + wk.row_in_head0;
-    decode_mfma_body<D, GP, FMT, false, W16, false, true>(p, wk);
+    decode_mfma_body<D, GP, FMT, false, W16, false, true, false, TAIL>(p, wk);
 }
 
 // Merge launch of the above: grid (kv_heads * row groups, batch, rows of a group), D threads.
@@ -2366,7 +2366,10 @@ int launch_quant(const DecodeDev &p, int gp, dim3 grid, hipStream_t s) {
 
 template <int D, int GP, int FMT>
 int launch_rows(const DecodeDev &p, dim3 grid, hipStream_t s) {
-    hipLaunchKernelGGL((sdpa_decode_rows_kernel<D, GP, FMT, (GP <= 16)>), grid, dim3(kThreads), 0, s, p);
+    if (GP > 8 && p.counters)
+        hipLaunchKernelGGL((sdpa_decode_rows_kernel<D, GP, FMT, (GP <= 16), (GP > 8)>), grid, dim3(kThreads), 0, s, p);
+    else
+        hipLaunchKernelGGL((sdpa_decode_rows_kernel<D, GP, FMT, (GP <= 16)>), grid, dim3(kThreads), 0, s, p);
     if (p.nsplit > 1 && p.counters == nullptr)
         hipLaunchKernelGGL((sdpa_decode_rows_merge_kernel<D, GP>), dim3(grid.y, grid.z, p.g_real), dim3(D), 0, s, p);
     hipError_t e = hipGetLastError();
