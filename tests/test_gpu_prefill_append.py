@@ -94,6 +94,17 @@ def test_rows_that_the_launch_does_not_take(rt, dtype, Hq, past, n):
         assert got.tobytes() == _over_one_tensor(q, k, v, True).tobytes()
 
 
+# f32 rows that would begin a fifth tile of keys in one range, or a ninth, where a workgroup's four waves take four at once: an append launch,
+# then whole tiles
+@pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [(1, 40, 8, 64, 56, 71), (1, 32, 32, 128, 100, 10), (2, 32, 8, 128, 97, 3), (1, 14, 2, 64, 65, 63), (16, 32, 32, 64, 250, 4)])
+def test_rounds_of_four_tiles_stay_full(rt, B, Hq, Hkv, D, past, n):
+    q, k, v = _inputs(np.float32, B, Hq, Hkv, D, past, n)
+    st = _state(k, v, past, n, True)
+    got = st.eval([q, np.ascontiguousarray(k[:, :, past:]), np.ascontiguousarray(v[:, :, past:])]).to_numpy()
+    assert st.k.valid_contiguous().tobytes() == k.tobytes() and st.v.valid_contiguous().tobytes() == v.tobytes()
+    assert got.tobytes() == _over_one_tensor(q, k, v, True).tobytes()
+
+
 # f32 rows behind a cache whose last tile of keys is not full (the call's rows begin a tile of their own): one row and all but one of a tile,
 # up to 32 rows per kv head and more, ranges of keys, 1 to 8 query heads per kv head
 @pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [(1, 8, 2, 128, 1, 3), (2, 4, 4, 64, 31, 2), (1, 14, 2, 128, 348, 10), (3, 32, 8, 64, 801, 11), (6, 32, 8, 128, 910, 3), (1, 8, 2, 128, 33, 200),

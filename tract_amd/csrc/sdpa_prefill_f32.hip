@@ -832,6 +832,11 @@ int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
         };
         const int64_t most = n_wg < want ? (want + n_wg - 1) / n_wg : 1, fours = cut_tiles < 8 ? 1 : (cut_tiles + 3) / 4;
         ns = not_empty(std::min(most, n_wg * fours <= cus || (fours <= 4 && n_wg * fours <= want) ? fours : cut_tiles / 4));
+        // An append launch instead where the tile that is not full would be a fifth in the one range of keys, which four waves take twice, or
+        // a ninth, a thirteenth and so on where whole rows keep all units busy.  (us, append launch | in here: 32 heads over 32, 10
+        // queries behind 100 tokens 13.3 | 15.8, 64 over 8, 40 behind 70 13.9 | 16.4, 40 over 8 of 64 features, 71 behind 56 10.0 | 10.6; 16 x 32 over
+        // 32, 4 behind 250 36.8 | 40.2, behind 760 84.1 | 86.4; no tile more: 14 over 2, 20 behind 90 13.7 | 11.7.)
+        if (a.k_new && ns == 1 && (cut_tiles + 3) / 4 > (tiles + 3) / 4) return 2;
     }
     ns = ns < kMaxSplits ? ns : kMaxSplits;
     p.paired = pairs && a.causal && n_wg <= want;
