@@ -91,7 +91,9 @@ def test_shapes_of_the_f32_product(rt, m, n, k):
 
 
 # f16 rows with k shared among waves: 32 x 16, 48 x 32, 64 x 32 and 32 x 64 (planes), 6 to 8 rows of tiles, and 16 x 64 of tall ones
-@pytest.mark.parametrize("m,n,k", [(90, 1010, 1056), (290, 1010, 160), (290, 1001, 2080), (450, 1010, 1056), (470, 1001, 96), (150, 3001, 160), (149, 3000, 1056), (6, 4112, 1152), (7, 5136, 384), (8, 272, 2176), (8, 12240, 384), (9, 14352, 1152), (16, 16384, 256), (16, 8208, 128)])
+@pytest.mark.parametrize("m,n,k", [(90, 1010, 1056), (290, 1010, 160), (290, 1001, 2080), (450, 1010, 1056), (470, 1001, 96), (150, 3001, 160), (149, 3000, 1056), (6, 4112, 1152), (7, 5136, 384), (8, 272, 2176), (8, 12240, 384), (9, 14352, 1152), (16, 16384, 256), (16, 8208, 128),
+                                   # ... and those beside them that stay in one pass of the streaming kernel: all features in LDS, and four tiles a wave
+                                   (6, 272, 12288), (7, 1040, 9216), (8, 528, 8192), (8, 4096, 4096), (6, 16, 4096)])
 def test_shapes_with_k_shared_among_waves(rt, m, n, k):
     rng = np.random.default_rng(n + k + m)
     blocks = orc.quant(orc.FMT_Q4_0, (0.05 * rng.standard_normal((n, k), dtype=np.float32)).astype(np.float32))

@@ -538,9 +538,13 @@ int launch_q4_0_tiled_matvec(const void *tiles, int64_t w_batch, int64_t n, int6
     // (a row group's records are addressed through one buffer descriptor: 32-bit offsets)
     if ((k / 128) * kTile >= (1ll << 31)) return fail("q4_0_matvec: rows of %lld features are too long for the tiled layout", (long long)k);
     // 6 f16 rows and more with few tiles (us, the kernel above | there: 5 rows of 4096 x 14336 11.5 | 11.9, of 1024 x 14336 10.9 | 11.4; 6 rows
-    // 14.4 | 12.2, 13.4 | 11.9, of 5120 x 5120 8.7 | 7.0, of 8192 x 8192 11.5 | 10.7, of 4096 x 4096 5.6 | 5.4; 8 rows of 4096 x 14336 15.3 |
-    // 12.7, of 1024 x 4096 5.4 | 5.5; 16 rows 23.1 | 18.3, of 4096 x 4096 8.3 | 8.0)
-    if (act_dtype == TROCM_F16 && m >= 6 && q4_0_matmul_waves_fits(n, m, act_batch, true)) {
+    // 14.4 | 12.2, 13.4 | 11.9, of 5120 x 5120 8.7 | 7.0, of 4096 x 2048 4.5 | 4.0; 8 rows of 4096 x 14336 15.3 | 12.7, of 6144 x 4096 7.9 | 6.5;
+    // 16 rows 23.1 | 18.3, of 4096 x 4096 8.3 | 8.0).  Up to 8 rows whose features are many and yet all fit LDS here stay, and those of 32 tiles,
+    // four for each of a row group's 8 waves, where no unit has a second group (6 rows of 4096 x 12288 10.9 | 12.9, of 12288 x 8192 16.6 |
+    // 18.1, of 1024 x 10240 8.6 | 9.2; 7 of 4096 x 9216 8.8 | 8.9; 8 of 6144 x 8192 11.6 | 12.2, of 2048 x 4096 5.3 | 5.6).
+    const bool whole = m * k * 2 + 16 * 1024 <= 160 * 1024;
+    const bool stays = m <= 8 && whole && (k >= 8192 || (k == 4096 && n / 16 * act_batch <= num_compute_units()));
+    if (act_dtype == TROCM_F16 && m >= 6 && !stays && q4_0_matmul_waves_fits(n, m, act_batch, true)) {
         const int rc = launch_q4_0_matmul_waves(tiles, nullptr, w_batch, n, k, act, act_batch, m, out, s, 1);
         if (rc != 2) return rc;
     }
