@@ -54,8 +54,9 @@ for n, k, m in [(4096, 1024, 49), (2816, 1024, 131), (4096, 4096, 260)]:   # cho
 
 # the sets of waves walk 1 to 7 tiles of k each (fewer than, as many as and more than are on their way at a time, and none behind the
 # last): the shapes of 32, 64 and 64 rows in 8 or 4, 4 and 2 sets
-@pytest.mark.parametrize("n,m", [(2816, 49), (2816, 131), (2832, 299), (5136, 388)])
-@pytest.mark.parametrize("tiles", [4, 8, 12, 16, 20, 24, 28])
+@pytest.mark.parametrize("n,m,tiles", [(n, m, t) for n, m in [(2816, 49), (2816, 131), (2832, 299), (5136, 388)] for t in (4, 8, 12, 16, 20, 24, 28)] +
+                         # ... and one or two sets of one or two waves, of 32 and 64 rows, with one to three tiles, and with more
+                         [(n, m, t) for n, m in [(2416, 616), (3072, 150), (12016, 32), (5008, 40)] for t in (1, 2, 3, 6, 7, 10)])
 def test_short_walks_of_k(rt, n, m, tiles):
     rng = np.random.default_rng(n + tiles)
     k = 128 * tiles

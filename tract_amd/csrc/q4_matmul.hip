@@ -195,8 +195,9 @@ constexpr int AROW = HK + 8;                 // halves per activation row in LDS
 // launches with so few workgroups that each compute unit would otherwise hold four waves that walk all of k alone.
 // NW: waves per set (4; 2 or 1 -- 64 or 32 rows of the weights per workgroup -- when even the smallest tile above leaves
 // compute units without a workgroup: the time of such a launch is the work of one compute unit).
-// SHORT: a set has one or two tiles, all asked for at the start (the general loop's code, and its loads past the end, cost 0.05 to 0.1 us
-// of 4 there).
+// SHORT: a set has one or two tiles, up to three where one or two sets of one or two waves walk k, all asked for at the start (the general
+// loop's code, and its loads past the end, cost 0.05 to 0.1 us of 4 there, and of those of three 0.2 to 0.4: 616 rows of 2416 x 384, with
+// conditions in one loop | the general loop | so: 6.1 | 6.3 | 5.9 us, 150 of 3072 x 768 6.2 | 6.5 | 6.2, 300 of 3008 x 384 5.5 | 5.4 | 5.2).
 template <int BM, int NI, int KS, int NW, bool SHORT = false>
 __global__ __launch_bounds__(64 * NW * KS, BM == 32 && NW * KS >= 8 && NI == 1 ? 4 : NW * KS >= 8 ? 1 : 2) void q4_0_tiled_matmul_kernel(MatMulDev p) {
     constexpr int MS = BM / 32;                  // 32-row subtiles of m
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(64 * NW * KS, BM == 32 && NW * KS >= 8 && NI == 1 ?
     // for launches in which a workgroup walks k alone, and a half tile's arithmetic is shorter than a trip to the L2.
     constexpr int PA = BM == 128 ? 1 : 2;
     // Tiles of the weights on their way from HBM, likewise: one tile's arithmetic of a small shape is about half of that trip.
-    constexpr int PW = SHORT ? 2 : BM == 128 ? 1 : (BM == 64 && NW == 4) || KS == 8 ? 2 : 3;
+    constexpr int PW = SHORT ? (KS > 2 ? 2 : 3) : BM == 128 ? 1 : (BM == 64 && NW == 4) || KS == 8 ? 2 : 3;
     constexpr int AP = BM * 8 / TS;              // 16-byte activation pieces per thread and half tile
     constexpr int RPP = TS / 8;                  // activation rows that the set's threads stage in one pass
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];   // [KS][2][BM AROW] halves; then the sums
@@ -331,12 +332,18 @@ __global__ __launch_bounds__(64 * NW * KS, BM == 32 && NW * KS >= 8 && NI == 1 ?
             if (STEADY ? !LAST || hh == 0 : 2 * t + hh + 1 < 2 * Tg) stage_a(PA == 2 ? hh ^ 1 : 0, hh ^ 1);
         }
     };
-    if constexpr (SHORT) {
+    if constexpr (SHORT && KS > 2) {   // (written as below: 0.1 us more of 4)
         if (Tg > 1) {
             tile(std::false_type{}, 0, ring[0], ring[0]);
             tile(std::true_type{}, 1, ring[1], ring[1]);
         } else {
             tile(std::true_type{}, 0, ring[0], ring[0]);
+        }
+    } else if constexpr (SHORT) {
+#pragma unroll
+        for (int u = 0; u < PW; u++) {
+            if (u + 1 < Tg) tile(std::false_type{}, u, ring[u], ring[u]);
+            else if (u + 1 == Tg) tile(std::true_type{}, u, ring[u], ring[u]);
         }
     } else if constexpr (!STEADY) {
         for (int t = 0; t < Tg; t++) {   // (PW = 1)
@@ -530,6 +537,8 @@ int launch_q4_0_matmul(const void *codes, const void *scales, int64_t w_batch, i
                 if (ks == 8) return few ? launch(q4_0_tiled_matmul_kernel<BMc, 1, 8, 1, true>) : launch(q4_0_tiled_matmul_kernel<BMc, 1, 8, 1>);
             if constexpr (NWc == 2)
                 if (ks == 4 && few) return launch(q4_0_tiled_matmul_kernel<BMc, 1, 4, 2, true>);
+            if constexpr (NWc <= 2)
+                if (ks <= 2 && k / TK <= 3 * ks) return ks == 2 ? launch(q4_0_tiled_matmul_kernel<BMc, 1, 2, NWc, true>) : launch(q4_0_tiled_matmul_kernel<BMc, 1, 1, NWc, true>);
             return ks == 4 ? launch(q4_0_tiled_matmul_kernel<BMc, 1, 4, NWc>) : ks == 2 ? launch(q4_0_tiled_matmul_kernel<BMc, 1, 2, NWc>)
                                                                                         : launch(q4_0_tiled_matmul_kernel<BMc, 1, 1, NWc>);
         };
