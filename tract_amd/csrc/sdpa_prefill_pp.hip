@@ -1128,7 +1128,7 @@ int64_t choose_splits(const PrefillPP &p, int D, int block_m, int64_t wgs1, int6
 // `whole` tiles, `per_q` workgroups each, stay whole.  A cut costs about 10 us (f32 partials written through, the arrival, the other
 // parts read back), and units that would idle leave power to the others, so that half of the time it takes off the last round is
 // gained: from 16 us on, at 1.8 us for a tile of 64 keys.  (32 heads over 8, no causal mask, 2 x 1500: 108.7 -> 101 us; behind past
-// tokens 3 x 900 after 2000 152 -> 142, 2 x 1400 after 3000 214 -> 194, 64 over 8, 1300 after 4000 261 -> 224.)  Causal prompts
+// tokens 3 x 900 after 2000 162 -> 151, 2 x 1400 after 3000 217 -> 199, 64 over 8, 1300 after 4000 266 -> 233.)  Causal prompts
 // behind little, whose longest tile takes longer than all of them spread over the units, lose what they gain: 2048 queries 63 -> 67,
 // 2 x 1500 55 -> 64 with all tiles longer than that share cut in two.
 // All but one of a tile's parts are stored (merge_parts): at most kCutPlaces of them, which a decode step's workspace of the same heads
