@@ -187,9 +187,9 @@ def test_scratch_limits_and_strided_rows(rt, dtype, Hq, n, causal):
 
 # 9 to 32 rows per kv head in 2, 3 and 4 ranges of keys, which the last workgroup to arrive merges (and 5 and more: the launch), a last
 # group of fewer rows, 64 features; an infinity of V in a range of its own stays one, calls repeated on the same counters
-@pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [(8, 32, 8, 128, 2200, 8), (8, 24, 8, 128, 2300, 5), (10, 32, 8, 128, 2600, 3), (16, 32, 8, 64, 2700, 4), (4, 10, 2, 128, 2100, 9),
-                                               (11, 32, 8, 128, 2400, 3), (5, 32, 32, 64, 1900, 11)])
-def test_ranges_merged_by_the_last_workgroup(rt, B, Hq, Hkv, D, past, n):
+@pytest.mark.parametrize("B,Hq,Hkv,D,past,n,ranges", [(8, 32, 8, 128, 2200, 8, 4), (8, 24, 8, 128, 2300, 5, 4), (10, 32, 8, 128, 2600, 3, 3), (16, 32, 8, 64, 2700, 4, 2),
+                                                      (4, 10, 2, 128, 2100, 9, 9), (11, 32, 8, 128, 2400, 3, 2), (5, 32, 32, 64, 1900, 11, 2)])
+def test_ranges_merged_by_the_last_workgroup(rt, B, Hq, Hkv, D, past, n, ranges):
     rng = np.random.default_rng(past + n)
     k, v = (rng.standard_normal((B, Hkv, past + n, D), dtype=np.float32).astype(np.float16) for _ in range(2))
     q = rng.standard_normal((B, Hq, n, D), dtype=np.float32).astype(np.float16)
@@ -198,9 +198,18 @@ def test_ranges_merged_by_the_last_workgroup(rt, B, Hq, Hkv, D, past, n):
     st.k.push(k[:, :, :past]), st.v.push(v[:, :, :past])
     kn, vn = np.ascontiguousarray(k[:, :, past:]), np.ascontiguousarray(v[:, :, past:])
     G = Hq // Hkv
+    groups = -(-G * n // 32)
+    record = 16 if -(-G * n // groups) <= 16 else 32   # rows of one
     for turn in range(3):
         st.k.truncate(past), st.v.truncate(past)
+        if turn == 1:
+            call("trocm_memset", C.c_void_p(st._ws.ptr.value + 64 * 1024), 0xA5, st._ws.nbytes - 64 * 1024, None)
         out = st.eval([q, kn, vn]).to_numpy().astype(np.float64)
+        if turn == 1:   # a record of every range has been stored, none behind the last, and the counters are zero again
+            kept, stored = st._ws.buf.to_numpy(), ranges * B * Hkv * groups * record * (D + 2) * 4
+            assert not kept[: 4 * B * Hkv * groups].any()
+            kept = kept[64 * 1024 :]
+            assert (kept[stored - 4 * D : stored] != 0xA5).any() and (kept[stored:] == 0xA5).all()
         for b in (0, B - 1):
             for h in (0, Hq - 1):
                 kh, vh = k[b, h // G].astype(np.float64), v[b, h // G].astype(np.float64)
