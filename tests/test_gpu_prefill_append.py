@@ -94,9 +94,10 @@ def test_rows_that_the_launch_does_not_take(rt, dtype, Hq, past, n):
         assert got.tobytes() == _over_one_tensor(q, k, v, True).tobytes()
 
 
-# f32 rows that would begin a fifth tile of keys in one range, or a ninth, where a workgroup's four waves take four at once: an append launch,
-# then whole tiles
-@pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [(1, 40, 8, 64, 56, 71), (1, 32, 32, 128, 100, 10), (2, 32, 8, 128, 97, 3), (1, 14, 2, 64, 65, 63), (16, 32, 32, 64, 250, 4)])
+# f32 rows that would begin a fifth tile of keys in a range, or a range more than the units take at once, where a workgroup's four waves take four
+# tiles at once: an append launch, then whole tiles
+@pytest.mark.parametrize("B,Hq,Hkv,D,past,n", [(1, 40, 8, 64, 56, 71), (1, 32, 32, 128, 100, 10), (2, 32, 8, 128, 97, 3), (1, 14, 2, 64, 65, 63), (16, 32, 32, 64, 250, 4), (3, 32, 32, 128, 244, 5), (2, 32, 32, 128, 500, 5),
+                                               (6, 32, 32, 64, 244, 5)])
 def test_rounds_of_four_tiles_stay_full(rt, B, Hq, Hkv, D, past, n):
     q, k, v = _inputs(np.float32, B, Hq, Hkv, D, past, n)
     st = _state(k, v, past, n, True)

@@ -826,17 +826,26 @@ int launch_sdpa_prefill_f32(const SdpaArgs &a, hipStream_t s) {
         // (A call with its append, us, ranges of five | of four: 2 x 32 heads over 8, 2 queries behind 618 tokens 19.7 | 15.2, 1 x 5 behind
         // 1910 21.4 | 17.0, 4 x 32 over 32, 6 behind 395 27.1 | 24.0; of four, more than a workgroup per unit, | of five: 3 x 64 over 8, 4 behind
         // 1405 24.8 | 22.8; a merge for two ranges | none: 6 x 4 over 184 tokens of 64 features 10.9 | 10.3.)
-        auto not_empty = [&](int64_t n) {
-            const int64_t longest = (cut_tiles + n - 1) / n;
-            return (cut_tiles + longest - 1) / longest;
+        auto ranges_of = [&](int64_t t) {
+            const int64_t most = n_wg < want ? (want + n_wg - 1) / n_wg : 1, fours = t < 8 ? 1 : (t + 3) / 4;
+            const int64_t n = std::min(most, n_wg * fours <= cus || (fours <= 4 && n_wg * fours <= want) ? fours : t / 4), longest = (t + n - 1) / n;
+            return (t + longest - 1) / longest;   // (none of them empty)
         };
-        const int64_t most = n_wg < want ? (want + n_wg - 1) / n_wg : 1, fours = cut_tiles < 8 ? 1 : (cut_tiles + 3) / 4;
-        ns = not_empty(std::min(most, n_wg * fours <= cus || (fours <= 4 && n_wg * fours <= want) ? fours : cut_tiles / 4));
-        // An append launch instead where the tile that is not full would be a fifth in the one range of keys, which four waves take twice, or
-        // a ninth, a thirteenth and so on where whole rows keep all units busy.  (us, append launch | in here: 32 heads over 32, 10
-        // queries behind 100 tokens 13.3 | 15.8, 64 over 8, 40 behind 70 13.9 | 16.4, 40 over 8 of 64 features, 71 behind 56 10.0 | 10.6; 16 x 32 over
-        // 32, 4 behind 250 36.8 | 40.2, behind 760 84.1 | 86.4; no tile more: 14 over 2, 20 behind 90 13.7 | 11.7.)
-        if (a.k_new && ns == 1 && (cut_tiles + 3) / 4 > (tiles + 3) / 4) return 2;
+        ns = ranges_of(cut_tiles);
+        // An append launch instead where one tile more costs more than that launch, by the rounds that four waves take a range's tiles in (us;
+        // `alone` on a compute unit or two of them sharing it, the last of five tiles in a round of its own, and `phase` where some wait for
+        // others to end).  Fitted to 40 calls of 5 queries of 16 to 192 kv heads over 8 to 24 whole tiles, each with an append launch and
+        // without: 0.6 us (64 features) and 1.6 off, and the slower side in two of the 40 (1.012, 1.046 of the faster).  Append launch | in here, us: 32
+        // heads over 32, 10 queries behind 100 tokens 13.3 | 15.8, 3 x 32 over 32, 5 behind 244 18.1 | 20.4, 2 x 32, 5 behind 500 18.9 | 20.7, 16 x 32, 4
+        // behind 760 84.1 | 86.4; kept: 3 x 32, 5 behind 756 35.3 | 28.3, 4 x 32, 5 behind 372 25.5 | 23.2, 14 over 2, 20 behind 90 13.7 | 11.7.
+        struct Rounds { float alone, shared, fifth, phase, range, append; };
+        const Rounds c = a.D == 64 ? Rounds{2.6f, 5.2f, 2.6f, 1.3f, 0.1f, 2.3f} : Rounds{5.2f, 12.8f, 8.0f, 2.5f, 0.2f, 3.1f};
+        auto expected = [&](int64_t t) {
+            const int64_t n = ranges_of(t), longest = (t + n - 1) / n, rounds = (longest + 3) / 4, wgs = n_wg * n, full = wgs / (2 * cus), rest = wgs - 2 * cus * full;
+            const float alone = c.alone * (float)rounds, shared = c.shared * (float)rounds - (longest > 4 && longest % 4 == 1 ? c.fifth : 0.0f);
+            return (float)full * shared + (rest > cus ? shared : rest > 0 ? alone : 0.0f) + c.phase * (float)(full + (rest > 0)) + c.range * (float)n;
+        };
+        if (cut_tiles > tiles && expected(cut_tiles) > expected(tiles) + c.append) return 2;
     }
     ns = ns < kMaxSplits ? ns : kMaxSplits;
     p.paired = pairs && a.causal && n_wg <= want;
